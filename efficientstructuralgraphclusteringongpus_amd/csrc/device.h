@@ -45,6 +45,10 @@ enum Counter {
   kCntRedo,     // deferred edges the union-find and border passes need: decided after all
   kCntRedoOwned,  // owned undecided entries of that second similarity round
   kCntDeferred,   // edges deferred by the core-check pruning and never needed
+  kCntFUnits1,    // units of the workgroup filter, and the next one to claim
+  kCntFUnits2,    // units of the large filter, and the next one to claim
+  kCntFQueue1,
+  kCntFQueue2,
   kCntTimer0 = 32,  // phase timers of debug builds (SGC_PHASE_TIMERS): 5 per tier
   kCntSlots = 48
 };
@@ -131,6 +135,11 @@ struct sgc_dgraph {
   // window boundary; the workgroup tier then streams exact window slices.
   uint32_t* woff = nullptr;
   uint32_t wcount = 0;
+  // Packed rows of the filter stage (filter.hip); graphs of a serving engine,
+  // and uploads without room, have none (null).  Row x is
+  // packed[gs[x], gs[x + 1]).
+  uint32_t* gs = nullptr;   // n + 1
+  uint4* packed = nullptr;  // packed_row_groups(n, m)
 };
 
 namespace sgc {
@@ -147,7 +156,7 @@ struct PassBuffers {
   uint32_t* cnt_u;   // n: undecided edges owned by each vertex (kFlagUDown entries)
   uint64_t* work_u;  // n: sum of the short-row lengths of those edges
   // m: owner b's undecided edges at [rb[b], rb[b] + cnt_u[b]) as (entry,
-  // its reverse entry, row start of a, d(a))
+  // its reverse entry, a, d(a))
   uint4* uedge;
   // ucap work units (begin, end in uedge, the owner's row begin and end):
   // small tier from the front, workgroup tier from the back
@@ -195,7 +204,11 @@ inline size_t unit_capacity(uint64_t m) { return (size_t)(m / 2) + 2; }
 // some entry has no reverse entry.  SGC_OK otherwise.
 int check_unit_overflow(const uint64_t* cnt_host, uint64_t m);
 
-// Kernel launchers (kernels.hip, similarity.hip).  All run on `s` and never
+// Uploads g; `scans`: also builds what only one-shot passes read (the packed
+// rows of the filter stage).
+int upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgraph** out);
+
+// Kernel launchers (kernels.hip, similarity.hip, filter.hip).  All run on `s` and never
 // synchronise.
 void launch_fill_src(const sgc_dgraph* g, hipStream_t s);
 // fills g->mirror (after launch_fill_src) by a search per entry; entries
@@ -215,6 +228,17 @@ uint32_t window_count(uint32_t n);
 // that is at most max(16 m, 1 GiB) bytes (four times the adjacency); else 0.
 uint64_t window_index_bytes(uint64_t n, uint64_t m);
 void launch_window_offsets(const sgc_dgraph* g, hipStream_t s);
+// Packed rows (filter.hip): groups to allocate, and the build (after the
+// reverse-entry and neighbour-degree indexes; leaves g without packed rows
+// when there is no room).  Synchronises the stream.
+uint64_t packed_row_groups(uint64_t n, uint64_t m);
+hipError_t build_packed_rows(sgc_dgraph* g, hipStream_t s);
+// Whether a pass runs the filter stage: its plan then comes from
+// launch_plan_filter, and launch_filter leaves the survivors as the exact
+// kernels' units.
+bool filter_stage(const sgc_dgraph* g, ScanParams p);
+void launch_plan_filter(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s);
+void launch_filter(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int cu_count, hipStream_t s);
 void launch_copy(const void* src, void* dst, uint64_t bytes, hipStream_t s);
 void launch_init(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s);
 // count_all: every edge is left to its owner (for exact common-neighbour

@@ -260,6 +260,10 @@ hipError_t upload_bytes(sgc_ctx* ctx, void* dst, const void* src, size_t bytes, 
 }  // namespace
 
 extern "C" int sgc_dgraph_upload(sgc_ctx* ctx, const sgc_host_graph* g, sgc_dgraph** out) {
+  return upload_graph(ctx, g, true, out);
+}
+
+int sgc::upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgraph** out) {
   clear_error();
   if (!ctx || !g || !out) return fail(SGC_EINVAL, "null argument");
   *out = nullptr;
@@ -279,6 +283,8 @@ extern "C" int sgc_dgraph_upload(sgc_ctx* ctx, const sgc_host_graph* g, sgc_dgra
     if (d->mirror) (void)hipFree(d->mirror);
     if (d->ndeg) (void)hipFree(d->ndeg);
     if (d->woff) (void)hipFree(d->woff);
+    if (d->gs) (void)hipFree(d->gs);
+    if (d->packed) (void)hipFree(d->packed);
     if (d->row_ptr) (void)hipFree(d->row_ptr);
     if (d->adj) (void)hipFree(d->adj);
     if (d->src) (void)hipFree(d->src);
@@ -328,6 +334,7 @@ extern "C" int sgc_dgraph_upload(sgc_ctx* ctx, const sgc_host_graph* g, sgc_dgra
     launch_neighbor_degrees(d, ctx->stream);
     launch_window_offsets(d, ctx->stream);
     e = hipGetLastError();
+    if (e == hipSuccess && scans) e = build_packed_rows(d, ctx->stream);
   }
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) {
@@ -345,6 +352,8 @@ extern "C" void sgc_dgraph_free(sgc_dgraph* d) {
   if (d->mirror) (void)hipFree(d->mirror);
   if (d->ndeg) (void)hipFree(d->ndeg);
   if (d->woff) (void)hipFree(d->woff);
+  if (d->gs) (void)hipFree(d->gs);
+  if (d->packed) (void)hipFree(d->packed);
   if (d->row_ptr) (void)hipFree(d->row_ptr);
   if (d->adj) (void)hipFree(d->adj);
   if (d->src) (void)hipFree(d->src);

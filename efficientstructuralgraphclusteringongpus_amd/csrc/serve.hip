@@ -739,7 +739,7 @@ extern "C" int sgc_server_add_graph(sgc_server* S, const sgc_host_graph* hg, uin
   sgc_ctx* ctx = S->ctx;
   SGC_HIP(hipSetDevice(ctx->device));
   Graph* G = new Graph();
-  int rc = sgc_dgraph_upload(ctx, hg, &G->dg);
+  int rc = upload_graph(ctx, hg, false, &G->dg);
   if (rc) {
     delete G;
     return rc;
