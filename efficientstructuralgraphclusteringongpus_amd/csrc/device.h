@@ -21,8 +21,17 @@ constexpr int kWave = 64;
 constexpr int32_t kNoLabel = 0x7FFFFFFF;
 
 
-// Counters written by the kernels (one 64-bit slot each).
+// Counters written by the kernels (64-bit words of one buffer).
+//
+// Atomics on one word are done one after the other, about 12 ns each on
+// this card, so a word that every block of a grid adds to costs 50 us per
+// 4096 blocks.  Sums are therefore kept in kStripes copies (count_add; a
+// block's copy goes by its index), read on the device by count_total /
+// count_any and summed on the host by fold_counters; counters whose atomics
+// return a value (queues, reservations) have a 128-byte line each.
+// k_finalize on 1M vertices: 101 us with single words, 9 with stripes.
 enum Counter {
+  // sums, striped
   kCntUEdges = 0,
   kCntSimilar,
   kCntCores,
@@ -31,27 +40,38 @@ enum Counter {
   kCntHubs,
   kCntOutliers,
   kCntProbes,
-  kCntUnits1,   // small-tier work units
-  kCntUnits2,   // workgroup-tier work units
-  kCntQueue1,   // next small-tier unit to claim
-  kCntQueue2,   // next workgroup-tier unit to claim
   kCntLoaded,   // short-row elements loaded by the claims (consumed or not)
   kCntClaims,   // claims taken
-  kCntDense,    // owned undecided entries listed for the one-wave-per-edge kernel
   kCntLabeled,  // entries of labelled rows (cores, borders): picks the classify pass's side
-  kCntTiny,     // tiny owners listed by the planner for the tiny-owner kernel
-  kCntOverflow, // owned undecided entries, when more than the unit array holds (asymmetric input)
   kCntMarked,   // cores marked by the core pass: none lets the later edge passes return at once
   kCntRedo,     // deferred edges the union-find and border passes need: decided after all
   kCntRedoOwned,  // owned undecided entries of that second similarity round
   kCntDeferred,   // edges deferred by the core-check pruning and never needed
-  kCntFUnits1,    // units of the workgroup filter, and the next one to claim
-  kCntFUnits2,    // units of the large filter, and the next one to claim
-  kCntFQueue1,
-  kCntFQueue2,
-  kCntTimer0 = 32,  // phase timers of debug builds (SGC_PHASE_TIMERS): 5 per tier
-  kCntSlots = 48
+  kStripeSlots = 16,
+  // single words
+  kCntOverflow = 16,  // owned undecided entries, when more than the unit array holds (asymmetric input)
+  kCntTimer0 = 32,    // phase timers of debug builds (SGC_PHASE_TIMERS): 5 per tier
+  kCntSlots = 48,     // host copies: the sums and single words above
+  kCntUnits1 = 48,    // small-tier work units
+  kCntUnits2 = 64,    // workgroup-tier work units
+  kCntQueue1 = 80,    // small-tier units claimed beyond each block's first
+  kCntQueue2 = 96,    // workgroup-tier units, likewise
+  kCntDense = 112,    // owned undecided entries listed for the one-wave-per-edge kernel
+  kCntTiny = 128,     // tiny owners listed by the planner for the tiny-owner kernel, or wave-filter owners
+  kCntFUnits1 = 144,  // units of the workgroup filter
+  kCntFUnits2 = 160,  // units of the large filter
+  kCntFQueue1 = 176,
+  kCntFQueue2 = 192,
+  kStripe0 = 208,
+  kStripes = 32,
+  kCntWords = kStripe0 + kStripes * kStripeSlots
 };
+
+// Adds the stripes of a counter buffer's host copy to its sums.
+inline void fold_counters(uint64_t* c) {
+  for (int i = 0; i < kStripes; ++i)
+    for (int q = 0; q < kStripeSlots; ++q) c[q] += c[kStripe0 + i * kStripeSlots + q];
+}
 
 // Similarity kernels selectable per context.
 enum SimImpl { kSimTiered = 0, kSimWavePerEdge = 1 };
@@ -70,7 +90,7 @@ struct sgc_ctx {
   char name[256] = {0};
   int cu_count = 0;
   sgc::DevBuf work;      // per-pass arrays
-  sgc::DevBuf counters;  // kCntSlots x uint64
+  sgc::DevBuf counters;  // kCntWords x uint64
   uint64_t* host_counters = nullptr;  // pinned mirror
   hipEvent_t ev[8] = {};
   int sim_impl = sgc::kSimTiered;
@@ -177,7 +197,7 @@ struct PassBuffers {
   void* scan_tmp = nullptr;
   size_t scan_tmp_bytes = 0;
   uint32_t ucap;
-  uint64_t* cnt;     // kCntSlots
+  uint64_t* cnt;     // kCntWords
 };
 
 struct ScanParams {
@@ -283,7 +303,7 @@ void launch_core_count(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s)
 // mu_dev (optional): read mu from device memory instead of p (captured launches)
 void launch_core_mark(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStream_t s,
                       const int32_t* mu_dev = nullptr);
-// gate >= 0: the kernel runs only when cnt[gate] is not 0
+// gate >= 0: the kernel runs only when the sum `gate` is not 0
 void launch_union(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s, int gate = -1);
 // marks the deferred edges a pruned pass needs after its union-find pass
 // (count in cnt[kCntRedo]); needs g->mirror

@@ -148,12 +148,12 @@ extern "C" int sgc_ctx_create(int device, sgc_ctx** out) {
   strncpy(ctx->name, prop.name[0] ? prop.name : prop.gcnArchName, sizeof(ctx->name) - 1);
   ctx->cu_count = prop.multiProcessorCount;
   SGC_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
-  int rc = ensure(ctx->counters, kCntSlots * sizeof(uint64_t));
+  int rc = ensure(ctx->counters, kCntWords * sizeof(uint64_t));
   if (rc) {
     delete ctx;
     return rc;
   }
-  SGC_HIP(hipHostMalloc((void**)&ctx->host_counters, kCntSlots * sizeof(uint64_t), hipHostMallocDefault));
+  SGC_HIP(hipHostMalloc((void**)&ctx->host_counters, kCntWords * sizeof(uint64_t), hipHostMallocDefault));
   for (auto& e : ctx->ev) SGC_HIP(hipEventCreate(&e));
   *out = ctx;
   return SGC_OK;
@@ -433,8 +433,9 @@ int run_pass(sgc_ctx* ctx, sgc_dgraph* g, double eps, int32_t mu, PassBuffers* p
   launch_classify(g, *pb, p, s);
   SGC_HIP(hipEventRecord(ctx->ev[6], s));
   SGC_HIP(hipGetLastError());
-  SGC_HIP(hipMemcpyAsync(ctx->host_counters, pb->cnt, kCntSlots * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+  SGC_HIP(hipMemcpyAsync(ctx->host_counters, pb->cnt, kCntWords * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
   SGC_HIP(hipStreamSynchronize(s));
+  fold_counters(ctx->host_counters);
   if (int rc = check_unit_overflow(ctx->host_counters, g->m)) return rc;
   if (st) {
     memset(st, 0, sizeof(*st));
@@ -491,8 +492,9 @@ int time_similarity(sgc_ctx* ctx, sgc_dgraph* g, double eps, PassBuffers* pb, do
   launch_similarity(g, *pb, p, ctx->cu_count, kSimTiered, nullptr, s);
   SGC_HIP(hipEventRecord(ctx->ev[2], s));
   SGC_HIP(hipGetLastError());
-  SGC_HIP(hipMemcpyAsync(ctx->host_counters, pb->cnt, kCntSlots * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+  SGC_HIP(hipMemcpyAsync(ctx->host_counters, pb->cnt, kCntWords * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
   SGC_HIP(hipStreamSynchronize(s));
+  fold_counters(ctx->host_counters);
   if (int rc = check_unit_overflow(ctx->host_counters, g->m)) return rc;
   *ms = elapsed(ctx->ev[1], ctx->ev[2]);
   return SGC_OK;

@@ -159,6 +159,46 @@ inline uint32_t grid_for(uint64_t items, uint32_t per_block) {
   return (uint32_t)g;
 }
 
+// Adds v[i] over the whole block to sum slot[i] (Counter) in the block's
+// stripe (all threads call it).
+template <int N>
+__device__ __forceinline__ void count_add(uint64_t* cnt, const int (&slot)[N], const uint64_t (&v)[N]) {
+  __shared__ unsigned long long part[N][1024 / kWave];
+  const uint32_t lane = lane_id(), w = threadIdx.x / kWave;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    unsigned long long s = v[i];
+    if (__ballot(s != 0))
+#pragma unroll
+      for (int off = kWave / 2; off > 0; off >>= 1) s += __shfl_down(s, off);
+    if (lane == 0) part[i][w] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x < N) {
+    unsigned long long t = 0;
+    for (uint32_t k = 0; k < (blockDim.x + kWave - 1) / kWave; ++k) t += part[threadIdx.x][k];
+    int at = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) at = (int)threadIdx.x == i ? slot[i] : at;
+    if (t)
+      atomicAdd((unsigned long long*)&cnt[kStripe0 + (blockIdx.x % kStripes) * kStripeSlots + (uint32_t)at], t);
+  }
+  __syncthreads();
+}
+
+// A sum's total, in every lane (whole waves call it).
+__device__ __forceinline__ uint64_t count_total(const uint64_t* cnt, int slot) {
+  uint64_t v = lane_id() < kStripes ? cnt[kStripe0 + lane_id() * kStripeSlots + slot] : 0ull;
+#pragma unroll
+  for (int off = 1; off < kStripes; off <<= 1) v += __shfl_xor(v, off);
+  return __shfl(v, 0);
+}
+
+// Whether a sum is not 0.
+__device__ __forceinline__ bool count_any(const uint64_t* cnt, int slot) {
+  return __ballot(lane_id() < kStripes && cnt[kStripe0 + lane_id() * kStripeSlots + slot] != 0) != 0;
+}
+
 // Adds v over the whole block to *dst with one atomic (all threads call it).
 __device__ __forceinline__ void block_atomic_add(unsigned long long* dst, unsigned long long v) {
   __shared__ unsigned long long part[1024 / kWave];

@@ -275,7 +275,7 @@ __global__ void __launch_bounds__(kBlock) k_plan_filter(uint32_t n, const uint32
                                                         uint32_t* __restrict__ wl_b, uint32_t* __restrict__ wl_e,
                                                         uint32_t* __restrict__ wl_k, uint64_t* __restrict__ cnt) {
   constexpr uint32_t V = 4;  // vertices per thread per block iteration
-  const uint64_t owned_all = cnt[kCntUEdges];
+  const uint64_t owned_all = count_total(cnt, kCntUEdges);
   if (owned_all > ucap) {  // asymmetric input: reported by the host, no unit is written
     if (blockIdx.x == 0 && threadIdx.x == 0) cnt[kCntOverflow] = owned_all;
     return;
@@ -587,9 +587,7 @@ __global__ void __launch_bounds__(LARGE ? 1024 : 256, 8)
     }
   }
   const uint64_t elements = tl == 0 ? (uint64_t)streamed * kGroup : 0ull;
-  block_atomic_add((unsigned long long*)&A.cnt[kCntProbes], elements);
-  block_atomic_add((unsigned long long*)&A.cnt[kCntLoaded], elements);
-  block_atomic_add((unsigned long long*)&A.cnt[kCntClaims], tl == 0 ? rounds : 0u);
+  count_add<3>(A.cnt, {kCntProbes, kCntLoaded, kCntClaims}, {elements, elements, tl == 0 ? rounds : 0u});
 }
 
 // Owners with short rows, one wave each: the row in LDS (sorted, for the
@@ -765,9 +763,7 @@ __global__ void __launch_bounds__(kBlock, 8)
     wave_lds_sync();
   }
   const uint64_t elements = tl == 0 ? (uint64_t)streamed * kGroup + probed : 0ull;
-  block_atomic_add((unsigned long long*)&A.cnt[kCntProbes], elements);
-  block_atomic_add((unsigned long long*)&A.cnt[kCntLoaded], elements);
-  block_atomic_add((unsigned long long*)&A.cnt[kCntClaims], tl == 0 ? rounds : 0u);
+  count_add<3>(A.cnt, {kCntProbes, kCntLoaded, kCntClaims}, {elements, elements, tl == 0 ? rounds : 0u});
 }
 
 // Temporary memory of build_packed_rows.

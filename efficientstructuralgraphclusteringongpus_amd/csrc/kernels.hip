@@ -182,7 +182,8 @@ __global__ void __launch_bounds__(kBlock) k_init(uint32_t n, uint32_t* __restric
     cnt_u[x] = 0;
     work_u[x] = 0;
   }
-  if (blockIdx.x == 0 && threadIdx.x < kCntSlots) cnt[threadIdx.x] = 0;
+  if (blockIdx.x == 0)
+    for (uint32_t t = threadIdx.x; t < kCntWords; t += kBlock) cnt[t] = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -284,7 +285,7 @@ __global__ void __launch_bounds__(kBlock) k_similarity_wave(const uint32_t* __re
       if (mpos < ae && adj[mpos] == (int32_t)b) flag[mpos] = f;
     }
   }
-  if (lane == 0 && probes) atomicAdd((unsigned long long*)&cnt[kCntProbes], (unsigned long long)probes);
+  count_add<1>(cnt, {kCntProbes}, {lane == 0 ? probes : 0ull});
 }
 
 // ---------------------------------------------------------------------------
@@ -326,7 +327,7 @@ __global__ void __launch_bounds__(kBlock) k_core_count(uint32_t m, const uint32_
 // similar edges, ed only discounts dissimilar ones, and every edge of a
 // still-undecided vertex is evaluated.
 // mu comes from mu_dev when given (parameters of a captured launch), else mu.
-// Also adds the entries of the core rows to cnt[kCntLabeled] when the row
+// Also adds the entries of the core rows to kCntLabeled when the row
 // offsets are given (rb null: views without them count nothing here).
 __global__ void __launch_bounds__(kBlock) k_core_mark(uint32_t n, const uint32_t* __restrict__ sd, int32_t mu,
                                                       const int32_t* __restrict__ mu_dev,
@@ -347,8 +348,7 @@ __global__ void __launch_bounds__(kBlock) k_core_mark(uint32_t n, const uint32_t
     labeled += core_mark_vertex(v, (uint32_t)x, mu, &mk);
     marked += mk;
   }
-  block_atomic_add((unsigned long long*)&cnt[kCntLabeled], labeled);
-  block_atomic_add((unsigned long long*)&cnt[kCntMarked], marked);
+  count_add<2>(cnt, {kCntLabeled, kCntMarked}, {labeled, marked});
 }
 
 // ---------------------------------------------------------------------------
@@ -356,14 +356,14 @@ __global__ void __launch_bounds__(kBlock) k_core_mark(uint32_t n, const uint32_t
 // (GPUSCAN++/GPUScan.cu:465-528, :632-652; scan_phases.h)
 // ---------------------------------------------------------------------------
 
-// gate >= 0: runs only when cnt[gate] is not 0 (the union-find pass repeated
+// gate >= 0: runs only when the sum `gate` is not 0 (the union-find pass repeated
 // after the second similarity round of a pruned pass).
 __global__ void __launch_bounds__(kBlock) k_union(uint32_t m, const uint32_t* __restrict__ src,
                                                   const int32_t* __restrict__ adj, const uint8_t* __restrict__ flag,
                                                   const uint8_t* __restrict__ core, int32_t* parent,
                                                   const uint64_t* __restrict__ cnt, int gate) {
-  if (cnt[kCntMarked] == 0) return;  // no core: no core-core edge to join
-  if (gate >= 0 && cnt[gate] == 0) return;
+  if (!count_any(cnt, kCntMarked)) return;  // no core: no core-core edge to join
+  if (gate >= 0 && !count_any(cnt, gate)) return;
   PhaseView v{};
   v.m = m, v.src = src, v.adj = adj, v.flag = flag, v.core = const_cast<uint8_t*>(core), v.parent = parent;
   const uint64_t stride = (uint64_t)gridDim.x * kBlock;
@@ -385,7 +385,7 @@ __global__ void __launch_bounds__(kBlock) k_flatten(uint32_t n, const uint8_t* _
 // 557-585 computes these on demand) and a core-non-core edge (a border
 // candidate, :692-719).  They are marked undecided again (owner side
 // kFlagUDown, the other kFlagUUp) for a second similarity round and counted
-// in cnt[kCntRedo].  A non-core-non-core edge is never needed: classify
+// in kCntRedo.  A non-core-non-core edge is never needed: classify
 // reads labels only.  Edges deferred with both endpoints in one tree cannot
 // join anything.
 __global__ void __launch_bounds__(kBlock) k_redo_mark(uint32_t m, const uint32_t* __restrict__ src,
@@ -393,7 +393,7 @@ __global__ void __launch_bounds__(kBlock) k_redo_mark(uint32_t m, const uint32_t
                                                       const uint32_t* __restrict__ mirror, uint8_t* flag,
                                                       const uint8_t* __restrict__ core, int32_t* parent,
                                                       uint64_t* __restrict__ cnt) {
-  if (cnt[kCntMarked] == 0 || cnt[kCntDeferred] == 0) return;
+  if (!count_any(cnt, kCntMarked) || !count_any(cnt, kCntDeferred)) return;
   constexpr uint32_t C = kEdgeChunks;
   const uint64_t stride = (uint64_t)gridDim.x * kBlock;
   uint32_t redo = 0;
@@ -421,7 +421,7 @@ __global__ void __launch_bounds__(kBlock) k_redo_mark(uint32_t m, const uint32_t
       ++redo;
     }
   }
-  block_atomic_add((unsigned long long*)&cnt[kCntRedo], redo);
+  count_add<1>(cnt, {kCntRedo}, {redo});
 }
 
 // ---------------------------------------------------------------------------
@@ -433,7 +433,7 @@ __global__ void __launch_bounds__(kBlock) k_border(uint32_t m, const uint32_t* _
                                                    const uint8_t* __restrict__ core, const uint32_t* __restrict__ rb,
                                                    const uint32_t* __restrict__ re, int32_t* label,
                                                    uint64_t* __restrict__ cnt) {
-  if (cnt[kCntMarked] == 0) return;  // no core: no border
+  if (!count_any(cnt, kCntMarked)) return;  // no core: no border
   PhaseView v{};
   v.m = m, v.src = src, v.adj = adj, v.flag = flag, v.core = const_cast<uint8_t*>(core), v.rb = rb, v.re = re;
   v.label = label;
@@ -444,7 +444,7 @@ __global__ void __launch_bounds__(kBlock) k_border(uint32_t m, const uint32_t* _
   for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * (kWave * kEdgeChunks);
        base < m; base += waves * kWave * kEdgeChunks)
     labeled += border_chunk(v, base);
-  block_atomic_add((unsigned long long*)&cnt[kCntLabeled], labeled);
+  count_add<1>(cnt, {kCntLabeled}, {labeled});
 }
 
 // ---------------------------------------------------------------------------
@@ -459,10 +459,10 @@ __global__ void __launch_bounds__(kBlock) k_classify(uint32_t m, uint64_t m_all,
                                                      const int32_t* __restrict__ label, int32_t* __restrict__ lo,
                                                      int32_t* __restrict__ hi, const uint64_t* __restrict__ cnt) {
   // no core means no label anywhere: lo and hi keep their initial values
-  if (cnt[kCntMarked] == 0) return;
+  if (!count_any(cnt, kCntMarked)) return;
   PhaseView v{};
   v.m = m, v.src = src, v.adj = adj, v.label = const_cast<int32_t*>(label), v.lo = lo, v.hi = hi;
-  const bool from_labeled = 3 * cnt[kCntLabeled] < m_all;
+  const bool from_labeled = 3 * count_total(cnt, kCntLabeled) < m_all;
   const uint64_t waves = (uint64_t)gridDim.x * (kBlock / kWave);
   for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * (kWave * kEdgeChunks);
        base < m; base += waves * kWave * kEdgeChunks)
@@ -482,12 +482,7 @@ __global__ void __launch_bounds__(kBlock) k_finalize(uint32_t n, int32_t mu, con
   const uint64_t stride = (uint64_t)gridDim.x * kBlock;
   for (uint64_t x = (uint64_t)blockIdx.x * kBlock + threadIdx.x; x < n; x += stride)
     finalize_vertex(v, (uint32_t)x, mu, &rc);
-  block_atomic_add((unsigned long long*)&cnt[kCntCores], rc.cores);
-  block_atomic_add((unsigned long long*)&cnt[kCntClusters], rc.clusters);
-  block_atomic_add((unsigned long long*)&cnt[kCntBorders], rc.borders);
-  block_atomic_add((unsigned long long*)&cnt[kCntHubs], rc.hubs);
-  block_atomic_add((unsigned long long*)&cnt[kCntOutliers], rc.outliers);
-  block_atomic_add((unsigned long long*)&cnt[kCntSimilar], rc.similar);
+  count_roles(cnt, rc);
 }
 
 // Plain streaming copy (16 bytes per lane per step), the reference point for

@@ -63,7 +63,8 @@ __global__ void __launch_bounds__(kBlock) k_chip_init(uint32_t a0, uint32_t a1, 
     cnt_u[x] = 0;
     work_u[x] = 0;
   }
-  if (blockIdx.x == 0 && threadIdx.x < kCntSlots) cnt[threadIdx.x] = 0;
+  if (blockIdx.x == 0)
+    for (uint32_t t = threadIdx.x; t < kCntWords; t += kBlock) cnt[t] = 0;
 }
 
 // src[k] = r0 + i for the entries [off[i], off[i+1]) of chip row i; one wave
@@ -114,7 +115,7 @@ constexpr uint64_t kRowChipBytesPerEntry = 4 + 4 + 1;
 constexpr uint64_t kMaxChipEntries = 0xFFFFFFF0ull;
 
 struct ResidentLayout {
-  size_t rb, re, sd, par, lab, lo, hi, core, cntu, work, cnt, scan, scan_bytes, bytes;
+  size_t rb, re, sd, par, lab, lo, hi, core, cntu, work, scan, scan_bytes, bytes;
 };
 
 ResidentLayout resident_layout(uint32_t n) {
@@ -123,7 +124,7 @@ ResidentLayout resident_layout(uint32_t n) {
   r.rb = L.take((size_t)n * 4), r.re = L.take((size_t)n * 4);
   r.sd = L.take((size_t)n * 4), r.par = L.take((size_t)n * 4), r.lab = L.take((size_t)n * 4);
   r.lo = L.take((size_t)n * 4), r.hi = L.take((size_t)n * 4), r.core = L.take(n);
-  r.cntu = L.take((size_t)n * 4), r.work = L.take((size_t)n * 8), r.cnt = L.take(kCntSlots * 8);
+  r.cntu = L.take((size_t)n * 4), r.work = L.take((size_t)n * 8);
   r.scan_bytes = std::max<size_t>(scan_scratch_bytes(n), 1);
   r.scan = L.take(r.scan_bytes);
   r.bytes = L.bytes;
@@ -341,7 +342,7 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
   pb.core = (uint8_t*)(base + RLay.core);
   pb.cnt_u = (uint32_t*)(base + RLay.cntu);
   pb.work_u = (uint64_t*)(base + RLay.work);
-  pb.cnt = (uint64_t*)(base + RLay.cnt);
+  pb.cnt = (uint64_t*)ctx->counters.ptr;
   // packed records of the similarity chips: first record and cursor of each
   // owner in lo's and sd's memory (free until the core phase)
   pb.rec_start = (uint32_t*)pb.lo;
@@ -372,7 +373,7 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
   SGC_HIP(hipEventCreateWithFlags(&R.back_i, hipEventDisableTiming));
   for (int i = 0; i < 2; ++i) {
     if (hipHostMalloc((void**)&R.h_flag[i], std::max<uint64_t>(J, 1)) != hipSuccess ||
-        hipHostMalloc((void**)&R.h_cnt[i], kCntSlots * 8) != hipSuccess) {
+        hipHostMalloc((void**)&R.h_cnt[i], kCntWords * 8) != hipSuccess) {
       (void)hipGetLastError();
       return fail(SGC_ENOMEM, "pinned host flag staging of %llu bytes failed", (unsigned long long)J);
     }
@@ -442,6 +443,7 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
     SGC_HIP(hipEventSynchronize(R.back[b]));
     const double tb = now_ms();
     if (c.mj) ooc_merge_rows(g, c.r0j, c.r1j, R.h_flag[b], R.flag);
+    fold_counters(R.h_cnt[b]);
     for (int q = 0; q < kCntSlots; ++q) totals[q] += R.h_cnt[b][q];
     R.ms_host += now_ms() - tb;
     ms_sim += elapsed(R.t0[b], R.t1[b]);
@@ -554,7 +556,7 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
       SGC_HIP(hipEventRecord(R.t1[b], s));
       SGC_HIP(hipGetLastError());
       // the counters before the next chip's init clears them
-      SGC_HIP(hipMemcpyAsync(R.h_cnt[b], pb.cnt, kCntSlots * 8, hipMemcpyDeviceToHost, s));
+      SGC_HIP(hipMemcpyAsync(R.h_cnt[b], pb.cnt, kCntWords * 8, hipMemcpyDeviceToHost, s));
       SGC_HIP(hipEventRecord(R.comp[b], s));
       SGC_HIP(hipStreamWaitEvent(R.d2h, R.comp[b], 0));
       if (c.mj) SGC_HIP(hipMemcpyAsync(R.h_flag[b], A.flag + jpos, c.mj, hipMemcpyDeviceToHost, R.d2h));
@@ -648,8 +650,9 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
   // classify to see: the three passes over the row chips would return at
   // once, so their uploads are skipped (every vertex ends as an outlier, or
   // as the hub that mu <= 0 makes it, in finalize)
-  SGC_HIP(hipMemcpyAsync(R.h_cnt[0], pb.cnt, kCntSlots * 8, hipMemcpyDeviceToHost, s));
+  SGC_HIP(hipMemcpyAsync(R.h_cnt[0], pb.cnt, kCntWords * 8, hipMemcpyDeviceToHost, s));
   SGC_HIP(hipStreamSynchronize(s));
+  fold_counters(R.h_cnt[0]);
   const bool any_core = R.h_cnt[0][kCntMarked] != 0;
   progress("ooc: core check over %zu row chips, %llu cores", nrow, (unsigned long long)R.h_cnt[0][kCntMarked]);
   SGC_HIP(hipEventRecord(ctx->ev[4], s));
@@ -672,7 +675,7 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
   launch_finalize(&whole, rb, p, s);
   SGC_HIP(hipEventRecord(ctx->ev[0], s));
   SGC_HIP(hipGetLastError());
-  SGC_HIP(hipMemcpyAsync(R.h_cnt[0], pb.cnt, kCntSlots * 8, hipMemcpyDeviceToHost, s));
+  SGC_HIP(hipMemcpyAsync(R.h_cnt[0], pb.cnt, kCntWords * 8, hipMemcpyDeviceToHost, s));
   if (labels) SGC_HIP(hipMemcpyAsync(labels, pb.label, (size_t)n * 4, hipMemcpyDeviceToHost, s));
   if (core_out) SGC_HIP(hipMemcpyAsync(core_out, pb.core, n, hipMemcpyDeviceToHost, s));
   SGC_HIP(hipStreamSynchronize(s));
@@ -686,6 +689,7 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
   const double ms_phases = now_ms() - t_phase;
   if (sim_out && g->m) memcpy(sim_out, R.flag, g->m);
 
+  fold_counters(R.h_cnt[0]);
   const uint64_t* c = R.h_cnt[0];
   if (st) {
     memset(st, 0, sizeof(*st));

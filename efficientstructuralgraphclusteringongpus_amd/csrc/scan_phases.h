@@ -195,6 +195,11 @@ struct RoleCounts {
   uint64_t similar = 0;
 };
 
+__device__ __forceinline__ void count_roles(uint64_t* cnt, const RoleCounts& rc) {
+  count_add<6>(cnt, {kCntCores, kCntClusters, kCntBorders, kCntHubs, kCntOutliers, kCntSimilar},
+               {rc.cores, rc.clusters, rc.borders, rc.hubs, rc.outliers, rc.similar});
+}
+
 __device__ __forceinline__ int32_t finalize_vertex(const PhaseView& v, uint32_t x, int32_t mu, RoleCounts* rc) {
   rc->similar += v.sd[x];
   int32_t l = v.label[x];

@@ -110,7 +110,8 @@ __global__ void __launch_bounds__(kBlock) k_query_init(uint32_t n, uint32_t* __r
     lo[x] = kNoLabel;
     hi[x] = -1;
   }
-  if (blockIdx.x == 0 && threadIdx.x < kCntSlots) cnt[threadIdx.x] = 0;
+  if (blockIdx.x == 0)
+    for (uint32_t t = threadIdx.x; t < kCntWords; t += kBlock) cnt[t] = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -190,7 +191,8 @@ __global__ void __launch_bounds__(kBlock) k_batch_init(const BatchTable* __restr
       Q.lo[x] = kNoLabel;
       Q.hi[x] = -1;
     }
-    if (T0 == 0 && threadIdx.x < kCntSlots) Q.cnt[threadIdx.x] = 0;
+    if (T0 == 0)
+      for (uint32_t w = threadIdx.x; w < kCntWords; w += kBlock) Q.cnt[w] = 0;
   }
 }
 
@@ -207,14 +209,13 @@ __global__ void __launch_bounds__(kBlock) k_batch_core_mark(const BatchTable* __
     const uint64_t x = T0 + threadIdx.x;
     uint32_t marked = 0, labeled = 0;
     if (x < Q.n) labeled = core_mark_vertex(v, (uint32_t)x, Q.mu, &marked);
-    block_atomic_add((unsigned long long*)&Q.cnt[kCntLabeled], labeled);
-    block_atomic_add((unsigned long long*)&Q.cnt[kCntMarked], marked);
+    count_add<2>(Q.cnt, {kCntLabeled, kCntMarked}, {labeled, marked});
   }
 }
 
 __global__ void __launch_bounds__(kBlock) k_batch_union(const BatchTable* __restrict__ bt) {
   SGC_BATCH_TILES(bt, e_tiles, true, kEdgeTile) {
-    if (Q.cnt[kCntMarked] == 0) continue;  // no core: no core-core edge to join
+    if (!count_any(Q.cnt, kCntMarked)) continue;  // no core: no core-core edge to join
     union_entries(item_view(Q), T0 + threadIdx.x, kBlock);
   }
 }
@@ -228,16 +229,16 @@ __global__ void __launch_bounds__(kBlock) k_batch_flatten(const BatchTable* __re
 
 __global__ void __launch_bounds__(kBlock) k_batch_border(const BatchTable* __restrict__ bt) {
   SGC_BATCH_TILES(bt, e_tiles, true, kEdgeTile) {
-    if (Q.cnt[kCntMarked] == 0) continue;  // no core: no border
+    if (!count_any(Q.cnt, kCntMarked)) continue;  // no core: no border
     const uint32_t labeled = border_chunk(item_view(Q), T0 + (threadIdx.x / kWave) * (kWave * kEdgeChunks));
-    block_atomic_add((unsigned long long*)&Q.cnt[kCntLabeled], labeled);
+    count_add<1>(Q.cnt, {kCntLabeled}, {labeled});
   }
 }
 
 __global__ void __launch_bounds__(kBlock) k_batch_classify(const BatchTable* __restrict__ bt) {
   SGC_BATCH_TILES(bt, e_tiles, true, kEdgeTile) {
-    if (Q.cnt[kCntMarked] == 0) continue;  // no label anywhere
-    classify_chunk(item_view(Q), T0 + (threadIdx.x / kWave) * (kWave * kEdgeChunks), 3 * Q.cnt[kCntLabeled] < Q.m);
+    if (!count_any(Q.cnt, kCntMarked)) continue;  // no label anywhere
+    classify_chunk(item_view(Q), T0 + (threadIdx.x / kWave) * (kWave * kEdgeChunks), 3 * count_total(Q.cnt, kCntLabeled) < Q.m);
   }
 }
 
@@ -248,19 +249,21 @@ __global__ void __launch_bounds__(kBlock) k_batch_finalize(const BatchTable* __r
     const uint64_t x = T0 + threadIdx.x;
     RoleCounts rc;
     if (x < Q.n) Q.out_labels[x] = finalize_vertex(v, (uint32_t)x, Q.mu, &rc);
-    block_atomic_add((unsigned long long*)&Q.cnt[kCntCores], rc.cores);
-    block_atomic_add((unsigned long long*)&Q.cnt[kCntClusters], rc.clusters);
-    block_atomic_add((unsigned long long*)&Q.cnt[kCntBorders], rc.borders);
-    block_atomic_add((unsigned long long*)&Q.cnt[kCntHubs], rc.hubs);
-    block_atomic_add((unsigned long long*)&Q.cnt[kCntOutliers], rc.outliers);
-    block_atomic_add((unsigned long long*)&Q.cnt[kCntSimilar], rc.similar);
+    count_roles(Q.cnt, rc);
   }
 }
 
-// Each query's counters to its slot's page-locked copy (block q: query q).
+// Each query's counters, stripes folded, to its slot's page-locked copy
+// (block q: query q).
 __global__ void __launch_bounds__(kBlock) k_batch_publish(const BatchTable* __restrict__ bt) {
   for (uint32_t q = blockIdx.x; q < bt->count; q += gridDim.x)
-    if (threadIdx.x < kCntSlots) bt->items[q].out_cnt[threadIdx.x] = bt->items[q].cnt[threadIdx.x];
+    if (threadIdx.x < kCntSlots) {
+      const uint64_t* const c = bt->items[q].cnt;
+      uint64_t v = c[threadIdx.x];
+      if (threadIdx.x < kStripeSlots)
+        for (uint32_t i = 0; i < kStripes; ++i) v += c[kStripe0 + i * kStripeSlots + threadIdx.x];
+      bt->items[q].out_cnt[threadIdx.x] = v;
+    }
 }
 
 #undef SGC_BATCH_TILES
@@ -297,6 +300,7 @@ struct Graph {
   sgc_dgraph* dg = nullptr;
   uint32_t* cn = nullptr;
   void* slot_mem = nullptr;
+  uint64_t* cnt_mem = nullptr;  // kCntWords per slot
   size_t bytes = 0;
   std::vector<Slot> slots;
   double precompute_ms = 0;
@@ -379,6 +383,7 @@ void free_graph(Graph* G) {
     if (s.done) (void)hipEventDestroy(s.done);
   }
   if (G->slot_mem) (void)hipFree(G->slot_mem);
+  if (G->cnt_mem) (void)hipFree(G->cnt_mem);
   if (G->cn) (void)hipFree(G->cn);
   if (G->dg) sgc_dgraph_free(G->dg);
   delete G;
@@ -402,7 +407,7 @@ void enqueue_query(const Graph* G, const Slot& sl, const ScanParams* p, hipStrea
   launch_classify_edges(g, sl.pb, st);
   launch_finalize(g, sl.pb, pv, st, mu_dev);
   (void)hipMemcpyAsync(sl.h_labels, sl.pb.label, (size_t)g->n * 4, hipMemcpyDeviceToHost, st);
-  (void)hipMemcpyAsync(sl.h_cnt, sl.pb.cnt, kCntSlots * 8, hipMemcpyDeviceToHost, st);
+  (void)hipMemcpyAsync(sl.h_cnt, sl.pb.cnt, kCntWords * 8, hipMemcpyDeviceToHost, st);
 }
 
 // Captures the slot's query work into an executable graph.  Capture runs at
@@ -612,6 +617,7 @@ int dispatch(sgc_server* S) {
 // Retires finished slots; with wait, blocks for the oldest in-flight query
 // first.  Returns the number retired.
 Result slot_result(const Graph* G, const Slot& s, double ms_device) {
+  if (!s.batched) fold_counters(s.h_cnt);  // a batch's counters are folded on the device
   Result r;
   r.labels.assign(s.h_labels, s.h_labels + G->dg->n);
   memset(&r.st, 0, sizeof(r.st));
@@ -746,7 +752,8 @@ extern "C" int sgc_server_add_graph(sgc_server* S, const sgc_host_graph* hg, uin
   }
   const uint32_t n = G->dg->n, m = G->dg->m;
   if (hipMalloc(&G->cn, std::max<size_t>(m, 1) * 4) != hipSuccess ||
-      hipMalloc(&G->slot_mem, S->slots_per_graph * slot_bytes(n, m)) != hipSuccess) {
+      hipMalloc(&G->slot_mem, S->slots_per_graph * slot_bytes(n, m)) != hipSuccess ||
+      hipMalloc(&G->cnt_mem, S->slots_per_graph * kCntWords * 8) != hipSuccess) {
     (void)hipGetLastError();
     free_graph(G);
     return fail(SGC_ENOMEM, "device allocation for graph of %u vertices failed", n);
@@ -771,7 +778,7 @@ extern "C" int sgc_server_add_graph(sgc_server* S, const sgc_host_graph* hg, uin
       free_graph(G);
       return fail(SGC_EDEVICE, "common-neighbour pass failed: %s", hipGetErrorString(e));
     }
-    uint64_t c[kCntSlots];
+    uint64_t c[kCntWords];
     if (hipMemcpy(c, pb.cnt, sizeof(c), hipMemcpyDeviceToHost) != hipSuccess) {
       (void)hipGetLastError();
       free_graph(G);
@@ -803,13 +810,13 @@ extern "C" int sgc_server_add_graph(sgc_server* S, const sgc_host_graph* hg, uin
     p += align256((size_t)n * 4 + 4);
     sl.pb.core = (uint8_t*)p;
     p += align256((size_t)n + 1);
-    sl.pb.cnt = (uint64_t*)p;
+    sl.pb.cnt = G->cnt_mem + (size_t)i * kCntWords;
     p += align256(kCntSlots * 8);
     sl.d_params = (QueryParams*)p;
     sl.stream = S->next_stream;
     S->next_stream = (S->next_stream + 1) % kStreams;
     if (hipHostMalloc((void**)&sl.h_labels, std::max<size_t>(n, 1) * 4) != hipSuccess ||
-        hipHostMalloc((void**)&sl.h_cnt, kCntSlots * 8) != hipSuccess ||
+        hipHostMalloc((void**)&sl.h_cnt, kCntWords * 8) != hipSuccess ||
         hipHostMalloc((void**)&sl.h_params, sizeof(QueryParams)) != hipSuccess ||
         hipEventCreate(&sl.start) != hipSuccess || hipEventCreate(&sl.done) != hipSuccess) {
       (void)hipGetLastError();

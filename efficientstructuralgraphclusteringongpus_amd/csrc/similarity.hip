@@ -84,7 +84,7 @@ __device__ __forceinline__ uint32_t log2_pow2(uint32_t t) { return 31 - __clz(t)
 // entries are added to its vertex's counts.  redo (the second round of a
 // pruned pass): the degree-only test is not rerun; the entries the round
 // marked kFlagUDown are planned as owned, their count goes to
-// cnt[kCntRedoOwned], and the kernel returns at once when cnt[kCntRedo] is 0.
+// kCntRedoOwned, and the kernel returns at once when kCntRedo is 0.
 // Where k_prep puts each owner's edge records:
 //   kRecRow     at the owner's own row range, uedge[rb[b] + slot];
 //   kRecCount   nowhere: flags and per-owner counts only (first of two passes);
@@ -112,8 +112,8 @@ __global__ void __launch_bounds__(kBlock) k_prep(uint32_t m, const uint32_t* __r
                                                  uint32_t w = 0) {
   constexpr bool redo = REDO;
   constexpr bool from_flags = REDO || REC == kRecCompact;  // owned entries from the flags already written
-  if (redo && cnt[kCntRedo] == 0) return;
-  if (REC == kRecCompact && r0 >= cnt[kCntUEdges]) return;  // a round past the chip's records
+  if (redo && !count_any(cnt, kCntRedo)) return;
+  if (REC == kRecCompact && r0 >= count_total(cnt, kCntUEdges)) return;  // a round past the chip's records
   constexpr uint32_t C = kEdgeChunks;
   const uint32_t lane = lane_id();
   const uint64_t waves = (uint64_t)gridDim.x * (kBlock / kWave);
@@ -228,7 +228,7 @@ __global__ void __launch_bounds__(kBlock) k_prep(uint32_t m, const uint32_t* __r
     }
   }
   if (REC != kRecCompact)
-    block_atomic_add((unsigned long long*)&cnt[redo ? kCntRedoOwned : kCntUEdges], owned_total);
+    count_add<1>(cnt, {redo ? kCntRedoOwned : kCntUEdges}, {owned_total});
 }
 
 // ---------------------------------------------------------------------------
@@ -254,8 +254,8 @@ __device__ __forceinline__ uint32_t edges_per_unit(uint32_t cnt, uint64_t work, 
 // vstate (pruned passes, first round): every vertex's state from its
 // degree-decided counts: core once ny >= mu, not core once d - nn < mu
 // (GPUSCAN++/GPUScan.cu:140-169).  redo: the second round of a pruned pass
-// (owned entries counted in cnt[kCntRedoOwned]; nothing to do when
-// cnt[kCntRedo] is 0).
+// (owned entries counted in kCntRedoOwned; nothing to do when kCntRedo is
+// 0).
 __global__ void __launch_bounds__(kBlock) k_plan(uint32_t x0, uint32_t x1, const uint32_t* __restrict__ rb,
                                                  const uint32_t* __restrict__ re, SimTuning tune,
                                                  const uint32_t* __restrict__ cnt_u,
@@ -267,14 +267,14 @@ __global__ void __launch_bounds__(kBlock) k_plan(uint32_t x0, uint32_t x1, const
                                                  const uint32_t* __restrict__ rec_start = nullptr, uint32_t r0 = 0,
                                                  uint32_t w = 0) {
   constexpr uint32_t V = 4;  // vertices per thread per block iteration
-  if (redo && cnt[kCntRedo] == 0) return;
+  if (redo && !count_any(cnt, kCntRedo)) return;
   // Every unit holds at least one owned entry, so ucap units always suffice
   // when each undecided edge is owned once.  An input without a reverse
   // entry for every entry can own more: then no unit is written (the
   // regions from both ends would meet), and the host reports the count.
   // A round of packed records (rec_start) plans the owners whose records
   // start in [r0, r0 + w), which hold fewer than ucap records.
-  const uint64_t owned_all = cnt[redo ? kCntRedoOwned : kCntUEdges];
+  const uint64_t owned_all = count_total(cnt, redo ? kCntRedoOwned : kCntUEdges);
   if (rec_start && r0 >= owned_all) return;
   if (!rec_start && owned_all > ucap) {
     if (blockIdx.x == 0 && threadIdx.x == 0) cnt[kCntOverflow] = owned_all;
@@ -791,22 +791,21 @@ __global__ void __launch_bounds__(T::kThreads, T::kMinWaves)
   do {              \
   } while (0)
 #endif
-  // Units come from a shared queue (their work varies widely).  Thread 0
-  // takes the next unit while the current one runs and puts its descriptor
-  // into s_next once its own streaming is done, so neither round trip sits
-  // at the top of a unit.
-  uint32_t nxt = 0;
+  // A block's first unit is its own; the others come from a shared queue
+  // (their work varies widely).  Thread 0 takes the next unit while the
+  // current one runs and puts its descriptor into s_next once its own
+  // streaming is done, so neither round trip sits at the top of a unit.
+  uint32_t nxt = blockIdx.x;
   auto fetch_next = [&]() {
     if (nxt < nunits) s_next = units[T::kBitmap ? ucap - 1 - nxt : nxt];
   };
-  if (threadIdx.x == 0) {
-    nxt = (uint32_t)atomicAdd((unsigned long long*)&cnt[queue_slot], 1ull);
-    fetch_next();
-  }
+  if (threadIdx.x == 0) fetch_next();
   for (;;) {
     if (threadIdx.x == 0) {
       s_unit = nxt;
-      if (nxt < nunits) nxt = (uint32_t)atomicAdd((unsigned long long*)&cnt[queue_slot], 1ull);
+      if (nxt < nunits)
+        nxt = nunits > gridDim.x ? gridDim.x + (uint32_t)atomicAdd((unsigned long long*)&cnt[queue_slot], 1ull)
+                                 : kNone;
     }
     __syncthreads();
     const uint32_t u = s_unit;
@@ -1186,12 +1185,8 @@ __global__ void __launch_bounds__(T::kThreads, T::kMinWaves)
       atomicAdd((unsigned long long*)&cnt[kCntTimer0 + (T::kBitmap ? 0 : 5) + i], (unsigned long long)tm[i]);
 #endif
 #undef SGC_TICK
-  if (threadIdx.x == 0 && deferred) atomicAdd((unsigned long long*)&cnt[kCntDeferred], (unsigned long long)deferred);
-  if (lane == 0 && claims) {
-    atomicAdd((unsigned long long*)&cnt[kCntProbes], (unsigned long long)streamed);
-    atomicAdd((unsigned long long*)&cnt[kCntLoaded], (unsigned long long)loaded);
-    atomicAdd((unsigned long long*)&cnt[kCntClaims], (unsigned long long)claims);
-  }
+  if (lane != 0) streamed = loaded = claims = 0;  // counted by every lane alike
+  count_add<4>(cnt, {kCntDeferred, kCntProbes, kCntLoaded, kCntClaims}, {deferred, streamed, loaded, claims});
 }
 
 // Window-offset index: woff[x * (W + 1) + w] = first position of row x whose
@@ -1416,9 +1411,8 @@ __global__ void __launch_bounds__(kBlock) k_redo_init(uint32_t n, uint32_t* __re
     cnt[kCntUnits1] = cnt[kCntUnits2] = 0;
     cnt[kCntQueue1] = cnt[kCntQueue2] = 0;
     cnt[kCntTiny] = 0;
-    cnt[kCntRedoOwned] = 0;
   }
-  if (cnt[kCntRedo] == 0) return;
+  if (!count_any(cnt, kCntRedo)) return;
   const uint64_t stride = (uint64_t)gridDim.x * kBlock;
   for (uint64_t x = (uint64_t)blockIdx.x * kBlock + threadIdx.x; x < n; x += stride) {
     cnt_u[x] = 0;
