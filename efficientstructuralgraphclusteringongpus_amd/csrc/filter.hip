@@ -43,7 +43,6 @@ constexpr uint32_t kNone = 0xFFFFFFFFu;
 constexpr uint32_t kGroup = 7;            // elements per group
 constexpr uint32_t kClasses = 16;
 constexpr uint32_t kWideRow = 512;        // rows of at least this many entries are ordered by class
-constexpr uint32_t kPadWord = 0xFFFFFFFFu;  // two padding elements
 constexpr uint32_t kWindowWords16 = 2048;   // 2^16 bits
 constexpr uint32_t kDegBuckets = 512;       // degree buckets: 16 per power of two
 
@@ -365,10 +364,12 @@ constexpr uint32_t kTeamLoads = 4;  // groups per lane and round
 // windows.
 enum FilterKind { kFilterWave, kFilterFold, kFilterWindows };
 
-// Misses of one group against a filter whose set bits are the absent
-// elements.
+// The absence bits of one group's seven elements in the top bits of a word,
+// against a filter whose set bits are the absent elements.  An element costs
+// four VALU instructions and one LDS read: address shift and mask, the word
+// shifted by the element, and its low bit funnelled into the result.
 template <int KIND>
-__device__ __forceinline__ uint32_t group_misses(const uint4 v, const uint32_t* filt) {
+__device__ __forceinline__ uint32_t group_absent(const uint4 v, const uint32_t* filt) {
   constexpr uint32_t mask = KIND == kFilterWave ? 0x3FCu : 0x1FFCu;
   const uint32_t base = KIND == kFilterWindows ? (v.x & 0x1Eu) << 12 : 0u;  // window (header >> 1) x 8 KB
   const char* const f = reinterpret_cast<const char*>(filt);
@@ -379,13 +380,13 @@ __device__ __forceinline__ uint32_t group_misses(const uint4 v, const uint32_t* 
     if (q) lo[q] = *reinterpret_cast<const uint32_t*>(f + (((w[q] >> 3) & mask) | base));
     hi[q] = *reinterpret_cast<const uint32_t*>(f + (((w[q] >> 19) & mask) | base));
   }
-  uint32_t miss = 0;
+  uint32_t bits = 0;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    if (q) miss += __builtin_amdgcn_ubfe(lo[q], w[q], 1);
-    miss += __builtin_amdgcn_ubfe(hi[q], w[q] >> 16, 1);
+    if (q) bits = __builtin_amdgcn_alignbit(lo[q] >> (w[q] & 31), bits, 1);
+    bits = __builtin_amdgcn_alignbit(hi[q] >> ((w[q] >> 16) & 31), bits, 1);
   }
-  return miss;
+  return bits;
 }
 
 // Loads of a round: as many as reach `need` misses if an eighth of the
@@ -395,24 +396,25 @@ __device__ __forceinline__ uint32_t round_loads(uint32_t need) {
   return nl < kTeamLoads ? nl : kTeamLoads;
 }
 
-// One round of a team at groups [g, ge) with `need` misses to go: returns
-// the misses found in the next round_loads() x 16 groups.
+// One round of a team at group g: the misses found in the next `take`
+// groups.  Lanes past them load the last one again (every address is valid,
+// also a resting team's) and are left out of the count.
 template <int KIND>
-__device__ __forceinline__ uint32_t filter_round(bool act, uint32_t nl, uint32_t g, uint32_t ge,
-                                                 const uint4* __restrict__ packed, const uint32_t* filt) {
-  const uint32_t tl = lane_id() & (kTeam - 1);
+__device__ __forceinline__ uint32_t filter_round(uint32_t g, uint32_t take, const uint4* __restrict__ packed,
+                                                 const uint32_t* filt) {
+  const uint32_t tl = lane_id() & (kTeam - 1), last = take ? take - 1 : 0u;
   uint4 v[kTeamLoads];
 #pragma unroll
   for (uint32_t j = 0; j < kTeamLoads; ++j) {
-    v[j] = make_uint4(0xFFFF0000u, kPadWord, kPadWord, kPadWord);
-    const uint32_t i = j * kTeam + tl;
-    if (act && j < nl && i < ge - g) v[j] = packed[g + i];
+    if (j && !__ballot(j * kTeam < take)) break;
+    v[j] = packed[g + min(j * kTeam + tl, last)];
   }
   uint32_t miss = 0;
 #pragma unroll
   for (uint32_t j = 0; j < kTeamLoads; ++j) {
-    if (j && !__ballot(act && j < nl)) break;
-    miss += group_misses<KIND>(v[j], filt);
+    if (j && !__ballot(j * kTeam < take)) break;
+    const uint32_t bits = group_absent<KIND>(v[j], filt);
+    miss += (uint32_t)__popc(j * kTeam + tl < take ? bits : 0u);
   }
   return team_sum(miss);
 }
@@ -462,8 +464,10 @@ __global__ void __launch_bounds__(LARGE ? 1024 : 256, 8)
   constexpr uint32_t MAXE = LARGE ? kLargeEdges : kSmallEdges;
   constexpr uint32_t WORDS = LARGE ? 9 * kWindowWords16 : kWindowWords16;
   __shared__ __align__(16) uint32_t filt[WORDS];
-  __shared__ uint2 e_q[MAXE];  // (first group, groups << 16 | misses needed)
-  __shared__ uint32_t s_surv[MAXE / 32], s_part[T / kWave];
+  // the edges to stream, longest first: (first group, groups << 16 | misses
+  // needed)
+  __shared__ uint2 e_q[MAXE];
+  __shared__ uint32_t s_surv[MAXE / 32], s_part[T / kWave], s_hist[32];
   __shared__ uint32_t s_unit, s_cursor;
   const uint32_t lane = lane_id(), tl = lane & (kTeam - 1), tid = threadIdx.x;
   const uint64_t nunits = A.cnt[LARGE ? kCntFUnits2 : kCntFUnits1];
@@ -491,6 +495,7 @@ __global__ void __launch_bounds__(LARGE ? 1024 : 256, 8)
     for (uint32_t t = tid; t < WORDS / 4; t += T)
       f4[t] = make_uint4(~0u, ~0u, ~0u, t % (kWindowWords16 / 4) == kWindowWords16 / 4 - 1 ? 0x7FFFFFFFu : ~0u);
     if (tid < MAXE / 32) s_surv[tid] = 0;
+    if (tid < 32) s_hist[tid] = 0;
     uint32_t g0 = 0, g1 = 0;
     if (mine) {
       g0 = A.gs[ed.z];
@@ -510,44 +515,54 @@ __global__ void __launch_bounds__(LARGE ? 1024 : 256, 8)
         atomicAnd(&filt[h >> 5], ~(1u << (h & 31)));
       }
     }
+    // Edges in order of the misses they need (two buckets per power of two),
+    // most first: the teams of a wave then take edges of about the same
+    // length, end their rounds and fetch their next edges together, and the
+    // longest edges do not start last.
+    bool keep = false;  // survives
+    uint32_t need0 = 0, rank = 0, slot = 0;
     if (mine) {
       uint32_t cstar;
-      bool survive;
-      const uint32_t need = misses_needed(A.eps, ed.w, l, &cstar, &survive);
-      e_q[tid] = make_uint2(g0, need ? ((g1 - g0) << 16) | need : 0u);
-      if (!need && survive) atomicOr(&s_surv[tid >> 5], 1u << (tid & 31));
+      need0 = misses_needed(A.eps, ed.w, l, &cstar, &keep);
     }
+    const uint32_t lg = need0 ? 31 - __clz(need0) : 0u;  // need0 < 2^16
+    const uint32_t bucket = 31 - (lg ? lg * 2 + ((need0 >> (lg - 1)) & 1) : 0u);
+    if (need0) {
+      keep = false;
+      rank = atomicAdd(&s_hist[bucket], 1u);
+    }
+    __syncthreads();
+    const uint32_t incl = wave_incl_scan(lane < 32 ? s_hist[lane] : 0u);
+    const uint32_t todo = __builtin_amdgcn_readlane(incl, 31);
+    slot = (uint32_t)__shfl((int)incl, (int)bucket) - s_hist[bucket] + rank;
+    if (need0) e_q[slot] = make_uint2(g0, ((g1 - g0) << 16) | need0);
     __syncthreads();
     // ---- stream
     bool act = false, out = false;  // this team has an edge; the cursor is at its end
-    uint32_t e = 0, g = 0, ge = 0, need = 0;
+    uint32_t e = 0, g = bg0, ge = 0, need = 0;
     for (;;) {
       if (!act && !out) {
         uint32_t t = 0;
         if (tl == 0) t = atomicAdd(&s_cursor, 1u);
         t = (uint32_t)__shfl((int)t, (int)(lane & ~(kTeam - 1)));
-        if (t < ne) {
+        if (t < todo) {
           const uint2 q = e_q[t];
           e = t;
           g = q.x;
           ge = q.x + (q.y >> 16);
           need = q.y & 0xFFFFu;
-          act = need != 0;
+          act = true;
         } else {
           out = true;
         }
       }
-      if (!__ballot(act)) {
-        if (!__ballot(!out)) break;
-        continue;
-      }
-      const uint32_t nl = round_loads(need);
-      const uint32_t miss = filter_round<LARGE ? kFilterWindows : kFilterFold>(act, nl, g, ge, A.packed, filt);
+      if (!__ballot(act)) break;
+      const uint32_t take = act ? min(round_loads(need) * kTeam, ge - g) : 0u;
+      const uint32_t miss = filter_round<LARGE ? kFilterWindows : kFilterFold>(g, take, A.packed, filt);
       if (act) {
-        const uint32_t took = min(nl * kTeam, ge - g);
-        streamed += took;
+        streamed += take;
         ++rounds;
-        g += took;
+        g += take;
         if (miss >= need) {
           act = false;
         } else {
@@ -561,7 +576,7 @@ __global__ void __launch_bounds__(LARGE ? 1024 : 256, 8)
     }
     __syncthreads();
     // ---- results, and the survivors' records to the front of the range
-    const bool keep = mine && ((s_surv[tid >> 5] >> (tid & 31)) & 1u);
+    if (need0) keep = (s_surv[slot >> 5] >> (slot & 31)) & 1u;
     if (mine && !keep) {
       if (ed.x < A.m) A.flag[ed.x] = kFlagN;
       if (ed.y < A.m) A.flag[ed.y] = kFlagN;
@@ -665,13 +680,12 @@ __global__ void __launch_bounds__(kBlock, 8)
           if (next >= ne) break;
           continue;
         }
-        const uint32_t nl = round_loads(need);
-        const uint32_t miss = filter_round<kFilterWave>(act, nl, g, ge, A.packed, filt);
+        const uint32_t take = act ? min(round_loads(need) * kTeam, ge - g) : 0u;
+        const uint32_t miss = filter_round<kFilterWave>(g, take, A.packed, filt);
         if (act) {
-          const uint32_t took = min(nl * kTeam, ge - g);
-          streamed += took;
+          streamed += take;
           ++rounds;
-          g += took;
+          g += take;
           if (miss >= need) {
             act = false;
           } else {
