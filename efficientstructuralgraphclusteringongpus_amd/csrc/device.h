@@ -59,10 +59,12 @@ enum Counter {
   kCntDense = 112,    // owned undecided entries listed for the one-wave-per-edge kernel
   kCntTiny = 128,     // tiny owners listed by the planner for the tiny-owner kernel, or wave-filter owners
   kCntFUnits1 = 144,  // units of the workgroup filter
-  kCntFUnits2 = 160,  // units of the large filter
+  kCntFUnits2 = 160,  // units of the large owners
   kCntFQueue1 = 176,
   kCntFQueue2 = 192,
-  kStripe0 = 208,
+  kCntHUnits = 208,   // units of the hash filter
+  kCntHQueue = 224,
+  kStripe0 = 240,
   kStripes = 32,
   kCntWords = kStripe0 + kStripes * kStripeSlots
 };
@@ -155,11 +157,10 @@ struct sgc_dgraph {
   // window boundary; the workgroup tier then streams exact window slices.
   uint32_t* woff = nullptr;
   uint32_t wcount = 0;
-  // Packed rows of the filter stage (filter.hip); graphs of a serving engine,
-  // and uploads without room, have none (null).  Row x is
-  // packed[gs[x], gs[x + 1]).
-  uint32_t* gs = nullptr;   // n + 1
-  uint4* packed = nullptr;  // packed_row_groups(n, m)
+  // Compact copies of the rows for the filter stages (filter.hip: bitmaps
+  // and hash groups, 9 bytes per entry); graphs of a serving engine, and
+  // uploads without room, have none (null).
+  char* packed = nullptr;
 };
 
 namespace sgc {
@@ -176,7 +177,7 @@ struct PassBuffers {
   uint32_t* cnt_u;   // n: undecided edges owned by each vertex (kFlagUDown entries)
   uint64_t* work_u;  // n: sum of the short-row lengths of those edges
   // m: owner b's undecided edges at [rb[b], rb[b] + cnt_u[b]) as (entry,
-  // its reverse entry, a, d(a))
+  // its reverse entry, row start of a, d(a))
   uint4* uedge;
   // ucap work units (begin, end in uedge, the owner's row begin and end):
   // small tier from the front, workgroup tier from the back
@@ -248,10 +249,9 @@ uint32_t window_count(uint32_t n);
 // that is at most max(16 m, 1 GiB) bytes (four times the adjacency); else 0.
 uint64_t window_index_bytes(uint64_t n, uint64_t m);
 void launch_window_offsets(const sgc_dgraph* g, hipStream_t s);
-// Packed rows (filter.hip): groups to allocate, and the build (after the
-// reverse-entry and neighbour-degree indexes; leaves g without packed rows
-// when there is no room).  Synchronises the stream.
-uint64_t packed_row_groups(uint64_t n, uint64_t m);
+// Compact row copies (filter.hip), after the reverse-entry and
+// neighbour-degree indexes; leaves g without them when there is no room.
+// Synchronises the stream.
 hipError_t build_packed_rows(sgc_dgraph* g, hipStream_t s);
 // Whether a pass runs the filter stage: its plan then comes from
 // launch_plan_filter, and launch_filter leaves the survivors as the exact

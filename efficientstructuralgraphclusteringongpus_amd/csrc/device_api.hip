@@ -283,7 +283,6 @@ int sgc::upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgr
     if (d->mirror) (void)hipFree(d->mirror);
     if (d->ndeg) (void)hipFree(d->ndeg);
     if (d->woff) (void)hipFree(d->woff);
-    if (d->gs) (void)hipFree(d->gs);
     if (d->packed) (void)hipFree(d->packed);
     if (d->row_ptr) (void)hipFree(d->row_ptr);
     if (d->adj) (void)hipFree(d->adj);
@@ -352,7 +351,6 @@ extern "C" void sgc_dgraph_free(sgc_dgraph* d) {
   if (d->mirror) (void)hipFree(d->mirror);
   if (d->ndeg) (void)hipFree(d->ndeg);
   if (d->woff) (void)hipFree(d->woff);
-  if (d->gs) (void)hipFree(d->gs);
   if (d->packed) (void)hipFree(d->packed);
   if (d->row_ptr) (void)hipFree(d->row_ptr);
   if (d->adj) (void)hipFree(d->adj);

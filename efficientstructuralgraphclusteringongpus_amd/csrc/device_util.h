@@ -116,6 +116,31 @@ __device__ __forceinline__ void block_reserve(uint32_t (&v)[N], unsigned long lo
   __syncthreads();
 }
 
+// Two-table cuckoo hashes in LDS (tables of `slots` words at offsets 0 and
+// slots, hashed by the top bits of two multiplicative hashes, shift = 32 -
+// log2(slots)); empty slots hold kEmptySlot, which is no vertex.  An insertion
+// evicts along a chain of at most kCuckooKicks; false if the chain fails.
+constexpr uint32_t kEmptySlot = 0xFFFFFFFFu;
+constexpr int kCuckooKicks = 128;
+
+__device__ __forceinline__ uint32_t cuckoo_h0(uint32_t x, uint32_t shift) { return (x * 0x9E3779B1u) >> shift; }
+__device__ __forceinline__ uint32_t cuckoo_h1(uint32_t x, uint32_t shift) {
+  return ((x ^ (x >> 16)) * 0x85EBCA77u) >> shift;
+}
+
+__device__ __forceinline__ bool cuckoo_insert(uint32_t* tab, uint32_t key, uint32_t slots, uint32_t shift,
+                                              uint32_t side = 0) {
+  uint32_t k = key;
+  for (int i = 0; i < kCuckooKicks; ++i) {
+    const uint32_t slot = side ? slots + cuckoo_h1(k, shift) : cuckoo_h0(k, shift);
+    const uint32_t old = atomicExch(&tab[slot], k);
+    if (old == kEmptySlot) return true;
+    k = old;  // the evicted key moves to its slot in the other table
+    side ^= 1u;
+  }
+  return false;
+}
+
 struct OpAdd {
   template <typename T>
   __device__ T operator()(T a, T b) const { return a + b; }

@@ -37,7 +37,6 @@ namespace sgc {
 
 namespace {
 
-constexpr uint32_t kEmptySlot = 0xFFFFFFFFu;
 constexpr uint32_t kNone = 0xFFFFFFFFu;
 
 constexpr uint32_t kT1MaxDeg = 1024;  // small-tier tables are sized for this
@@ -216,15 +215,16 @@ __global__ void __launch_bounds__(kBlock) k_prep(uint32_t m, const uint32_t* __r
       }
     }
     // owner b's undecided edges go to uedge[rb[b] + slot], slot < cnt_u[b],
-    // as (entry, its reverse entry or kNone without the index, a, d(a))
+    // as (entry, its reverse entry or kNone without the index, row start of
+    // a, d(a))
 #pragma unroll
     for (uint32_t j = 0; j < C; ++j) {
       if (REC == kRecCount || !om[j]) continue;
       const uint32_t slot = __shfl(sb[j], rank[j] >> 24) + (rank[j] & 0xFFFFFFu);
       if ((om[j] >> lane) & 1ull)
         uedge[(REC == kRecCompact ? 0u - r0 : ub[j]) + slot] =
-            make_uint4((uint32_t)(base + j * kWave + lane), mirror ? mirror[base + j * kWave + lane] : kNone, v[j],
-                       dv[j]);
+            make_uint4((uint32_t)(base + j * kWave + lane), mirror ? mirror[base + j * kWave + lane] : kNone,
+                       rb[v[j]], dv[j]);
     }
   }
   if (REC != kRecCompact)
@@ -351,16 +351,14 @@ __global__ void __launch_bounds__(kBlock) k_plan(uint32_t x0, uint32_t x1, const
 // and the owner row with the same exact threshold and early exit as the
 // tiered kernels, and writes both entries.
 __device__ __forceinline__ void tiny_edge(uint32_t m, uint32_t x, uint32_t bb, uint32_t be, uint32_t rs,
-                                          uint32_t i, const uint32_t* __restrict__ rb,
-                                          const int32_t* __restrict__ adj,
+                                          uint32_t i, const int32_t* __restrict__ adj,
                                           const uint32_t* __restrict__ mirror, double eps,
                                           const uint4* __restrict__ uedge, uint8_t* __restrict__ flag,
                                           uint32_t* __restrict__ cn_out) {
   const uint32_t l = be - bb;
-  const uint4 ed = uedge[rs + i];  // (entry, reverse entry, a, d(a)); rs: x's first record
-  const uint32_t k = ed.x, s = ed.w;
+  const uint4 ed = uedge[rs + i];  // (entry, reverse entry, row start of a, d(a)); rs: x's first record
+  const uint32_t k = ed.x, ab = ed.z, s = ed.w, ae = ab + s;
   if (k >= m) return;
-  const uint32_t ab = rb[ed.z], ae = ab + s;
   const double rhs = predicate_rhs(eps, s, l);
   const uint32_t cstar = s <= kMaxThresholdRow && !cn_out ? min_common_threshold(rhs, s) : kNone;
   // merge in blocks of 4 entries per row: count the matches between the
@@ -466,8 +464,8 @@ __global__ void __launch_bounds__(kBlock) k_sim_tiny(uint32_t m, const uint32_t*
           lo = mid + 1;
       }
       const uint32_t first = lo ? s_incl[w0 + lo - 1] : 0u;
-      tiny_edge(m, s_x[w0 + lo], s_bb[w0 + lo], s_be[w0 + lo], s_rs[w0 + lo], idx - first, rb, adj, mirror, eps,
-                uedge, flag, cn_out);
+      tiny_edge(m, s_x[w0 + lo], s_bb[w0 + lo], s_be[w0 + lo], s_rs[w0 + lo], idx - first, adj, mirror, eps, uedge,
+                flag, cn_out);
     }
     __builtin_amdgcn_wave_barrier();  // every lane is done with the rows before the next group overwrites them
   }
@@ -593,31 +591,13 @@ struct ClaimTable {
 //   Small tier: 2 x 2^bits slots with 2^bits >= 2 d(b) (at most a quarter
 //   full), in place of linear probing, whose lock-step rounds last as long
 //   as the wave's longest probe.
-// Insertion evicts along a chain of at most kCuckooKicks; a failed chain
-// (never observed at these loads) sends the unit to bitmap windows (large
-// tier) or linear probing (small tier).
+// Insertion evicts along a chain of at most kCuckooKicks (device_util.h); a
+// failed chain
+// (never observed at these loads) sends the unit to bitmap windows
+// (large tier) or linear probing (small tier).
 constexpr uint32_t kCuckooSlots = 16384;
 constexpr uint32_t kCuckooShift = 18;  // 32 - log2(kCuckooSlots)
 constexpr uint32_t kCuckooMaxKeys = 8192;
-constexpr int kCuckooKicks = 128;
-
-__device__ __forceinline__ uint32_t cuckoo_h0(uint32_t x, uint32_t shift) { return (x * 0x9E3779B1u) >> shift; }
-__device__ __forceinline__ uint32_t cuckoo_h1(uint32_t x, uint32_t shift) {
-  return ((x ^ (x >> 16)) * 0x85EBCA77u) >> shift;
-}
-
-__device__ __forceinline__ bool cuckoo_insert(uint32_t* tab, uint32_t key, uint32_t slots, uint32_t shift,
-                                              uint32_t side = 0) {
-  uint32_t k = key;
-  for (int i = 0; i < kCuckooKicks; ++i) {
-    const uint32_t slot = side ? slots + cuckoo_h1(k, shift) : cuckoo_h0(k, shift);
-    const uint32_t old = atomicExch(&tab[slot], k);
-    if (old == kEmptySlot) return true;
-    k = old;  // the evicted key moves to its slot in the other table
-    side ^= 1u;
-  }
-  return false;
-}
 
 // Inserts this thread's N keys (kEmptySlot: none): every first placement
 // into table 0 is issued before any result is looked at, so a thread's keys
@@ -747,8 +727,7 @@ __device__ __forceinline__ uint32_t count_dispatch(uint32_t nl, const ClaimTable
 // (s > kMaxThresholdRow) are counted fully.
 template <class T>
 __global__ void __launch_bounds__(T::kThreads, T::kMinWaves)
-    k_sim_units(uint32_t n, uint32_t m, const uint32_t* __restrict__ rb, const uint32_t* __restrict__ src,
-                const int32_t* __restrict__ adj,
+    k_sim_units(uint32_t n, uint32_t m, const uint32_t* __restrict__ src, const int32_t* __restrict__ adj,
                 const uint32_t* __restrict__ mirror, double eps, uint8_t* __restrict__ flag,
                 uint32_t* __restrict__ cn_out, const uint32_t* __restrict__ woff, uint32_t wstride,
                 const uint4* __restrict__ uedge, const uint4* __restrict__ units, uint32_t ucap,
@@ -837,12 +816,12 @@ __global__ void __launch_bounds__(T::kThreads, T::kMinWaves)
     if (vstate && threadIdx.x == 0) s_by = s_bn = s_def = 0;
     if (threadIdx.x < ne) {
       const uint32_t t = threadIdx.x;
-      const uint4 ed = uedge[un.x + t];  // (entry, reverse entry, a, d(a))
+      const uint4 ed = uedge[un.x + t];  // (entry, reverse entry, row start of a, d(a))
       const uint32_t k = ed.x;
       uint32_t ab = 0, s = 0, cstar = 0, a = 0;
       if (k < m) {
-        a = ed.z;
-        ab = rb[a];
+        if (T::kBitmap && (woff || vstate)) a = (uint32_t)adj[k];  // window-offset index, vertex state
+        ab = ed.z;
         s = ed.w;
         if (vstate) {
           my_a = a;
@@ -1284,13 +1263,13 @@ void launch_similarity(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, 
   // the core-check pruning runs in the workgroup tier, which launches first
   // and holds the long rows; the later tiers decide every edge they own
   const bool prune = p.prune && !cn_out && g->mirror;
-  k_sim_units<LargeTier><<<cus, LargeTier::kThreads, 0, s>>>(g->n, g->m, g->row_begin, g->src, g->adj, g->mirror, p.eps, b.flag,
+  k_sim_units<LargeTier><<<cus, LargeTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps, b.flag,
                                                              cn_out, g->woff, window_count(g->n) + 1, b.uedge, units,
                                                              ucap, b.cnt, kCntUnits2, kCntQueue2,
                                                              g->tuning.hash_tables != 0, prune ? b.core : nullptr,
                                                              b.ny, b.nn, p.mu);
   if (mid) (void)hipEventRecord(mid, s);
-  k_sim_units<SmallTier><<<cus * 8, SmallTier::kThreads, 0, s>>>(g->n, g->m, g->row_begin, g->src, g->adj, g->mirror, p.eps,
+  k_sim_units<SmallTier><<<cus * 8, SmallTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps,
                                                                  b.flag, cn_out, nullptr, 0, b.uedge, units, ucap,
                                                                  b.cnt, kCntUnits1, kCntQueue1, g->tuning.hash_tables != 0,
                                                                  nullptr, nullptr, nullptr, 0);
@@ -1381,13 +1360,13 @@ void launch_similarity_packed(const sgc_dgraph* g, const PassBuffers& b, ScanPar
         k_plan<<<grid_for(rr.hi[q] - rr.lo[q], kBlock), kBlock, 0, s>>>(
             rr.lo[q], rr.hi[q], g->row_begin, g->row_end, t, b.cnt_u, b.work_u, b.units, b.ucap, b.tiny, b.cnt, nullptr,
             nullptr, nullptr, p.mu, false, b.rec_start, r0, w);
-    k_sim_units<LargeTier><<<cus, LargeTier::kThreads, 0, s>>>(g->n, g->m, g->row_begin, g->src, g->adj, g->mirror, p.eps, b.flag,
+    k_sim_units<LargeTier><<<cus, LargeTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps, b.flag,
                                                                nullptr, g->woff, window_count(g->n) + 1, b.uedge, b.units,
                                                                b.ucap, b.cnt, kCntUnits2, kCntQueue2,
                                                                g->tuning.hash_tables != 0, nullptr, nullptr, nullptr,
                                                                0);
     if (r == 0 && mid) (void)hipEventRecord(mid, s);
-    k_sim_units<SmallTier><<<cus * 8, SmallTier::kThreads, 0, s>>>(g->n, g->m, g->row_begin, g->src, g->adj, g->mirror, p.eps,
+    k_sim_units<SmallTier><<<cus * 8, SmallTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps,
                                                                    b.flag, nullptr, nullptr, 0, b.uedge, b.units,
                                                                    b.ucap, b.cnt, kCntUnits1, kCntQueue1,
                                                                    g->tuning.hash_tables != 0, nullptr, nullptr,
@@ -1436,11 +1415,11 @@ void launch_redo(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int cu
   k_plan<<<grid_for(g->n, kBlock), kBlock, 0, s>>>(0, g->n, g->row_begin, g->row_end, t, b.cnt_u, b.work_u, b.units,
                                                    b.ucap, b.tiny, b.cnt, nullptr, nullptr, nullptr, p.mu, true);
   const uint32_t cus = (uint32_t)(cu_count > 0 ? cu_count : 256);
-  k_sim_units<LargeTier><<<cus, LargeTier::kThreads, 0, s>>>(g->n, g->m, g->row_begin, g->src, g->adj, g->mirror, p.eps, b.flag,
+  k_sim_units<LargeTier><<<cus, LargeTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps, b.flag,
                                                              nullptr, g->woff, window_count(g->n) + 1, b.uedge, b.units,
                                                              b.ucap, b.cnt, kCntUnits2, kCntQueue2,
                                                              g->tuning.hash_tables != 0, nullptr, nullptr, nullptr, 0);
-  k_sim_units<SmallTier><<<cus * 8, SmallTier::kThreads, 0, s>>>(g->n, g->m, g->row_begin, g->src, g->adj, g->mirror, p.eps,
+  k_sim_units<SmallTier><<<cus * 8, SmallTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps,
                                                                  b.flag, nullptr, nullptr, 0, b.uedge, b.units,
                                                                  b.ucap, b.cnt, kCntUnits1, kCntQueue1,
                                                                  g->tuning.hash_tables != 0, nullptr, nullptr, nullptr,
