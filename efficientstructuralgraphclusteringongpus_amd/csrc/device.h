@@ -64,7 +64,8 @@ enum Counter {
   kCntFQueue2 = 192,
   kCntHUnits = 208,   // units of the hash filter
   kCntHQueue = 224,
-  kStripe0 = 240,
+  kCntPieces = 240,   // pieces of labelled rows for the classify pass
+  kStripe0 = 256,
   kStripes = 32,
   kCntWords = kStripe0 + kStripes * kStripeSlots
 };

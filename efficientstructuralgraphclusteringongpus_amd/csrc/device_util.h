@@ -68,19 +68,26 @@ __device__ __forceinline__ T wave_seg_reduce(uint32_t row, T val, Op op) {
   return val;
 }
 
+// The value of the lane below (DPP wave_shr: no LDS permute); all 64 lanes
+// must call it.
+__device__ __forceinline__ uint32_t wave_prev(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xf, 0xf, true);
+}
+
 __device__ __forceinline__ bool wave_seg_head(uint32_t row) {
-  uint32_t prev = __shfl_up(row, 1);
+  const uint32_t prev = wave_prev(row);
   return lane_id() == 0 || prev != row;
 }
 
-// Inclusive prefix sum over the wave.
+// Inclusive prefix sum over the wave, by DPP row shifts and broadcasts; all
+// 64 lanes must call it.
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
-  const uint32_t lane = lane_id();
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    uint32_t o = __shfl_up(v, off);
-    if (lane >= (uint32_t)off) v += o;
-  }
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);   // row_shr:1
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);   // row_shr:2
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);   // row_shr:4
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);   // row_shr:8
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15 to rows 1, 3
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31 to rows 2, 3
   return v;
 }
 

@@ -5,6 +5,8 @@
 // consecutive lanes) so each row issues at most one atomic per wave.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include <hipcub/device/device_radix_sort.hpp>
 
 #include "device.h"
@@ -292,33 +294,24 @@ __global__ void __launch_bounds__(kBlock) k_similarity_wave(const uint32_t* __re
 // Core check (GPUSCAN++/GPUScan.cu:115-131, :276-367)
 // ---------------------------------------------------------------------------
 
-__global__ void __launch_bounds__(kBlock) k_core_count(uint32_t m, const uint32_t* __restrict__ src,
+// Similar entries per row, from the flags' similar entries alone: one
+// atomic per run of a row's entries in a wave's 64.
+__global__ void __launch_bounds__(kBlock) k_core_count(uint64_t m, const uint32_t* __restrict__ src,
                                                        const uint8_t* __restrict__ flag, uint32_t* __restrict__ sd) {
-  constexpr uint32_t C = kEdgeChunks;
-  const uint32_t lane = lane_id();
-  const uint64_t waves = (uint64_t)gridDim.x * (kBlock / kWave);
-  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * (kWave * C); base < m;
-       base += waves * kWave * C) {
-    uint32_t row[C], y[C];
-#pragma unroll
-    for (uint32_t j = 0; j < C; ++j) {
-      const uint64_t k = base + j * kWave + lane;
-      y[j] = k < m && flag[k] == kFlagY ? 1u : 0u;
-    }
-    // rows of similar entries only; the others get a marker row, so one
-    // row's similar entries may form several runs of lanes: each run's first
-    // lane adds the run's count (ballot over [first lane, next run))
-#pragma unroll
-    for (uint32_t j = 0; j < C; ++j) row[j] = y[j] ? src[base + j * kWave + lane] : 0xFFFFFFFFu;
-#pragma unroll
-    for (uint32_t j = 0; j < C; ++j) {
-      const uint64_t ym = __ballot(y[j]);
-      if (!ym) continue;
-      const bool head = wave_seg_head(row[j]);
+  __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
+  const uint32_t lane = lane_id(), wv = threadIdx.x / kWave;
+  const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * kFlagTile;
+  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * kFlagTile; base < m; base += step) {
+    const uint32_t total = similar_tile(flag, m, base, s_at[wv]);
+    for (uint32_t i0 = 0; i0 < total; i0 += kWave) {
+      const bool on = i0 + lane < total;
+      const uint32_t row = on ? src[base + s_at[wv][i0 + lane]] : 0xFFFFFFFFu;
+      const bool head = wave_seg_head(row);
       const uint64_t after = __ballot(head) & ~lanemask_le(lane);
-      const uint64_t run = (after ? lanemask_lt((uint32_t)(__ffsll((long long)after) - 1)) : ~0ull) & ~lanemask_lt(lane);
-      if (head && y[j]) atomicAdd(&sd[row[j]], (uint32_t)__popcll(ym & run));
+      const uint32_t stop = after ? (uint32_t)(__ffsll((long long)after) - 1) : (uint32_t)kWave;
+      if (head && on) atomicAdd(&sd[row], stop - lane);
     }
+    wave_lds_sync();  // the list is rewritten
   }
 }
 
@@ -356,19 +349,58 @@ __global__ void __launch_bounds__(kBlock) k_core_mark(uint32_t n, const uint32_t
 // (GPUSCAN++/GPUScan.cu:465-528, :632-652; scan_phases.h)
 // ---------------------------------------------------------------------------
 
-// gate >= 0: runs only when the sum `gate` is not 0 (the union-find pass repeated
-// after the second similarity round of a pruned pass).
-__global__ void __launch_bounds__(kBlock) k_union(uint32_t m, const uint32_t* __restrict__ src,
+// Two rounds over the similar core-core edges, each visited from its larger
+// endpoint: the first joins one edge per run of a row's entries (HEADS), then
+// k_compress points every core at its root, and the second joins what is
+// left; by then nearly every edge's endpoints have the same parent, which two
+// plain loads show (a parent read from a stale cache line is still an
+// ancestor).  Joining every edge at once met in long chains and contended
+// swaps: on planted communities (n = 3e5, 3.6e6 similar edges, 64k cores)
+// 0.97 ms, 0.26 in two rounds.
+// gate >= 0: runs only when the sum `gate` is not 0 (the union-find pass
+// repeated after the second similarity round of a pruned pass).
+constexpr uint64_t kFewCores = 1024;  // up to here the first round costs more than it saves
+
+template <bool HEADS>
+__global__ void __launch_bounds__(kBlock) k_union(uint64_t m, const uint32_t* __restrict__ src,
                                                   const int32_t* __restrict__ adj, const uint8_t* __restrict__ flag,
                                                   const uint8_t* __restrict__ core, int32_t* parent,
                                                   const uint64_t* __restrict__ cnt, int gate) {
-  if (!count_any(cnt, kCntMarked)) return;  // no core: no core-core edge to join
+  const uint64_t cores = count_total(cnt, kCntMarked);
+  if (cores == 0) return;  // no core-core edge to join
+  if (HEADS && cores <= kFewCores) return;
   if (gate >= 0 && !count_any(cnt, gate)) return;
-  PhaseView v{};
-  v.m = m, v.src = src, v.adj = adj, v.flag = flag, v.core = const_cast<uint8_t*>(core), v.parent = parent;
+  __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
+  const uint32_t lane = lane_id(), wv = threadIdx.x / kWave;
+  const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * kFlagTile;
+  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * kFlagTile; base < m; base += step) {
+    const uint32_t total = similar_tile(flag, m, base, s_at[wv]);
+    for (uint32_t i0 = 0; i0 < total; i0 += kWave) {
+      bool on = i0 + lane < total;
+      const uint64_t k = base + (on ? s_at[wv][i0 + lane] : 0);
+      const uint32_t u = on ? src[k] : 0u;
+      const int32_t w = on ? adj[k] : 0;
+      on = on && (uint32_t)w < u && core[u] && core[w];
+      if (HEADS) {
+        // the first of the row's entries among the lanes that are on
+        const uint64_t below = __ballot(on) & lanemask_lt(lane);
+        const uint32_t prev = below ? 63u - (uint32_t)__clzll((long long)below) : lane;
+        const uint32_t pu = (uint32_t)__shfl((int)u, (int)prev);
+        if (on && (!below || pu != u)) uf_union(parent, (int32_t)u, w);
+      } else if (on && parent[u] != parent[w]) {
+        uf_union(parent, (int32_t)u, w);
+      }
+    }
+    wave_lds_sync();  // the list is rewritten
+  }
+}
+
+__global__ void __launch_bounds__(kBlock) k_compress(uint32_t n, const uint8_t* __restrict__ core, int32_t* parent,
+                                                     const uint64_t* __restrict__ cnt) {
+  if (count_total(cnt, kCntMarked) <= kFewCores) return;
   const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-  for (uint64_t k0 = (uint64_t)blockIdx.x * kBlock + threadIdx.x; k0 < m; k0 += stride * kEdgeChunks)
-    union_entries(v, k0, stride);
+  for (uint64_t x = (uint64_t)blockIdx.x * kBlock + threadIdx.x; x < n; x += stride)
+    if (core[x]) st_coherent(parent + x, uf_find(parent, (int32_t)x));
 }
 
 __global__ void __launch_bounds__(kBlock) k_flatten(uint32_t n, const uint8_t* __restrict__ core, int32_t* parent,
@@ -428,22 +460,28 @@ __global__ void __launch_bounds__(kBlock) k_redo_mark(uint32_t m, const uint32_t
 // Borders (GPUSCAN++/GPUScan.cu:654-730): minimum candidate cluster id
 // ---------------------------------------------------------------------------
 
-__global__ void __launch_bounds__(kBlock) k_border(uint32_t m, const uint32_t* __restrict__ src,
+__global__ void __launch_bounds__(kBlock) k_border(uint64_t m, const uint32_t* __restrict__ src,
                                                    const int32_t* __restrict__ adj, const uint8_t* __restrict__ flag,
                                                    const uint8_t* __restrict__ core, const uint32_t* __restrict__ rb,
                                                    const uint32_t* __restrict__ re, int32_t* label,
                                                    uint64_t* __restrict__ cnt) {
   if (!count_any(cnt, kCntMarked)) return;  // no core: no border
+  __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
   PhaseView v{};
-  v.m = m, v.src = src, v.adj = adj, v.flag = flag, v.core = const_cast<uint8_t*>(core), v.rb = rb, v.re = re;
-  v.label = label;
-  const uint64_t waves = (uint64_t)gridDim.x * (kBlock / kWave);
+  v.src = src, v.adj = adj, v.core = const_cast<uint8_t*>(core), v.rb = rb, v.re = re, v.label = label;
+  const uint32_t lane = lane_id(), wv = threadIdx.x / kWave;
+  const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * kFlagTile;
   // entries of the border rows this lane labels first; the core rows'
   // entries were counted by k_core_mark
-  uint32_t labeled = 0;
-  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * (kWave * kEdgeChunks);
-       base < m; base += waves * kWave * kEdgeChunks)
-    labeled += border_chunk(v, base);
+  uint64_t labeled = 0;
+  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * kFlagTile; base < m; base += step) {
+    const uint32_t total = similar_tile(flag, m, base, s_at[wv]);
+    for (uint32_t i0 = 0; i0 < total; i0 += kWave) {
+      const bool on = i0 + lane < total;
+      labeled += border_entry(v, base + (on ? s_at[wv][i0 + lane] : 0), on);
+    }
+    wave_lds_sync();  // the list is rewritten
+  }
   count_add<1>(cnt, {kCntLabeled}, {labeled});
 }
 
@@ -451,22 +489,94 @@ __global__ void __launch_bounds__(kBlock) k_border(uint32_t m, const uint32_t* _
 // Hubs and outliers (GPUSCAN++/GPUScan.cu:732-798)
 // ---------------------------------------------------------------------------
 
-// Every launch over the graph's entries (m_all of them, maybe in several row
-// chips) takes the same side: from the labelled rows when they hold fewer
-// than a third of the entries.
+// The side of the classify pass, the same for every launch over the graph's
+// m_all entries (maybe in several row chips): from the labelled rows when
+// they hold fewer than a third of the entries.
+__device__ __forceinline__ bool classify_from_labeled(const uint64_t* cnt, uint64_t m_all) {
+  return 3 * count_total(cnt, kCntLabeled) < m_all;
+}
+
+// listed: the labelled side is left to k_classify_rows.
 __global__ void __launch_bounds__(kBlock) k_classify(uint32_t m, uint64_t m_all, const uint32_t* __restrict__ src,
                                                      const int32_t* __restrict__ adj,
                                                      const int32_t* __restrict__ label, int32_t* __restrict__ lo,
-                                                     int32_t* __restrict__ hi, const uint64_t* __restrict__ cnt) {
+                                                     int32_t* __restrict__ hi, const uint64_t* __restrict__ cnt,
+                                                     bool listed) {
   // no core means no label anywhere: lo and hi keep their initial values
   if (!count_any(cnt, kCntMarked)) return;
   PhaseView v{};
   v.m = m, v.src = src, v.adj = adj, v.label = const_cast<int32_t*>(label), v.lo = lo, v.hi = hi;
-  const bool from_labeled = 3 * count_total(cnt, kCntLabeled) < m_all;
+  const bool from_labeled = classify_from_labeled(cnt, m_all);
+  if (from_labeled && listed) return;
   const uint64_t waves = (uint64_t)gridDim.x * (kBlock / kWave);
   for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * (kWave * kEdgeChunks);
        base < m; base += waves * kWave * kEdgeChunks)
     classify_chunk(v, base, from_labeled);
+}
+
+// The labelled side without a walk over all entries: the labelled rows in
+// pieces of kRowPiece entries, listed, then one wave per piece.  At most one
+// piece per labelled row and one per kRowPiece entries: under m of them.
+// R-MAT-24 with 304 cores: 1.45 ms for the walk, 0.73 listed.
+constexpr uint32_t kRowPiece = 1024;
+
+__global__ void __launch_bounds__(kBlock) k_label_pieces(uint32_t n, uint64_t m, const uint32_t* __restrict__ rb,
+                                                         const uint32_t* __restrict__ re,
+                                                         const int32_t* __restrict__ label, uint2* __restrict__ piece,
+                                                         uint64_t* __restrict__ cnt) {
+  if (!count_any(cnt, kCntMarked) || !classify_from_labeled(cnt, m)) return;
+  constexpr uint32_t V = 8;
+  unsigned long long* const ctr[1] = {(unsigned long long*)&cnt[kCntPieces]};
+  const uint64_t tile = (uint64_t)kBlock * V;
+  for (uint64_t base = (uint64_t)blockIdx.x * tile; base < n; base += (uint64_t)gridDim.x * tile) {  // block-uniform
+    uint32_t len[V], need[1] = {0};
+#pragma unroll
+    for (uint32_t j = 0; j < V; ++j) {
+      const uint64_t x = base + j * kBlock + threadIdx.x;
+      len[j] = x < n && label[x] != kNoLabel ? re[x] - rb[x] : 0u;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < V; ++j) need[0] += (len[j] + kRowPiece - 1) / kRowPiece;
+    if (!__syncthreads_or(need[0] != 0)) continue;
+    block_reserve<1>(need, ctr);
+#pragma unroll
+    for (uint32_t j = 0; j < V; ++j)
+      for (uint32_t at = 0; at < len[j]; at += kRowPiece)
+        piece[need[0]++] = make_uint2((uint32_t)(base + j * kBlock + threadIdx.x), at);
+  }
+}
+
+__global__ void __launch_bounds__(kBlock) k_classify_rows(const uint32_t* __restrict__ rb,
+                                                          const uint32_t* __restrict__ re,
+                                                          const int32_t* __restrict__ adj,
+                                                          const int32_t* __restrict__ label, int32_t* lo, int32_t* hi,
+                                                          const uint2* __restrict__ piece,
+                                                          const uint64_t* __restrict__ cnt) {
+  const uint64_t count = cnt[kCntPieces];  // 0 when the other side is taken
+  const uint64_t waves = (uint64_t)gridDim.x * (kBlock / kWave);
+  for (uint64_t i = (uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; i < count; i += waves) {
+    const uint2 p = piece[i];
+    const uint32_t b = rb[p.x] + p.y, len = min(re[p.x] - b, kRowPiece);
+    const int32_t l = label[p.x];
+    for (uint32_t t0 = lane_id(); t0 < len; t0 += kWave * kEdgeChunks) {
+      int32_t nb[kEdgeChunks];
+      bool to[kEdgeChunks];
+#pragma unroll
+      for (uint32_t j = 0; j < kEdgeChunks; ++j) {
+        to[j] = t0 + j * kWave < len;
+        nb[j] = to[j] ? adj[b + t0 + j * kWave] : 0;
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < kEdgeChunks; ++j) to[j] = to[j] && label[nb[j]] == kNoLabel;
+      // a bound that is there already needs no atomic (a stale one is looser)
+#pragma unroll
+      for (uint32_t j = 0; j < kEdgeChunks; ++j)
+        if (to[j]) {
+          if (l < lo[nb[j]]) atomicMin(&lo[nb[j]], l);
+          if (l > hi[nb[j]]) atomicMax(&hi[nb[j]], l);
+        }
+    }
+  }
 }
 
 // Also counts the similar entries: sd[x] holds those of row x.
@@ -570,10 +680,18 @@ void launch_similarity_wave(const sgc_dgraph* g, const PassBuffers& b, ScanParam
                                               b.cnt);
 }
 
+// Graphs below this many entries skip the launches that only pay on large
+// ones (the first union round, the list of labelled rows): a launch costs 4-5
+// us, a whole pass over a million flags no more than that.
+constexpr uint64_t kSmallGraph = 1u << 20;
+
+// Blocks of a pass over the flags by similar_tile.
+static uint32_t flag_grid(uint64_t m) { return std::min(grid_for(m, kFlagTile * (kBlock / kWave)), 2048u); }
+
 // Edge passes take the entries [0, g->m) of g (a whole graph or one chip of
 // rows); vertex passes cover all g->n vertices.
 void launch_core_count(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s) {
-  if (g->m) k_core_count<<<grid_for(g->m, kBlock), kBlock, 0, s>>>(g->m, g->src, b.flag, b.sd);
+  if (g->m) k_core_count<<<flag_grid(g->m), kBlock, 0, s>>>(g->m, g->src, b.flag, b.sd);
 }
 
 void launch_core_mark(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStream_t s,
@@ -583,8 +701,13 @@ void launch_core_mark(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, h
 }
 
 void launch_union(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s, int gate) {
-  if (g->m)
-    k_union<<<grid_for(g->m, kBlock), kBlock, 0, s>>>(g->m, g->src, g->adj, b.flag, b.core, b.parent, b.cnt, gate);
+  if (!g->m) return;
+  const uint32_t grid = flag_grid(g->m);
+  if (g->m >= kSmallGraph) {
+    k_union<true><<<grid, kBlock, 0, s>>>(g->m, g->src, g->adj, b.flag, b.core, b.parent, b.cnt, gate);
+    k_compress<<<grid_for(g->n, kBlock), kBlock, 0, s>>>(g->n, b.core, b.parent, b.cnt);
+  }
+  k_union<false><<<grid, kBlock, 0, s>>>(g->m, g->src, g->adj, b.flag, b.core, b.parent, b.cnt, gate);
 }
 
 void launch_redo_mark(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s) {
@@ -598,14 +721,24 @@ void launch_flatten(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s) {
 }
 
 void launch_border(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s) {
-  if (g->m) k_border<<<grid_for(g->m, kBlock), kBlock, 0, s>>>(g->m, g->src, g->adj, b.flag, b.core, g->row_begin,
-                                                     g->row_end, b.label, b.cnt);
+  if (g->m)
+    k_border<<<flag_grid(g->m), kBlock, 0, s>>>(g->m, g->src, g->adj, b.flag, b.core, g->row_begin, g->row_end, b.label,
+                                                b.cnt);
 }
 
 void launch_classify_edges(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s, uint64_t m_all) {
-  if (g->m)
-    k_classify<<<grid_for(g->m, kBlock), kBlock, 0, s>>>(g->m, m_all ? m_all : g->m, g->src, g->adj, b.label, b.lo,
-                                                         b.hi, b.cnt);
+  if (!g->m) return;
+  // a whole graph lists its labelled rows, in the edge records' memory (free
+  // by now; serving slots have none)
+  const bool listed = !m_all && b.uedge && g->row_begin && g->m >= kSmallGraph;
+  if (listed) {
+    uint2* const piece = reinterpret_cast<uint2*>(b.uedge);
+    k_label_pieces<<<grid_for(g->n, kBlock * 8), kBlock, 0, s>>>(g->n, g->m, g->row_begin, g->row_end, b.label, piece,
+                                                                 b.cnt);
+    k_classify_rows<<<2048, kBlock, 0, s>>>(g->row_begin, g->row_end, g->adj, b.label, b.lo, b.hi, piece, b.cnt);
+  }
+  k_classify<<<grid_for(g->m, kBlock), kBlock, 0, s>>>(g->m, m_all ? m_all : g->m, g->src, g->adj, b.label, b.lo, b.hi,
+                                                       b.cnt, listed);
 }
 
 void launch_finalize(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStream_t s,

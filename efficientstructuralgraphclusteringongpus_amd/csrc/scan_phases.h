@@ -67,6 +67,46 @@ __device__ __forceinline__ void uf_union(int32_t* parent, int32_t a, int32_t b) 
   }
 }
 
+// The similar entries of the wave's tile [base, base + kFlagTile) of the flag
+// array, ascending, into `at` (the wave's kFlagTile words of LDS, offsets from
+// base); returns their number (uniform).  Flags come 16 to a load (flag must
+// be 16-byte aligned and readable up to the next multiple of 16): a byte a
+// lane read them at 0.9 TB/s.
+constexpr uint32_t kFlagTile = 2048;
+
+__device__ __forceinline__ uint32_t similar_tile(const uint8_t* __restrict__ flag, uint64_t m, uint64_t base,
+                                                 uint16_t* at) {
+  constexpr uint32_t L = kFlagTile / (kWave * 16);
+  const uint32_t lane = lane_id();
+  uint4 w[L];
+#pragma unroll
+  for (uint32_t j = 0; j < L; ++j) {
+    const uint64_t k = base + (j * kWave + lane) * 16;
+    w[j] = k < m ? *reinterpret_cast<const uint4*>(flag + k) : make_uint4(0, 0, 0, 0);
+  }
+  uint32_t total = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < L; ++j) {
+    const uint64_t k = base + (j * kWave + lane) * 16;
+    const uint32_t x[4] = {w[j].x, w[j].y, w[j].z, w[j].w};
+    uint32_t mask = 0;  // bit i: entry k + i is similar
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q) {
+      const uint32_t z = x[q] ^ (0x01010101u * kFlagY);
+      const uint32_t t = ~(((z & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | z | 0x7F7F7F7Fu);  // 0x80 in zero bytes
+      mask |= (((t >> 7) & 1u) | ((t >> 14) & 2u) | ((t >> 21) & 4u) | ((t >> 28) & 8u)) << (4 * q);
+    }
+    if (k + 16 > m) mask &= k < m ? (1u << (uint32_t)(m - k)) - 1u : 0u;
+    if (!__ballot(mask != 0)) continue;
+    const uint32_t incl = wave_incl_scan((uint32_t)__popc(mask));
+    uint32_t pos = total + incl - (uint32_t)__popc(mask);
+    for (uint32_t b = mask; b; b &= b - 1) at[pos++] = (uint16_t)((j * kWave + lane) * 16 + (uint32_t)__ffs(b) - 1);
+    total += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+  }
+  wave_lds_sync();
+  return total;
+}
+
 // Joins the similar core-core edges among entries k_j = k0 + j * step
 // (j < kEdgeChunks), each visited from its larger endpoint.
 __device__ __forceinline__ void union_entries(const PhaseView& v, uint64_t k0, uint64_t step) {
@@ -94,6 +134,25 @@ __device__ __forceinline__ void union_entries(const PhaseView& v, uint64_t k0, u
 // ancestors only), which must not land on a finished label.
 __device__ __forceinline__ void flatten_vertex(const PhaseView& v, uint32_t x) {
   if (v.core[x]) v.label[x] = uf_find(v.parent, (int32_t)x);
+}
+
+// ---- borders: the minimum candidate cluster id over similar edges to cores,
+// for one similar entry k per lane (on; ascending over the lanes).  A row's
+// candidates may lie in several runs of lanes (other entries between them get
+// a marker row), each run's minimum is added.  Returns the entries of the
+// border rows this lane labelled first (rows known only).  All 64 lanes must
+// call it.
+__device__ __forceinline__ uint32_t border_entry(const PhaseView& v, uint64_t k, bool on) {
+  const uint32_t row = on ? v.src[k] : 0xFFFFFFFFu;
+  const int32_t c = on ? v.adj[k] : 0;
+  const bool y = on && v.core[c] && !v.core[row];
+  if (!__ballot(y)) return 0;
+  const int32_t cand = y ? v.label[c] : kNoLabel;
+  const uint32_t r = y ? row : 0xFFFFFFFFu;
+  const int32_t best = wave_seg_reduce(r, cand, OpMin());
+  if (wave_seg_head(r) && best != kNoLabel && atomicMin(&v.label[r], best) == kNoLabel && v.rb)
+    return v.re[r] - v.rb[r];
+  return 0;
 }
 
 // ---- borders: the minimum candidate cluster id over similar edges to cores,

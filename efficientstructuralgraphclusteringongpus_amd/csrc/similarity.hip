@@ -195,13 +195,16 @@ __global__ void __launch_bounds__(kBlock) k_prep(uint32_t m, const uint32_t* __r
         if (lane == 0) owned_total += (uint32_t)__popcll(om[j]);
         // this lane's row segment [h, next head): owned count at the head,
         // this lane's rank among the owned entries below it
-        const uint64_t ws = wave_seg_reduce(row, owned ? (uint64_t)dv[j] : 0ull, OpAdd());
+        // (the work sums only steer the planner: lengths are clamped so that
+        // 64 of them fit 32 bits, and their sums come from one prefix sum)
+        const uint32_t len = owned ? min(dv[j], 1u << 25) : 0u, incl = wave_incl_scan(len);
         const bool head = wave_seg_head(row);
         const uint64_t hm = __ballot(head);
         const uint32_t h = 63 - __clzll((long long)(hm & lanemask_le(lane)));
         const uint64_t after = hm & ~lanemask_le(lane);
-        const uint64_t seg =
-            (after ? lanemask_lt((uint32_t)(__ffsll((long long)after) - 1)) : ~0ull) & ~lanemask_lt(h);
+        const uint32_t stop = after ? (uint32_t)(__ffsll((long long)after) - 1) : (uint32_t)kWave;
+        const uint64_t seg = (after ? lanemask_lt(stop) : ~0ull) & ~lanemask_lt(h);
+        const uint32_t ws = (uint32_t)__shfl((int)incl, (int)(stop - 1)) - (incl - len);
         const uint32_t c = (uint32_t)__popcll(om[j] & seg);
         rank[j] = (uint32_t)__popcll(om[j] & seg & lanemask_lt(lane)) | (h << 24);
         if (head && c) {
