@@ -50,6 +50,7 @@ enum Counter {
   kStripeSlots = 16,
   // single words
   kCntOverflow = 16,  // owned undecided entries, when more than the unit array holds (asymmetric input)
+  kCntStamp0 = 17,    // device clock when each phase's first kernel started (Stamp; 0: it was not launched)
   kCntTimer0 = 32,    // phase timers of debug builds (SGC_PHASE_TIMERS): 5 per tier
   kCntSlots = 48,     // host copies: the sums and single words above
   kCntUnits1 = 48,    // small-tier work units
@@ -70,6 +71,23 @@ enum Counter {
   kCntWords = kStripe0 + kStripes * kStripeSlots
 };
 
+// Phase times come from the device clock, read by the first block of a phase's
+// first kernel: an event between two kernels holds the second back by about
+// 2 us, which a pass of 150 us feels.
+enum Stamp {
+  kStampInit = 0,
+  kStampSim,         // first similarity kernel
+  kStampSimRest,     // first similarity kernel of the short owners
+  kStampExactLarge,  // workgroup-tier exact kernel
+  kStampExactSmall,
+  kStampCore,
+  kStampCluster,
+  kStampBorder,
+  kStampClassify,
+  kStampEnd,
+  kStamps
+};
+
 // Adds the stripes of a counter buffer's host copy to its sums.
 inline void fold_counters(uint64_t* c) {
   for (int i = 0; i < kStripes; ++i)
@@ -78,6 +96,10 @@ inline void fold_counters(uint64_t* c) {
 
 // Similarity kernels selectable per context.
 enum SimImpl { kSimTiered = 0, kSimWavePerEdge = 1 };
+
+// Results of a pass up to this size go to host memory through the context's
+// page-locked staging, written by the pass's last kernel.
+constexpr size_t kStageBytes = 256u << 10;
 
 // Grow-only device allocation owned by a context.
 struct DevBuf {
@@ -94,7 +116,9 @@ struct sgc_ctx {
   int cu_count = 0;
   sgc::DevBuf work;      // per-pass arrays
   sgc::DevBuf counters;  // kCntWords x uint64
-  uint64_t* host_counters = nullptr;  // pinned mirror
+  uint64_t* host_counters = nullptr;  // page-locked: kCntWords words, then kStageBytes for small results
+  uint64_t* host_counters_dev = nullptr;  // its device address
+  double clock_khz = 100000.0;  // rate of the device clock (Stamp)
   hipEvent_t ev[8] = {};
   int sim_impl = sgc::kSimTiered;
   void* scratch = nullptr;  // this GPU's static scratch (sgc_scan_device_noalloc)
@@ -260,6 +284,8 @@ hipError_t build_packed_rows(sgc_dgraph* g, hipStream_t s);
 bool filter_stage(const sgc_dgraph* g, ScanParams p);
 void launch_plan_filter(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s);
 void launch_filter(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int cu_count, hipStream_t s);
+// Whether launch_filter can leave units to the exact kernels.
+bool filter_leaves_units(const sgc_dgraph* g);
 void launch_copy(const void* src, void* dst, uint64_t bytes, hipStream_t s);
 void launch_init(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s);
 // count_all: every edge is left to its owner (for exact common-neighbour
@@ -294,8 +320,10 @@ void launch_similarity(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, 
                        hipStream_t s, uint32_t* cn_out = nullptr);
 void launch_similarity_wave(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int cu_count, hipStream_t s);
 void launch_core(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStream_t s);
-void launch_cluster(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s);
-void launch_border(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s);
+// flatten: launch_flatten's work too (small graphs: a launch less)
+void launch_border(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s, bool flatten = false);
+// Graphs on which a launch costs more than what it saves.
+bool small_graph(const sgc_dgraph* g);
 void launch_classify(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStream_t s);
 // The single kernels the four launchers above are made of (edge passes over
 // entries [0, g->m), vertex passes over all g->n vertices); the out-of-core
@@ -312,6 +340,11 @@ void launch_redo_mark(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s);
 void launch_flatten(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s);
 // m_all: entries of the whole graph when g is one of several row chips
 void launch_classify_edges(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s, uint64_t m_all = 0);
+// The pass's end: counters (sums folded) to host_cnt (page-locked, device
+// address), and the results to the device addresses given (any may be null);
+// after an overflow (kCntOverflow) the results are left alone.
+void launch_publish(const sgc_dgraph* g, const PassBuffers& b, uint64_t* host_cnt, int32_t* labels, uint8_t* core,
+                    uint8_t* sim, hipStream_t s);
 void launch_finalize(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStream_t s,
                      const int32_t* mu_dev = nullptr);
 

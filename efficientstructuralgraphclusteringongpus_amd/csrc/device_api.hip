@@ -153,7 +153,12 @@ extern "C" int sgc_ctx_create(int device, sgc_ctx** out) {
     delete ctx;
     return rc;
   }
-  SGC_HIP(hipHostMalloc((void**)&ctx->host_counters, kCntWords * sizeof(uint64_t), hipHostMallocDefault));
+  SGC_HIP(hipHostMalloc((void**)&ctx->host_counters, kCntWords * sizeof(uint64_t) + kStageBytes,
+                        hipHostMallocDefault));
+  SGC_HIP(hipHostGetDevicePointer((void**)&ctx->host_counters_dev, ctx->host_counters, 0));
+  int clock_khz = 0;
+  if (hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && clock_khz > 0)
+    ctx->clock_khz = clock_khz;
   for (auto& e : ctx->ev) SGC_HIP(hipEventCreate(&e));
   *out = ctx;
   return SGC_OK;
@@ -400,51 +405,103 @@ int check_unit_overflow(const uint64_t* c, uint64_t m) {
 
 namespace {
 
-// One plain pass over g with the arrays in *pb (carved by the caller).
-// want_flags: the caller takes the similarity flags, so every edge is
+// Where a pass's results go (any pointer may be null).
+struct PassOut {
+  int32_t* labels;
+  uint8_t* core;
+  uint8_t* sim;
+  bool device;  // device addresses (else host)
+};
+
+// Whether the pass's own kernels may write to p: memory of the context's
+// device.
+bool on_device(const sgc_ctx* ctx, const void* p) {
+  if (!p) return true;
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice && a.device == ctx->device;
+}
+
+// Milliseconds from the phase stamp a to the first stamp set from b on.
+double phase_ms(const sgc_ctx* ctx, int a, int b) {
+  const uint64_t* t = ctx->host_counters + kCntStamp0;
+  if (!t[a]) return 0.0;
+  while (b < kStampEnd && !t[b]) ++b;
+  return t[b] > t[a] ? (double)(t[b] - t[a]) / ctx->clock_khz : 0.0;
+}
+
+// One plain pass over g with the arrays in *pb (carved by the caller), its
+// results to `out`.  A caller that takes the similarity flags has every edge
 // decided (no core-check pruning).
-int run_pass(sgc_ctx* ctx, sgc_dgraph* g, double eps, int32_t mu, PassBuffers* pb, sgc_stats* st,
-             bool want_flags) {
+int run_pass(sgc_ctx* ctx, sgc_dgraph* g, double eps, int32_t mu, PassBuffers* pb, sgc_stats* st, const PassOut& out) {
   SGC_HIP(hipSetDevice(ctx->device));
   // The reference's pruned core check (GPUSCAN++/GPUScan.cu:303) needs
   // mu >= 1 (for mu <= 0 no vertex is ever decided not core) and the
   // reverse-entry index of a resident graph.
-  const bool prune = ctx->prune && mu >= 1 && !want_flags && g->mirror && ctx->sim_impl == kSimTiered;
+  const bool prune = ctx->prune && mu >= 1 && !out.sim && g->mirror && ctx->sim_impl == kSimTiered;
   const ScanParams p{eps, mu, prune};
   hipStream_t s = ctx->stream;
-  SGC_HIP(hipEventRecord(ctx->ev[0], s));
+  const bool small = small_graph(g);
   launch_init(g, *pb, s);
   launch_prep(g, *pb, p, s);
   launch_plan(g, *pb, p, s);
-  SGC_HIP(hipEventRecord(ctx->ev[1], s));
-  launch_similarity(g, *pb, p, ctx->cu_count, ctx->sim_impl, ctx->ev[7], s);
-  SGC_HIP(hipEventRecord(ctx->ev[2], s));
+  launch_similarity(g, *pb, p, ctx->cu_count, ctx->sim_impl, nullptr, s);
   launch_core(g, *pb, p, s);
-  SGC_HIP(hipEventRecord(ctx->ev[3], s));
   launch_union(g, *pb, s);
   // deferred edges the clusters or borders need, decided now
   if (p.prune) launch_redo(g, *pb, p, ctx->cu_count, s);
-  launch_flatten(g, *pb, s);
-  SGC_HIP(hipEventRecord(ctx->ev[4], s));
-  launch_border(g, *pb, s);
-  SGC_HIP(hipEventRecord(ctx->ev[5], s));
+  if (!small) launch_flatten(g, *pb, s);
+  launch_border(g, *pb, s, small);
   launch_classify(g, *pb, p, s);
-  SGC_HIP(hipEventRecord(ctx->ev[6], s));
+  // The last kernel hands over the counters and what it can write itself:
+  // results in this device's memory, and small ones for the host by way of
+  // the page-locked staging (three copies and a second wait cost more than
+  // 50 us of a pass of 170).
+  const uint64_t n = g->n, m = g->m;
+  const size_t o_core = (out.labels ? n * 4 : 0), o_sim = o_core + (out.core ? n : 0), bytes = o_sim + (out.sim ? m : 0);
+  char* const stage = (char*)(ctx->host_counters + kCntWords);
+  char* const stage_dev = (char*)(ctx->host_counters_dev + kCntWords);
+  const bool staged = !out.device && bytes <= kStageBytes;
+  const bool direct = out.device && on_device(ctx, out.labels) && on_device(ctx, out.core) && on_device(ctx, out.sim);
+  if (staged)
+    launch_publish(g, *pb, ctx->host_counters_dev, out.labels ? (int32_t*)stage_dev : nullptr,
+                   out.core ? (uint8_t*)stage_dev + o_core : nullptr, out.sim ? (uint8_t*)stage_dev + o_sim : nullptr, s);
+  else
+    launch_publish(g, *pb, ctx->host_counters_dev, direct ? out.labels : nullptr, direct ? out.core : nullptr,
+                   direct ? out.sim : nullptr, s);
   SGC_HIP(hipGetLastError());
-  SGC_HIP(hipMemcpyAsync(ctx->host_counters, pb->cnt, kCntWords * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
   SGC_HIP(hipStreamSynchronize(s));
-  fold_counters(ctx->host_counters);
   if (int rc = check_unit_overflow(ctx->host_counters, g->m)) return rc;
+  if (staged) {
+    if (out.labels) memcpy(out.labels, stage, n * 4);
+    if (out.core) memcpy(out.core, stage + o_core, n);
+    if (out.sim) memcpy(out.sim, stage + o_sim, m);
+  } else if (!direct) {
+    const hipMemcpyKind kind = out.device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
+    if (out.labels) SGC_HIP(hipMemcpyAsync(out.labels, pb->label, n * 4, kind, s));
+    if (out.core) SGC_HIP(hipMemcpyAsync(out.core, pb->core, n, kind, s));
+    if (out.sim && m) SGC_HIP(hipMemcpyAsync(out.sim, pb->flag, m, kind, s));
+    SGC_HIP(hipStreamSynchronize(s));
+  }
   if (st) {
     memset(st, 0, sizeof(*st));
-    st->ms_prep = elapsed(ctx->ev[0], ctx->ev[1]);
-    st->ms_similarity = elapsed(ctx->ev[1], ctx->ev[2]);
-    st->ms_similarity_large = g->m ? elapsed(ctx->ev[1], ctx->ev[7]) : 0.0;
-    st->ms_core = elapsed(ctx->ev[2], ctx->ev[3]);
-    st->ms_cluster = elapsed(ctx->ev[3], ctx->ev[4]);
-    st->ms_border = elapsed(ctx->ev[4], ctx->ev[5]);
-    st->ms_classify = elapsed(ctx->ev[5], ctx->ev[6]);
-    st->ms_total = elapsed(ctx->ev[0], ctx->ev[6]);
+    st->ms_total = phase_ms(ctx, kStampInit, kStampEnd);
+    if (g->m) {
+      st->ms_prep = phase_ms(ctx, kStampInit, kStampSim);
+      const uint64_t* const t = ctx->host_counters + kCntStamp0;
+      int sim0 = kStampSim;
+      while (sim0 < kStampCore && !t[sim0]) ++sim0;
+      st->ms_similarity = phase_ms(ctx, sim0, kStampCore);
+      // owners of long rows: their filters (if any) and their exact kernel
+      st->ms_similarity_large = phase_ms(ctx, kStampSim, kStampSimRest) + phase_ms(ctx, kStampExactLarge, kStampExactSmall);
+      st->ms_core = phase_ms(ctx, kStampCore, kStampCluster);
+      st->ms_cluster = phase_ms(ctx, kStampCluster, kStampBorder);
+      st->ms_border = phase_ms(ctx, kStampBorder, kStampClassify);
+      st->ms_classify = phase_ms(ctx, kStampClassify, kStampEnd);
+    }
     const uint64_t* c = ctx->host_counters;
     st->edges = g->m / 2;
     st->u_edges = c[kCntUEdges];
@@ -587,14 +644,8 @@ extern "C" int sgc_scan_device(sgc_ctx* ctx, sgc_dgraph* g, double eps, int32_t 
   SGC_HIP(hipSetDevice(ctx->device));
   PassBuffers pb;
   int rc = carve(ctx, g, &pb);
-  if (!rc) rc = run_pass(ctx, g, eps, mu, &pb, st, d_sim != nullptr);
   if (rc) return rc;
-  hipStream_t s = ctx->stream;
-  if (d_labels) SGC_HIP(hipMemcpyAsync(d_labels, pb.label, (size_t)g->n * 4, hipMemcpyDeviceToDevice, s));
-  if (d_core) SGC_HIP(hipMemcpyAsync(d_core, pb.core, g->n, hipMemcpyDeviceToDevice, s));
-  if (d_sim && g->m) SGC_HIP(hipMemcpyAsync(d_sim, pb.flag, g->m, hipMemcpyDeviceToDevice, s));
-  SGC_HIP(hipStreamSynchronize(s));
-  return SGC_OK;
+  return run_pass(ctx, g, eps, mu, &pb, st, PassOut{d_labels, d_core, d_sim, true});
 }
 
 extern "C" int sgc_scan(sgc_ctx* ctx, sgc_dgraph* g, double eps, int32_t mu, int32_t* labels, uint8_t* core,
@@ -605,14 +656,8 @@ extern "C" int sgc_scan(sgc_ctx* ctx, sgc_dgraph* g, double eps, int32_t mu, int
   SGC_HIP(hipSetDevice(ctx->device));
   PassBuffers pb;
   int rc = carve(ctx, g, &pb);
-  if (!rc) rc = run_pass(ctx, g, eps, mu, &pb, st, sim != nullptr);
   if (rc) return rc;
-  hipStream_t s = ctx->stream;
-  if (labels) SGC_HIP(hipMemcpyAsync(labels, pb.label, (size_t)g->n * 4, hipMemcpyDeviceToHost, s));
-  if (core) SGC_HIP(hipMemcpyAsync(core, pb.core, g->n, hipMemcpyDeviceToHost, s));
-  if (sim && g->m) SGC_HIP(hipMemcpyAsync(sim, pb.flag, g->m, hipMemcpyDeviceToHost, s));
-  SGC_HIP(hipStreamSynchronize(s));
-  return SGC_OK;
+  return run_pass(ctx, g, eps, mu, &pb, st, PassOut{labels, core, sim, false});
 }
 
 extern "C" uint64_t sgc_noalloc_max_bytes(void) { return kScratchBytes; }
@@ -639,14 +684,7 @@ extern "C" int sgc_scan_device_noalloc(sgc_ctx* ctx, sgc_dgraph* g, double eps, 
   SGC_HIP(hipSetDevice(ctx->device));
   PassBuffers pb;
   bind_pass((char*)ctx->scratch, L, g, (uint64_t*)ctx->counters.ptr, &pb);
-  int rc = run_pass(ctx, g, eps, mu, &pb, st, d_sim != nullptr);
-  if (rc) return rc;
-  hipStream_t s = ctx->stream;
-  if (d_labels) SGC_HIP(hipMemcpyAsync(d_labels, pb.label, (size_t)g->n * 4, hipMemcpyDeviceToDevice, s));
-  if (d_core) SGC_HIP(hipMemcpyAsync(d_core, pb.core, g->n, hipMemcpyDeviceToDevice, s));
-  if (d_sim && g->m) SGC_HIP(hipMemcpyAsync(d_sim, pb.flag, g->m, hipMemcpyDeviceToDevice, s));
-  SGC_HIP(hipStreamSynchronize(s));
-  return SGC_OK;
+  return run_pass(ctx, g, eps, mu, &pb, st, PassOut{d_labels, d_core, d_sim, true});
 }
 
 extern "C" int sgc_copy_bench(sgc_ctx* ctx, uint64_t bytes, double* ms) {

@@ -218,6 +218,13 @@ __device__ __forceinline__ void count_add(uint64_t* cnt, const int (&slot)[N], c
   __syncthreads();
 }
 
+// The device clock at the start of a phase (the first kernel that sets it
+// counts).
+__device__ __forceinline__ void stamp(uint64_t* cnt, int which) {
+  if (blockIdx.x == 0 && threadIdx.x == 0 && cnt[kCntStamp0 + which] == 0)
+    cnt[kCntStamp0 + which] = (uint64_t)wall_clock64();
+}
+
 // A sum's total, in every lane (whole waves call it).
 __device__ __forceinline__ uint64_t count_total(const uint64_t* cnt, int slot) {
   uint64_t v = lane_id() < kStripes ? cnt[kStripe0 + lane_id() * kStripeSlots + slot] : 0ull;

@@ -624,6 +624,7 @@ __device__ __forceinline__ void emit_unit(const FilterArgs& A, const UnitIO& io,
 // then folded level by level ([w, 2 w) for M = 128 w).
 template <bool LARGE>
 __global__ void __launch_bounds__(LARGE ? 1024 : 256, 8) k_bitmap_units(FilterArgs A, UnitIO io) {
+  stamp(A.cnt, LARGE ? kStampSim : kStampSimRest);
   constexpr uint32_t T = LARGE ? 1024 : 256, TEAM = 16;
   constexpr uint32_t MAXE = LARGE ? kLargeEdges : kSmallEdges;
   // 16-byte words of the largest M: M(46338) = 2^18 bits; 4 M(1024) = 2^14
@@ -756,6 +757,7 @@ __global__ void __launch_bounds__(LARGE ? 1024 : 256, 8) k_bitmap_units(FilterAr
 // Hash filter of the large owners, unit by unit as above.  Bound by the reads
 // of the groups past L2: half of the workgroups take the same time.
 __global__ void __launch_bounds__(1024, 8) k_hash_units(FilterArgs A, UnitIO io) {
+  stamp(A.cnt, kStampSim);
   constexpr uint32_t T = 1024, TEAM = 16, MAXE = kLargeEdges;
   constexpr uint32_t WORDS = 9 * kWindowWords16;
   __shared__ __align__(16) uint32_t filt[WORDS];
@@ -888,6 +890,7 @@ __device__ __noinline__ bool row_contains(const int32_t* __restrict__ adj, uint3
 __global__ void __launch_bounds__(kBlock, 6)
     k_bitmap_wave(FilterArgs A, const uint32_t* __restrict__ wl_b, const uint32_t* __restrict__ wl_e,
                   const uint32_t* __restrict__ wl_k) {
+  stamp(A.cnt, kStampSimRest);
   // 16-byte words of the largest M: 4 M(256) = 2^12 bits; slots of each hash table
   constexpr uint32_t W = kBlock / kWave, TOP = 32, SLOTS = 2 * kWaveRow, SHIFT = 23;
   static_assert(SLOTS == 1u << (32 - SHIFT), "cuckoo hash shift");
@@ -1165,6 +1168,8 @@ void launch_plan_filter(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s
                                                           (uint32_t*)b.lo, b.cnt);
 }
 
+bool filter_leaves_units(const sgc_dgraph* g) { return g->max_degree > std::min(kWaveRow, kWaveEdges); }
+
 void launch_filter(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int cu_count, hipStream_t s) {
   const uint32_t cus = (uint32_t)(cu_count > 0 ? cu_count : 256);
   const PackLayout L = pack_layout(g->m);
@@ -1186,14 +1191,17 @@ void launch_filter(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int 
   const bool coarse = p.eps >= kCoarseEps;
   io.in = b.units + fcap - 1, io.in_step = -1, io.in_count = kCntFUnits2, io.queue = kCntFQueue2;
   io.next = coarse ? hash_units : nullptr;
-  if (coarse) {
+  // kernels whose owners the graph cannot have are not launched (an owner
+  // with more than kWaveEdges edges has a longer row than that)
+  const bool has_large = g->max_degree > kSmallRow, has_small = g->max_degree > std::min(kWaveRow, kWaveEdges);
+  if (coarse && has_large) {
     k_bitmap_units<true><<<cus * 2, 1024, 0, s>>>(A, io);
     io.in = hash_units, io.in_step = 1, io.in_count = kCntHUnits, io.queue = kCntHQueue;
-    io.next = nullptr;
   }
-  k_hash_units<<<cus * 2, 1024, 0, s>>>(A, io);
+  io.next = nullptr;
+  if (has_large) k_hash_units<<<cus * 2, 1024, 0, s>>>(A, io);
   io.in = b.units, io.in_step = 1, io.in_count = kCntFUnits1, io.queue = kCntFQueue1;
-  k_bitmap_units<false><<<cus * 8, 256, 0, s>>>(A, io);
+  if (has_small) k_bitmap_units<false><<<cus * 8, 256, 0, s>>>(A, io);
   const uint64_t want = ((uint64_t)g->n + kBlock / kWave - 1) / (kBlock / kWave), cap = (uint64_t)cus * 6;
   k_bitmap_wave<<<(uint32_t)(want < cap ? want : cap), kBlock, 0, s>>>(A, (const uint32_t*)b.label,
                                                                        (const uint32_t*)b.parent,

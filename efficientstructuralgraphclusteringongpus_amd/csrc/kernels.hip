@@ -184,8 +184,11 @@ __global__ void __launch_bounds__(kBlock) k_init(uint32_t n, uint32_t* __restric
     cnt_u[x] = 0;
     work_u[x] = 0;
   }
-  if (blockIdx.x == 0)
+  if (blockIdx.x == 0) {
     for (uint32_t t = threadIdx.x; t < kCntWords; t += kBlock) cnt[t] = 0;
+    __syncthreads();
+    stamp(cnt, kStampInit);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -197,6 +200,7 @@ __global__ void __launch_bounds__(kBlock) k_init(uint32_t n, uint32_t* __restric
 // append per block iteration.
 __global__ void __launch_bounds__(kBlock) k_list_owned(uint32_t m, const uint8_t* __restrict__ flag,
                                                        uint32_t* __restrict__ list, uint64_t* __restrict__ cnt) {
+  stamp(cnt, kStampSim);
   constexpr uint32_t E = 16;
   unsigned long long* const ctr[1] = {(unsigned long long*)&cnt[kCntDense]};
   const uint64_t tile = (uint64_t)kBlock * E;
@@ -297,7 +301,9 @@ __global__ void __launch_bounds__(kBlock) k_similarity_wave(const uint32_t* __re
 // Similar entries per row, from the flags' similar entries alone: one
 // atomic per run of a row's entries in a wave's 64.
 __global__ void __launch_bounds__(kBlock) k_core_count(uint64_t m, const uint32_t* __restrict__ src,
-                                                       const uint8_t* __restrict__ flag, uint32_t* __restrict__ sd) {
+                                                       const uint8_t* __restrict__ flag, uint32_t* __restrict__ sd,
+                                                       uint64_t* __restrict__ cnt) {
+  stamp(cnt, kStampCore);
   __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
   const uint32_t lane = lane_id(), wv = threadIdx.x / kWave;
   const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * kFlagTile;
@@ -365,7 +371,8 @@ template <bool HEADS>
 __global__ void __launch_bounds__(kBlock) k_union(uint64_t m, const uint32_t* __restrict__ src,
                                                   const int32_t* __restrict__ adj, const uint8_t* __restrict__ flag,
                                                   const uint8_t* __restrict__ core, int32_t* parent,
-                                                  const uint64_t* __restrict__ cnt, int gate) {
+                                                  uint64_t* __restrict__ cnt, int gate) {
+  stamp(cnt, kStampCluster);
   const uint64_t cores = count_total(cnt, kCntMarked);
   if (cores == 0) return;  // no core-core edge to join
   if (HEADS && cores <= kFewCores) return;
@@ -460,15 +467,27 @@ __global__ void __launch_bounds__(kBlock) k_redo_mark(uint32_t m, const uint32_t
 // Borders (GPUSCAN++/GPUScan.cu:654-730): minimum candidate cluster id
 // ---------------------------------------------------------------------------
 
-__global__ void __launch_bounds__(kBlock) k_border(uint64_t m, const uint32_t* __restrict__ src,
+template <bool FLATTEN>
+__global__ void __launch_bounds__(kBlock) k_border(uint32_t n, uint64_t m, int32_t* parent,
+                                                   const uint32_t* __restrict__ src,
                                                    const int32_t* __restrict__ adj, const uint8_t* __restrict__ flag,
                                                    const uint8_t* __restrict__ core, const uint32_t* __restrict__ rb,
                                                    const uint32_t* __restrict__ re, int32_t* label,
                                                    uint64_t* __restrict__ cnt) {
+  stamp(cnt, kStampBorder);
   if (!count_any(cnt, kCntMarked)) return;  // no core: no border
+  // FLATTEN: cluster ids of the cores too (roots go to label, as k_flatten
+  // does for larger graphs); the edges below then find a core's root themselves
+  if (FLATTEN) {
+    PhaseView f{};
+    f.core = const_cast<uint8_t*>(core), f.parent = parent, f.label = label;
+    const uint64_t stride = (uint64_t)gridDim.x * kBlock;
+    for (uint64_t x = (uint64_t)blockIdx.x * kBlock + threadIdx.x; x < n; x += stride) flatten_vertex(f, (uint32_t)x);
+  }
   __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
   PhaseView v{};
   v.src = src, v.adj = adj, v.core = const_cast<uint8_t*>(core), v.rb = rb, v.re = re, v.label = label;
+  v.parent = parent;
   const uint32_t lane = lane_id(), wv = threadIdx.x / kWave;
   const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * kFlagTile;
   // entries of the border rows this lane labels first; the core rows'
@@ -478,7 +497,7 @@ __global__ void __launch_bounds__(kBlock) k_border(uint64_t m, const uint32_t* _
     const uint32_t total = similar_tile(flag, m, base, s_at[wv]);
     for (uint32_t i0 = 0; i0 < total; i0 += kWave) {
       const bool on = i0 + lane < total;
-      labeled += border_entry(v, base + (on ? s_at[wv][i0 + lane] : 0), on);
+      labeled += border_entry<FLATTEN>(v, base + (on ? s_at[wv][i0 + lane] : 0), on);
     }
     wave_lds_sync();  // the list is rewritten
   }
@@ -500,8 +519,9 @@ __device__ __forceinline__ bool classify_from_labeled(const uint64_t* cnt, uint6
 __global__ void __launch_bounds__(kBlock) k_classify(uint32_t m, uint64_t m_all, const uint32_t* __restrict__ src,
                                                      const int32_t* __restrict__ adj,
                                                      const int32_t* __restrict__ label, int32_t* __restrict__ lo,
-                                                     int32_t* __restrict__ hi, const uint64_t* __restrict__ cnt,
+                                                     int32_t* __restrict__ hi, uint64_t* __restrict__ cnt,
                                                      bool listed) {
+  stamp(cnt, kStampClassify);
   // no core means no label anywhere: lo and hi keep their initial values
   if (!count_any(cnt, kCntMarked)) return;
   PhaseView v{};
@@ -524,6 +544,7 @@ __global__ void __launch_bounds__(kBlock) k_label_pieces(uint32_t n, uint64_t m,
                                                          const uint32_t* __restrict__ re,
                                                          const int32_t* __restrict__ label, uint2* __restrict__ piece,
                                                          uint64_t* __restrict__ cnt) {
+  stamp(cnt, kStampClassify);
   if (!count_any(cnt, kCntMarked) || !classify_from_labeled(cnt, m)) return;
   constexpr uint32_t V = 8;
   unsigned long long* const ctr[1] = {(unsigned long long*)&cnt[kCntPieces]};
@@ -593,6 +614,38 @@ __global__ void __launch_bounds__(kBlock) k_finalize(uint32_t n, int32_t mu, con
   for (uint64_t x = (uint64_t)blockIdx.x * kBlock + threadIdx.x; x < n; x += stride)
     finalize_vertex(v, (uint32_t)x, mu, &rc);
   count_roles(cnt, rc);
+}
+
+// Copies `bytes` bytes by the whole grid: 16 at a time where both ends allow
+// it.
+__device__ __forceinline__ void grid_copy(const void* __restrict__ from, void* __restrict__ to, uint64_t bytes) {
+  const uint64_t at = (uint64_t)blockIdx.x * kBlock + threadIdx.x, stride = (uint64_t)gridDim.x * kBlock;
+  uint64_t done = 0;
+  if ((((uintptr_t)from | (uintptr_t)to) & 15) == 0) {
+    const uint64_t v = bytes / 16;
+    for (uint64_t i = at; i < v; i += stride) ((uint4*)to)[i] = ((const uint4*)from)[i];
+    done = v * 16;
+  }
+  for (uint64_t i = done + at; i < bytes; i += stride) ((uint8_t*)to)[i] = ((const uint8_t*)from)[i];
+}
+
+__global__ void __launch_bounds__(kBlock) k_publish(uint32_t n, uint64_t m, uint64_t* cnt, uint64_t* host_cnt,
+                                                    const int32_t* label, const uint8_t* core, const uint8_t* flag,
+                                                    int32_t* to_label, uint8_t* to_core, uint8_t* to_sim) {
+  stamp(cnt, kStampEnd);
+  if (blockIdx.x == 0) {
+    __syncthreads();
+    if (threadIdx.x < kCntSlots) {
+      uint64_t v = cnt[threadIdx.x];
+      if (threadIdx.x < kStripeSlots)
+        for (uint32_t i = 0; i < kStripes; ++i) v += cnt[kStripe0 + i * kStripeSlots + threadIdx.x];
+      host_cnt[threadIdx.x] = v;
+    }
+  }
+  if (cnt[kCntOverflow]) return;
+  if (to_label) grid_copy(label, to_label, (uint64_t)n * 4);
+  if (to_core) grid_copy(core, to_core, n);
+  if (to_sim) grid_copy(flag, to_sim, m);
 }
 
 // Plain streaming copy (16 bytes per lane per step), the reference point for
@@ -691,7 +744,7 @@ static uint32_t flag_grid(uint64_t m) { return std::min(grid_for(m, kFlagTile * 
 // Edge passes take the entries [0, g->m) of g (a whole graph or one chip of
 // rows); vertex passes cover all g->n vertices.
 void launch_core_count(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s) {
-  if (g->m) k_core_count<<<flag_grid(g->m), kBlock, 0, s>>>(g->m, g->src, b.flag, b.sd);
+  if (g->m) k_core_count<<<flag_grid(g->m), kBlock, 0, s>>>(g->m, g->src, b.flag, b.sd, b.cnt);
 }
 
 void launch_core_mark(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStream_t s,
@@ -720,11 +773,17 @@ void launch_flatten(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s) {
   k_flatten<<<grid_for(g->n, kBlock), kBlock, 0, s>>>(g->n, b.core, b.parent, b.label);
 }
 
-void launch_border(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s) {
-  if (g->m)
-    k_border<<<flag_grid(g->m), kBlock, 0, s>>>(g->m, g->src, g->adj, b.flag, b.core, g->row_begin, g->row_end, b.label,
-                                                b.cnt);
+void launch_border(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s, bool flatten) {
+  if (!g->m) return;
+  if (flatten)
+    k_border<true><<<std::max(flag_grid(g->m), std::min(grid_for(g->n, kBlock), 1024u)), kBlock, 0, s>>>(
+        g->n, g->m, b.parent, g->src, g->adj, b.flag, b.core, g->row_begin, g->row_end, b.label, b.cnt);
+  else
+    k_border<false><<<flag_grid(g->m), kBlock, 0, s>>>(g->n, g->m, b.parent, g->src, g->adj, b.flag, b.core,
+                                                       g->row_begin, g->row_end, b.label, b.cnt);
 }
+
+bool small_graph(const sgc_dgraph* g) { return g->m < kSmallGraph; }
 
 void launch_classify_edges(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s, uint64_t m_all) {
   if (!g->m) return;
@@ -747,14 +806,16 @@ void launch_finalize(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hi
 }
 
 
+void launch_publish(const sgc_dgraph* g, const PassBuffers& b, uint64_t* host_cnt, int32_t* labels, uint8_t* core,
+                    uint8_t* sim, hipStream_t s) {
+  const uint64_t bytes = (labels ? (uint64_t)g->n * 4 : 0) + (core ? g->n : 0) + (sim ? g->m : 0);
+  k_publish<<<std::min(grid_for(bytes / 16, kBlock), 2048u), kBlock, 0, s>>>(g->n, g->m, b.cnt, host_cnt, b.label,
+                                                                             b.core, b.flag, labels, core, sim);
+}
+
 void launch_core(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStream_t s) {
   launch_core_count(g, b, s);
   launch_core_mark(g, b, p, s);
-}
-
-void launch_cluster(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s) {
-  launch_union(g, b, s);
-  launch_flatten(g, b, s);
 }
 
 void launch_classify(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStream_t s) {

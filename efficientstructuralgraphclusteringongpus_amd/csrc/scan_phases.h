@@ -140,14 +140,15 @@ __device__ __forceinline__ void flatten_vertex(const PhaseView& v, uint32_t x) {
 // for one similar entry k per lane (on; ascending over the lanes).  A row's
 // candidates may lie in several runs of lanes (other entries between them get
 // a marker row), each run's minimum is added.  Returns the entries of the
-// border rows this lane labelled first (rows known only).  All 64 lanes must
-// call it.
+// border rows this lane labelled first (rows known only).  FIND: the cores'
+// cluster ids are not in label yet.  All 64 lanes must call it.
+template <bool FIND>
 __device__ __forceinline__ uint32_t border_entry(const PhaseView& v, uint64_t k, bool on) {
   const uint32_t row = on ? v.src[k] : 0xFFFFFFFFu;
   const int32_t c = on ? v.adj[k] : 0;
   const bool y = on && v.core[c] && !v.core[row];
   if (!__ballot(y)) return 0;
-  const int32_t cand = y ? v.label[c] : kNoLabel;
+  const int32_t cand = !y ? kNoLabel : FIND ? uf_find(v.parent, c) : v.label[c];
   const uint32_t r = y ? row : 0xFFFFFFFFu;
   const int32_t best = wave_seg_reduce(r, cand, OpMin());
   if (wave_seg_head(r) && best != kNoLabel && atomicMin(&v.label[r], best) == kNoLabel && v.rb)

@@ -736,6 +736,7 @@ __global__ void __launch_bounds__(T::kThreads, T::kMinWaves)
                 const uint4* __restrict__ uedge, const uint4* __restrict__ units, uint32_t ucap,
                 uint64_t* __restrict__ cnt, int units_slot, int queue_slot, bool hash_tables,
                 uint8_t* __restrict__ vstate, uint32_t* __restrict__ ny, uint32_t* __restrict__ nn, int32_t mu) {
+  stamp(cnt, T::kBitmap ? kStampExactLarge : kStampExactSmall);
   __shared__ __align__(16) uint32_t tab[T::kTableWords];
   __shared__ unsigned long long e_state[T::kMaxEdges];  // hits << 32 | consumed
   // (c*, d(a), claim cap, slice end) of each edge: what a wave needs to size
@@ -1262,7 +1263,13 @@ void launch_similarity(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, 
   const bool filtered = filter_stage(g, p) && !cn_out;
   const uint32_t half = filtered ? b.ucap / 2 : 0, ucap = b.ucap - half;
   const uint4* const units = b.units + half;
-  if (filtered) launch_filter(g, b, p, cu_count, s);
+  if (filtered) {
+    launch_filter(g, b, p, cu_count, s);
+    if (!filter_leaves_units(g)) {
+      if (mid) (void)hipEventRecord(mid, s);
+      return;
+    }
+  }
   // the core-check pruning runs in the workgroup tier, which launches first
   // and holds the long rows; the later tiers decide every edge they own
   const bool prune = p.prune && !cn_out && g->mirror;

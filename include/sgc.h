@@ -215,8 +215,10 @@ uint64_t sgc_dgraph_m(const sgc_dgraph* dg);
 /* ------------------------------------------------------------------------ */
 
 typedef struct {
-  /* Device time from resident CSR to resident labels, hipEvent-timed on the
-   * context stream, and its phases. */
+  /* Device time from resident CSR to resident labels and its phases, by the
+   * device clock from each phase's first kernel to the next one's.  In a pass
+   * over a small graph the cores' cluster ids are written with the borders
+   * (ms_border). */
   double ms_total;
   double ms_prep;       /* orientation + degree-only pre-decision */
   double ms_similarity; /* common-neighbour kernels */
