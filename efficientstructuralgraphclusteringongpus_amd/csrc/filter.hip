@@ -333,7 +333,9 @@ constexpr double kCoarseEps = 0.27;
 
 // Units of the workgroup and large filters (small from the front of funits,
 // large from the back) and the wave list.  A unit's edges are capped so that
-// a small graph still gives every workgroup slot several units.
+// a small graph still gives every workgroup slot several units; below 96
+// edges a unit's row load and empty lanes cost more than the balance gives
+// (at least 32 / 96 edges: R-MAT-14 177 / 151 us, R-MAT-16 250 / 246).
 __global__ void __launch_bounds__(kBlock) k_plan_filter(uint32_t n, const uint32_t* __restrict__ rb,
                                                         const uint32_t* __restrict__ re,
                                                         const uint32_t* __restrict__ cnt_u,
@@ -347,7 +349,7 @@ __global__ void __launch_bounds__(kBlock) k_plan_filter(uint32_t n, const uint32
     if (blockIdx.x == 0 && threadIdx.x == 0) cnt[kCntOverflow] = owned_all;
     return;
   }
-  const uint32_t cap_s = (uint32_t)min((uint64_t)kSmallEdges, max((uint64_t)32, owned_all / 8192));
+  const uint32_t cap_s = (uint32_t)min((uint64_t)kSmallEdges, max((uint64_t)96, owned_all / 8192));
   const uint32_t cap_l = (uint32_t)min((uint64_t)kLargeEdges, max((uint64_t)64, owned_all / 2048));
   unsigned long long* const ctr[3] = {(unsigned long long*)&cnt[kCntFUnits1], (unsigned long long*)&cnt[kCntFUnits2],
                                       (unsigned long long*)&cnt[kCntTiny]};
@@ -1180,7 +1182,7 @@ void launch_filter(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int 
                      b.uedge,  b.flag,
                      b.cnt};
   // Units of owners above kWaveRow entries: fewer than m / 50 of each kind
-  // (an owner has its row's entries, a unit 32 edges unless it is an owner's
+  // (an owner has its row's entries, a unit 64 edges unless it is an owner's
   // last), so each of the four lists has room in an eighth of the array.
   const uint32_t fcap = b.ucap / 2;
   UnitIO io;
