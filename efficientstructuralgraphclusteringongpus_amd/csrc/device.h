@@ -102,7 +102,11 @@ enum SimImpl { kSimTiered = 0, kSimWavePerEdge = 1 };
 // 246 us through two pageable copies, 215 staged).
 constexpr size_t kStageBytes = 512u << 10;
 
-// Grow-only device allocation owned by a context.
+// Page-locked staging of a context: kBounces buffers of kBounceBytes.
+constexpr int kBounces = 4;
+constexpr size_t kBounceBytes = 8u << 20;
+
+// Grow-only device (or page-locked host) allocation owned by a context.
 struct DevBuf {
   void* ptr = nullptr;
   size_t bytes = 0;
@@ -123,10 +127,12 @@ struct sgc_ctx {
   hipEvent_t ev[8] = {};
   int sim_impl = sgc::kSimTiered;
   void* scratch = nullptr;  // this GPU's static scratch (sgc_scan_device_noalloc)
-  // page-locked staging for graph uploads from pageable memory (two
-  // buffers, allocated at the first such upload and kept until destroy)
-  void* bounce[2] = {nullptr, nullptr};
-  hipEvent_t bounce_done[2] = {nullptr, nullptr};
+  // page-locked staging for copies from and to pageable memory (one
+  // allocation of sgc::kBounces buffers, made at the first such copy and
+  // kept until destroy)
+  char* bounce = nullptr;
+  hipEvent_t bounce_done[sgc::kBounces] = {};
+  sgc::DevBuf host_work;    // page-locked work memory of out-of-core passes
   bool prune = false;       // core-check pruning in passes that return no similarity flags (sgc_ctx_set_pruning)
 };
 
@@ -187,6 +193,9 @@ struct sgc_dgraph {
   // and hash groups, 9 bytes per entry); graphs of a serving engine, and
   // uploads without room, have none (null).
   char* packed = nullptr;
+  // the allocations that hold the arrays above: one for all of them, or,
+  // where that much was not free in one piece, one for each that was
+  void* blocks[5] = {};
 };
 
 namespace sgc {
@@ -251,6 +260,28 @@ inline size_t unit_capacity(uint64_t m) { return (size_t)(m / 2) + 2; }
 // some entry has no reverse entry.  SGC_OK otherwise.
 int check_unit_overflow(const uint64_t* cnt_host, uint64_t m);
 
+// The context's work buffer grown to at least `bytes`, or null when the
+// device has not that much.
+void* work_memory(sgc_ctx* ctx, size_t bytes);
+// At least `bytes` of page-locked host memory, the context's until
+// release_host_work; null when the system will not lock that much.
+void* host_work_memory(sgc_ctx* ctx, size_t bytes);
+// Gives that memory back if it is more than a context keeps.
+void release_host_work(sgc_ctx* ctx);
+// Copies between host memory and the device on the context stream.  Pageable
+// memory goes through the context's page-locked staging, chunk by chunk, the
+// host's share of one chunk overlapping the transfer of the others.  A
+// pageable source or destination is done with on return; a page-locked one
+// when the stream is.
+hipError_t upload_bytes(sgc_ctx* ctx, void* dst, const void* src, size_t bytes, bool src_pinned);
+struct HostCopy {
+  void* dst;
+  const void* src;
+  size_t bytes;
+};
+// Device to host; every copy is done on return.
+hipError_t download(sgc_ctx* ctx, const HostCopy* copies, int count);
+
 // Uploads g; `scans`: also builds what only one-shot passes read (the packed
 // rows of the filter stage).
 int upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgraph** out);
@@ -262,9 +293,10 @@ void launch_fill_src(const sgc_dgraph* g, hipStream_t s);
 // without a reverse entry get 0xFFFFFFFF
 void launch_mirror(const sgc_dgraph* g, hipStream_t s);
 // fills g->mirror (after launch_fill_src) by a stable sort of the entries by
-// neighbour, or by launch_mirror where the input is not symmetric or the
-// sort's memory is not there; synchronises the stream
-hipError_t build_mirror(const sgc_dgraph* g, hipStream_t s);
+// neighbour in the context's work buffer, or by launch_mirror where the input
+// is not symmetric or the buffer's memory is not there; synchronises the
+// stream
+hipError_t build_mirror(sgc_ctx* ctx, const sgc_dgraph* g);
 // fills g->ndeg
 void launch_neighbor_degrees(const sgc_dgraph* g, hipStream_t s);
 // 2^20-id windows of the large-tier bitmap covering n ids, and the kernel
@@ -275,10 +307,12 @@ uint32_t window_count(uint32_t n);
 // that is at most max(16 m, 1 GiB) bytes (four times the adjacency); else 0.
 uint64_t window_index_bytes(uint64_t n, uint64_t m);
 void launch_window_offsets(const sgc_dgraph* g, hipStream_t s);
-// Compact row copies (filter.hip), after the reverse-entry and
-// neighbour-degree indexes; leaves g without them when there is no room.
-// Synchronises the stream.
-hipError_t build_packed_rows(sgc_dgraph* g, hipStream_t s);
+// Bytes of the compact row copies (filter.hip) of m entries, and the kernels
+// that write them, after the reverse-entry and neighbour-degree indexes;
+// they use the context's work buffer and leave g without the copies when its
+// memory is not there.
+size_t packed_bytes(uint64_t m);
+hipError_t build_packed_rows(sgc_ctx* ctx, sgc_dgraph* g);
 // Whether a pass runs the filter stage: its plan then comes from
 // launch_plan_filter, and launch_filter leaves the survivors as the exact
 // kernels' units.

@@ -173,10 +173,10 @@ extern "C" void sgc_ctx_destroy(sgc_ctx* ctx) {
   if (ctx->work.ptr) (void)hipFree(ctx->work.ptr);
   if (ctx->counters.ptr) (void)hipFree(ctx->counters.ptr);
   if (ctx->host_counters) (void)hipHostFree(ctx->host_counters);
-  for (int i = 0; i < 2; ++i) {
-    if (ctx->bounce[i]) (void)hipHostFree(ctx->bounce[i]);
-    if (ctx->bounce_done[i]) (void)hipEventDestroy(ctx->bounce_done[i]);
-  }
+  if (ctx->bounce) (void)hipHostFree(ctx->bounce);
+  for (auto& e : ctx->bounce_done)
+    if (e) (void)hipEventDestroy(e);
+  if (ctx->host_work.ptr) (void)hipHostFree(ctx->host_work.ptr);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
 }
@@ -219,50 +219,137 @@ extern "C" int sgc_ctx_set_pruning(sgc_ctx* ctx, int enable) {
 }
 
 namespace {
-constexpr size_t kBounceBytes = 64u << 20;
 
-// Host-to-device copy on the context stream.  A pageable source goes through
-// the context's two page-locked buffers: the next chunk is copied in while
-// the previous one is sent (the runtime's own staging of a pageable copy
-// runs about a third slower).  The buffers are free again on return.
-hipError_t upload_bytes(sgc_ctx* ctx, void* dst, const void* src, size_t bytes, bool src_pinned) {
-  if (!bytes) return hipSuccess;
-  if (!src_pinned && !ctx->bounce[0]) {
-    bool ok = true;
-    for (int i = 0; i < 2 && ok; ++i)
-      ok = hipHostMalloc(&ctx->bounce[i], kBounceBytes) == hipSuccess &&
-           hipEventCreateWithFlags(&ctx->bounce_done[i], hipEventDisableTiming) == hipSuccess;
-    if (!ok) {  // the runtime stages the copy instead
-      (void)hipGetLastError();
-      for (int i = 0; i < 2; ++i) {
-        if (ctx->bounce[i]) (void)hipHostFree(ctx->bounce[i]);
-        if (ctx->bounce_done[i]) (void)hipEventDestroy(ctx->bounce_done[i]);
-        ctx->bounce[i] = nullptr;
-        ctx->bounce_done[i] = nullptr;
-      }
-    }
+// The context's page-locked staging, allocated on first use; null when the
+// system will not lock it (the runtime stages the copies instead).
+char* bounce_buffers(sgc_ctx* ctx) {
+  if (ctx->bounce) return ctx->bounce;
+  void* p = nullptr;
+  bool ok = hipHostMalloc(&p, kBounces * kBounceBytes) == hipSuccess;
+  for (int i = 0; i < kBounces && ok; ++i)
+    if (!ctx->bounce_done[i]) ok = hipEventCreateWithFlags(&ctx->bounce_done[i], hipEventDisableTiming) == hipSuccess;
+  if (!ok) {
+    (void)hipGetLastError();
+    if (p) (void)hipHostFree(p);
+    return nullptr;
   }
-  if (src_pinned || !ctx->bounce[0]) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream);
-  bool used[2] = {false, false};
+  ctx->bounce = (char*)p;
+  return ctx->bounce;
+}
+
+// Waits for the transfers issued from or to the staging buffers.
+hipError_t bounce_wait(sgc_ctx* ctx, const bool* used) {
   hipError_t e = hipSuccess;
-  for (size_t off = 0, i = 0; off < bytes && e == hipSuccess; off += kBounceBytes, ++i) {
-    const int b = (int)(i & 1);
-    const size_t len = std::min(kBounceBytes, bytes - off);
-    if (used[b]) e = hipEventSynchronize(ctx->bounce_done[b]);  // its last chunk is on the device
-    if (e != hipSuccess) break;
-    parallel_copy(ctx->bounce[b], (const char*)src + off, len);
-    e = hipMemcpyAsync((char*)dst + off, ctx->bounce[b], len, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) e = hipEventRecord(ctx->bounce_done[b], ctx->stream);
-    used[b] = true;
-  }
-  for (int b = 0; b < 2; ++b)
+  for (int b = 0; b < kBounces; ++b)
     if (used[b]) {
       const hipError_t w = hipEventSynchronize(ctx->bounce_done[b]);
       if (e == hipSuccess) e = w;
     }
   return e;
 }
+
+bool host_pinned(const void* p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeHost;
+}
 }  // namespace
+
+hipError_t sgc::upload_bytes(sgc_ctx* ctx, void* dst, const void* src, size_t bytes, bool src_pinned) {
+  if (!bytes) return hipSuccess;
+  char* const ring = src_pinned ? nullptr : bounce_buffers(ctx);
+  if (!ring) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream);
+  bool used[kBounces] = {};
+  hipError_t e = hipSuccess;
+  for (size_t off = 0, i = 0; off < bytes && e == hipSuccess; off += kBounceBytes, ++i) {
+    const int b = (int)(i % kBounces);
+    const size_t len = std::min(kBounceBytes, bytes - off);
+    if (used[b]) e = hipEventSynchronize(ctx->bounce_done[b]);  // its last chunk is on the device
+    if (e != hipSuccess) break;
+    parallel_copy(ring + b * kBounceBytes, (const char*)src + off, len);
+    e = hipMemcpyAsync((char*)dst + off, ring + b * kBounceBytes, len, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) e = hipEventRecord(ctx->bounce_done[b], ctx->stream);
+    used[b] = true;
+  }
+  const hipError_t w = bounce_wait(ctx, used);
+  return e != hipSuccess ? e : w;
+}
+
+hipError_t sgc::download(sgc_ctx* ctx, const HostCopy* copies, int count) {
+  hipStream_t s = ctx->stream;
+  struct Chunk {
+    char* dst;
+    size_t bytes;
+  } held[kBounces];
+  bool used[kBounces] = {};
+  hipError_t e = hipSuccess;
+  size_t i = 0;
+  // the chunk in buffer b goes to its destination
+  auto drain = [&](int b) {
+    const hipError_t w = hipEventSynchronize(ctx->bounce_done[b]);
+    used[b] = false;
+    if (w == hipSuccess) parallel_copy(held[b].dst, ctx->bounce + b * kBounceBytes, held[b].bytes);
+    return w;
+  };
+  for (int c = 0; c < count && e == hipSuccess; ++c) {
+    const HostCopy& h = copies[c];
+    if (!h.bytes || !h.dst) continue;
+    char* const ring = host_pinned(h.dst) ? nullptr : bounce_buffers(ctx);
+    if (!ring) {
+      e = hipMemcpyAsync(h.dst, h.src, h.bytes, hipMemcpyDeviceToHost, s);
+      continue;
+    }
+    for (size_t off = 0; off < h.bytes && e == hipSuccess; off += kBounceBytes, ++i) {
+      const int b = (int)(i % kBounces);
+      if (used[b]) e = drain(b);
+      if (e != hipSuccess) break;
+      held[b] = Chunk{(char*)h.dst + off, std::min(kBounceBytes, h.bytes - off)};
+      e = hipMemcpyAsync(ring + b * kBounceBytes, (const char*)h.src + off, held[b].bytes, hipMemcpyDeviceToHost, s);
+      if (e == hipSuccess) e = hipEventRecord(ctx->bounce_done[b], s);
+      used[b] = e == hipSuccess;
+    }
+  }
+  for (int k = 0; k < kBounces; ++k, ++i)
+    if (used[i % kBounces]) {
+      const hipError_t w = drain((int)(i % kBounces));
+      if (e == hipSuccess) e = w;
+    }
+  const hipError_t w = hipStreamSynchronize(s);
+  return e != hipSuccess ? e : w;
+}
+
+void* sgc::work_memory(sgc_ctx* ctx, size_t bytes) {
+  if (ensure(ctx->work, bytes) == SGC_OK) return ctx->work.ptr;
+  clear_error();
+  return nullptr;
+}
+
+// Page-locked work memory a context keeps between out-of-core passes.
+constexpr size_t kHostWorkKept = 256u << 20;
+
+void* sgc::host_work_memory(sgc_ctx* ctx, size_t bytes) {
+  DevBuf& b = ctx->host_work;
+  if (b.bytes >= bytes) return b.ptr;
+  if (b.ptr) (void)hipHostFree(b.ptr);
+  b = DevBuf();
+  if (hipHostMalloc(&b.ptr, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    b.ptr = nullptr;
+    return nullptr;
+  }
+  b.bytes = bytes;
+  return b.ptr;
+}
+
+void sgc::release_host_work(sgc_ctx* ctx) {
+  DevBuf& b = ctx->host_work;
+  if (b.bytes <= kHostWorkKept) return;
+  (void)hipHostFree(b.ptr);
+  b = DevBuf();
+}
 
 extern "C" int sgc_dgraph_upload(sgc_ctx* ctx, const sgc_host_graph* g, sgc_dgraph** out) {
   return upload_graph(ctx, g, true, out);
@@ -285,60 +372,64 @@ int sgc::upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgr
   narrow_row_ptr(g, rp32.data(), &maxd);
   d->max_degree = (uint32_t)maxd;
   auto cleanup = [d]() {
-    if (d->mirror) (void)hipFree(d->mirror);
-    if (d->ndeg) (void)hipFree(d->ndeg);
-    if (d->woff) (void)hipFree(d->woff);
-    if (d->packed) (void)hipFree(d->packed);
-    if (d->row_ptr) (void)hipFree(d->row_ptr);
-    if (d->adj) (void)hipFree(d->adj);
-    if (d->src) (void)hipFree(d->src);
+    for (void* p : d->blocks)
+      if (p) (void)hipFree(p);
     delete d;
   };
-  const size_t m_bytes = std::max<size_t>(g->m, 1) * 4;
-  if (hipMalloc(&d->row_ptr, (g->n + 1) * 4) != hipSuccess || hipMalloc(&d->adj, m_bytes) != hipSuccess ||
-      hipMalloc(&d->src, m_bytes) != hipSuccess) {
+  // What a graph keeps: its CSR with each entry's row; then, where there is
+  // room, the reverse-entry index (without it the similarity kernels search
+  // the second entry of an edge), the neighbour degrees (the prep kernel
+  // gathers them), the window-offset index (the kernels find window
+  // boundaries while streaming; it grows with n^2: R-MAT-26 at edge factor 16
+  // needs 17 GB, twice its adjacency, and a pass there runs 2.5 times faster
+  // with it) and the filter stages' compact rows (every edge goes to the
+  // exact kernels).  One allocation for all: seven of them cost an upload of
+  // R-MAT-20 and its release 1.9 ms, one 0.6.
+  const size_t rp_bytes = align_up((g->n + 1) * 4, 256), m_bytes = align_up(std::max<size_t>(g->m, 1) * 4, 256);
+  const size_t need[5] = {rp_bytes + 2 * m_bytes, g->m ? m_bytes : 0, g->m ? m_bytes : 0,
+                          align_up(window_index_bytes(d->n, g->m), 256), scans && g->m ? packed_bytes(g->m) : 0};
+  char* at[5] = {};
+  if (hipMalloc(&d->blocks[0], need[0] + need[1] + need[2] + need[3] + need[4]) == hipSuccess) {
+    char* p = (char*)d->blocks[0];
+    for (int i = 0; i < 5; p += need[i++]) at[i] = need[i] ? p : nullptr;
+  } else {
     (void)hipGetLastError();
-    cleanup();
-    return fail(SGC_ENOMEM, "device allocation for graph (n=%llu, m=%llu) failed", (unsigned long long)g->n,
-                (unsigned long long)g->m);
-  }
-  d->row_begin = d->row_ptr;
-  d->row_end = d->row_ptr + 1;
-  // reverse-entry index: the similarity kernels write both entries of an
-  // edge without searching for the second
-  if (g->m && hipMalloc(&d->mirror, m_bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    d->mirror = nullptr;  // the kernels find the reverse entry themselves
-  }
-  // neighbour degrees, streamed by the prep kernel on every pass
-  if (g->m && hipMalloc(&d->ndeg, m_bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    d->ndeg = nullptr;  // the prep kernel gathers them
-  }
-  // window-offset index when there is more than one window and it takes at
-  // most four times the adjacency's bytes (it grows with n^2: R-MAT-26 at
-  // edge factor 16 needs 17 GB, twice its adjacency, and a pass there runs
-  // 2.5 times faster with it)
-  const uint64_t woff_bytes = window_index_bytes(d->n, g->m);
-  if (woff_bytes) {
-    if (hipMalloc(&d->woff, woff_bytes) == hipSuccess) {
-      d->wcount = window_count(d->n);
-    } else {
-      (void)hipGetLastError();
-      d->woff = nullptr;  // the kernels find window boundaries while streaming instead
+    for (int i = 0; i < 5; ++i) {
+      d->blocks[i] = nullptr;
+      if (need[i] && hipMalloc(&d->blocks[i], need[i]) != hipSuccess) {
+        (void)hipGetLastError();
+        d->blocks[i] = nullptr;
+        if (i) continue;
+        cleanup();
+        return fail(SGC_ENOMEM, "device allocation for graph (n=%llu, m=%llu) failed", (unsigned long long)g->n,
+                    (unsigned long long)g->m);
+      }
+      at[i] = (char*)d->blocks[i];
     }
   }
+  d->row_ptr = (uint32_t*)at[0];
+  d->adj = (int32_t*)(at[0] + rp_bytes);
+  d->src = (uint32_t*)(at[0] + rp_bytes + m_bytes);
+  d->row_begin = d->row_ptr;
+  d->row_end = d->row_ptr + 1;
+  d->mirror = (uint32_t*)at[1];
+  d->ndeg = (uint32_t*)at[2];
+  d->woff = (uint32_t*)at[3];
+  if (d->woff) d->wcount = window_count(d->n);
+  d->packed = at[4];
+  // the indexes are built in the buffer a pass works in, sized for that at once
+  (void)work_memory(ctx, pass_layout(d).bytes);
   hipError_t e = upload_bytes(ctx, d->row_ptr, rp32.data(), (g->n + 1) * 4, false);
   if (e == hipSuccess && g->m) e = upload_bytes(ctx, d->adj, g->adj, g->m * 4, g->pinned);
   if (e == hipSuccess) {
     launch_fill_src(d, ctx->stream);
-    e = build_mirror(d, ctx->stream);
+    e = build_mirror(ctx, d);
   }
   if (e == hipSuccess) {
     launch_neighbor_degrees(d, ctx->stream);
     launch_window_offsets(d, ctx->stream);
     e = hipGetLastError();
-    if (e == hipSuccess && scans) e = build_packed_rows(d, ctx->stream);
+    if (e == hipSuccess) e = build_packed_rows(ctx, d);
   }
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) {
@@ -353,13 +444,8 @@ extern "C" void sgc_dgraph_free(sgc_dgraph* d) {
   if (!d) return;
   (void)hipSetDevice(d->ctx->device);
   (void)hipStreamSynchronize(d->ctx->stream);
-  if (d->mirror) (void)hipFree(d->mirror);
-  if (d->ndeg) (void)hipFree(d->ndeg);
-  if (d->woff) (void)hipFree(d->woff);
-  if (d->packed) (void)hipFree(d->packed);
-  if (d->row_ptr) (void)hipFree(d->row_ptr);
-  if (d->adj) (void)hipFree(d->adj);
-  if (d->src) (void)hipFree(d->src);
+  for (void* p : d->blocks)
+    if (p) (void)hipFree(p);
   delete d;
 }
 
@@ -480,11 +566,14 @@ int run_pass(sgc_ctx* ctx, sgc_dgraph* g, double eps, int32_t mu, PassBuffers* p
     if (out.core) memcpy(out.core, stage + o_core, n);
     if (out.sim) memcpy(out.sim, stage + o_sim, m);
   } else if (!direct) {
-    const hipMemcpyKind kind = out.device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
-    if (out.labels) SGC_HIP(hipMemcpyAsync(out.labels, pb->label, n * 4, kind, s));
-    if (out.core) SGC_HIP(hipMemcpyAsync(out.core, pb->core, n, kind, s));
-    if (out.sim && m) SGC_HIP(hipMemcpyAsync(out.sim, pb->flag, m, kind, s));
-    SGC_HIP(hipStreamSynchronize(s));
+    const HostCopy copies[3] = {{out.labels, pb->label, n * 4}, {out.core, pb->core, n}, {out.sim, pb->flag, m}};
+    if (!out.device) {
+      SGC_HIP(download(ctx, copies, 3));
+    } else {
+      for (const HostCopy& c : copies)
+        if (c.dst && c.bytes) SGC_HIP(hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyDeviceToDevice, s));
+      SGC_HIP(hipStreamSynchronize(s));
+    }
   }
   if (st) {
     memset(st, 0, sizeof(*st));

@@ -1130,17 +1130,19 @@ PackLayout pack_layout(uint64_t m) {
 
 }  // namespace
 
-hipError_t build_packed_rows(sgc_dgraph* g, hipStream_t s) {
-  if (!g->m || !g->mirror || !g->ndeg) return hipSuccess;
+size_t packed_bytes(uint64_t m) { return pack_layout(m).bytes; }
+
+hipError_t build_packed_rows(sgc_ctx* ctx, sgc_dgraph* g) {
+  if (!g->packed) return hipSuccess;
+  hipStream_t s = ctx->stream;
   const uint32_t n = g->n, m = g->m;
   const PackLayout L = pack_layout(m);
-  char *mem = nullptr, *out = nullptr;
-  if (hipMalloc(&out, L.bytes) != hipSuccess || hipMalloc(&mem, L.tmp_bytes) != hipSuccess) {
-    (void)hipGetLastError();  // no room: every edge goes to the exact kernels
-    if (out) (void)hipFree(out);
+  char* const mem = g->mirror && g->ndeg ? (char*)work_memory(ctx, L.tmp_bytes) : nullptr;
+  if (!mem) {  // every edge goes to the exact kernels
+    g->packed = nullptr;
     return hipSuccess;
   }
-  g->packed = out;
+  char* const out = g->packed;
   PackArgs A;
   A.n = n;
   A.rp = g->row_ptr, A.adj = g->adj, A.ndeg = g->ndeg;
@@ -1153,10 +1155,7 @@ hipError_t build_packed_rows(sgc_dgraph* g, hipStream_t s) {
   k_pack_table<<<1, kDegBuckets, 0, s>>>(A);
   k_pack_narrow<<<grid_for(std::min(n, m / kMinRow + 1), kBlock / kWave), kBlock, 0, s>>>(A);
   k_pack_wide<<<grid_for(std::min(n, m / kWideRow + 1), 1), kBlock, 0, s>>>(A);
-  const hipError_t e = hipGetLastError();
-  const hipError_t w = hipStreamSynchronize(s);
-  (void)hipFree(mem);
-  return e != hipSuccess ? e : w;
+  return hipGetLastError();
 }
 
 bool filter_stage(const sgc_dgraph* g, ScanParams p) {

@@ -112,9 +112,9 @@ void narrow_row_ptr(const sgc_host_graph* g, uint32_t* out, uint64_t* max_degree
 }
 
 void parallel_copy(void* dst, const void* src, size_t bytes) {
-  const size_t piece = 1 << 20;
+  const size_t piece = 256 << 10;
   const int64_t pieces = (int64_t)((bytes + piece - 1) / piece);
-#pragma omp parallel for schedule(static)
+#pragma omp parallel for schedule(static) if (pieces > 2)
   for (int64_t p = 0; p < pieces; ++p) {
     const size_t off = (size_t)p * piece;
     memcpy((char*)dst + off, (const char*)src + off, std::min(piece, bytes - off));

@@ -679,8 +679,9 @@ void launch_mirror(const sgc_dgraph* g, hipStream_t s) {
   k_mirror<<<grid_for(g->m, kBlock), kBlock, 0, s>>>(g->m, g->row_ptr, g->src, g->adj, g->mirror);
 }
 
-hipError_t build_mirror(const sgc_dgraph* g, hipStream_t s) {
+hipError_t build_mirror(sgc_ctx* ctx, const sgc_dgraph* g) {
   if (!g->m || !g->mirror) return hipSuccess;
+  hipStream_t s = ctx->stream;
   const uint32_t m = g->m;
   int bits = 1;
   while (bits < 32 && (1ull << bits) < (uint64_t)g->n) ++bits;
@@ -688,11 +689,10 @@ hipError_t build_mirror(const sgc_dgraph* g, hipStream_t s) {
   (void)hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, (const uint32_t*)nullptr, (uint32_t*)nullptr,
                                            (const uint64_t*)nullptr, (uint64_t*)nullptr, m, 0, bits, s);
   // keys out, values in and out, the sort's scratch and the mismatch count
-  char* mem = nullptr;
   const size_t o_keys = 0, o_vin = ((size_t)m * 4 + 255) / 256 * 256, o_vout = o_vin + (size_t)m * 8,
                o_tmp = o_vout + (size_t)m * 8, o_bad = o_tmp + (tmp_bytes + 255) / 256 * 256;
-  if (hipMalloc(&mem, o_bad + 256) != hipSuccess) {
-    (void)hipGetLastError();
+  char* const mem = (char*)work_memory(ctx, o_bad + 256);
+  if (!mem) {
     launch_mirror(g, s);  // not enough room to sort: search each reverse entry
     return hipGetLastError();
   }
@@ -711,7 +711,6 @@ hipError_t build_mirror(const sgc_dgraph* g, hipStream_t s) {
   unsigned long long h_bad = 0;
   if (e == hipSuccess) e = hipMemcpyAsync(&h_bad, bad, 8, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)hipFree(mem);
   if (e == hipSuccess && h_bad) {  // some entry lacks its reverse: the search finds those that exist
     launch_mirror(g, s);
     e = hipGetLastError();

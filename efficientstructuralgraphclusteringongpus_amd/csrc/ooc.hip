@@ -33,6 +33,7 @@
 
 #include "device.h"
 #include "device_util.h"
+#include "graph_host.h"
 #include "ooc_host.h"
 
 namespace sgc {
@@ -176,7 +177,8 @@ size_t row_chip_bytes(uint64_t cap, uint64_t rows) {
 size_t offsets_slice(uint64_t rows) { return ((rows + 1) * 4 + 255) / 256 * 256; }
 size_t offsets_bytes(uint64_t rows_i, uint64_t rows_j) { return offsets_slice(rows_i) + 2 * offsets_slice(rows_j); }
 
-// Pinned copy of one row block, free again once its upload has run.
+// Pinned copy of one row block (in the context's page-locked work memory),
+// free again once its upload has run.
 struct Staging {
   int32_t* adj = nullptr;
   uint32_t* off = nullptr;
@@ -217,21 +219,16 @@ struct OocRun {
         (void)hipStreamDestroy(st);
       }
     for (Staging& st : stage) {
-      if (st.adj) (void)hipHostFree(st.adj);
-      if (st.off) (void)hipHostFree(st.off);
       if (st.free) (void)hipEventDestroy(st.free);
     }
     if (up_i) (void)hipEventDestroy(up_i);
     if (back_i) (void)hipEventDestroy(back_i);
-    if (h_iflag) (void)hipHostFree(h_iflag);
     for (int i = 0; i < 2; ++i) {
-      if (h_flag[i]) (void)hipHostFree(h_flag[i]);
-      if (h_cnt[i]) (void)hipHostFree(h_cnt[i]);
       for (hipEvent_t e : {up_j[i], comp[i], back[i], t0[i], tm[i], t1[i]})
         if (e) (void)hipEventDestroy(e);
     }
-    if (flag && flag_pageable) free(flag);
-    else if (flag) (void)hipHostFree(flag);
+    if (flag_pageable) free(flag);
+    if (ctx) release_host_work(ctx);
     if (dev) (void)hipFree(dev);
   }
 };
@@ -260,12 +257,9 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
                 (unsigned long long)budget, (unsigned long long)resident, n);
   const uint64_t room = budget - resident - 8192;
   double t0 = now_ms();
-  std::vector<uint32_t> deg(n);
-  ooc_degrees(g, deg.data());
   std::vector<uint64_t> blocks, row_bounds;
   uint64_t block_rows = 0, row_max = 0, row_rows = 0;
-  uint64_t maxd = 1;
-  for (uint32_t x = 0; x < n; ++x) maxd = std::max<uint64_t>(maxd, deg[x]);
+  const uint64_t maxd = std::max<uint64_t>(1, ooc_max_degree(g));
   // Row blocks as large as the room allows once the records of the largest
   // degree and the row offsets are counted in (a block holds at most as many
   // rows as entries), in groups of the largest size whose chips still fit
@@ -354,29 +348,38 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
   // a page-locked graph is sent as it lies: only row offsets are staged.
   // Staging 0 holds a group (and the row chips' offsets), 1 and 2 a row
   // block each.
+  // The whole-graph flags only meet the device through the staged chip flags
+  // and the row chips' uploads: ordinary memory serves when the system will
+  // not lock m more bytes (the row-chip uploads then go through the context's
+  // staging).
+  Layout HL;
+  size_t o_adj[3], o_off[3], o_flag[2], o_cnt[2];
   for (int q = 0; q < 3; ++q) {
-    Staging& sg = R.stage[q];
-    const uint64_t entries = g->pinned ? 0 : std::max<uint64_t>(q ? J : I, 1);
-    const uint64_t rows = std::max<uint64_t>(q ? block_rows : std::max(rows_i, row_rows), 1);
-    if ((entries && hipHostMalloc((void**)&sg.adj, entries * 4) != hipSuccess) ||
-        hipHostMalloc((void**)&sg.off, (rows + 1) * 4) != hipSuccess) {
-      (void)hipGetLastError();
-      return fail(SGC_ENOMEM, "pinned host staging of %llu bytes failed",
-                  (unsigned long long)(entries * 4 + (rows + 1) * 4));
-    }
-    SGC_HIP(hipEventCreateWithFlags(&sg.free, hipEventDisableTiming));
+    o_adj[q] = HL.take((g->pinned ? 0 : std::max<uint64_t>(q ? J : I, 1)) * 4);
+    o_off[q] = HL.take((std::max<uint64_t>(q ? block_rows : std::max(rows_i, row_rows), 1) + 1) * 4);
   }
-  if (hipHostMalloc((void**)&R.h_iflag, std::max<uint64_t>(I, 1)) != hipSuccess) {
-    (void)hipGetLastError();
-    return fail(SGC_ENOMEM, "pinned host flag staging of %llu bytes failed", (unsigned long long)I);
+  const size_t o_iflag = HL.take(std::max<uint64_t>(I, 1));
+  for (int i = 0; i < 2; ++i) o_flag[i] = HL.take(std::max<uint64_t>(J, 1)), o_cnt[i] = HL.take(kCntWords * 8);
+  char* host = (char*)host_work_memory(ctx, HL.bytes + std::max<uint64_t>(g->m, 1));
+  if (host) {
+    R.flag = (uint8_t*)host + HL.bytes;
+  } else {
+    host = (char*)host_work_memory(ctx, HL.bytes);
+    if (!host) return fail(SGC_ENOMEM, "pinned host staging of %llu bytes failed", (unsigned long long)HL.bytes);
+    R.flag = (uint8_t*)malloc(std::max<uint64_t>(g->m, 1));
+    if (!R.flag) return fail(SGC_ENOMEM, "host flag array of %llu bytes failed", (unsigned long long)g->m);
+    R.flag_pageable = true;
   }
+  for (int q = 0; q < 3; ++q) {
+    if (!g->pinned) R.stage[q].adj = (int32_t*)(host + o_adj[q]);
+    R.stage[q].off = (uint32_t*)(host + o_off[q]);
+    SGC_HIP(hipEventCreateWithFlags(&R.stage[q].free, hipEventDisableTiming));
+  }
+  R.h_iflag = (uint8_t*)host + o_iflag;
   SGC_HIP(hipEventCreateWithFlags(&R.back_i, hipEventDisableTiming));
   for (int i = 0; i < 2; ++i) {
-    if (hipHostMalloc((void**)&R.h_flag[i], std::max<uint64_t>(J, 1)) != hipSuccess ||
-        hipHostMalloc((void**)&R.h_cnt[i], kCntWords * 8) != hipSuccess) {
-      (void)hipGetLastError();
-      return fail(SGC_ENOMEM, "pinned host flag staging of %llu bytes failed", (unsigned long long)J);
-    }
+    R.h_flag[i] = (uint8_t*)host + o_flag[i];
+    R.h_cnt[i] = (uint64_t*)(host + o_cnt[i]);
     SGC_HIP(hipEventCreateWithFlags(&R.up_j[i], hipEventDisableTiming));
     SGC_HIP(hipEventCreateWithFlags(&R.comp[i], hipEventDisableTiming));
     SGC_HIP(hipEventCreateWithFlags(&R.back[i], hipEventDisableTiming));
@@ -387,17 +390,6 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
   SGC_HIP(hipEventCreateWithFlags(&R.up_i, hipEventDisableTiming));
   SGC_HIP(hipStreamCreateWithFlags(&R.h2d, hipStreamNonBlocking));
   SGC_HIP(hipStreamCreateWithFlags(&R.d2h, hipStreamNonBlocking));
-  // the whole-graph flags only meet the device through the staged chip
-  // flags and the row chips' uploads: ordinary memory serves when the system
-  // will not lock m more bytes (the row-chip uploads then copy through the
-  // runtime's own staging)
-  if (hipHostMalloc((void**)&R.flag, std::max<uint64_t>(g->m, 1)) != hipSuccess) {
-    (void)hipGetLastError();
-    R.flag = nullptr;
-    R.flag = (uint8_t*)malloc(std::max<uint64_t>(g->m, 1));
-    if (!R.flag) return fail(SGC_ENOMEM, "host flag array of %llu bytes failed", (unsigned long long)g->m);
-    R.flag_pageable = true;
-  }
 
   const ScanParams p{eps, mu};
   uint64_t totals[kCntSlots] = {0};
@@ -409,24 +401,26 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
   const size_t P = blocks.size() - 1;
   const SimChipArrays A = sim_arrays(R.chip, I, J, RC, nullptr);
   auto range_m = [&](size_t b0, size_t b1) { return g->row_ptr[blocks[b1]] - g->row_ptr[blocks[b0]]; };
-  // rows of blocks [b0, b1) into pinned staging (offsets only for a
-  // page-locked graph)
-  auto stage_rows = [&](Staging& sg, size_t b0, size_t b1) -> int {
-    if (sg.pending) SGC_HIP(hipEventSynchronize(sg.free));
-    sg.pending = false;
-    const double tb = now_ms();
-    ooc_copy_rows(g, blocks[b0], blocks[b1], 0, g->pinned ? nullptr : sg.adj, sg.off);
-    R.ms_host += now_ms() - tb;
-    return SGC_OK;
-  };
   // blocks [b0, b1) to chip entries [pos, pos + their entries), their
-  // offsets (from their first entry) to off_dev; `done` is recorded on the
-  // upload stream
+  // offsets (from their first entry) to off_dev, through pinned staging piece
+  // by piece (a page-locked graph as it lies: only the offsets are staged),
+  // so that all but the first piece's host copy overlaps the transfer; `done`
+  // is recorded on the upload stream
   auto upload_rows = [&](Staging& sg, size_t b0, size_t b1, uint64_t pos, uint32_t* off_dev, hipEvent_t done) -> int {
     const uint64_t mb = range_m(b0, b1);
     const uint32_t nr = (uint32_t)(blocks[b1] - blocks[b0]);
-    const int32_t* from = g->pinned ? g->adj + g->row_ptr[blocks[b0]] : sg.adj;
-    if (mb) SGC_HIP(hipMemcpyAsync(A.adj + pos, from, mb * 4, hipMemcpyHostToDevice, R.h2d));
+    if (sg.pending) SGC_HIP(hipEventSynchronize(sg.free));
+    sg.pending = false;
+    const double tb = now_ms();
+    ooc_offsets(g, blocks[b0], blocks[b1], sg.off);
+    const int32_t* const from = g->adj + g->row_ptr[blocks[b0]];
+    const uint64_t piece = g->pinned ? std::max<uint64_t>(mb, 1) : kBounceBytes / 4;
+    for (uint64_t k = 0; k < mb; k += piece) {
+      const uint64_t len = std::min(piece, mb - k);
+      if (!g->pinned) parallel_copy(sg.adj + k, from + k, len * 4);
+      SGC_HIP(hipMemcpyAsync(A.adj + pos + k, (g->pinned ? from : sg.adj) + k, len * 4, hipMemcpyHostToDevice, R.h2d));
+    }
+    R.ms_host += now_ms() - tb;
     SGC_HIP(hipMemcpyAsync(off_dev, sg.off, ((size_t)nr + 1) * 4, hipMemcpyHostToDevice, R.h2d));
     SGC_HIP(hipEventRecord(sg.free, R.h2d));
     sg.pending = true;
@@ -476,7 +470,6 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
     const uint32_t nri = (uint32_t)(c.r1i - c.r0i);
     // the group goes to chip entries [J, J + mi) once every chip of the
     // previous group has run
-    if ((rc = stage_rows(R.stage[0], gi, ge))) return rc;
     for (int b = 0; b < 2; ++b)
       if (used[b]) SGC_HIP(hipStreamWaitEvent(R.h2d, R.comp[b], 0));
     if ((rc = upload_rows(R.stage[0], gi, ge, J, R.off_i, R.up_i))) return rc;
@@ -501,7 +494,6 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
         // run
         jpos = b == 0 ? J - c.mj : J + c.mi;
         Staging& sj = R.stage[1 + b];
-        if ((rc = stage_rows(sj, j, j + 1))) return rc;
         if (used[b]) SGC_HIP(hipStreamWaitEvent(R.h2d, R.comp[b], 0));
         if ((rc = upload_rows(sj, j, j + 1, jpos, R.off_j[b], R.up_j[b]))) return rc;
         SGC_HIP(hipStreamWaitEvent(s, R.up_j[b], 0));
@@ -623,14 +615,14 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
       uint32_t* ho = R.stage[0].off;
       for (uint32_t k = 0; k <= nr; ++k) ho[k] = (uint32_t)(g->row_ptr[r0 + k] - b0);
       SGC_HIP(hipMemcpyAsync(c_off, ho, ((size_t)nr + 1) * 4, hipMemcpyHostToDevice, s));
-      if (mc) SGC_HIP(hipMemcpyAsync(c_flag, R.flag + b0, mc, hipMemcpyHostToDevice, s));
+      SGC_HIP(upload_bytes(ctx, c_flag, R.flag + b0, mc, !R.flag_pageable));
       R.bytes_h2d += (double)mc + (double)(nr + 1) * 4;
       if (nr) k_fill_src_rows<<<grid_for(nr, kBlock / kWave), kBlock, 0, s>>>((uint32_t)r0, nr, c_off, c_src);
       loaded = i;
       loaded_adj = false;
     }
     if (with_adj && !loaded_adj) {
-      if (mc) SGC_HIP(hipMemcpyAsync(c_adj, g->adj + b0, mc * 4, hipMemcpyHostToDevice, s));
+      SGC_HIP(upload_bytes(ctx, c_adj, g->adj + b0, mc * 4, g->pinned));
       R.bytes_h2d += (double)mc * 4;
       loaded_adj = true;
     }
@@ -676,9 +668,8 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
   SGC_HIP(hipEventRecord(ctx->ev[0], s));
   SGC_HIP(hipGetLastError());
   SGC_HIP(hipMemcpyAsync(R.h_cnt[0], pb.cnt, kCntWords * 8, hipMemcpyDeviceToHost, s));
-  if (labels) SGC_HIP(hipMemcpyAsync(labels, pb.label, (size_t)n * 4, hipMemcpyDeviceToHost, s));
-  if (core_out) SGC_HIP(hipMemcpyAsync(core_out, pb.core, n, hipMemcpyDeviceToHost, s));
-  SGC_HIP(hipStreamSynchronize(s));
+  const HostCopy results[2] = {{labels, pb.label, (size_t)n * 4}, {core_out, pb.core, n}};
+  SGC_HIP(download(ctx, results, 2));
   R.bytes_d2h += (labels ? (double)n * 4 : 0) + (core_out ? (double)n : 0);
   if (nrow == 1) {
     ms_core = elapsed(ctx->ev[3], ctx->ev[4]);
@@ -687,7 +678,7 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
     ms_classify = elapsed(ctx->ev[6], ctx->ev[0]);
   }
   const double ms_phases = now_ms() - t_phase;
-  if (sim_out && g->m) memcpy(sim_out, R.flag, g->m);
+  if (sim_out && g->m) parallel_copy(sim_out, R.flag, g->m);
 
   fold_counters(R.h_cnt[0]);
   const uint64_t* c = R.h_cnt[0];

@@ -22,6 +22,7 @@
 
 #include <algorithm>
 #include <deque>
+#include <memory>
 #include <unordered_map>
 #include <vector>
 
@@ -298,9 +299,8 @@ struct Slot {
 struct Graph {
   uint32_t id = 0;
   sgc_dgraph* dg = nullptr;
-  uint32_t* cn = nullptr;
-  void* slot_mem = nullptr;
-  uint64_t* cnt_mem = nullptr;  // kCntWords per slot
+  uint32_t* cn = nullptr;  // start of the graph's device memory: then the slots, then kCntWords per slot
+  char* host_mem = nullptr;  // page-locked: the slots' labels, counters and parameters
   size_t bytes = 0;
   std::vector<Slot> slots;
   double precompute_ms = 0;
@@ -315,7 +315,7 @@ struct Query {
 };
 
 struct Result {
-  std::vector<int32_t> labels;
+  std::unique_ptr<int32_t[]> labels;  // st.n of them
   sgc_query_stats st;
 };
 
@@ -376,14 +376,10 @@ namespace {
 void free_graph(Graph* G) {
   for (Slot& s : G->slots) {
     if (s.exec) (void)hipGraphExecDestroy(s.exec);
-    if (s.h_params) (void)hipHostFree(s.h_params);
-    if (s.h_labels) (void)hipHostFree(s.h_labels);
-    if (s.h_cnt) (void)hipHostFree(s.h_cnt);
     if (s.start) (void)hipEventDestroy(s.start);
     if (s.done) (void)hipEventDestroy(s.done);
   }
-  if (G->slot_mem) (void)hipFree(G->slot_mem);
-  if (G->cnt_mem) (void)hipFree(G->cnt_mem);
+  if (G->host_mem) (void)hipHostFree(G->host_mem);
   if (G->cn) (void)hipFree(G->cn);
   if (G->dg) sgc_dgraph_free(G->dg);
   delete G;
@@ -619,7 +615,8 @@ int dispatch(sgc_server* S) {
 Result slot_result(const Graph* G, const Slot& s, double ms_device) {
   if (!s.batched) fold_counters(s.h_cnt);  // a batch's counters are folded on the device
   Result r;
-  r.labels.assign(s.h_labels, s.h_labels + G->dg->n);
+  r.labels.reset(new int32_t[std::max<uint32_t>(G->dg->n, 1)]);
+  parallel_copy(r.labels.get(), s.h_labels, (size_t)G->dg->n * 4);
   memset(&r.st, 0, sizeof(r.st));
   r.st.status = SGC_OK;
   r.st.graph = G->id;
@@ -751,9 +748,10 @@ extern "C" int sgc_server_add_graph(sgc_server* S, const sgc_host_graph* hg, uin
     return rc;
   }
   const uint32_t n = G->dg->n, m = G->dg->m;
-  if (hipMalloc(&G->cn, std::max<size_t>(m, 1) * 4) != hipSuccess ||
-      hipMalloc(&G->slot_mem, S->slots_per_graph * slot_bytes(n, m)) != hipSuccess ||
-      hipMalloc(&G->cnt_mem, S->slots_per_graph * kCntWords * 8) != hipSuccess) {
+  // one device and one page-locked allocation for all slots
+  const size_t cn_bytes = align256(std::max<size_t>(m, 1) * 4), label_bytes = align256(std::max<size_t>(n, 1) * 4),
+               host_bytes = label_bytes + align256(kCntWords * 8) + align256(sizeof(QueryParams));
+  if (hipMalloc((void**)&G->cn, cn_bytes + S->slots_per_graph * (slot_bytes(n, m) + kCntWords * 8)) != hipSuccess) {
     (void)hipGetLastError();
     free_graph(G);
     return fail(SGC_ENOMEM, "device allocation for graph of %u vertices failed", n);
@@ -791,8 +789,14 @@ extern "C" int sgc_server_add_graph(sgc_server* S, const sgc_host_graph* hg, uin
   }
   G->precompute_ms = now_ms() - t0;
   // query slots
+  if (hipHostMalloc((void**)&G->host_mem, S->slots_per_graph * host_bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    free_graph(G);
+    return fail(SGC_ENOMEM, "query slot set-up failed");
+  }
   G->slots.resize(S->slots_per_graph);
-  char* base = (char*)G->slot_mem;
+  char* const base = (char*)G->cn + cn_bytes;
+  uint64_t* const cnt_mem = (uint64_t*)(base + S->slots_per_graph * slot_bytes(n, m));
   for (uint32_t i = 0; i < S->slots_per_graph; ++i) {
     Slot& sl = G->slots[i];
     char* p = base + i * slot_bytes(n, m);
@@ -810,15 +814,16 @@ extern "C" int sgc_server_add_graph(sgc_server* S, const sgc_host_graph* hg, uin
     p += align256((size_t)n * 4 + 4);
     sl.pb.core = (uint8_t*)p;
     p += align256((size_t)n + 1);
-    sl.pb.cnt = G->cnt_mem + (size_t)i * kCntWords;
+    sl.pb.cnt = cnt_mem + (size_t)i * kCntWords;
     p += align256(kCntSlots * 8);
     sl.d_params = (QueryParams*)p;
     sl.stream = S->next_stream;
     S->next_stream = (S->next_stream + 1) % kStreams;
-    if (hipHostMalloc((void**)&sl.h_labels, std::max<size_t>(n, 1) * 4) != hipSuccess ||
-        hipHostMalloc((void**)&sl.h_cnt, kCntWords * 8) != hipSuccess ||
-        hipHostMalloc((void**)&sl.h_params, sizeof(QueryParams)) != hipSuccess ||
-        hipEventCreate(&sl.start) != hipSuccess || hipEventCreate(&sl.done) != hipSuccess) {
+    char* const h = G->host_mem + i * host_bytes;
+    sl.h_labels = (int32_t*)h;
+    sl.h_cnt = (uint64_t*)(h + label_bytes);
+    sl.h_params = (QueryParams*)(h + label_bytes + align256(kCntWords * 8));
+    if (hipEventCreate(&sl.start) != hipSuccess || hipEventCreate(&sl.done) != hipSuccess) {
       (void)hipGetLastError();
       free_graph(G);
       return fail(SGC_ENOMEM, "query slot set-up failed");
@@ -1021,8 +1026,9 @@ extern "C" int sgc_server_result(sgc_server* S, uint64_t ticket, int32_t* labels
   }
   const Result& r = it->second;
   if (labels) {
-    if (capacity < r.labels.size()) return fail(SGC_EINVAL, "labels buffer holds %llu < %zu", (unsigned long long)capacity, r.labels.size());
-    memcpy(labels, r.labels.data(), r.labels.size() * 4);
+    const uint64_t n = r.labels ? r.st.n : 0;  // a query on a removed graph has none
+    if (capacity < n) return fail(SGC_EINVAL, "labels buffer holds %llu < %llu", (unsigned long long)capacity, (unsigned long long)n);
+    parallel_copy(labels, r.labels.get(), n * 4);
   }
   if (st) *st = r.st;
   const int status = r.st.status;
