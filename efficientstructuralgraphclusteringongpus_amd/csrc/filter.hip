@@ -322,6 +322,7 @@ __global__ void __launch_bounds__(kBlock) k_pack_wide(PackArgs A) {
 //   workgroup  up to kSmallRow entries (or many edges): 256 threads
 //   large      1024 threads
 constexpr uint32_t kWaveRow = 256;
+constexpr uint32_t kXcds = 8;  // blocks go to the XCDs in turn
 constexpr uint32_t kWaveEdges = 256;
 constexpr uint32_t kSmallRow = 1024;
 constexpr uint32_t kSmallEdges = 256;  // edges per unit
@@ -621,9 +622,11 @@ __device__ __forceinline__ void emit_unit(const FilterArgs& A, const UnitIO& io,
 }
 
 // Bitmap filter of one unit at a time: an owner and up to MAXE of its edges;
-// teams of 16 lanes take edges from the unit's cursor.  The owner's row goes
+// teams of 16 lanes take edges from the unit's cursor.  The owner's bitmap goes
 // into LDS at the largest M needed (at LDS words [top, 2 top) of 16 bytes),
-// then folded level by level ([w, 2 w) for M = 128 w).
+// then folded level by level ([w, 2 w) for M = 128 w).  Loading the stored
+// bitmap instead of hashing the row again: R-MAT-22 shuffled, eps 0.6, large
+// owners 632 -> 593 us.
 template <bool LARGE>
 __global__ void __launch_bounds__(LARGE ? 1024 : 256, 8) k_bitmap_units(FilterArgs A, UnitIO io) {
   stamp(A.cnt, LARGE ? kStampSim : kStampSimRest);
@@ -663,14 +666,19 @@ __global__ void __launch_bounds__(LARGE ? 1024 : 256, 8) k_bitmap_units(FilterAr
     uint32_t top = coarse_words(min(l, kMaxThresholdRow));
     const uint32_t tf = 4 * coarse_words(min(l, FINE));
     top = top > tf ? top : tf;
-    for (uint32_t t = tid; t < top; t += T) s_own[top + t] = make_uint4(0, 0, 0, 0);
+    // that is the row's own stored bitmap, but for rows that have none
+    const bool stored = LARGE ? l > kSmallRow && l <= kMaxThresholdRow : l >= kMinRow && l <= kFineRow;
+    const uint4* const row = A.bits + (LARGE ? coarse_at(bb) : A.fine0 + 4 * coarse_at(bb));
+    for (uint32_t t = tid; t < top; t += T) s_own[top + t] = stored ? row[t] : make_uint4(0, 0, 0, 0);
     if (tid < MAXE / 32) s_surv[tid] = 0;
     if (tid < 32) s_hist[tid] = 0;
     __syncthreads();
-    const uint32_t mask = top * 128 - 1;
-    for (uint32_t t = tid; t < l; t += T) {
-      const uint32_t h = vertex_hash((uint32_t)A.adj[bb + t]) & mask;
-      atomicOr(&own[top * 4 + (h >> 5)], 1u << (h & 31));
+    if (!stored) {
+      const uint32_t mask = top * 128 - 1;
+      for (uint32_t t = tid; t < l; t += T) {
+        const uint32_t h = vertex_hash((uint32_t)A.adj[bb + t]) & mask;
+        atomicOr(&own[top * 4 + (h >> 5)], 1u << (h & 31));
+      }
     }
     bool keep = false;  // survives
     uint32_t need = 0;
@@ -881,14 +889,17 @@ __device__ __noinline__ bool row_contains(const int32_t* __restrict__ adj, uint3
   return lo < e && adj[lo] == x;
 }
 
-// Owners with short rows, one wave each: the row's bitmaps in LDS; 64 edges
-// at a time, eight teams of 8 lanes.  What the bitmaps do not reject is
+// Owners with short rows, one wave each: the row's stored bitmap and its folds
+// in LDS; 64 edges at a time, eight teams of 8 lanes.  What the bitmaps do not reject is
 // counted element by element in a cuckoo hash of the owner's row (a quarter
 // full at most, built when the first edge needs it), four teams of 16, so
 // nothing is left to the exact kernels.  Planted communities (n = 3e5, eps
-// 0.35, 2.8e7 undecided edges of rows around 185, an eighth similar): 2.9 ms,
+// 0.35, 2.8e7 undecided edges of rows around 185, an eighth similar): 2.7 ms,
 // of which about half are the exact counts; 5.3 with binary searches in a
-// sorted LDS row instead of the hash.
+// sorted LDS row instead of the hash.  Waits for loads take two thirds of the
+// wave cycles and the VALU is half busy: five waves a SIMD instead of six take
+// 3.5 ms.  With the row hashed again for every owner, the owners dealt to the
+// XCDs one by one and no owner fetched ahead: 2.85.
 __global__ void __launch_bounds__(kBlock, 6)
     k_bitmap_wave(FilterArgs A, const uint32_t* __restrict__ wl_b, const uint32_t* __restrict__ wl_e,
                   const uint32_t* __restrict__ wl_k) {
@@ -911,19 +922,27 @@ __global__ void __launch_bounds__(kBlock, 6)
   const uint32_t count = (uint32_t)A.cnt[kCntTiny];
   const uint32_t waves = gridDim.x * W;
   uint32_t streamed = 0, rounds = 0, probed = 0;
-  for (uint32_t idx = blockIdx.x * W + wv; idx < count; idx += waves) {
-    const uint32_t bb = __builtin_amdgcn_readfirstlane(wl_b[idx]), be = __builtin_amdgcn_readfirstlane(wl_e[idx]);
-    const uint32_t owned = __builtin_amdgcn_readfirstlane(wl_k[idx]), l = be - bb;
+  // blocks of one XCD (every eighth) take neighbouring owners of the list,
+  // whose edges share rows: its L2 then serves more of them
+  const uint32_t per = gridDim.x / kXcds, vb = gridDim.x % kXcds ? blockIdx.x : blockIdx.x % kXcds * per + blockIdx.x / kXcds;
+  uint32_t idx = vb * W + wv, n_b = 0, n_e = 0, n_k = 0;  // the next owner, fetched one ahead
+  if (idx < count) n_b = wl_b[idx], n_e = wl_e[idx], n_k = wl_k[idx];
+  for (; idx < count; idx += waves) {
+    const uint32_t bb = __builtin_amdgcn_readfirstlane(n_b), be = __builtin_amdgcn_readfirstlane(n_e);
+    const uint32_t owned = __builtin_amdgcn_readfirstlane(n_k), l = be - bb;
+    if (idx + waves < count) n_b = wl_b[idx + waves], n_e = wl_e[idx + waves], n_k = wl_k[idx + waves];
     uint4 ed = make_uint4(kNone, kNone, 0, 0);  // (entry, reverse entry, row start of a, d(a))
     if (lane < owned) ed = A.uedge[bb + lane];
     const uint32_t top = 4 * coarse_words(l), mask = top * 128 - 1;
-    if (lane < top) own4[top + lane] = make_uint4(0, 0, 0, 0);
+    if (lane < top) own4[top + lane] = l >= kMinRow ? A.bits[A.fine0 + 4 * coarse_at(bb) + lane] : make_uint4(0, 0, 0, 0);
     wave_lds_sync();
-    for (uint32_t t = lane; t < l; t += kWave) {
-      const uint32_t h = vertex_hash((uint32_t)A.adj[bb + t]) & mask;
-      atomicOr(&own[top * 4 + (h >> 5)], 1u << (h & 31));
+    if (l < kMinRow) {
+      if (lane < l) {
+        const uint32_t h = vertex_hash((uint32_t)A.adj[bb + lane]) & mask;
+        atomicOr(&own[top * 4 + (h >> 5)], 1u << (h & 31));
+      }
+      wave_lds_sync();
     }
-    wave_lds_sync();
     for (uint32_t w = top >> 1; w; w >>= 1) {
       if (lane < w) {
         const uint4 x = own4[2 * w + lane], y = own4[3 * w + lane];
