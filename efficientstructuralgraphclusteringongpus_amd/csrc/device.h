@@ -321,6 +321,11 @@ void launch_plan_filter(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s
 void launch_filter(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int cu_count, hipStream_t s);
 // Whether launch_filter can leave units to the exact kernels.
 bool filter_leaves_units(const sgc_dgraph* g);
+// Exact units by teams (exact.hip): whether it takes the small or large units
+// of a graph of n vertices, and the kernel.
+bool exact_units_cover(uint32_t n, bool large);
+void launch_exact_units(const sgc_dgraph* g, const PassBuffers& b, const uint4* units, uint32_t ucap, ScanParams p,
+                        int cu_count, hipStream_t s, bool large, uint32_t* cn_out);
 void launch_copy(const void* src, void* dst, uint64_t bytes, hipStream_t s);
 void launch_init(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s);
 // count_all: every edge is left to its owner (for exact common-neighbour

@@ -431,16 +431,6 @@ struct FilterArgs {
   uint64_t* cnt;
 };
 
-// Sum over each team of 8 or 16 lanes, in all of them.
-template <uint32_t TEAM>
-__device__ __forceinline__ uint32_t team_sum(uint32_t v) {
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true);   // quad_perm 1 0 3 2
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, true);   // quad_perm 2 3 0 1
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true);  // row_half_mirror
-  if (TEAM == 16) v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, true);  // row_mirror
-  return v;
-}
-
 constexpr uint32_t kTeamLoads = 4;  // 16-byte loads per lane and round
 
 // Misses that make an edge (s = d(a), threshold c*) dissimilar; 0: decided
@@ -555,22 +545,6 @@ __device__ __forceinline__ uint32_t group_round(uint32_t g, uint32_t take, const
     miss += (uint32_t)__popc(j * TEAM + tl < take ? bits : 0u);
   }
   return team_sum<TEAM>(miss);
-}
-
-// Position of each thread's edge among the unit's edges in order of `size`
-// (about two buckets per power of two, largest first): the teams of a wave
-// then take edges of about the same length, end their rounds and fetch their
-// next edges together, and the longest do not start last.  hist: 32 zeroed
-// words; called by every thread, with two barriers.  *todo: edges with size
-// > 0 (size < 2^16).
-__device__ __forceinline__ uint32_t order_by_size(uint32_t size, uint32_t* hist, uint32_t* todo) {
-  const uint32_t lg = size ? 31 - __clz(size) : 0u;
-  const uint32_t bucket = 31 - (lg ? lg * 2 + ((size >> (lg - 1)) & 1) : 0u);
-  const uint32_t rank = size ? atomicAdd(&hist[bucket], 1u) : 0u;
-  __syncthreads();
-  const uint32_t incl = wave_incl_scan(lane_id() < 32 ? hist[lane_id()] : 0u);
-  *todo = __builtin_amdgcn_readlane(incl, 31);
-  return (uint32_t)__shfl((int)incl, (int)bucket) - hist[bucket] + rank;
 }
 
 // Ends a unit: edges of `mine` threads with !keep are rejected (flags), the
@@ -873,20 +847,6 @@ __global__ void __launch_bounds__(1024, 8) k_hash_units(FilterArgs A, UnitIO io)
   }
   const uint64_t elements = tl == 0 ? (uint64_t)streamed * kGroup : 0ull;
   count_add<3>(A.cnt, {kCntProbes, kCntLoaded, kCntClaims}, {elements, elements, tl == 0 ? rounds : 0u});
-}
-
-// Whether x is in the sorted row adj[b, e) (the wave tier's way out when a
-// cuckoo insertion fails).
-__device__ __noinline__ bool row_contains(const int32_t* __restrict__ adj, uint32_t b, uint32_t e, int32_t x) {
-  uint32_t lo = b, hi = e;
-  while (lo < hi) {
-    const uint32_t mid = lo + ((hi - lo) >> 1);
-    if (adj[mid] < x)
-      lo = mid + 1;
-    else
-      hi = mid;
-  }
-  return lo < e && adj[lo] == x;
 }
 
 // Owners with short rows, one wave each: the row's stored bitmap and its folds

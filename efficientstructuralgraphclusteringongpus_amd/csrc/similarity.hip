@@ -10,16 +10,15 @@
 // 2. k_plan: each owner's edges are cut into units of bounded work.
 //    Owners with d(b) <= the tuned cut-off (at most kT1MaxDeg) go to the
 //    small tier, the rest to the workgroup tier.
-// 3. Counting (k_sim_units): the owner's row N(b) is put into LDS and the
-//    short rows N(a) of the unit's edges are streamed through it in claims
+// 3. Counting (exact.hip; k_sim_units for what it does not take): the owner's
+//    row N(b) is put into LDS and, in k_sim_units, the short rows N(a) of the unit's edges are streamed through it in claims
 //    that every wave of the workgroup takes dynamically (up to 16 coalesced
 //    loads per lane in flight in the large tier).  Per edge the running
 //    (hits, consumed) pair decides early: reached -> similar, unreachable ->
 //    not similar (the reference's predicate in its exact threshold form).
 //    The result is written to both directed entries.
 //    Small tier: owners of degree <= 1024, 256-thread workgroups, the row as
-//    a two-table cuckoo hash (linear probing if an insertion chain fails).
-//    Large tier: 1024-thread workgroups, the row as a cuckoo hash (whole, or
+//    a linear-probing hash.  Large tier: 1024-thread workgroups, the row as a cuckoo hash (whole, or
 //    in runs of 2^20-id windows) or one window at a time as an exact 128 KB
 //    bitmap.
 // 4. k_sim_tiny: owners whose edges' whole merge work is small, one edge per
@@ -578,7 +577,7 @@ struct ClaimTable {
   const int32_t* adj;
   const uint32_t* tab;
   uint32_t wlo, whi;    // large tier: the window [wlo, whi)
-  uint32_t mask, shift;  // hash table shape (cuckoo: second table's offset, hash shift)
+  uint32_t mask, shift;  // small tier: hash table shape
   uint32_t b;            // the owner
   bool last;             // no later window
   bool mir_here;         // the table's id range holds b
@@ -591,13 +590,9 @@ struct ClaimTable {
 //   hold their whole row (at most half full), longer rows hold runs of
 //   consecutive windows with at most that many keys, so a claim is cut at
 //   the run's end instead of at every window's.
-//   Small tier: 2 x 2^bits slots with 2^bits >= 2 d(b) (at most a quarter
-//   full), in place of linear probing, whose lock-step rounds last as long
-//   as the wave's longest probe.
 // Insertion evicts along a chain of at most kCuckooKicks (device_util.h); a
 // failed chain
-// (never observed at these loads) sends the unit to bitmap windows
-// (large tier) or linear probing (small tier).
+// (never observed at these loads) sends the unit to bitmap windows.
 constexpr uint32_t kCuckooSlots = 16384;
 constexpr uint32_t kCuckooShift = 18;  // 32 - log2(kCuckooSlots)
 constexpr uint32_t kCuckooMaxKeys = 8192;
@@ -654,10 +649,8 @@ __device__ __forceinline__ uint32_t count_claim(const ClaimTable& c, uint32_t s0
     uint32_t v0[NL], v1[NL];
 #pragma unroll
     for (uint32_t j = 0; j < NL; ++j) {
-      // workgroup tier: the fixed table shape as constants
-      const uint32_t shift = T::kBitmap ? kCuckooShift : c.shift, second = T::kBitmap ? kCuckooSlots : c.mask;
-      v0[j] = c.tab[cuckoo_h0((uint32_t)x[j], shift)];
-      v1[j] = c.tab[second + cuckoo_h1((uint32_t)x[j], shift)];
+      v0[j] = c.tab[cuckoo_h0((uint32_t)x[j], kCuckooShift)];
+      v1[j] = c.tab[kCuckooSlots + cuckoo_h1((uint32_t)x[j], kCuckooShift)];
     }
 #pragma unroll
     for (uint32_t j = 0; j < NL; ++j) {
@@ -712,7 +705,9 @@ __device__ __forceinline__ uint32_t count_dispatch(uint32_t nl, const ClaimTable
 }
 
 // One unit = one owner b and up to MAX_EDGES of its undecided edges (a, b).
-// The owner row N(b) goes into LDS (small tier: hash table; large tier: the
+// The owner row N(b) goes into LDS (small tier: linear-probing hash table, for
+// graphs tuned to hash_tables = 0; the others' small units go to
+// k_exact_units; large tier: the
 // whole row or runs of 2^20-id windows as a cuckoo hash, else one window at a
 // time as an exact bitmap).  The short rows N(a) are
 // streamed in claims that every wave of the workgroup takes dynamically: a
@@ -938,8 +933,6 @@ __global__ void __launch_bounds__(T::kThreads, T::kMinWaves)
             tab4[t] = make_uint4(kEmptySlot, kEmptySlot, kEmptySlot, kEmptySlot);
           if (threadIdx.x == 0) s_fail = 0;
           __syncthreads();
-          mask = kCuckooSlots;
-          shift = kCuckooShift;
           const bool ok = cuckoo_insert_all<KB>(tab, kk, kCuckooSlots, kCuckooShift);
           if (!ok) s_fail = 1;
           __syncthreads();
@@ -961,27 +954,6 @@ __global__ void __launch_bounds__(T::kThreads, T::kMinWaves)
             atomicOr(&tab[x >> 5], 1u << (x & 31));
           }
         }
-      } else if (hash_ok) {
-        // two tables of 2^bits >= 2l slots each
-        const uint32_t slots = table_size_for(l);
-        mask = slots;
-        shift = 32 - log2_pow2(slots);
-        uint4* tab4 = reinterpret_cast<uint4*>(tab);  // 2 * slots is a multiple of 128
-        for (uint32_t t = threadIdx.x; t < 2 * slots / 4; t += T::kThreads)
-          tab4[t] = make_uint4(kEmptySlot, kEmptySlot, kEmptySlot, kEmptySlot);
-        if (threadIdx.x == 0) s_fail = 0;
-        __syncthreads();
-        bool ok = true;  // key by key: batched placements cost this tier register spills
-#pragma unroll
-        for (uint32_t j = 0; j < KPT; ++j)
-          if (threadIdx.x + j * T::kThreads < l) ok = cuckoo_insert(tab, key[j], slots, shift) && ok;
-        if (!ok) s_fail = 1;
-        __syncthreads();
-        if (s_fail) {  // redo with linear probing
-          hash_ok = false;
-          continue;
-        }
-        hashed = true;
       } else {
         const uint32_t TS = table_size_for(2 * l);
         mask = TS - 1;
@@ -1082,8 +1054,8 @@ __global__ void __launch_bounds__(T::kThreads, T::kMinWaves)
         uint32_t used;
         const uint32_t nl = (len + kWave - 1) / kWave;
         uint32_t h;
-        if (hashed)
-          h = count_dispatch<T, true>(nl, cc, s0, len, &e_mir[e], &e_q[e].w, &used);
+        if (T::kBitmap && hashed)
+          h = count_dispatch<T, T::kBitmap>(nl, cc, s0, len, &e_mir[e], &e_q[e].w, &used);
         else
           h = count_dispatch<T, false>(nl, cc, s0, len, &e_mir[e], &e_q[e].w, &used);
         if (lane == 0) atomicAdd(&e_state[e], ((unsigned long long)h << 32) | (unsigned long long)used);
@@ -1249,6 +1221,29 @@ void launch_plan(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStr
                                                    p.mu, false);
 }
 
+namespace {
+// The units of both tiers, by the team kernels where they take them.
+void launch_units(const sgc_dgraph* g, const PassBuffers& b, const uint4* units, uint32_t ucap, ScanParams p,
+                  uint32_t cus, bool prune, hipEvent_t mid, hipStream_t s, uint32_t* cn_out) {
+  const bool hash = g->tuning.hash_tables != 0;
+  if (hash && !prune && exact_units_cover(g->n, true))
+    launch_exact_units(g, b, units, ucap, p, (int)cus, s, true, cn_out);
+  else
+    k_sim_units<LargeTier><<<cus, LargeTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps, b.flag,
+                                                               cn_out, g->woff, window_count(g->n) + 1, b.uedge, units,
+                                                               ucap, b.cnt, kCntUnits2, kCntQueue2, hash,
+                                                               prune ? b.core : nullptr, b.ny, b.nn, p.mu);
+  if (mid) (void)hipEventRecord(mid, s);
+  if (hash)
+    launch_exact_units(g, b, units, ucap, p, (int)cus, s, false, cn_out);
+  else
+    k_sim_units<SmallTier><<<cus * 8, SmallTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps, b.flag,
+                                                                   cn_out, nullptr, 0, b.uedge, units, ucap, b.cnt,
+                                                                   kCntUnits1, kCntQueue1, hash, nullptr, nullptr,
+                                                                   nullptr, 0);
+}
+}  // namespace
+
 void launch_similarity(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int cu_count, int impl, hipEvent_t mid,
                        hipStream_t s, uint32_t* cn_out) {
   if (g->m == 0) return;
@@ -1273,16 +1268,7 @@ void launch_similarity(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, 
   // the core-check pruning runs in the workgroup tier, which launches first
   // and holds the long rows; the later tiers decide every edge they own
   const bool prune = p.prune && !cn_out && g->mirror;
-  k_sim_units<LargeTier><<<cus, LargeTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps, b.flag,
-                                                             cn_out, g->woff, window_count(g->n) + 1, b.uedge, units,
-                                                             ucap, b.cnt, kCntUnits2, kCntQueue2,
-                                                             g->tuning.hash_tables != 0, prune ? b.core : nullptr,
-                                                             b.ny, b.nn, p.mu);
-  if (mid) (void)hipEventRecord(mid, s);
-  k_sim_units<SmallTier><<<cus * 8, SmallTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps,
-                                                                 b.flag, cn_out, nullptr, 0, b.uedge, units, ucap,
-                                                                 b.cnt, kCntUnits1, kCntQueue1, g->tuning.hash_tables != 0,
-                                                                 nullptr, nullptr, nullptr, 0);
+  launch_units(g, b, units, ucap, p, cus, prune, mid, s, cn_out);
   if (g->tuning.tiny_work && !filtered) {
     // the list's length is on the device: enough threads for every owner of
     // the chip's vertices, grid-striding beyond two per CU slot
@@ -1370,17 +1356,7 @@ void launch_similarity_packed(const sgc_dgraph* g, const PassBuffers& b, ScanPar
         k_plan<<<grid_for(rr.hi[q] - rr.lo[q], kBlock), kBlock, 0, s>>>(
             rr.lo[q], rr.hi[q], g->row_begin, g->row_end, t, b.cnt_u, b.work_u, b.units, b.ucap, b.tiny, b.cnt, nullptr,
             nullptr, nullptr, p.mu, false, b.rec_start, r0, w);
-    k_sim_units<LargeTier><<<cus, LargeTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps, b.flag,
-                                                               nullptr, g->woff, window_count(g->n) + 1, b.uedge, b.units,
-                                                               b.ucap, b.cnt, kCntUnits2, kCntQueue2,
-                                                               g->tuning.hash_tables != 0, nullptr, nullptr, nullptr,
-                                                               0);
-    if (r == 0 && mid) (void)hipEventRecord(mid, s);
-    k_sim_units<SmallTier><<<cus * 8, SmallTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps,
-                                                                   b.flag, nullptr, nullptr, 0, b.uedge, b.units,
-                                                                   b.ucap, b.cnt, kCntUnits1, kCntQueue1,
-                                                                   g->tuning.hash_tables != 0, nullptr, nullptr,
-                                                                   nullptr, 0);
+    launch_units(g, b, b.units, b.ucap, p, cus, false, r == 0 ? mid : nullptr, s, nullptr);
     if (t.tiny_work) {
       const uint64_t want = ((uint64_t)g->n + kBlock - 1) / kBlock, cap = (uint64_t)cus * 32;
       k_sim_tiny<<<(uint32_t)(want < cap ? want : cap), kBlock, 0, s>>>(g->m, g->row_begin, g->row_end, g->adj,
@@ -1425,15 +1401,7 @@ void launch_redo(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int cu
   k_plan<<<grid_for(g->n, kBlock), kBlock, 0, s>>>(0, g->n, g->row_begin, g->row_end, t, b.cnt_u, b.work_u, b.units,
                                                    b.ucap, b.tiny, b.cnt, nullptr, nullptr, nullptr, p.mu, true);
   const uint32_t cus = (uint32_t)(cu_count > 0 ? cu_count : 256);
-  k_sim_units<LargeTier><<<cus, LargeTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps, b.flag,
-                                                             nullptr, g->woff, window_count(g->n) + 1, b.uedge, b.units,
-                                                             b.ucap, b.cnt, kCntUnits2, kCntQueue2,
-                                                             g->tuning.hash_tables != 0, nullptr, nullptr, nullptr, 0);
-  k_sim_units<SmallTier><<<cus * 8, SmallTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps,
-                                                                 b.flag, nullptr, nullptr, 0, b.uedge, b.units,
-                                                                 b.ucap, b.cnt, kCntUnits1, kCntQueue1,
-                                                                 g->tuning.hash_tables != 0, nullptr, nullptr, nullptr,
-                                                                 0);
+  launch_units(g, b, b.units, b.ucap, p, cus, false, nullptr, s, nullptr);
   launch_union(g, b, s, kCntRedo);
 }
 
