@@ -383,6 +383,12 @@ void launch_classify_edges(const sgc_dgraph* g, const PassBuffers& b, hipStream_
 // The pass's end: counters (sums folded) to host_cnt (page-locked, device
 // address), and the results to the device addresses given (any may be null);
 // after an overflow (kCntOverflow) the results are left alone.
+// All that follows the similarity phase, and the pass's end, in one launch:
+// graphs of few vertices and entries (tiny_graph), without the core-check
+// pruning.
+bool tiny_graph(const sgc_dgraph* g);
+void launch_tail(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, uint64_t* host_cnt, int32_t* labels,
+                 uint8_t* core, uint8_t* sim, hipStream_t s);
 void launch_publish(const sgc_dgraph* g, const PassBuffers& b, uint64_t* host_cnt, int32_t* labels, uint8_t* core,
                     uint8_t* sim, hipStream_t s);
 void launch_finalize(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStream_t s,

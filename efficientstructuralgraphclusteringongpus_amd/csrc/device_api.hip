@@ -535,29 +535,35 @@ int run_pass(sgc_ctx* ctx, sgc_dgraph* g, double eps, int32_t mu, PassBuffers* p
   launch_prep(g, *pb, p, s);
   launch_plan(g, *pb, p, s);
   launch_similarity(g, *pb, p, ctx->cu_count, ctx->sim_impl, nullptr, s);
-  launch_core(g, *pb, p, s);
-  launch_union(g, *pb, s);
-  // deferred edges the clusters or borders need, decided now
-  if (p.prune) launch_redo(g, *pb, p, ctx->cu_count, s);
-  if (!small) launch_flatten(g, *pb, s);
-  launch_border(g, *pb, s, small);
-  launch_classify(g, *pb, p, s);
-  // The last kernel hands over the counters and what it can write itself:
-  // results in this device's memory, and small ones for the host by way of
-  // the page-locked staging (three copies and a second wait cost more than
-  // 50 us of a pass of 170).
+  // Small results for the host go by way of the page-locked staging, those in
+  // this device's memory to their place, written by the pass's last kernel
+  // (three copies and a second wait cost more than 50 us of a pass of 170).
   const uint64_t n = g->n, m = g->m;
   const size_t o_core = (out.labels ? n * 4 : 0), o_sim = o_core + (out.core ? n : 0), bytes = o_sim + (out.sim ? m : 0);
   char* const stage = (char*)(ctx->host_counters + kCntWords);
   char* const stage_dev = (char*)(ctx->host_counters_dev + kCntWords);
   const bool staged = !out.device && bytes <= kStageBytes;
   const bool direct = out.device && on_device(ctx, out.labels) && on_device(ctx, out.core) && on_device(ctx, out.sim);
-  if (staged)
-    launch_publish(g, *pb, ctx->host_counters_dev, out.labels ? (int32_t*)stage_dev : nullptr,
-                   out.core ? (uint8_t*)stage_dev + o_core : nullptr, out.sim ? (uint8_t*)stage_dev + o_sim : nullptr, s);
-  else
-    launch_publish(g, *pb, ctx->host_counters_dev, direct ? out.labels : nullptr, direct ? out.core : nullptr,
-                   direct ? out.sim : nullptr, s);
+  int32_t* to_labels = staged || direct ? out.labels : nullptr;
+  uint8_t* to_core = staged || direct ? out.core : nullptr;
+  uint8_t* to_sim = staged || direct ? out.sim : nullptr;
+  if (staged) {
+    if (to_labels) to_labels = (int32_t*)stage_dev;
+    if (to_core) to_core = (uint8_t*)stage_dev + o_core;
+    if (to_sim) to_sim = (uint8_t*)stage_dev + o_sim;
+  }
+  if (tiny_graph(g) && !p.prune) {
+    launch_tail(g, *pb, p, ctx->host_counters_dev, to_labels, to_core, to_sim, s);
+  } else {
+    launch_core(g, *pb, p, s);
+    launch_union(g, *pb, s);
+    // deferred edges the clusters or borders need, decided now
+    if (p.prune) launch_redo(g, *pb, p, ctx->cu_count, s);
+    if (!small) launch_flatten(g, *pb, s);
+    launch_border(g, *pb, s, small);
+    launch_classify(g, *pb, p, s);
+    launch_publish(g, *pb, ctx->host_counters_dev, to_labels, to_core, to_sim, s);
+  }
   SGC_HIP(hipGetLastError());
   SGC_HIP(hipStreamSynchronize(s));
   if (int rc = check_unit_overflow(ctx->host_counters, g->m)) return rc;

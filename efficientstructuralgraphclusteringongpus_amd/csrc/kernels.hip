@@ -648,6 +648,190 @@ __global__ void __launch_bounds__(kBlock) k_publish(uint32_t n, uint64_t m, uint
   if (to_sim) grid_copy(flag, to_sim, m);
 }
 
+// Everything after the similarity phase of a tiny graph, from the core count
+// to the results, by one workgroup with the per-vertex state in LDS: the seven
+// kernels it replaces do less than a microsecond of work each in launches 2-5
+// us apart.  LDS: sd, then the lower label bound; parent, then the upper
+// bound; label; core.  Bound by the latency of one CU's loads, so only where
+// the entries are few: R-MAT with 10 / 12 thousand entries 67 / 66 -> 54 / 56
+// us a pass on the device, but 40 / 80 / 120 thousand 148 / 110 / 120 ->
+// 154 / 114 / 136.
+constexpr uint32_t kTailVertices = 8192, kTailEntries = 1u << 15;
+
+struct TailArgs {
+  uint32_t n, m;
+  const uint32_t* src;
+  const int32_t* adj;
+  const uint32_t* rb;
+  const uint32_t* re;
+  const uint8_t* flag;
+  int32_t mu;
+  int32_t* label;
+  uint8_t* core;
+  const uint64_t* cnt;
+  uint64_t* host_cnt;
+  int32_t* to_label;
+  uint8_t* to_core;
+  uint8_t* to_sim;
+};
+
+__global__ void __launch_bounds__(1024) k_tail(TailArgs a) {
+  constexpr uint32_t T = 1024;
+  extern __shared__ __align__(16) int32_t sh[];
+  __shared__ uint64_t s_stamp[4];
+  __shared__ unsigned long long s_sum[kStripeSlots];  // this kernel's share of the striped sums
+  const uint32_t tid = threadIdx.x, n = a.n, m = a.m;
+  int32_t* const lo = sh;
+  int32_t* const hi = sh + n;
+  int32_t* const label = sh + 2 * n;
+  uint8_t* const core = (uint8_t*)(sh + 3 * n);
+  uint32_t* const sd = (uint32_t*)lo;
+  volatile int32_t* const parent = hi;
+  auto start = [&](int i) {
+    __syncthreads();
+    if (tid == 0) s_stamp[i] = (uint64_t)wall_clock64();
+  };
+  // fn(k) for this thread's similar entries
+  auto for_similar = [&](auto fn) {
+    for (uint32_t k0 = tid * 16; k0 < m; k0 += T * 16) {
+      uint32_t mask = similar_mask(*reinterpret_cast<const uint4*>(a.flag + k0));
+      if (k0 + 16 > m) mask &= (1u << (m - k0)) - 1u;
+      for (; mask; mask &= mask - 1) fn(k0 + (uint32_t)__ffs(mask) - 1);
+    }
+  };
+  auto sum = [&](int slot, unsigned long long v) {
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_down(v, off);
+    if (lane_id() == 0 && v) atomicAdd(&s_sum[slot], v);
+  };
+  auto find = [&](int32_t x) {
+    int32_t p = parent[x];
+    while (p != x) {
+      const int32_t gp = parent[p];
+      if (gp != p) parent[x] = gp;  // path splitting
+      x = p;
+      p = gp;
+    }
+    return x;
+  };
+  for (uint32_t x = tid; x < n; x += T) sd[x] = 0;
+  if (tid < kStripeSlots) s_sum[tid] = 0;
+  start(0);
+  // ---- cores
+  for_similar([&](uint32_t k) { atomicAdd(&sd[a.src[k]], 1u); });
+  __syncthreads();
+  const uint32_t thr = a.mu >= 1 ? (uint32_t)a.mu : 1u;
+  uint32_t marked = 0, labeled = 0, similar = 0;
+  for (uint32_t x = tid; x < n; x += T) {
+    const bool c = sd[x] >= thr;
+    similar += sd[x];
+    core[x] = c;
+    marked += c;
+    if (c) labeled += a.re[x] - a.rb[x];
+    lo[x] = kNoLabel;
+    parent[x] = (int32_t)x;
+    label[x] = kNoLabel;
+  }
+  sum(kCntMarked, marked);
+  sum(kCntLabeled, labeled);
+  sum(kCntSimilar, similar);
+  start(1);
+  const bool any = s_sum[kCntMarked] != 0;
+  if (any) {
+    // ---- clusters
+    for_similar([&](uint32_t k) {
+      const uint32_t u = a.src[k];
+      const int32_t w = a.adj[k];
+      if ((uint32_t)w >= u || !core[u] || !core[w]) return;
+      for (;;) {
+        const int32_t ru = find((int32_t)u), rw = find(w);
+        if (ru == rw) return;
+        const int32_t top = ru > rw ? ru : rw, low = ru > rw ? rw : ru;
+        if (atomicCAS((int32_t*)&parent[top], top, low) == top) return;
+      }
+    });
+    __syncthreads();
+    for (uint32_t x = tid; x < n; x += T)
+      if (core[x]) label[x] = find((int32_t)x);
+    start(2);
+    // ---- borders: the minimum candidate id; core labels do not change
+    labeled = 0;
+    for_similar([&](uint32_t k) {
+      const uint32_t u = a.src[k];
+      const int32_t w = a.adj[k];
+      if (core[u] || !core[w]) return;
+      if (atomicMin(&label[u], label[w]) == kNoLabel) labeled += a.re[u] - a.rb[u];
+    });
+    sum(kCntLabeled, labeled);
+    for (uint32_t x = tid; x < n; x += T) hi[x] = -1;
+    start(3);
+    // ---- hubs and outliers, from the same side as k_classify
+    const bool from_labeled = 3 * s_sum[kCntLabeled] < m;
+    constexpr uint32_t C = 8;
+    for (uint32_t k0 = tid; k0 < m; k0 += T * C) {
+      uint32_t row[C];
+      int32_t nb[C];
+#pragma unroll
+      for (uint32_t j = 0; j < C; ++j) {
+        const uint32_t k = k0 + j * T;
+        row[j] = k < m ? a.src[k] : 0u;
+        nb[j] = k < m ? a.adj[k] : 0;
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < C; ++j) {
+        if (k0 + j * T >= m) continue;
+        const uint32_t from = from_labeled ? row[j] : (uint32_t)nb[j], to = from_labeled ? (uint32_t)nb[j] : row[j];
+        const int32_t l = label[from];
+        if (l == kNoLabel || label[to] != kNoLabel) continue;
+        if (l < lo[to]) atomicMin(&lo[to], l);
+        if (l > hi[to]) atomicMax(&hi[to], l);
+      }
+    }
+  } else {
+    start(2);
+    start(3);
+  }
+  __syncthreads();
+  // ---- roles and results
+  const bool publish = a.cnt[kCntOverflow] == 0;
+  RoleCounts rc;
+  PhaseView v{};
+  v.sd = nullptr, v.core = core, v.label = label, v.lo = lo, v.hi = hi;
+  for (uint32_t x = tid; x < n; x += T) {
+    const int32_t l = role_label(v, x, a.mu, &rc);
+    a.label[x] = l;
+    a.core[x] = core[x];
+    if (publish && a.to_label) a.to_label[x] = l;
+    if (publish && a.to_core) a.to_core[x] = core[x];
+  }
+  if (publish && a.to_sim) {
+    uint32_t done = 0;
+    if (((uintptr_t)a.to_sim & 15) == 0) {
+      done = m / 16 * 16;
+      for (uint32_t k = tid * 16; k < done; k += T * 16)
+        *reinterpret_cast<uint4*>(a.to_sim + k) = *reinterpret_cast<const uint4*>(a.flag + k);
+    }
+    for (uint32_t k = done + tid; k < m; k += T) a.to_sim[k] = a.flag[k];
+  }
+  sum(kCntCores, rc.cores);
+  sum(kCntClusters, rc.clusters);
+  sum(kCntBorders, rc.borders);
+  sum(kCntHubs, rc.hubs);
+  sum(kCntOutliers, rc.outliers);
+  __syncthreads();
+  if (tid < kCntSlots) {
+    uint64_t v = a.cnt[tid];
+    if (tid < kStripeSlots) {
+      for (uint32_t i = 0; i < kStripes; ++i) v += a.cnt[kStripe0 + i * kStripeSlots + tid];
+      v += s_sum[tid];
+    }
+    const int i = (int)tid - kCntStamp0;
+    if (i >= kStampCore && i < kStampEnd) v = s_stamp[i - kStampCore];
+    if (i == kStampEnd) v = (uint64_t)wall_clock64();
+    a.host_cnt[tid] = v;
+  }
+}
+
 // Plain streaming copy (16 bytes per lane per step), the reference point for
 // the HBM byte counters.
 __global__ void __launch_bounds__(kBlock) k_copy(const uint4* __restrict__ src, uint4* __restrict__ dst, uint64_t n) {
@@ -804,6 +988,15 @@ void launch_finalize(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hi
   k_finalize<<<grid_for(g->n, kBlock), kBlock, 0, s>>>(g->n, p.mu, mu_dev, b.sd, b.lo, b.hi, b.core, b.label, b.cnt);
 }
 
+
+bool tiny_graph(const sgc_dgraph* g) { return g->m && g->n <= kTailVertices && g->m <= kTailEntries; }
+
+void launch_tail(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, uint64_t* host_cnt, int32_t* labels,
+                 uint8_t* core, uint8_t* sim, hipStream_t s) {
+  const TailArgs a{g->n, g->m, g->src, g->adj, g->row_begin, g->row_end, b.flag, p.mu, b.label, b.core, b.cnt,
+                   host_cnt, labels, core, sim};
+  k_tail<<<1, 1024, (size_t)g->n * 13, s>>>(a);
+}
 
 void launch_publish(const sgc_dgraph* g, const PassBuffers& b, uint64_t* host_cnt, int32_t* labels, uint8_t* core,
                     uint8_t* sim, hipStream_t s) {

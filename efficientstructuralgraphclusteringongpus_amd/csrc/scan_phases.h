@@ -67,6 +67,19 @@ __device__ __forceinline__ void uf_union(int32_t* parent, int32_t a, int32_t b) 
   }
 }
 
+// Bit i: flag i of 16 says similar.
+__device__ __forceinline__ uint32_t similar_mask(const uint4 w) {
+  const uint32_t x[4] = {w.x, w.y, w.z, w.w};
+  uint32_t mask = 0;
+#pragma unroll
+  for (uint32_t q = 0; q < 4; ++q) {
+    const uint32_t z = x[q] ^ (0x01010101u * kFlagY);
+    const uint32_t t = ~(((z & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | z | 0x7F7F7F7Fu);  // 0x80 in zero bytes
+    mask |= (((t >> 7) & 1u) | ((t >> 14) & 2u) | ((t >> 21) & 4u) | ((t >> 28) & 8u)) << (4 * q);
+  }
+  return mask;
+}
+
 // The similar entries of the wave's tile [base, base + kFlagTile) of the flag
 // array, ascending, into `at` (the wave's kFlagTile words of LDS, offsets from
 // base); returns their number (uniform).  Flags come 16 to a load (flag must
@@ -88,14 +101,7 @@ __device__ __forceinline__ uint32_t similar_tile(const uint8_t* __restrict__ fla
 #pragma unroll
   for (uint32_t j = 0; j < L; ++j) {
     const uint64_t k = base + (j * kWave + lane) * 16;
-    const uint32_t x[4] = {w[j].x, w[j].y, w[j].z, w[j].w};
-    uint32_t mask = 0;  // bit i: entry k + i is similar
-#pragma unroll
-    for (uint32_t q = 0; q < 4; ++q) {
-      const uint32_t z = x[q] ^ (0x01010101u * kFlagY);
-      const uint32_t t = ~(((z & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | z | 0x7F7F7F7Fu);  // 0x80 in zero bytes
-      mask |= (((t >> 7) & 1u) | ((t >> 14) & 2u) | ((t >> 21) & 4u) | ((t >> 28) & 8u)) << (4 * q);
-    }
+    uint32_t mask = similar_mask(w[j]);
     if (k + 16 > m) mask &= k < m ? (1u << (uint32_t)(m - k)) - 1u : 0u;
     if (!__ballot(mask != 0)) continue;
     const uint32_t incl = wave_incl_scan((uint32_t)__popc(mask));
@@ -260,8 +266,7 @@ __device__ __forceinline__ void count_roles(uint64_t* cnt, const RoleCounts& rc)
                {rc.cores, rc.clusters, rc.borders, rc.hubs, rc.outliers, rc.similar});
 }
 
-__device__ __forceinline__ int32_t finalize_vertex(const PhaseView& v, uint32_t x, int32_t mu, RoleCounts* rc) {
-  rc->similar += v.sd[x];
+__device__ __forceinline__ int32_t role_label(const PhaseView& v, uint32_t x, int32_t mu, RoleCounts* rc) {
   int32_t l = v.label[x];
   if (v.core[x]) {
     ++rc->cores;
@@ -278,6 +283,11 @@ __device__ __forceinline__ int32_t finalize_vertex(const PhaseView& v, uint32_t 
     rc->outliers += !hub;
   }
   return l;
+}
+
+__device__ __forceinline__ int32_t finalize_vertex(const PhaseView& v, uint32_t x, int32_t mu, RoleCounts* rc) {
+  rc->similar += v.sd[x];
+  return role_label(v, x, mu, rc);
 }
 
 }  // namespace sgc

@@ -1226,7 +1226,12 @@ namespace {
 void launch_units(const sgc_dgraph* g, const PassBuffers& b, const uint4* units, uint32_t ucap, ScanParams p,
                   uint32_t cus, bool prune, hipEvent_t mid, hipStream_t s, uint32_t* cn_out) {
   const bool hash = g->tuning.hash_tables != 0;
-  if (hash && !prune && exact_units_cover(g->n, true))
+  // no launch for units that no row is long enough for (a chip's longest row
+  // is not known)
+  const bool any_large = !g->max_degree || g->max_degree > std::min(g->tuning.small_max_degree, kT1MaxDeg);
+  if (!any_large)
+    ;
+  else if (hash && !prune && exact_units_cover(g->n, true))
     launch_exact_units(g, b, units, ucap, p, (int)cus, s, true, cn_out);
   else
     k_sim_units<LargeTier><<<cus, LargeTier::kThreads, 0, s>>>(g->n, g->m, g->src, g->adj, g->mirror, p.eps, b.flag,
