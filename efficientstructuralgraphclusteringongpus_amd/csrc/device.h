@@ -288,11 +288,12 @@ int upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgraph**
 
 // Kernel launchers (kernels.hip, similarity.hip, filter.hip).  All run on `s` and never
 // synchronise.
-void launch_fill_src(const sgc_dgraph* g, hipStream_t s);
-// fills g->mirror (after launch_fill_src) by a search per entry; entries
+// src[k] = base + the row of entry k, for n rows that start at rp[0 .. n]
+void launch_fill_rows(const uint32_t* rp, uint32_t n, uint32_t m, uint32_t base, uint32_t* src, hipStream_t s);
+// fills g->mirror (after g->src) by a search per entry; entries
 // without a reverse entry get 0xFFFFFFFF
 void launch_mirror(const sgc_dgraph* g, hipStream_t s);
-// fills g->mirror (after launch_fill_src) by a stable sort of the entries by
+// fills g->mirror (after g->src), on large graphs by a stable sort of the entries by
 // neighbour in the context's work buffer, or by launch_mirror where the input
 // is not symmetric or the buffer's memory is not there; synchronises the
 // stream

@@ -422,7 +422,7 @@ int sgc::upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgr
   hipError_t e = upload_bytes(ctx, d->row_ptr, rp32.data(), (g->n + 1) * 4, false);
   if (e == hipSuccess && g->m) e = upload_bytes(ctx, d->adj, g->adj, g->m * 4, g->pinned);
   if (e == hipSuccess) {
-    launch_fill_src(d, ctx->stream);
+    launch_fill_rows(d->row_ptr, d->n, d->m, 0, d->src, ctx->stream);
     e = build_mirror(ctx, d);
   }
   if (e == hipSuccess) {

@@ -21,14 +21,52 @@ namespace {
 // Graph preparation
 // ---------------------------------------------------------------------------
 
-// src[k] = row of entry k; one wave per vertex, lanes stride the row.
-__global__ void __launch_bounds__(kBlock) k_fill_src(uint32_t n, const uint32_t* __restrict__ rp,
-                                                     uint32_t* __restrict__ src) {
+// The last of rows [lo, hi] that starts at k or before, given that lo does: 64
+// pivots to a round.
+__device__ __forceinline__ uint32_t wave_row_of(const uint32_t* __restrict__ rp, uint32_t lo, uint32_t hi, uint32_t k) {
   const uint32_t lane = lane_id();
-  const uint64_t waves = (uint64_t)gridDim.x * (kBlock / kWave);
-  for (uint64_t x = (uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; x < n; x += waves) {
-    const uint32_t b = rp[x], e = rp[x + 1];
-    for (uint32_t k = b + lane; k < e; k += kWave) src[k] = (uint32_t)x;
+  while (hi - lo >= kWave) {
+    const uint64_t w = (uint64_t)hi - lo + 1;
+    const uint32_t le = (uint32_t)__popcll(__ballot(rp[lo + (uint32_t)(w * lane / kWave)] <= k));  // at least 1
+    const uint32_t at = lo;
+    lo = at + (uint32_t)(w * (le - 1) / kWave);
+    if (le < kWave) hi = at + (uint32_t)(w * le / kWave) - 1;
+  }
+  return lo + (uint32_t)__popcll(__ballot(lane <= hi - lo && rp[lo + lane] <= k)) - 1;
+}
+
+// src[k] = base + the row of entry k.  A wave takes 1024 entries, finds the
+// rows of the first and the last and searches the others between them: stores
+// are whole lines and no row is long or short for it.  A wave to a row took
+// 256 us on R-MAT-20 (3.1e7 entries) and 59 on R-MAT-18.
+constexpr uint32_t kFillTile = 1024;
+
+__global__ void __launch_bounds__(kBlock) k_fill_rows(uint32_t n, uint32_t m, uint32_t base,
+                                                      const uint32_t* __restrict__ rp, uint32_t* __restrict__ src) {
+  constexpr uint32_t C = 4;
+  const uint32_t lane = lane_id();
+  const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * kFillTile;
+  for (uint64_t t = ((uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * kFillTile; t < m; t += step) {
+    const uint32_t t0 = (uint32_t)t, len = min(m - t0, kFillTile);
+    const uint32_t first = wave_row_of(rp, 0, n - 1, t0), last = wave_row_of(rp, first, n - 1, t0 + len - 1);
+    for (uint32_t i = lane; i < len; i += kWave * C) {
+      uint32_t lo[C], hi[C];
+#pragma unroll
+      for (uint32_t j = 0; j < C; ++j) lo[j] = first, hi[j] = last;
+      for (uint32_t left = last - first; left; left >>= 1) {
+#pragma unroll
+        for (uint32_t j = 0; j < C; ++j) {
+          const uint32_t mid = lo[j] + ((hi[j] - lo[j] + 1) >> 1);
+          if (rp[mid] <= t0 + min(i + j * kWave, len - 1))
+            lo[j] = mid;
+          else
+            hi[j] = mid - 1;  // above lo: mid = lo only when lo = hi, and then rp[lo] <= k
+        }
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < C; ++j)
+        if (i + j * kWave < len) src[t0 + i + j * kWave] = base + lo[j];
+    }
   }
 }
 
@@ -846,9 +884,8 @@ void launch_copy(const void* src, void* dst, uint64_t bytes, hipStream_t s) {
   if (n) k_copy<<<grid_for(n, kBlock), kBlock, 0, s>>>((const uint4*)src, (uint4*)dst, n);
 }
 
-void launch_fill_src(const sgc_dgraph* g, hipStream_t s) {
-  if (g->n == 0 || g->m == 0) return;
-  k_fill_src<<<grid_for(g->n, kBlock / kWave), kBlock, 0, s>>>(g->n, g->row_ptr, g->src);
+void launch_fill_rows(const uint32_t* rp, uint32_t n, uint32_t m, uint32_t base, uint32_t* src, hipStream_t s) {
+  if (n && m) k_fill_rows<<<grid_for(m, kFillTile * (kBlock / kWave)), kBlock, 0, s>>>(n, m, base, rp, src);
 }
 
 void launch_neighbor_degrees(const sgc_dgraph* g, hipStream_t s) {
@@ -863,10 +900,20 @@ void launch_mirror(const sgc_dgraph* g, hipStream_t s) {
   k_mirror<<<grid_for(g->m, kBlock), kBlock, 0, s>>>(g->m, g->row_ptr, g->src, g->adj, g->mirror);
 }
 
+// Up to here the search is the faster (the sort takes ten launches and more
+// each of a fixed time; the search's loads fall out of L2 later): R-MAT-14 14
+// us against 160, R-MAT-18 (7.6e6 entries) 323 against 358, R-MAT-20 1800
+// against 1270.
+constexpr uint32_t kSearchEntries = 1u << 23;
+
 hipError_t build_mirror(sgc_ctx* ctx, const sgc_dgraph* g) {
   if (!g->m || !g->mirror) return hipSuccess;
   hipStream_t s = ctx->stream;
   const uint32_t m = g->m;
+  if (m <= kSearchEntries) {
+    launch_mirror(g, s);
+    return hipGetLastError();
+  }
   int bits = 1;
   while (bits < 32 && (1ull << bits) < (uint64_t)g->n) ++bits;
   size_t tmp_bytes = 0;

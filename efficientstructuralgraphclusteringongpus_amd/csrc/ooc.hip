@@ -68,18 +68,6 @@ __global__ void __launch_bounds__(kBlock) k_chip_init(uint32_t a0, uint32_t a1, 
     for (uint32_t t = threadIdx.x; t < kCntWords; t += kBlock) cnt[t] = 0;
 }
 
-// src[k] = r0 + i for the entries [off[i], off[i+1]) of chip row i; one wave
-// per row.
-__global__ void __launch_bounds__(kBlock) k_fill_src_rows(uint32_t r0, uint32_t nr, const uint32_t* __restrict__ off,
-                                                          uint32_t* __restrict__ src) {
-  const uint32_t lane = lane_id();
-  const uint64_t waves = (uint64_t)gridDim.x * (kBlock / kWave);
-  for (uint64_t i = (uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; i < nr; i += waves) {
-    const uint32_t b = off[i], e = off[i + 1];
-    for (uint32_t k = b + lane; k < e; k += kWave) src[k] = r0 + (uint32_t)i;
-  }
-}
-
 float elapsed(hipEvent_t a, hipEvent_t b) {
   float ms = 0.f;
   return hipEventElapsedTime(&ms, a, b) == hipSuccess ? ms : 0.f;
@@ -474,7 +462,7 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
       if (used[b]) SGC_HIP(hipStreamWaitEvent(R.h2d, R.comp[b], 0));
     if ((rc = upload_rows(R.stage[0], gi, ge, J, R.off_i, R.up_i))) return rc;
     SGC_HIP(hipStreamWaitEvent(s, R.up_i, 0));
-    if (nri) k_fill_src_rows<<<grid_for(nri, kBlock / kWave), kBlock, 0, s>>>((uint32_t)c.r0i, nri, R.off_i, A.src + J);
+    launch_fill_rows(R.off_i, nri, (uint32_t)c.mi, (uint32_t)c.r0i, A.src + J, s);
     // the group's flags are rewritten once the previous group's are back
     if (any_group) SGC_HIP(hipStreamWaitEvent(s, R.back_i, 0));
     any_group = true;
@@ -497,9 +485,7 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
         if (used[b]) SGC_HIP(hipStreamWaitEvent(R.h2d, R.comp[b], 0));
         if ((rc = upload_rows(sj, j, j + 1, jpos, R.off_j[b], R.up_j[b]))) return rc;
         SGC_HIP(hipStreamWaitEvent(s, R.up_j[b], 0));
-        if (nrj)
-          k_fill_src_rows<<<grid_for(nrj, kBlock / kWave), kBlock, 0, s>>>((uint32_t)c.r0j, nrj, R.off_j[b],
-                                                                           A.src + jpos);
+        launch_fill_rows(R.off_j[b], nrj, (uint32_t)c.mj, (uint32_t)c.r0j, A.src + jpos, s);
         if (b == 0) {
           base = jpos;
           c.j_first = true;
@@ -617,7 +603,7 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
       SGC_HIP(hipMemcpyAsync(c_off, ho, ((size_t)nr + 1) * 4, hipMemcpyHostToDevice, s));
       SGC_HIP(upload_bytes(ctx, c_flag, R.flag + b0, mc, !R.flag_pageable));
       R.bytes_h2d += (double)mc + (double)(nr + 1) * 4;
-      if (nr) k_fill_src_rows<<<grid_for(nr, kBlock / kWave), kBlock, 0, s>>>((uint32_t)r0, nr, c_off, c_src);
+      launch_fill_rows(c_off, nr, (uint32_t)mc, (uint32_t)r0, c_src, s);
       loaded = i;
       loaded_adj = false;
     }
