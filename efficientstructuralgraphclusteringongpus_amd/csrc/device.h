@@ -290,16 +290,11 @@ int upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgraph**
 // synchronise.
 // src[k] = base + the row of entry k, for n rows that start at rp[0 .. n]
 void launch_fill_rows(const uint32_t* rp, uint32_t n, uint32_t m, uint32_t base, uint32_t* src, hipStream_t s);
-// fills g->mirror (after g->src) by a search per entry; entries
-// without a reverse entry get 0xFFFFFFFF
-void launch_mirror(const sgc_dgraph* g, hipStream_t s);
-// fills g->mirror (after g->src), on large graphs by a stable sort of the entries by
-// neighbour in the context's work buffer, or by launch_mirror where the input
-// is not symmetric or the buffer's memory is not there; synchronises the
-// stream
-hipError_t build_mirror(sgc_ctx* ctx, const sgc_dgraph* g);
-// fills g->ndeg
-void launch_neighbor_degrees(const sgc_dgraph* g, hipStream_t s);
+// Fills g->ndeg and g->mirror (after g->src), whichever are there.  Entries
+// without a reverse entry get mirror word 0xFFFFFFFF.  Works in the context's
+// work buffer; without its memory the reverse entries are searched one by
+// one.  May synchronise the stream.
+hipError_t build_indexes(sgc_ctx* ctx, const sgc_dgraph* g);
 // 2^20-id windows of the large-tier bitmap covering n ids, and the kernel
 // filling g->woff (see sgc_dgraph).
 uint32_t window_count(uint32_t n);

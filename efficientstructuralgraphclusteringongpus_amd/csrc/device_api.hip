@@ -423,10 +423,9 @@ int sgc::upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgr
   if (e == hipSuccess && g->m) e = upload_bytes(ctx, d->adj, g->adj, g->m * 4, g->pinned);
   if (e == hipSuccess) {
     launch_fill_rows(d->row_ptr, d->n, d->m, 0, d->src, ctx->stream);
-    e = build_mirror(ctx, d);
+    e = build_indexes(ctx, d);
   }
   if (e == hipSuccess) {
-    launch_neighbor_degrees(d, ctx->stream);
     launch_window_offsets(d, ctx->stream);
     e = hipGetLastError();
     if (e == hipSuccess) e = build_packed_rows(ctx, d);

@@ -190,6 +190,132 @@ __global__ void __launch_bounds__(kBlock) k_mirror_from_sorted(uint32_t m, const
   block_atomic_add(bad, miss);
 }
 
+// The reverse-entry index of mid-size graphs by splitting: the searches of
+// k_mirror whose rows start in the same 2^15 entries of the adjacency meet in
+// one bucket, whose rows then lie in LDS.  k_split_searches writes one item a
+// search, (entry, its row, where its neighbour's row starts in the bucket and
+// its length), in runs of a tile's items for a bucket, and the neighbour
+// degrees on the way; k_bucket_searches finds and writes.  Searches in rows
+// over kBucketRow, and those a bucket has no room for (input whose entries
+// lack their reverse), are done on the spot.  Bound by the item and index
+// traffic, about 40 bytes an entry: R-MAT-20 (3.1e7 entries) 0.64 ms with the
+// neighbour degrees, 1.44 by the sort; R-MAT-22 2.9 and 4.8.
+constexpr uint32_t kBucketBits = 15, kBucketRow = 4096;
+constexpr uint32_t kBucketCap = (1u << kBucketBits) + kBucketRow;  // a bucket's rows hold no more
+constexpr uint32_t kBuckets = 4096;
+constexpr uint32_t kSplitEntries = kBuckets << kBucketBits;  // largest graph
+
+// The position of x in the sorted row a[lo, hi), or 0xFFFFFFFF.
+__device__ __forceinline__ uint32_t find_in_row(const int32_t* a, uint32_t lo, uint32_t hi, int32_t x) {
+  const uint32_t end = hi;
+  while (lo < hi) {
+    const uint32_t mid = lo + ((hi - lo) >> 1);
+    if (a[mid] < x)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  return lo < end && a[lo] == x ? lo : 0xFFFFFFFFu;
+}
+
+struct SplitItem {
+  uint32_t k, u, row;  // row: its start in the bucket, length << kBucketBits
+};
+
+__global__ void __launch_bounds__(1024) k_split_searches(uint32_t m, const uint32_t* __restrict__ rp,
+                                                         const uint32_t* __restrict__ src,
+                                                         const int32_t* __restrict__ adj, uint32_t* __restrict__ ndeg,
+                                                         uint32_t* __restrict__ mirror, uint32_t* __restrict__ cursor,
+                                                         SplitItem* __restrict__ items, uint32_t buckets) {
+  constexpr uint32_t T = 1024, C = 16;
+  __shared__ uint32_t s_count[kBuckets], s_base[kBuckets];
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t b = tid; b < buckets; b += T) s_count[b] = 0;
+  __syncthreads();
+  for (uint64_t t0 = (uint64_t)blockIdx.x * T * C; t0 < m; t0 += (uint64_t)gridDim.x * T * C) {  // block-uniform
+    uint32_t u[C], start[C], len[C], at[C];  // len 0: no search; at: its place among the tile's items of its bucket
+#pragma unroll
+    for (uint32_t j = 0; j < C; ++j) {
+      const uint64_t k = t0 + j * T + tid;
+      u[j] = k < m ? src[k] : 0u;
+      at[j] = k < m ? (uint32_t)adj[k] : 0u;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < C; ++j) {
+      const uint64_t k = t0 + j * T + tid;
+      const uint32_t v = at[j], du = rp[u[j] + 1] - rp[u[j]];
+      start[j] = rp[v];
+      const uint32_t dv = rp[v + 1] - start[j];
+      if (k < m) ndeg[k] = dv;
+      len[j] = k < m && (dv < du || (dv == du && v <= u[j])) ? dv : 0u;
+      if (len[j] > kBucketRow) {
+        const uint32_t p = find_in_row(adj, start[j], start[j] + dv, (int32_t)u[j]);
+        if (p != 0xFFFFFFFFu) {
+          mirror[k] = p;
+          mirror[p] = (uint32_t)k;
+        }
+        len[j] = 0;
+      }
+      if (len[j]) at[j] = atomicAdd(&s_count[start[j] >> kBucketBits], 1u);
+    }
+    __syncthreads();
+    for (uint32_t b = tid; b < buckets; b += T) {
+      const uint32_t c = s_count[b];
+      if (c) s_base[b] = atomicAdd(&cursor[b], c);
+      s_count[b] = 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < C; ++j) {
+      if (!len[j]) continue;
+      const uint32_t k = (uint32_t)(t0 + j * T + tid), b = start[j] >> kBucketBits, i = s_base[b] + at[j];
+      if (i < kBucketCap) {
+        items[(uint64_t)b * kBucketCap + i] =
+            SplitItem{k, u[j], (start[j] & ((1u << kBucketBits) - 1)) | len[j] << kBucketBits};
+      } else {
+        const uint32_t p = find_in_row(adj, start[j], start[j] + len[j], (int32_t)u[j]);
+        if (p != 0xFFFFFFFFu) {
+          mirror[k] = p;
+          mirror[p] = k;
+        }
+      }
+    }
+    __syncthreads();  // s_base is rewritten
+  }
+}
+
+// Block b: bucket b.
+__global__ void __launch_bounds__(1024) k_bucket_searches(uint32_t m, const int32_t* __restrict__ adj,
+                                                          const uint32_t* __restrict__ cursor,
+                                                          const SplitItem* __restrict__ items,
+                                                          uint32_t* __restrict__ mirror) {
+  constexpr uint32_t T = 1024, C = 4;
+  __shared__ __align__(16) int32_t rows[kBucketCap];
+  const uint32_t b0 = blockIdx.x << kBucketBits, span = min(m - b0, kBucketCap), tid = threadIdx.x;
+  const uint32_t count = min(cursor[blockIdx.x], kBucketCap);
+  if (!count) return;
+  for (uint32_t t = tid * 4; t < span / 4 * 4; t += T * 4)
+    *reinterpret_cast<int4*>(rows + t) = *reinterpret_cast<const int4*>(adj + b0 + t);
+  if (tid < span % 4) rows[span / 4 * 4 + tid] = adj[b0 + span / 4 * 4 + tid];
+  __syncthreads();
+  const SplitItem* const it = items + (uint64_t)blockIdx.x * kBucketCap;
+  for (uint32_t i0 = tid; i0 < count; i0 += T * C) {
+    SplitItem q[C];
+#pragma unroll
+    for (uint32_t j = 0; j < C; ++j) q[j] = it[min(i0 + j * T, count - 1)];
+#pragma unroll
+    for (uint32_t j = 0; j < C; ++j) {
+      if (i0 + j * T >= count) break;
+      const uint32_t lo = q[j].row & ((1u << kBucketBits) - 1);
+      const uint32_t p = find_in_row(rows, lo, lo + (q[j].row >> kBucketBits), (int32_t)q[j].u);
+      if (p != 0xFFFFFFFFu) {
+        mirror[q[j].k] = b0 + p;
+        mirror[b0 + p] = q[j].k;
+      }
+    }
+  }
+}
+
 // ndeg[k] = d(adj[k]), so the prep kernel streams the neighbour degrees
 // instead of gathering two row offsets per entry on every pass.
 __global__ void __launch_bounds__(kBlock) k_neighbor_degrees(uint32_t m, const uint32_t* __restrict__ rp,
@@ -888,25 +1014,48 @@ void launch_fill_rows(const uint32_t* rp, uint32_t n, uint32_t m, uint32_t base,
   if (n && m) k_fill_rows<<<grid_for(m, kFillTile * (kBlock / kWave)), kBlock, 0, s>>>(n, m, base, rp, src);
 }
 
-void launch_neighbor_degrees(const sgc_dgraph* g, hipStream_t s) {
+static void launch_neighbor_degrees(const sgc_dgraph* g, hipStream_t s) {
   if (g->m && g->ndeg)
     k_neighbor_degrees<<<grid_for(g->m, kBlock), kBlock, 0, s>>>(g->m, g->row_ptr, g->adj, g->ndeg);
 }
 
-void launch_mirror(const sgc_dgraph* g, hipStream_t s) {
+static void launch_mirror(const sgc_dgraph* g, hipStream_t s) {
   if (!g->m || !g->mirror) return;
   // words of entries without a reverse entry are never written by k_mirror
   (void)hipMemsetAsync(g->mirror, 0xFF, (size_t)g->m * 4, s);
   k_mirror<<<grid_for(g->m, kBlock), kBlock, 0, s>>>(g->m, g->row_ptr, g->src, g->adj, g->mirror);
 }
 
-// Up to here the search is the faster (the sort takes ten launches and more
-// each of a fixed time; the search's loads fall out of L2 later): R-MAT-14 14
-// us against 160, R-MAT-18 (7.6e6 entries) 323 against 358, R-MAT-20 1800
-// against 1270.
-constexpr uint32_t kSearchEntries = 1u << 23;
+// Up to here one search an entry is as fast (its rows come from L2): with the
+// neighbour degrees, 1.8e6 entries 65 us against 63 split, but 4e6 161 against
+// 76, 7.6e6 (R-MAT-18) 366 / 145.  Above kSplitEntries the sort takes over: a
+// bucket's rows no longer fit LDS, or its items come one by one.
+constexpr uint32_t kSearchEntries = 1u << 21;
 
-hipError_t build_mirror(sgc_ctx* ctx, const sgc_dgraph* g) {
+static hipError_t build_mirror(sgc_ctx* ctx, const sgc_dgraph* g);
+
+hipError_t build_indexes(sgc_ctx* ctx, const sgc_dgraph* g) {
+  hipStream_t s = ctx->stream;
+  const uint32_t m = g->m;
+  if (m > kSearchEntries && m <= kSplitEntries && g->mirror && g->ndeg) {
+    const uint32_t buckets = (m + (1u << kBucketBits) - 1) >> kBucketBits;
+    char* const mem = (char*)work_memory(ctx, (size_t)buckets * (kBucketCap * sizeof(SplitItem) + 4));
+    if (mem) {
+      uint32_t* const cursor = (uint32_t*)(mem + (size_t)buckets * kBucketCap * sizeof(SplitItem));
+      hipError_t e = hipMemsetAsync(cursor, 0, (size_t)buckets * 4, s);
+      if (e == hipSuccess) e = hipMemsetAsync(g->mirror, 0xFF, (size_t)m * 4, s);
+      if (e != hipSuccess) return e;
+      k_split_searches<<<std::min(grid_for(m, 16384), 1024u), 1024, 0, s>>>(m, g->row_ptr, g->src, g->adj, g->ndeg,
+                                                                             g->mirror, cursor, (SplitItem*)mem, buckets);
+      k_bucket_searches<<<buckets, 1024, 0, s>>>(m, g->adj, cursor, (const SplitItem*)mem, g->mirror);
+      return hipGetLastError();
+    }
+  }
+  launch_neighbor_degrees(g, s);
+  return build_mirror(ctx, g);
+}
+
+static hipError_t build_mirror(sgc_ctx* ctx, const sgc_dgraph* g) {
   if (!g->m || !g->mirror) return hipSuccess;
   hipStream_t s = ctx->stream;
   const uint32_t m = g->m;
