@@ -462,13 +462,6 @@ __global__ void __launch_bounds__(kBlock) k_similarity_wave(const uint32_t* __re
 // Core check (GPUSCAN++/GPUScan.cu:115-131, :276-367)
 // ---------------------------------------------------------------------------
 
-// The core count and the union-find take this many wave loads of listed
-// entries at a time: each entry costs two to four dependent gathers, and one
-// load at a time left them waiting (planted communities, n = 3e5, 7e6 similar
-// entries: core count 65 -> 39 us, union-find 260 -> 225; the border pass,
-// whose entries rarely pass the first gather, gains nothing: 72 / 76).
-constexpr uint32_t kListed = 4;
-
 // Similar entries per row, from the flags' similar entries alone: one
 // atomic per run of a row's entries in a wave's 64.
 __global__ void __launch_bounds__(kBlock) k_core_count(uint64_t m, const uint32_t* __restrict__ src,
@@ -476,28 +469,12 @@ __global__ void __launch_bounds__(kBlock) k_core_count(uint64_t m, const uint32_
                                                        uint64_t* __restrict__ cnt) {
   stamp(cnt, kStampCore);
   __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
-  const uint32_t lane = lane_id(), wv = threadIdx.x / kWave;
+  const uint32_t wv = threadIdx.x / kWave;
+  PhaseView v{};
+  v.m = (uint32_t)m, v.src = src, v.flag = flag, v.sd = sd;
   const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * kFlagTile;
-  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * kFlagTile; base < m; base += step) {
-    const uint32_t total = similar_tile(flag, m, base, s_at[wv]);
-    for (uint32_t i0 = 0; i0 < total; i0 += kWave * kListed) {
-      uint32_t row[kListed];
-#pragma unroll
-      for (uint32_t j = 0; j < kListed; ++j) {
-        const uint32_t i = i0 + j * kWave + lane;
-        row[j] = i < total ? src[base + s_at[wv][i]] : 0xFFFFFFFFu;
-      }
-#pragma unroll
-      for (uint32_t j = 0; j < kListed; ++j) {
-        if (i0 + j * kWave >= total) break;
-        const bool head = wave_seg_head(row[j]);
-        const uint64_t after = __ballot(head) & ~lanemask_le(lane);
-        const uint32_t stop = after ? (uint32_t)(__ffsll((long long)after) - 1) : (uint32_t)kWave;
-        if (head && row[j] != 0xFFFFFFFFu) atomicAdd(&sd[row[j]], stop - lane);
-      }
-    }
-    wave_lds_sync();  // the list is rewritten
-  }
+  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * kFlagTile; base < m; base += step)
+    core_count_tile(v, base, s_at[wv]);
 }
 
 // core(x) <=> #similar neighbours >= mu (mu <= 0: >= 1).  The reference's
@@ -557,41 +534,12 @@ __global__ void __launch_bounds__(kBlock) k_union(uint64_t m, const uint32_t* __
   if (HEADS && cores <= kFewCores) return;
   if (gate >= 0 && !count_any(cnt, gate)) return;
   __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
-  const uint32_t lane = lane_id(), wv = threadIdx.x / kWave;
+  const uint32_t wv = threadIdx.x / kWave;
+  PhaseView v{};
+  v.m = (uint32_t)m, v.src = src, v.adj = adj, v.flag = flag, v.core = const_cast<uint8_t*>(core), v.parent = parent;
   const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * kFlagTile;
-  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * kFlagTile; base < m; base += step) {
-    const uint32_t total = similar_tile(flag, m, base, s_at[wv]);
-    for (uint32_t i0 = 0; i0 < total; i0 += kWave * kListed) {
-      uint32_t u[kListed];
-      int32_t w[kListed];
-      bool on[kListed];
-#pragma unroll
-      for (uint32_t j = 0; j < kListed; ++j) {
-        const uint32_t i = i0 + j * kWave + lane;
-        const uint64_t k = base + (i < total ? s_at[wv][i] : 0);
-        u[j] = i < total ? src[k] : 0u;
-        w[j] = i < total ? adj[k] : 0;
-      }
-#pragma unroll
-      for (uint32_t j = 0; j < kListed; ++j) on[j] = (uint32_t)w[j] < u[j] && core[u[j]] && core[w[j]];
-      if (!HEADS) {
-#pragma unroll
-        for (uint32_t j = 0; j < kListed; ++j) on[j] = on[j] && parent[u[j]] != parent[w[j]];
-      }
-#pragma unroll
-      for (uint32_t j = 0; j < kListed; ++j) {
-        if (HEADS) {
-          // the first of the row's entries among the lanes that are on
-          const uint64_t below = __ballot(on[j]) & lanemask_lt(lane);
-          const uint32_t prev = below ? 63u - (uint32_t)__clzll((long long)below) : lane;
-          const uint32_t pu = (uint32_t)__shfl((int)u[j], (int)prev);
-          on[j] = on[j] && (!below || pu != u[j]);
-        }
-        if (on[j]) uf_union(parent, (int32_t)u[j], w[j]);
-      }
-    }
-    wave_lds_sync();  // the list is rewritten
-  }
+  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * kFlagTile; base < m; base += step)
+    union_tile<HEADS>(v, base, s_at[wv]);
 }
 
 __global__ void __launch_bounds__(kBlock) k_compress(uint32_t n, const uint8_t* __restrict__ core, int32_t* parent,
@@ -678,21 +626,15 @@ __global__ void __launch_bounds__(kBlock) k_border(uint32_t n, uint64_t m, int32
   }
   __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
   PhaseView v{};
-  v.src = src, v.adj = adj, v.core = const_cast<uint8_t*>(core), v.rb = rb, v.re = re, v.label = label;
-  v.parent = parent;
-  const uint32_t lane = lane_id(), wv = threadIdx.x / kWave;
+  v.m = (uint32_t)m, v.src = src, v.adj = adj, v.flag = flag, v.core = const_cast<uint8_t*>(core);
+  v.rb = rb, v.re = re, v.label = label, v.parent = parent;
+  const uint32_t wv = threadIdx.x / kWave;
   const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * kFlagTile;
   // entries of the border rows this lane labels first; the core rows'
   // entries were counted by k_core_mark
   uint64_t labeled = 0;
-  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * kFlagTile; base < m; base += step) {
-    const uint32_t total = similar_tile(flag, m, base, s_at[wv]);
-    for (uint32_t i0 = 0; i0 < total; i0 += kWave) {
-      const bool on = i0 + lane < total;
-      labeled += border_entry<FLATTEN>(v, base + (on ? s_at[wv][i0 + lane] : 0), on);
-    }
-    wave_lds_sync();  // the list is rewritten
-  }
+  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * kFlagTile; base < m; base += step)
+    labeled += border_tile<FLATTEN>(v, base, s_at[wv]);
   count_add<1>(cnt, {kCntLabeled}, {labeled});
 }
 

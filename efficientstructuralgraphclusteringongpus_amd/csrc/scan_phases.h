@@ -113,27 +113,73 @@ __device__ __forceinline__ uint32_t similar_tile(const uint8_t* __restrict__ fla
   return total;
 }
 
-// Joins the similar core-core edges among entries k_j = k0 + j * step
-// (j < kEdgeChunks), each visited from its larger endpoint.
-__device__ __forceinline__ void union_entries(const PhaseView& v, uint64_t k0, uint64_t step) {
-  constexpr uint32_t C = kEdgeChunks;
-  uint32_t u[C];
-  int32_t w[C];
-  bool y[C];
+// The core count and the union-find take this many wave loads of listed
+// entries at a time: each entry costs two to four dependent gathers, and one
+// load at a time left them waiting (planted communities, n = 3e5, 7e6 similar
+// entries: core count 65 -> 39 us, union-find 260 -> 225; the border pass,
+// whose entries rarely pass the first gather, gains nothing: 72 / 76).
+constexpr uint32_t kListed = 4;
+
+// Similar entries per row among the wave's tile at `base`: one atomic per run
+// of a row's entries in a wave's 64.
+__device__ __forceinline__ void core_count_tile(const PhaseView& v, uint64_t base, uint16_t* at) {
+  const uint32_t lane = lane_id();
+  const uint32_t total = similar_tile(v.flag, v.m, base, at);
+  for (uint32_t i0 = 0; i0 < total; i0 += kWave * kListed) {
+    uint32_t row[kListed];
 #pragma unroll
-  for (uint32_t j = 0; j < C; ++j) {
-    const uint64_t k = k0 + j * step;
-    y[j] = k < v.m && v.flag[k] == kFlagY;
-    u[j] = y[j] ? v.src[k] : 0u;
-    w[j] = y[j] ? v.adj[k] : 0;
-    y[j] = y[j] && (uint32_t)w[j] < u[j];
+    for (uint32_t j = 0; j < kListed; ++j) {
+      const uint32_t i = i0 + j * kWave + lane;
+      row[j] = i < total ? v.src[base + at[i]] : 0xFFFFFFFFu;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kListed; ++j) {
+      if (i0 + j * kWave >= total) break;
+      const bool head = wave_seg_head(row[j]);
+      const uint64_t after = __ballot(head) & ~lanemask_le(lane);
+      const uint32_t stop = after ? (uint32_t)(__ffsll((long long)after) - 1) : (uint32_t)kWave;
+      if (head && row[j] != 0xFFFFFFFFu) atomicAdd(&v.sd[row[j]], stop - lane);
+    }
   }
-  bool cc[C];
+  wave_lds_sync();  // the list is rewritten
+}
+
+// Joins the similar core-core edges of the wave's tile, each visited from its
+// larger endpoint.  HEADS: one edge per run of a row's entries only.
+template <bool HEADS>
+__device__ __forceinline__ void union_tile(const PhaseView& v, uint64_t base, uint16_t* at) {
+  const uint32_t lane = lane_id();
+  const uint32_t total = similar_tile(v.flag, v.m, base, at);
+  for (uint32_t i0 = 0; i0 < total; i0 += kWave * kListed) {
+    uint32_t u[kListed];
+    int32_t w[kListed];
+    bool on[kListed];
 #pragma unroll
-  for (uint32_t j = 0; j < C; ++j) cc[j] = y[j] && v.core[u[j]] && v.core[w[j]];
+    for (uint32_t j = 0; j < kListed; ++j) {
+      const uint32_t i = i0 + j * kWave + lane;
+      const uint64_t k = base + (i < total ? at[i] : 0);
+      u[j] = i < total ? v.src[k] : 0u;
+      w[j] = i < total ? v.adj[k] : 0;
+    }
 #pragma unroll
-  for (uint32_t j = 0; j < C; ++j)
-    if (cc[j]) uf_union(v.parent, (int32_t)u[j], w[j]);
+    for (uint32_t j = 0; j < kListed; ++j) on[j] = (uint32_t)w[j] < u[j] && v.core[u[j]] && v.core[w[j]];
+    if (!HEADS) {
+#pragma unroll
+      for (uint32_t j = 0; j < kListed; ++j) on[j] = on[j] && v.parent[u[j]] != v.parent[w[j]];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kListed; ++j) {
+      if (HEADS) {
+        // the first of the row's entries among the lanes that are on
+        const uint64_t below = __ballot(on[j]) & lanemask_lt(lane);
+        const uint32_t prev = below ? 63u - (uint32_t)__clzll((long long)below) : lane;
+        const uint32_t pu = (uint32_t)__shfl((int)u[j], (int)prev);
+        on[j] = on[j] && (!below || pu != u[j]);
+      }
+      if (on[j]) uf_union(v.parent, (int32_t)u[j], w[j]);
+    }
+  }
+  wave_lds_sync();  // the list is rewritten
 }
 
 // Roots go to label: the finds keep splitting paths in parent (stores of
@@ -162,43 +208,16 @@ __device__ __forceinline__ uint32_t border_entry(const PhaseView& v, uint64_t k,
   return 0;
 }
 
-// ---- borders: the minimum candidate cluster id over similar edges to cores,
-// for the wave chunk of kEdgeChunks x 64 entries at `base`.  Only similar
-// entries read rows and neighbours; the others get a marker row, so one
-// row's lanes may form several runs, whose minimum may also take lanes of
-// the same row from another run (that row's candidates too).  Returns the
-// entries of the border rows this lane labelled first (rows known only).
-__device__ __forceinline__ uint32_t border_chunk(const PhaseView& v, uint64_t base) {
-  constexpr uint32_t C = kEdgeChunks;
-  const uint32_t lane = lane_id();
+// The same for the wave's tile at `base`.
+template <bool FIND>
+__device__ __forceinline__ uint32_t border_tile(const PhaseView& v, uint64_t base, uint16_t* at) {
+  const uint32_t total = similar_tile(v.flag, v.m, base, at);
   uint32_t labeled = 0;
-  bool y[C];
-#pragma unroll
-  for (uint32_t j = 0; j < C; ++j) {
-    const uint64_t k = base + j * kWave + lane;
-    y[j] = k < v.m && v.flag[k] == kFlagY;
+  for (uint32_t i0 = 0; i0 < total; i0 += kWave) {
+    const bool on = i0 + lane_id() < total;
+    labeled += border_entry<FIND>(v, base + (on ? at[i0 + lane_id()] : 0), on);
   }
-  uint32_t row[C];
-  int32_t c[C];
-#pragma unroll
-  for (uint32_t j = 0; j < C; ++j) {
-    const uint64_t k = base + j * kWave + lane;
-    row[j] = y[j] ? v.src[k] : 0xFFFFFFFFu;
-    c[j] = y[j] ? v.adj[k] : 0;
-  }
-#pragma unroll
-  for (uint32_t j = 0; j < C; ++j) y[j] = y[j] && v.core[c[j]] && !v.core[row[j]];
-  int32_t cand[C];
-#pragma unroll
-  for (uint32_t j = 0; j < C; ++j) cand[j] = y[j] ? v.label[c[j]] : kNoLabel;
-#pragma unroll
-  for (uint32_t j = 0; j < C; ++j) {
-    if (!__ballot(y[j])) continue;
-    const uint32_t r = y[j] ? row[j] : 0xFFFFFFFFu;
-    const int32_t best = wave_seg_reduce(r, cand[j], OpMin());
-    if (wave_seg_head(r) && best != kNoLabel && atomicMin(&v.label[r], best) == kNoLabel && v.rb)
-      labeled += v.re[r] - v.rb[r];
-  }
+  wave_lds_sync();  // the list is rewritten
   return labeled;
 }
 

@@ -6,10 +6,12 @@
 // A graph is admitted if it fits the engine's HBM budget: its CSR, the row of
 // each entry, cn[] and a fixed number of query slots.  At admission every
 // edge's common-neighbour count |N(u) & N(v)| is computed once by the tiered
-// similarity kernels in their counting mode.  A query is then a threshold
-// pass over cn[] (the degree-only rule, then the reference's predicate in
-// its int32/double form) followed by the core, union-find, border and
-// classify kernels, all O(m) streaming passes on the slot's stream.
+// similarity kernels in their counting mode, and every entry's ratio
+// (cn + 2)^2 / ((d(u) + 1) (d(v) + 1)) from it.  A query is then a threshold
+// pass over the ratios (entries near the threshold from cn[]: the degree-only
+// rule, then the reference's predicate in its int32/double form) followed by
+// the core, union-find, border and classify kernels, all O(m) streaming passes
+// on the slot's stream.
 // Continuous batching: queries take free slots of their graph as they arrive
 // and are retired as their streams finish; queued queries start in the freed
 // slots, so several queries of different graphs overlap on the device.
@@ -43,64 +45,88 @@ struct QueryParams {
   int32_t pad;
 };
 
+// What a query's threshold pass reads of a graph.
+struct CountView {
+  uint32_t m;
+  const uint32_t* rp;
+  const uint32_t* src;
+  const int32_t* adj;
+  const uint32_t* ndeg;  // or null
+  const uint32_t* cn;
+  const float* ratio;    // or null
+};
+
+// ratio[k] = (cn + 2)^2 / ((d(u) + 1) (d(v) + 1)) of entry k = (u, v), within
+// one part in 2^23: away from eps^2 by more than that it decides the entry.
+// The predicate, and both degree rules before it (cn + 2 <= min(d) + 1, and
+// (cn + 2)^2 >= 4), say the same in exact arithmetic, and their roundings are
+// of one part in 2^50.  NaN where they might not: counts whose square the
+// reference's int32 wraps, and counts no symmetric graph has.
+__global__ void __launch_bounds__(kBlock) k_ratios(CountView g, float* __restrict__ ratio) {
+  const uint64_t stride = (uint64_t)gridDim.x * kBlock;
+  for (uint64_t k = (uint64_t)blockIdx.x * kBlock + threadIdx.x; k < g.m; k += stride) {
+    const uint32_t u = g.src[k], v = (uint32_t)g.adj[k], c = g.cn[k];
+    const uint32_t du = g.rp[u + 1] - g.rp[u], dv = g.ndeg ? g.ndeg[k] : g.rp[v + 1] - g.rp[v];
+    const double t = (double)c + 2.0, ab = ((double)du + 1.0) * ((double)dv + 1.0);
+    const bool plain = c < 46338u && c < min(du, dv);
+    ratio[k] = plain ? (float)(t * t / ab) : __int_as_float(0x7FC00000);
+  }
+}
+
 // flag[k] for one query from cn[]: the degree-only rule first
 // (GPUSCAN++/GPUScan.cu:143-169), then for undecided edges the predicate
 // `(cn+2)*(cn+2) < eps*eps*(s+1)*(l+1)` -> not similar (GPUScan.cu:220-221).
-// The same pass counts each row's similar entries into sd (the core count).
-// The neighbour degree comes from ndeg when the graph has it.  One wave,
-// kEdgeChunks x 64 entries at `base`.
-__device__ __forceinline__ void threshold_chunk(uint32_t m, uint64_t base, const uint32_t* __restrict__ rp,
-                                                const uint32_t* __restrict__ src, const int32_t* __restrict__ adj,
-                                                const uint32_t* __restrict__ ndeg, const uint32_t* __restrict__ cn,
-                                                double eps, uint8_t* __restrict__ flag, uint32_t* __restrict__ sd) {
-  constexpr uint32_t C = kEdgeChunks;
+__device__ __forceinline__ uint8_t threshold_entry(const CountView& g, uint64_t k, double eps) {
+  const uint32_t u = g.src[k], v = (uint32_t)g.adj[k];
+  const uint32_t du = g.rp[u + 1] - g.rp[u], dv = g.ndeg ? g.ndeg[k] : g.rp[v + 1] - g.rp[v];
+  const uint8_t f = prep_flag(u, v, du, dv, eps);
+  if (f < kFlagUUp) return f;
+  const uint32_t s = f == kFlagUUp ? du : dv, l = f == kFlagUUp ? dv : du;
+  return predicate_exact(g.cn[k], predicate_rhs(eps, s, l)) ? kFlagY : kFlagN;
+}
+
+// The flags of one wave's tile of kFlagTile entries at `base`, four entries a
+// lane and step.  Bound by the reads: 4 bytes an entry from the ratios and the
+// flag, where cn, the degrees and both ids are 16 (96 queries over eight
+// graphs of 2.4e5 to 3.1e7 entries: 6.9 -> 4.9 ms with the listed similar
+// entries of the passes after it).  Entries within two parts in 10^6 of the
+// threshold (or with no ratio) are decided in full.
+__device__ __forceinline__ void threshold_tile(const CountView& g, uint64_t base, double eps,
+                                               uint8_t* __restrict__ flag) {
+  constexpr uint32_t L = kFlagTile / (kWave * 4);
   const uint32_t lane = lane_id();
-  uint32_t u[C], v[C], du[C], dv[C];
+  const float hi = (float)(eps * eps * 1.000002), lo = (float)(eps * eps * 0.999998);
+  float4 q[L];
 #pragma unroll
-  for (uint32_t j = 0; j < C; ++j) {
-    const uint64_t k = base + j * kWave + lane;
-    u[j] = k < m ? src[k] : 0xFFFFFFFFu;  // rows must not decrease across lanes
-    v[j] = k < m ? (uint32_t)adj[k] : 0u;
-    dv[j] = k < m && ndeg ? ndeg[k] : 0u;
+  for (uint32_t j = 0; j < L; ++j) {
+    const uint64_t k = base + (j * kWave + lane) * 4;
+    q[j] = make_float4(0, 0, 0, 0);
+    if (g.ratio && k < g.m) q[j] = *reinterpret_cast<const float4*>(g.ratio + k);  // the array ends on 256 bytes
   }
 #pragma unroll
-  for (uint32_t j = 0; j < C; ++j) {
-    const bool in = u[j] != 0xFFFFFFFFu;
-    du[j] = in ? rp[u[j] + 1] - rp[u[j]] : 0u;
-    if (!ndeg) dv[j] = in ? rp[v[j] + 1] - rp[v[j]] : 0u;
-  }
+  for (uint32_t j = 0; j < L; ++j) {
+    const uint64_t k = base + (j * kWave + lane) * 4;
+    if (k >= g.m) break;
+    const float x[4] = {q[j].x, q[j].y, q[j].z, q[j].w};
+    uint32_t f = 0;
 #pragma unroll
-  for (uint32_t j = 0; j < C; ++j) {
-    const uint64_t k = base + j * kWave + lane;
-    uint32_t y = 0;
-    if (k < m) {
-      uint8_t f = prep_flag(u[j], v[j], du[j], dv[j], eps);
-      if (f >= kFlagUUp) {
-        const uint32_t s = f == kFlagUUp ? du[j] : dv[j], l = f == kFlagUUp ? dv[j] : du[j];
-        f = predicate_exact(cn[k], predicate_rhs(eps, s, l)) ? kFlagY : kFlagN;
-      }
-      flag[k] = f;
-      y = f == kFlagY;
+    for (uint32_t i = 0; i < 4; ++i) {
+      uint32_t v = x[i] > hi ? kFlagY : kFlagN;
+      if ((!(x[i] > hi || x[i] < lo) || !g.ratio) && k + i < g.m) v = threshold_entry(g, k + i, eps);
+      f |= v << (8 * i);
     }
-    if (!__ballot(y)) continue;
-    const uint32_t sum = wave_seg_reduce(u[j], y, OpAdd());
-    if (wave_seg_head(u[j]) && sum) atomicAdd(&sd[u[j]], sum);
+    *reinterpret_cast<uint32_t*>(flag + k) = f;  // the array ends on 256 bytes
   }
 }
 
 // eps comes from prm when given (captured launches), else eps.
-__global__ void __launch_bounds__(kBlock) k_threshold(uint32_t m, const uint32_t* __restrict__ rp,
-                                                      const uint32_t* __restrict__ src,
-                                                      const int32_t* __restrict__ adj,
-                                                      const uint32_t* __restrict__ ndeg,
-                                                      const uint32_t* __restrict__ cn, double eps,
-                                                      const QueryParams* __restrict__ prm,
-                                                      uint8_t* __restrict__ flag, uint32_t* __restrict__ sd) {
+__global__ void __launch_bounds__(kBlock) k_threshold(CountView g, double eps, const QueryParams* __restrict__ prm,
+                                                      uint8_t* __restrict__ flag) {
   if (prm) eps = prm->eps;
-  const uint64_t waves = (uint64_t)gridDim.x * (kBlock / kWave);
-  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * (kWave * kEdgeChunks);
-       base < m; base += waves * kWave * kEdgeChunks)
-    threshold_chunk(m, base, rp, src, adj, ndeg, cn, eps, flag, sd);
+  const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * kFlagTile;
+  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * kFlagTile; base < g.m;
+       base += step)
+    threshold_tile(g, base, eps, flag);
 }
 
 __global__ void __launch_bounds__(kBlock) k_query_init(uint32_t n, uint32_t* __restrict__ sd, int32_t* __restrict__ lo,
@@ -120,10 +146,10 @@ __global__ void __launch_bounds__(kBlock) k_query_init(uint32_t n, uint32_t* __r
 // ---------------------------------------------------------------------------
 
 // Queries per batch, and the tiles the batched kernels cut each query into:
-// a block takes 1024 entries (four waves of kEdgeChunks x 64) or 256
-// vertices of one query, so block-wide reductions never mix two queries.
+// a block takes 8192 entries (a flag tile a wave) or 256 vertices of one
+// query, so block-wide reductions never mix two queries.
 constexpr uint32_t kBatchMax = 64;
-constexpr uint32_t kEdgeTile = (kBlock / kWave) * kWave * kEdgeChunks;
+constexpr uint32_t kEdgeTile = (kBlock / kWave) * kFlagTile;
 constexpr uint32_t kVertexTile = kBlock;
 // Fixed grid of every batched kernel (grid-stride over the batch's tiles).
 constexpr uint32_t kBatchGrid = 1024;
@@ -137,6 +163,7 @@ struct BatchItem {
   const int32_t* adj;
   const uint32_t* ndeg;
   const uint32_t* cn;
+  const float* ratio;
   uint8_t* flag;
   uint32_t* sd;
   int32_t* parent;
@@ -199,8 +226,17 @@ __global__ void __launch_bounds__(kBlock) k_batch_init(const BatchTable* __restr
 
 __global__ void __launch_bounds__(kBlock) k_batch_threshold(const BatchTable* __restrict__ bt) {
   SGC_BATCH_TILES(bt, e_tiles, true, kEdgeTile) {
-    const uint64_t base = T0 + (threadIdx.x / kWave) * (kWave * kEdgeChunks);
-    threshold_chunk(Q.m, base, Q.rp, Q.src, Q.adj, Q.ndeg, Q.cn, Q.eps, Q.flag, Q.sd);
+    const CountView g{Q.m, Q.rp, Q.src, Q.adj, Q.ndeg, Q.cn, Q.ratio};
+    const uint64_t base = T0 + threadIdx.x / kWave * kFlagTile;
+    if (base < Q.m) threshold_tile(g, base, Q.eps, Q.flag);
+  }
+}
+
+__global__ void __launch_bounds__(kBlock) k_batch_core_count(const BatchTable* __restrict__ bt) {
+  __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
+  const uint32_t wv = threadIdx.x / kWave;
+  SGC_BATCH_TILES(bt, e_tiles, true, kEdgeTile) {
+    if (T0 + wv * kFlagTile < Q.m) core_count_tile(item_view(Q), T0 + wv * kFlagTile, s_at[wv]);
   }
 }
 
@@ -215,9 +251,11 @@ __global__ void __launch_bounds__(kBlock) k_batch_core_mark(const BatchTable* __
 }
 
 __global__ void __launch_bounds__(kBlock) k_batch_union(const BatchTable* __restrict__ bt) {
+  __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
+  const uint32_t wv = threadIdx.x / kWave;
   SGC_BATCH_TILES(bt, e_tiles, true, kEdgeTile) {
     if (!count_any(Q.cnt, kCntMarked)) continue;  // no core: no core-core edge to join
-    union_entries(item_view(Q), T0 + threadIdx.x, kBlock);
+    if (T0 + wv * kFlagTile < Q.m) union_tile<false>(item_view(Q), T0 + wv * kFlagTile, s_at[wv]);
   }
 }
 
@@ -229,9 +267,12 @@ __global__ void __launch_bounds__(kBlock) k_batch_flatten(const BatchTable* __re
 }
 
 __global__ void __launch_bounds__(kBlock) k_batch_border(const BatchTable* __restrict__ bt) {
+  __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
+  const uint32_t wv = threadIdx.x / kWave;
   SGC_BATCH_TILES(bt, e_tiles, true, kEdgeTile) {
     if (!count_any(Q.cnt, kCntMarked)) continue;  // no core: no border
-    const uint32_t labeled = border_chunk(item_view(Q), T0 + (threadIdx.x / kWave) * (kWave * kEdgeChunks));
+    uint32_t labeled = 0;
+    if (T0 + wv * kFlagTile < Q.m) labeled = border_tile<false>(item_view(Q), T0 + wv * kFlagTile, s_at[wv]);
     count_add<1>(Q.cnt, {kCntLabeled}, {labeled});
   }
 }
@@ -239,7 +280,10 @@ __global__ void __launch_bounds__(kBlock) k_batch_border(const BatchTable* __res
 __global__ void __launch_bounds__(kBlock) k_batch_classify(const BatchTable* __restrict__ bt) {
   SGC_BATCH_TILES(bt, e_tiles, true, kEdgeTile) {
     if (!count_any(Q.cnt, kCntMarked)) continue;  // no label anywhere
-    classify_chunk(item_view(Q), T0 + (threadIdx.x / kWave) * (kWave * kEdgeChunks), 3 * count_total(Q.cnt, kCntLabeled) < Q.m);
+    const bool from_labeled = 3 * count_total(Q.cnt, kCntLabeled) < Q.m;
+    for (uint64_t k = T0 + threadIdx.x / kWave * (kWave * kEdgeChunks); k < min(T0 + kEdgeTile, (uint64_t)Q.m);
+         k += kBlock * kEdgeChunks)
+      classify_chunk(item_view(Q), k, from_labeled);
   }
 }
 
@@ -300,6 +344,7 @@ struct Graph {
   uint32_t id = 0;
   sgc_dgraph* dg = nullptr;
   uint32_t* cn = nullptr;  // start of the graph's device memory: then the slots, then kCntWords per slot
+  float* ratio = nullptr;  // in the reverse-entry index's memory, which only the counting pass reads
   char* host_mem = nullptr;  // page-locked: the slots' labels, counters and parameters
   size_t bytes = 0;
   std::vector<Slot> slots;
@@ -385,6 +430,11 @@ void free_graph(Graph* G) {
   delete G;
 }
 
+CountView count_view(const Graph* G) {
+  const sgc_dgraph* g = G->dg;
+  return CountView{g->m, g->row_ptr, g->src, g->adj, g->ndeg, G->cn, G->ratio};
+}
+
 // The work of one query on stream st: eager (p given) or reading eps and mu
 // from the slot's parameter block (p null, for capture).
 void enqueue_query(const Graph* G, const Slot& sl, const ScanParams* p, hipStream_t st) {
@@ -394,8 +444,8 @@ void enqueue_query(const Graph* G, const Slot& sl, const ScanParams* p, hipStrea
   const int32_t* mu_dev = p ? nullptr : &sl.d_params->mu;
   k_query_init<<<grid_for(g->n, kBlock), kBlock, 0, st>>>(g->n, sl.pb.sd, sl.pb.lo, sl.pb.hi, sl.pb.cnt);
   if (g->m)
-    k_threshold<<<grid_for(g->m, kBlock), kBlock, 0, st>>>(g->m, g->row_ptr, g->src, g->adj, g->ndeg, G->cn, pv.eps,
-                                                            prm, sl.pb.flag, sl.pb.sd);
+    k_threshold<<<grid_for(g->m, kEdgeTile), kBlock, 0, st>>>(count_view(G), pv.eps, prm, sl.pb.flag);
+  launch_core_count(g, sl.pb, st);
   launch_core_mark(g, sl.pb, pv, st, mu_dev);
   launch_union(g, sl.pb, st);
   launch_flatten(g, sl.pb, st);
@@ -450,6 +500,7 @@ int ensure_lanes(sgc_server* S) {
       (void)hipMemcpyAsync(L.d_table, L.h_table, sizeof(BatchTable), hipMemcpyHostToDevice, st);
       k_batch_init<<<kBatchGrid, kBlock, 0, st>>>(L.d_table);
       k_batch_threshold<<<kBatchGrid, kBlock, 0, st>>>(L.d_table);
+      k_batch_core_count<<<kBatchGrid, kBlock, 0, st>>>(L.d_table);
       k_batch_core_mark<<<kBatchGrid, kBlock, 0, st>>>(L.d_table);
       k_batch_union<<<kBatchGrid, kBlock, 0, st>>>(L.d_table);
       k_batch_flatten<<<kBatchGrid, kBlock, 0, st>>>(L.d_table);
@@ -522,7 +573,7 @@ int launch_batch(sgc_server* S, BatchLane& L, const std::vector<double>& eps, co
     const sgc_dgraph* g = b.G->dg;
     const PassBuffers& pb = b.sl->pb;
     BatchItem& it = T->items[q];
-    it.rp = g->row_ptr, it.src = g->src, it.adj = g->adj, it.ndeg = g->ndeg, it.cn = b.G->cn;
+    it.rp = g->row_ptr, it.src = g->src, it.adj = g->adj, it.ndeg = g->ndeg, it.cn = b.G->cn, it.ratio = b.G->ratio;
     it.flag = pb.flag, it.sd = pb.sd, it.parent = pb.parent, it.label = pb.label, it.lo = pb.lo, it.hi = pb.hi;
     it.core = pb.core, it.cnt = pb.cnt;
     it.out_labels = b.sl->d_out_labels, it.out_cnt = b.sl->d_out_cnt;
@@ -771,6 +822,12 @@ extern "C" int sgc_server_add_graph(sgc_server* S, const sgc_host_graph* hg, uin
     launch_prep(G->dg, pb, p, s, true);
     launch_plan(G->dg, pb, p, s);
     launch_similarity(G->dg, pb, p, ctx->cu_count, kSimTiered, nullptr, s, G->cn);
+    if (G->dg->mirror) {
+      G->ratio = (float*)G->dg->mirror;
+      G->dg->mirror = nullptr;
+      CountView cv = count_view(G);
+      k_ratios<<<grid_for(m, kBlock), kBlock, 0, s>>>(cv, G->ratio);
+    }
     const hipError_t e = hipStreamSynchronize(s);
     if (e != hipSuccess || hipGetLastError() != hipSuccess) {
       free_graph(G);

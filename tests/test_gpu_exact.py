@@ -57,3 +57,33 @@ def test_exact_kernels_match_oracle(ctx, n):
             print("[case] eps", eps, "similar", st.similar_edges, "chips", info.similarity_chips, flush=True)
     finally:
         server.close()
+
+
+@pytest.mark.parametrize("batched", [False, True])
+def test_queries_at_the_thresholds_of_edges(ctx, batched):
+    """eps exactly at an edge's own (cn + 2) / sqrt((d(u) + 1) (d(v) + 1)),
+    the doubles beside it, and just outside the band in which a query decides
+    by the ratio alone; extreme eps."""
+    g = sgc.HostGraph.rmat(11, 12, seed=4)
+    rng = np.random.default_rng(5)
+    rows = [set(g.adj[g.row_ptr[u]:g.row_ptr[u + 1]].tolist()) for u in range(g.n)]
+    src = np.repeat(np.arange(g.n), np.diff(g.row_ptr).astype(np.int64))
+    eps = [0.0, 1e-200, 1e200, 1.0]
+    for k in rng.choice(g.m, 10, replace=False):
+        u, v = int(src[k]), int(g.adj[k])
+        e = (len(rows[u] & rows[v]) + 2) / np.sqrt(float(len(rows[u]) + 1) * float(len(rows[v]) + 1))
+        eps += [float(e), float(np.nextafter(e, 0)), float(np.nextafter(e, 2)), float(e * (1 - 2e-6)), float(e * (1 + 2e-6))]
+    server = sgc.Server(ctx, sgc.Server.graph_bytes(g) + (1 << 20))
+    try:
+        gid = server.add_graph(g)[0]
+        server.set_batching(g.m if batched else 0)
+        tickets = [server.submit(gid, e, 3) for e in eps]
+        while server.pending:
+            server.progress(wait=True)
+        for e, t in zip(eps, tickets):
+            labels, core, sim, _ = ob.orc_scan(g.row_ptr, g.adj, e, 3)
+            got, st = server.result(t, g.n)
+            assert np.array_equal(got, labels) and st.similar_edges == int(sim.sum()) // 2, e
+        print("[case] batched", batched, "queries", len(eps), flush=True)
+    finally:
+        server.close()
