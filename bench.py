@@ -11,16 +11,16 @@ does the same work whatever --steps is.
 
 value = E * passes / (wall time of the K steps) in GTEPS (1e9
 similarity-edges/s), passes = 12 K.
-roofline: the workgroup-tier similarity kernel (k_sim_units<LargeTier>,
-owners of degree > 1024), the dominant kernel of a pass.  Its DRAM bytes per
-launch come from the committed rocprofv3 counter summary of this workload
-(profiles/k_sim_units_large_rmat24_counters.md: FETCH_SIZE and WRITE_SIZE of
-each of the 12 configurations, scaled by the same counters of a plain copy),
-summed over the launches actually timed and divided by their hipEvent-timed
-durations on the library's stream: achieved GB/s, and frac against the
-8 TB/s peak.  The algorithmic-byte model (sum over the
-kernel's undecided edges of 4 * (s + min(l, s * ceil(log2(l + 1))))) is
-reported beside it under alg_model; early exit and LDS-resident owner rows
+roofline: the similarity of the large owners (degree > 1024), most of a pass:
+the bitmap filter, the hash filter and the exact kernel for what they leave.
+Their DRAM bytes per pass come from the committed rocprofv3 counter summary of
+this workload (profiles/large_owner_similarity_rmat24_counters.md: FETCH_SIZE
+and WRITE_SIZE of each of the 12 configurations, scaled by the same counters
+of a plain copy), summed over the passes actually timed and divided by their
+durations on the device clock: achieved GB/s, and frac against the 8 TB/s
+peak.  The algorithmic-byte model (sum over the owners' undecided edges of
+4 * (s + min(l, s * ceil(log2(l + 1))))) is reported beside it under
+alg_model; the filters' compact rows, early exits and LDS-resident owner rows
 move far fewer bytes than that model, so its ratio to the peak passes 1.
 cpu_baseline: the oracle's per-edge similarity (prep + merge intersection,
 OpenMP) over a uniform random sample of the same graph's edges, on this
@@ -410,11 +410,11 @@ def ooc_bench(sgc, ctx, args):
 
 
 def measured_traffic(args):
-    """DRAM bytes per launch of the workgroup-tier similarity kernel for each
+    """DRAM bytes per pass of the large owners' similarity kernels for each
     (eps, mu) of the default workload, from the committed rocprofv3 counter
     summary (FETCH_SIZE and WRITE_SIZE, each scaled by the plain-copy
     calibration); None for other workloads or without the summary."""
-    path = os.path.join(ROOT, "profiles", "k_sim_units_large_rmat24_counters.md")
+    path = os.path.join(ROOT, "profiles", "large_owner_similarity_rmat24_counters.md")
     default = (args.scale == 24 and args.edge_factor == 16 and args.seed == 1)
     if not default or not os.path.exists(path):
         return None
@@ -507,16 +507,15 @@ def main() -> int:
     wall = time.perf_counter() - t0
     for eps, mu, st in stats[: len(params)]:
         log(f"eps={eps} mu={mu}: pass {st.ms_total:.2f} ms, similarity {st.ms_similarity:.2f} ms "
-            f"(workgroup tier {st.ms_similarity_large:.2f}), U={st.u_edges} streamed={st.probe_elements:.3g} "
-            f"loaded={st.loaded_elements:.3g} claims={st.claims:.3g} "
-            f"({st.probe_elements * 4 / max(st.ms_similarity, 1e-9) / 1e6:.0f} GB/s) cores={st.cores} "
+            f"(large owners {st.ms_similarity_large:.2f}), U={st.u_edges} probed={st.probe_elements:.3g} "
+            f"claims={st.claims:.3g} cores={st.cores} "
             f"clusters={st.clusters} pruned={st.pruned} deferred={st.deferred_edges} redo={st.redo_edges}")
 
     passes = len(stats)
     ms_per_step = wall / args.steps * 1e3
     value = E * passes / wall / 1e9
-    # roofline: the workgroup-tier similarity kernel (owners of degree > 1024),
-    # the pass's dominant kernel, timed by hipEvents on the library's stream
+    # roofline: the similarity kernels of the large owners (degree > 1024),
+    # most of a pass, timed by the device clock
     sim_ms = sum(st.ms_similarity for _, _, st in stats)
     alg_bytes = sum(work[eps][1] for eps, _, _ in stats)
     large_ms = sum(st.ms_similarity_large for _, _, st in stats)
@@ -579,7 +578,8 @@ def main() -> int:
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": "k_sim_units<LargeTier> (similarity of edges whose owner has degree > 1024)",
+            "kernel": ("k_bitmap_units<true>, k_hash_units, k_sim_units<LargeTier> (similarity of edges whose owner "
+                       "has degree > 1024)"),
             "achieved": round(achieved, 2) if achieved else None,
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
@@ -588,21 +588,21 @@ def main() -> int:
             "traffic_source": traffic["source"] if traffic else None,
             "avg_launch_ms": round(launch_ms, 4),
             "launches": passes,
-            "note": ("achieved = DRAM bytes of the timed launches (rocprofv3 FETCH_SIZE and WRITE_SIZE per "
-                     "configuration, scaled by a plain copy's counters) / their summed hipEvent durations"),
+            "note": ("achieved = DRAM bytes of the timed passes' kernels (rocprofv3 FETCH_SIZE and WRITE_SIZE per "
+                     "configuration, scaled by a plain copy's counters) / their summed durations"),
             "alg_model": {
                 "bytes_per_launch": large_bytes / passes,
                 "achieved": round(alg_achieved, 2),
                 "frac": round(alg_achieved / HBM_PEAK_GBS, 4),
-                "note": ("sum over the kernel's undecided edges of 4 * (s + min(l, s * ceil(log2(l + 1)))), the "
-                         "reference's per-lane binary search; early exit and LDS-resident owner rows move fewer "
-                         "bytes, so this ratio passes 1"),
+                "note": ("sum over the owners' undecided edges of 4 * (s + min(l, s * ceil(log2(l + 1)))), the "
+                         "reference's per-lane binary search; compact rows, early exit and LDS-resident owner rows "
+                         "move fewer bytes, so this ratio passes 1"),
             },
         },
         "similarity_both_tiers": {
             "alg_bytes_per_launch": alg_bytes / len(stats),
             "avg_ms": round(sim_ms / len(stats), 4),
-            "streamed_bytes_per_launch": sum(4 * st.probe_elements for _, _, st in stats) / len(stats),
+            "elements_probed_per_pass": sum(st.probe_elements for _, _, st in stats) / len(stats),
         },
         "cpu_baseline": cpu,
         "serving": serving,

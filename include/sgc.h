@@ -178,10 +178,8 @@ typedef struct sgc_dgraph sgc_dgraph;
  * not in page-locked memory (sgc_graph_pin) is staged through the context's
  * 32 MB of page-locked buffers, allocated at the first such copy and kept
  * until sgc_ctx_destroy.  The indexes are built in the context's work memory,
- * which is grown to what a pass over the graph needs.  Without the room to
- * sort the entries there, or for an input whose entries lack their reverse,
- * the reverse-entry index is built by a search instead.  Synchronises the
- * context stream. */
+ * which is grown to what a pass over the graph needs; without that room the
+ * reverse entries are searched one by one.  Synchronises the context stream. */
 int sgc_dgraph_upload(sgc_ctx* ctx, const sgc_host_graph* g, sgc_dgraph** out);
 void sgc_dgraph_free(sgc_dgraph* dg);
 
@@ -193,9 +191,11 @@ typedef struct {
   uint32_t small_max_degree; /* owners of degree <= this take the small tier (1..1024; default 1024) */
   double small_unit_work;    /* short-row elements per small-tier work unit (default 262144) */
   double large_unit_work;    /* per workgroup-tier work unit (default 8388608) */
-  uint32_t hash_tables;      /* 1 (default): owner rows as cuckoo hashes where they fit (small tier; whole
-                                rows and runs of 2^20-id windows of <= 8192 keys in the workgroup tier);
-                                0: linear probing (small tier) and one bitmap window at a time only */
+  uint32_t hash_tables;      /* 1 (default): the filter stages first, and owner rows as cuckoo hashes or bit
+                                sets where they fit; 0: no filters, every edge counted, with linear probing
+                                (small tier) and one bitmap window at a time only.  The filter stages plan
+                                their own units: of the other knobs only small_max_degree acts on what they
+                                leave */
   uint32_t tiny_work;        /* owners whose edges' merge work, sum of d(a) + d(b), is at most this are
                                 decided by one thread each, without a work unit (0..65536; default 2048;
                                 0 turns this off) */
@@ -239,9 +239,9 @@ typedef struct {
   uint64_t hubs;
   uint64_t outliers;
   double alg_bytes;      /* algorithmic bytes of the similarity kernels */
-  double probe_elements; /* list elements consumed by them */
+  double probe_elements; /* list elements consumed by them (bitmap words count for the elements they hold) */
   double loaded_elements; /* list elements loaded by them (consumed or read past a window's end) */
-  double claims;          /* wave claims of the tiered kernels */
+  double claims;          /* rounds of loads: a wave's, or a team's of 8 or 16 lanes */
   /* Core-check pruning (GPUSCAN++/GPUScan.cu:303): in a pruned pass the
    * workgroup-tier similarity kernel defers an edge whose endpoints are both
    * already decided (core, or not core); after the union-find pass the
