@@ -415,7 +415,8 @@ def measured_traffic(args):
     summary (FETCH_SIZE and WRITE_SIZE, each scaled by the plain-copy
     calibration); None for other workloads or without the summary."""
     path = os.path.join(ROOT, "profiles", "large_owner_similarity_rmat24_counters.md")
-    default = (args.scale == 24 and args.edge_factor == 16 and args.seed == 1)
+    # pruned passes run the exact kernels on every edge: other traffic
+    default = (args.scale == 24 and args.edge_factor == 16 and args.seed == 1 and not args.prune)
     if not default or not os.path.exists(path):
         return None
     table = {}
