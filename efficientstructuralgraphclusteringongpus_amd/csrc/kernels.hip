@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include <hipcub/device/device_radix_sort.hpp>
 
@@ -464,17 +465,18 @@ __global__ void __launch_bounds__(kBlock) k_similarity_wave(const uint32_t* __re
 
 // Similar entries per row, from the flags' similar entries alone: one
 // atomic per run of a row's entries in a wave's 64.
+template <uint32_t TILE>
 __global__ void __launch_bounds__(kBlock) k_core_count(uint64_t m, const uint32_t* __restrict__ src,
                                                        const uint8_t* __restrict__ flag, uint32_t* __restrict__ sd,
                                                        uint64_t* __restrict__ cnt) {
   stamp(cnt, kStampCore);
-  __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
+  __shared__ uint16_t s_at[kBlock / kWave][TILE];
   const uint32_t wv = threadIdx.x / kWave;
   PhaseView v{};
   v.m = (uint32_t)m, v.src = src, v.flag = flag, v.sd = sd;
-  const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * kFlagTile;
-  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * kFlagTile; base < m; base += step)
-    core_count_tile(v, base, s_at[wv]);
+  const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * TILE;
+  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * TILE; base < m; base += step)
+    core_count_tile<TILE>(v, base, s_at[wv]);
 }
 
 // core(x) <=> #similar neighbours >= mu (mu <= 0: >= 1).  The reference's
@@ -523,7 +525,7 @@ __global__ void __launch_bounds__(kBlock) k_core_mark(uint32_t n, const uint32_t
 // repeated after the second similarity round of a pruned pass).
 constexpr uint64_t kFewCores = 1024;  // up to here the first round costs more than it saves
 
-template <bool HEADS>
+template <bool HEADS, uint32_t TILE>
 __global__ void __launch_bounds__(kBlock) k_union(uint64_t m, const uint32_t* __restrict__ src,
                                                   const int32_t* __restrict__ adj, const uint8_t* __restrict__ flag,
                                                   const uint8_t* __restrict__ core, int32_t* parent,
@@ -533,13 +535,13 @@ __global__ void __launch_bounds__(kBlock) k_union(uint64_t m, const uint32_t* __
   if (cores == 0) return;  // no core-core edge to join
   if (HEADS && cores <= kFewCores) return;
   if (gate >= 0 && !count_any(cnt, gate)) return;
-  __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
+  __shared__ uint16_t s_at[kBlock / kWave][TILE];
   const uint32_t wv = threadIdx.x / kWave;
   PhaseView v{};
   v.m = (uint32_t)m, v.src = src, v.adj = adj, v.flag = flag, v.core = const_cast<uint8_t*>(core), v.parent = parent;
-  const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * kFlagTile;
-  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * kFlagTile; base < m; base += step)
-    union_tile<HEADS>(v, base, s_at[wv]);
+  const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * TILE;
+  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * TILE; base < m; base += step)
+    union_tile<HEADS, TILE>(v, base, s_at[wv]);
 }
 
 __global__ void __launch_bounds__(kBlock) k_compress(uint32_t n, const uint8_t* __restrict__ core, int32_t* parent,
@@ -607,7 +609,7 @@ __global__ void __launch_bounds__(kBlock) k_redo_mark(uint32_t m, const uint32_t
 // Borders (GPUSCAN++/GPUScan.cu:654-730): minimum candidate cluster id
 // ---------------------------------------------------------------------------
 
-template <bool FLATTEN>
+template <bool FLATTEN, uint32_t TILE>
 __global__ void __launch_bounds__(kBlock) k_border(uint32_t n, uint64_t m, int32_t* parent,
                                                    const uint32_t* __restrict__ src,
                                                    const int32_t* __restrict__ adj, const uint8_t* __restrict__ flag,
@@ -624,17 +626,17 @@ __global__ void __launch_bounds__(kBlock) k_border(uint32_t n, uint64_t m, int32
     const uint64_t stride = (uint64_t)gridDim.x * kBlock;
     for (uint64_t x = (uint64_t)blockIdx.x * kBlock + threadIdx.x; x < n; x += stride) flatten_vertex(f, (uint32_t)x);
   }
-  __shared__ uint16_t s_at[kBlock / kWave][kFlagTile];
+  __shared__ uint16_t s_at[kBlock / kWave][TILE];
   PhaseView v{};
   v.m = (uint32_t)m, v.src = src, v.adj = adj, v.flag = flag, v.core = const_cast<uint8_t*>(core);
   v.rb = rb, v.re = re, v.label = label, v.parent = parent;
   const uint32_t wv = threadIdx.x / kWave;
-  const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * kFlagTile;
+  const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave) * TILE;
   // entries of the border rows this lane labels first; the core rows'
   // entries were counted by k_core_mark
   uint64_t labeled = 0;
-  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * kFlagTile; base < m; base += step)
-    labeled += border_tile<FLATTEN>(v, base, s_at[wv]);
+  for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / kWave) + wv) * TILE; base < m; base += step)
+    labeled += border_tile<FLATTEN, TILE>(v, base, s_at[wv]);
   count_add<1>(cnt, {kCntLabeled}, {labeled});
 }
 
@@ -1083,17 +1085,46 @@ void launch_similarity_wave(const sgc_dgraph* g, const PassBuffers& b, ScanParam
 }
 
 // Graphs below this many entries skip the launches that only pay on large
-// ones (the first union round, the list of labelled rows): a launch costs 4-5
-// us, a whole pass over a million flags no more than that.
-constexpr uint64_t kSmallGraph = 1u << 20;
+// ones (the list of labelled rows, a flatten kernel of its own): a launch
+// costs 2-5 us, and the walk of all entries it saves no more than that.
+// R-MAT with 1.8 / 3.8 million entries: 159 / 437 us a pass with them, 155 /
+// 405 without.
+constexpr uint64_t kSmallGraph = 1u << 22;
+
+// The first union round pays from here on: planted communities with 0.7 / 1.4
+// million entries 80 / 81 -> 37 / 37 us in two rounds (and 3.4 million 300 ->
+// 78); without cores the two launches cost 3.
+constexpr uint64_t kUnionRounds = 1u << 19;
+
+// Passes over fewer flags than this take the short tile: planted communities
+// with 0.7 / 3.4 / 8.1 million entries 109 / 121 / 143 us in the core count,
+// union-find and borders with the long one, 50 / 98 / 127 with the short (in
+// two union rounds).  Above, tiles keep every wave busy, and the short one
+// reads a graph with few similar entries at half the rate (R-MAT-20: 64 us
+// against 90; planted with 55 million entries 338 against 263).
+constexpr uint64_t kShortTiles = 1u << 24;
 
 // Blocks of a pass over the flags by similar_tile.
-static uint32_t flag_grid(uint64_t m) { return std::min(grid_for(m, kFlagTile * (kBlock / kWave)), 2048u); }
+static uint32_t flag_grid(uint64_t m) {
+  return std::min(grid_for(m, (m < kShortTiles ? kShortTile : kFlagTile) * (kBlock / kWave)), m < kShortTiles ? 4096u : 2048u);
+}
+
+// Calls fn with the tile's size as a constant.
+template <typename Fn>
+static void with_tile(uint64_t m, Fn fn) {
+  if (m < kShortTiles)
+    fn(std::integral_constant<uint32_t, kShortTile>());
+  else
+    fn(std::integral_constant<uint32_t, kFlagTile>());
+}
 
 // Edge passes take the entries [0, g->m) of g (a whole graph or one chip of
 // rows); vertex passes cover all g->n vertices.
 void launch_core_count(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s) {
-  if (g->m) k_core_count<<<flag_grid(g->m), kBlock, 0, s>>>(g->m, g->src, b.flag, b.sd, b.cnt);
+  if (!g->m) return;
+  with_tile(g->m, [&](auto tile) {
+    k_core_count<tile><<<flag_grid(g->m), kBlock, 0, s>>>(g->m, g->src, b.flag, b.sd, b.cnt);
+  });
 }
 
 void launch_core_mark(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStream_t s,
@@ -1105,11 +1136,13 @@ void launch_core_mark(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, h
 void launch_union(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s, int gate) {
   if (!g->m) return;
   const uint32_t grid = flag_grid(g->m);
-  if (g->m >= kSmallGraph) {
-    k_union<true><<<grid, kBlock, 0, s>>>(g->m, g->src, g->adj, b.flag, b.core, b.parent, b.cnt, gate);
-    k_compress<<<grid_for(g->n, kBlock), kBlock, 0, s>>>(g->n, b.core, b.parent, b.cnt);
-  }
-  k_union<false><<<grid, kBlock, 0, s>>>(g->m, g->src, g->adj, b.flag, b.core, b.parent, b.cnt, gate);
+  with_tile(g->m, [&](auto tile) {
+    if (g->m >= kUnionRounds) {
+      k_union<true, tile><<<grid, kBlock, 0, s>>>(g->m, g->src, g->adj, b.flag, b.core, b.parent, b.cnt, gate);
+      k_compress<<<grid_for(g->n, kBlock), kBlock, 0, s>>>(g->n, b.core, b.parent, b.cnt);
+    }
+    k_union<false, tile><<<grid, kBlock, 0, s>>>(g->m, g->src, g->adj, b.flag, b.core, b.parent, b.cnt, gate);
+  });
 }
 
 void launch_redo_mark(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s) {
@@ -1124,12 +1157,14 @@ void launch_flatten(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s) {
 
 void launch_border(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s, bool flatten) {
   if (!g->m) return;
-  if (flatten)
-    k_border<true><<<std::max(flag_grid(g->m), std::min(grid_for(g->n, kBlock), 1024u)), kBlock, 0, s>>>(
-        g->n, g->m, b.parent, g->src, g->adj, b.flag, b.core, g->row_begin, g->row_end, b.label, b.cnt);
-  else
-    k_border<false><<<flag_grid(g->m), kBlock, 0, s>>>(g->n, g->m, b.parent, g->src, g->adj, b.flag, b.core,
-                                                       g->row_begin, g->row_end, b.label, b.cnt);
+  with_tile(g->m, [&](auto tile) {
+    if (flatten)
+      k_border<true, tile><<<std::max(flag_grid(g->m), std::min(grid_for(g->n, kBlock), 1024u)), kBlock, 0, s>>>(
+          g->n, g->m, b.parent, g->src, g->adj, b.flag, b.core, g->row_begin, g->row_end, b.label, b.cnt);
+    else
+      k_border<false, tile><<<flag_grid(g->m), kBlock, 0, s>>>(g->n, g->m, b.parent, g->src, g->adj, b.flag, b.core,
+                                                               g->row_begin, g->row_end, b.label, b.cnt);
+  });
 }
 
 bool small_graph(const sgc_dgraph* g) { return g->m < kSmallGraph; }

@@ -80,33 +80,43 @@ __device__ __forceinline__ uint32_t similar_mask(const uint4 w) {
   return mask;
 }
 
-// The similar entries of the wave's tile [base, base + kFlagTile) of the flag
-// array, ascending, into `at` (the wave's kFlagTile words of LDS, offsets from
-// base); returns their number (uniform).  Flags come 16 to a load (flag must
-// be 16-byte aligned and readable up to the next multiple of 16): a byte a
-// lane read them at 0.9 TB/s.
-constexpr uint32_t kFlagTile = 2048;
+// The similar entries of the wave's tile [base, base + TILE) of the flag
+// array, ascending, into `at` (the wave's TILE words of LDS, offsets from
+// base); returns their number (uniform).  Flags come 16 to a load, or 4 in the
+// short tile (flag must be 16-byte aligned and readable up to the next
+// multiple of 16): a byte a lane read them at 0.9 TB/s.  The short tile is for
+// graphs that fill the chip with few waves otherwise, where a wave with 2048
+// similar entries is the whole pass.
+constexpr uint32_t kFlagTile = 2048, kShortTile = 256;
 
+template <uint32_t TILE>
 __device__ __forceinline__ uint32_t similar_tile(const uint8_t* __restrict__ flag, uint64_t m, uint64_t base,
                                                  uint16_t* at) {
-  constexpr uint32_t L = kFlagTile / (kWave * 16);
+  static_assert(TILE == kFlagTile || TILE == kShortTile, "flags per lane and load");
+  constexpr uint32_t F = TILE == kShortTile ? 4 : 16, L = TILE / (kWave * F);
   const uint32_t lane = lane_id();
   uint4 w[L];
 #pragma unroll
   for (uint32_t j = 0; j < L; ++j) {
-    const uint64_t k = base + (j * kWave + lane) * 16;
-    w[j] = k < m ? *reinterpret_cast<const uint4*>(flag + k) : make_uint4(0, 0, 0, 0);
+    const uint64_t k = base + (j * kWave + lane) * F;
+    w[j] = make_uint4(0, 0, 0, 0);
+    if (k < m) {
+      if (F == 16)
+        w[j] = *reinterpret_cast<const uint4*>(flag + k);
+      else
+        w[j].x = *reinterpret_cast<const uint32_t*>(flag + k);
+    }
   }
   uint32_t total = 0;
 #pragma unroll
   for (uint32_t j = 0; j < L; ++j) {
-    const uint64_t k = base + (j * kWave + lane) * 16;
+    const uint64_t k = base + (j * kWave + lane) * F;
     uint32_t mask = similar_mask(w[j]);
-    if (k + 16 > m) mask &= k < m ? (1u << (uint32_t)(m - k)) - 1u : 0u;
+    if (k + F > m) mask &= k < m ? (1u << (uint32_t)(m - k)) - 1u : 0u;
     if (!__ballot(mask != 0)) continue;
     const uint32_t incl = wave_incl_scan((uint32_t)__popc(mask));
     uint32_t pos = total + incl - (uint32_t)__popc(mask);
-    for (uint32_t b = mask; b; b &= b - 1) at[pos++] = (uint16_t)((j * kWave + lane) * 16 + (uint32_t)__ffs(b) - 1);
+    for (uint32_t b = mask; b; b &= b - 1) at[pos++] = (uint16_t)((j * kWave + lane) * F + (uint32_t)__ffs(b) - 1);
     total += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
   }
   wave_lds_sync();
@@ -122,9 +132,10 @@ constexpr uint32_t kListed = 4;
 
 // Similar entries per row among the wave's tile at `base`: one atomic per run
 // of a row's entries in a wave's 64.
+template <uint32_t TILE = kFlagTile>
 __device__ __forceinline__ void core_count_tile(const PhaseView& v, uint64_t base, uint16_t* at) {
   const uint32_t lane = lane_id();
-  const uint32_t total = similar_tile(v.flag, v.m, base, at);
+  const uint32_t total = similar_tile<TILE>(v.flag, v.m, base, at);
   for (uint32_t i0 = 0; i0 < total; i0 += kWave * kListed) {
     uint32_t row[kListed];
 #pragma unroll
@@ -146,10 +157,10 @@ __device__ __forceinline__ void core_count_tile(const PhaseView& v, uint64_t bas
 
 // Joins the similar core-core edges of the wave's tile, each visited from its
 // larger endpoint.  HEADS: one edge per run of a row's entries only.
-template <bool HEADS>
+template <bool HEADS, uint32_t TILE = kFlagTile>
 __device__ __forceinline__ void union_tile(const PhaseView& v, uint64_t base, uint16_t* at) {
   const uint32_t lane = lane_id();
-  const uint32_t total = similar_tile(v.flag, v.m, base, at);
+  const uint32_t total = similar_tile<TILE>(v.flag, v.m, base, at);
   for (uint32_t i0 = 0; i0 < total; i0 += kWave * kListed) {
     uint32_t u[kListed];
     int32_t w[kListed];
@@ -209,9 +220,9 @@ __device__ __forceinline__ uint32_t border_entry(const PhaseView& v, uint64_t k,
 }
 
 // The same for the wave's tile at `base`.
-template <bool FIND>
+template <bool FIND, uint32_t TILE = kFlagTile>
 __device__ __forceinline__ uint32_t border_tile(const PhaseView& v, uint64_t base, uint16_t* at) {
-  const uint32_t total = similar_tile(v.flag, v.m, base, at);
+  const uint32_t total = similar_tile<TILE>(v.flag, v.m, base, at);
   uint32_t labeled = 0;
   for (uint32_t i0 = 0; i0 < total; i0 += kWave) {
     const bool on = i0 + lane_id() < total;

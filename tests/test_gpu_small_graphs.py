@@ -1,5 +1,6 @@
 """The passes after the similarity phase at the sizes where they change: one
-workgroup for tiny graphs, fewer launches below 2^20 entries, results through
+workgroup for tiny graphs, one union round below 2^19 entries, fewer launches
+below 2^22, short flag tiles below 2^24, results through
 page-locked staging up to 512 KB, and results written by the pass itself to
 device addresses of any alignment (needs an MI355X).  All results are whole
 numbers: they must equal the oracle's."""
@@ -33,13 +34,14 @@ def communities(n, edges, seed):
 
 @pytest.mark.parametrize("n,edges", [(2, 1), (65, 300), (1003, 16383), (1003, 16384), (1003, 16385),
                                      (8192, 16384), (8193, 16384),
-                                     (30000, (1 << 19) - 1), (30000, 1 << 19)])
+                                     (20000, (1 << 18) - 1), (20000, 1 << 18), (60000, (1 << 21) - 1), (60000, 1 << 21),
+                                     (200003, (1 << 23) - 1), (200003, 1 << 23)])
 def test_results_at_every_size(ctx, n, edges):
     g = communities(n, edges, seed=n + edges)
     assert g.m == 2 * edges
     dg = sgc.DeviceGraph(ctx, g)
     try:
-        for eps, mu in ((0.3, 2), (0.5, 4), (0.35, 0), (0.2, 1000)):
+        for eps, mu in ((0.3, 2), (0.5, 4), (0.35, 0), (0.2, 1000))[:4 if edges <= 1 << 19 else 1]:
             labels, core, sim, _ = ob.orc_scan(g.row_ptr, g.adj, eps, mu)
             r = sgc.scan(ctx, dg, eps, mu, want_sim=True)
             print("[case] n", n, "m", g.m, "eps", eps, "mu", mu, "cores", r.stats.cores, "borders", r.stats.borders,
