@@ -247,7 +247,7 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
   double t0 = now_ms();
   std::vector<uint64_t> blocks, row_bounds;
   uint64_t block_rows = 0, row_max = 0, row_rows = 0;
-  const uint64_t maxd = std::max<uint64_t>(1, ooc_max_degree(g));
+  const uint64_t maxd = std::max<uint64_t>(1, ooc_degrees(g, nullptr));
   // Row blocks as large as the room allows once the records of the largest
   // degree and the row offsets are counted in (a block holds at most as many
   // rows as entries), in groups of the largest size whose chips still fit
@@ -400,7 +400,7 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
     if (sg.pending) SGC_HIP(hipEventSynchronize(sg.free));
     sg.pending = false;
     const double tb = now_ms();
-    ooc_offsets(g, blocks[b0], blocks[b1], sg.off);
+    ooc_copy_rows(g, blocks[b0], blocks[b1], 0, nullptr, sg.off);
     const int32_t* const from = g->adj + g->row_ptr[blocks[b0]];
     const uint64_t piece = g->pinned ? std::max<uint64_t>(mb, 1) : kBounceBytes / 4;
     for (uint64_t k = 0; k < mb; k += piece) {

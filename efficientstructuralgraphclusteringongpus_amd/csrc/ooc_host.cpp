@@ -12,11 +12,14 @@
 
 namespace sgc {
 
-uint64_t ooc_max_degree(const sgc_host_graph* g) {
+uint64_t ooc_degrees(const sgc_host_graph* g, uint32_t* deg) {
   const uint64_t* rp = g->row_ptr;
   uint64_t most = 0;
 #pragma omp parallel for schedule(static) reduction(max : most)
-  for (uint64_t x = 0; x < g->n; ++x) most = std::max(most, rp[x + 1] - rp[x]);
+  for (uint64_t x = 0; x < g->n; ++x) {
+    most = std::max(most, rp[x + 1] - rp[x]);
+    if (deg) deg[x] = (uint32_t)(rp[x + 1] - rp[x]);
+  }
   return most;
 }
 
@@ -47,11 +50,17 @@ int ooc_plan_rows(const sgc_host_graph* g, uint64_t cap, uint64_t row_cap, std::
   return SGC_OK;
 }
 
-void ooc_offsets(const sgc_host_graph* g, uint64_t r0, uint64_t r1, uint32_t* off) {
+void ooc_copy_rows(const sgc_host_graph* g, uint64_t r0, uint64_t r1, uint32_t base, int32_t* dst, uint32_t* off) {
   const uint64_t* rp = g->row_ptr;
-  const uint64_t b = rp[r0], nr = r1 - r0;
+  const uint64_t b = rp[r0], m = rp[r1] - b;
+  const uint64_t nr = r1 - r0;
 #pragma omp parallel for schedule(static)
-  for (uint64_t i = 0; i <= nr; ++i) off[i] = (uint32_t)(rp[r0 + i] - b);
+  for (uint64_t i = 0; i <= nr; ++i) off[i] = base + (uint32_t)(rp[r0 + i] - b);
+  if (!dst) return;
+  const uint64_t piece = 1 << 20;
+#pragma omp parallel for schedule(dynamic, 1)
+  for (uint64_t p = 0; p < m; p += piece)
+    memcpy(dst + p, g->adj + b + p, (size_t)std::min(piece, m - p) * sizeof(int32_t));
 }
 
 void ooc_merge_rows(const sgc_host_graph* g, uint64_t r0, uint64_t r1, const uint8_t* chip_flag, uint8_t* flag) {

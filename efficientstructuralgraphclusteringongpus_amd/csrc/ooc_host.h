@@ -1,5 +1,5 @@
 // Host half of the out-of-core tier: row-block planning, row
-// offsets and the merge of chip flags into the whole-graph flag array
+// copies and the merge of chip flags into the whole-graph flag array
 // (g++/OpenMP; the device half is in ooc.hip).
 #pragma once
 
@@ -11,7 +11,9 @@
 
 namespace sgc {
 
-uint64_t ooc_max_degree(const sgc_host_graph* g);
+// The largest degree; the degrees as uint32 to deg unless it is null (every
+// degree is < 2^31 for a graph the OOC tier takes).
+uint64_t ooc_degrees(const sgc_host_graph* g, uint32_t* deg);
 
 // Consecutive rows cut into blocks bounds[i] .. bounds[i+1] of at most cap
 // entries and at most row_cap rows each.  *max_entries and *max_rows receive
@@ -20,8 +22,9 @@ uint64_t ooc_max_degree(const sgc_host_graph* g);
 int ooc_plan_rows(const sgc_host_graph* g, uint64_t cap, uint64_t row_cap, std::vector<uint64_t>* bounds,
                   uint64_t* max_entries, uint64_t* max_rows);
 
-// Offsets of rows [r0, r1) from the first row's entries, to off[0 .. r1-r0].
-void ooc_offsets(const sgc_host_graph* g, uint64_t r0, uint64_t r1, uint32_t* off);
+// Copies the entries of rows [r0, r1) to dst (parallel; skipped for a null
+// dst) and writes their offsets, shifted by `base`, to off[0 .. r1-r0].
+void ooc_copy_rows(const sgc_host_graph* g, uint64_t r0, uint64_t r1, uint32_t base, int32_t* dst, uint32_t* off);
 
 // Copies the final flags (N or Y) of rows [r0, r1), held in chip_flag, into
 // the whole-graph flag array; entries the chip left undecided are skipped,
