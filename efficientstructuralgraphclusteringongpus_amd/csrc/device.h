@@ -66,6 +66,7 @@ enum Counter {
   kCntHUnits = 208,   // units of the hash filter
   kCntHQueue = 224,
   kCntPieces = 240,   // pieces of labelled rows for the classify pass
+  kCntWPieces = 248,  // pieces of wave-filter owners beyond their first (the line is the other's only later)
   kStripe0 = 256,
   kStripes = 32,
   kCntWords = kStripe0 + kStripes * kStripeSlots

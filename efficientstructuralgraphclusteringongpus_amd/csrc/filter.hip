@@ -332,6 +332,20 @@ constexpr uint32_t kLargeEdges = 768;
 // bitmaps first / without: eps 0.25 63.1 / 58.0 ms, eps 0.3 46.4 / 50.6.
 constexpr double kCoarseEps = 0.27;
 
+// Pieces an owner's edges are cut into for the wave filter, beyond its first
+// (row begin and end, first edge, edges): at most one for every 32 owned
+// edges, so under an eighth of the quarter of the unit array they have.  A
+// whole owner is a chain of waits of up to 256 edges, and with few owners the
+// longest chains are the kernel: pieces are sized for kWavePieces of them, two
+// to a wave slot.  Planted communities with 0.7 / 1.4 / 3.4 million entries,
+// similarity phase: 227 / 286 / 722 us whole, 161 / 183 / 610 in pieces.
+// Graphs of kPieceEntries and more have owners enough (8.1 million: 981 and
+// 1006), and the registers the piece costs slow them (R-MAT-22 shuffled 1.65 ->
+// 1.72 ms).
+constexpr uint32_t kWavePieces = 12288;
+constexpr uint32_t kPieceEntries = 1u << 22;
+__host__ __device__ __forceinline__ uint4* wave_pieces(uint4* funits, uint32_t fcap) { return funits + fcap / 2; }
+
 // Units of the workgroup and large filters (small from the front of funits,
 // large from the back) and the wave list.  A unit's edges are capped so that
 // a small graph still gives every workgroup slot several units; below 96
@@ -343,7 +357,8 @@ __global__ void __launch_bounds__(kBlock) k_plan_filter(uint32_t n, const uint32
                                                         const uint64_t* __restrict__ work_u,
                                                         uint4* __restrict__ funits, uint32_t fcap, uint32_t ucap,
                                                         uint32_t* __restrict__ wl_b, uint32_t* __restrict__ wl_e,
-                                                        uint32_t* __restrict__ wl_k, uint64_t* __restrict__ cnt) {
+                                                        uint32_t* __restrict__ wl_k, bool pieces,
+                                                        uint64_t* __restrict__ cnt) {
   constexpr uint32_t V = 4;  // vertices per thread per block iteration
   const uint64_t owned_all = count_total(cnt, kCntUEdges);
   if (owned_all > ucap) {  // asymmetric input: reported by the host, no unit is written
@@ -352,8 +367,10 @@ __global__ void __launch_bounds__(kBlock) k_plan_filter(uint32_t n, const uint32
   }
   const uint32_t cap_s = (uint32_t)min((uint64_t)kSmallEdges, max((uint64_t)96, owned_all / 8192));
   const uint32_t cap_l = (uint32_t)min((uint64_t)kLargeEdges, max((uint64_t)64, owned_all / 2048));
-  unsigned long long* const ctr[3] = {(unsigned long long*)&cnt[kCntFUnits1], (unsigned long long*)&cnt[kCntFUnits2],
-                                      (unsigned long long*)&cnt[kCntTiny]};
+  const uint32_t cap_w =
+      pieces ? (uint32_t)min((uint64_t)kWaveEdges, max((uint64_t)32, owned_all / kWavePieces)) : kWaveEdges;
+  unsigned long long* const ctr[4] = {(unsigned long long*)&cnt[kCntFUnits1], (unsigned long long*)&cnt[kCntFUnits2],
+                                      (unsigned long long*)&cnt[kCntTiny], (unsigned long long*)&cnt[kCntWPieces]};
   const uint64_t tile = (uint64_t)kBlock * V;
   for (uint64_t base = (uint64_t)blockIdx.x * tile; base < n; base += (uint64_t)gridDim.x * tile) {  // block-uniform
     uint32_t owned[V], c1[V], c2[V], c3[V], per[V], start[V], stop[V];
@@ -362,7 +379,7 @@ __global__ void __launch_bounds__(kBlock) k_plan_filter(uint32_t n, const uint32
       const uint64_t x = base + j * kBlock + threadIdx.x;
       owned[j] = x < n ? cnt_u[x] : 0u;
     }
-    uint32_t need[3] = {0, 0, 0};
+    uint32_t need[4] = {0, 0, 0, 0};
 #pragma unroll
     for (uint32_t j = 0; j < V; ++j) {
       const uint64_t x = base + j * kBlock + threadIdx.x;
@@ -391,8 +408,9 @@ __global__ void __launch_bounds__(kBlock) k_plan_filter(uint32_t n, const uint32
       need[0] += c1[j];
       need[1] += c2[j];
       need[2] += c3[j];
+      need[3] += c3[j] ? (owned[j] - 1) / cap_w : 0u;
     }
-    block_reserve<3>(need, ctr);
+    block_reserve<4>(need, ctr);
 #pragma unroll
     for (uint32_t j = 0; j < V; ++j) {
       const uint32_t cu = c1[j] + c2[j];
@@ -406,7 +424,9 @@ __global__ void __launch_bounds__(kBlock) k_plan_filter(uint32_t n, const uint32
       if (c3[j]) {
         wl_b[need[2]] = start[j];
         wl_e[need[2]] = stop[j];
-        wl_k[need[2]] = owned[j];
+        wl_k[need[2]] = min(owned[j], cap_w);
+        for (uint32_t at = cap_w; at < owned[j]; at += cap_w)
+          wave_pieces(funits, fcap)[need[3]++] = make_uint4(start[j], stop[j], at, min(owned[j] - at, cap_w));
       }
       need[0] += c1[j];
       need[1] += c2[j];
@@ -860,9 +880,10 @@ __global__ void __launch_bounds__(1024, 8) k_hash_units(FilterArgs A, UnitIO io)
 // wave cycles and the VALU is half busy: five waves a SIMD instead of six take
 // 3.5 ms.  With the row hashed again for every owner, the owners dealt to the
 // XCDs one by one and no owner fetched ahead: 2.85.
+template <bool PIECES>
 __global__ void __launch_bounds__(kBlock, 6)
     k_bitmap_wave(FilterArgs A, const uint32_t* __restrict__ wl_b, const uint32_t* __restrict__ wl_e,
-                  const uint32_t* __restrict__ wl_k) {
+                  const uint32_t* __restrict__ wl_k, const uint4* __restrict__ pieces) {
   stamp(A.cnt, kStampSimRest);
   // 16-byte words of the largest M: 4 M(256) = 2^12 bits; slots of each hash table
   constexpr uint32_t W = kBlock / kWave, TOP = 32, SLOTS = 2 * kWaveRow, SHIFT = 23;
@@ -879,20 +900,30 @@ __global__ void __launch_bounds__(kBlock, 6)
   uint2* const e_q = s_q[wv];
   uint16_t* const e_need = s_need[wv];
   uint16_t* const list = s_list[wv];
-  const uint32_t count = (uint32_t)A.cnt[kCntTiny];
+  const uint32_t owners = (uint32_t)A.cnt[kCntTiny], count = owners + (PIECES ? (uint32_t)A.cnt[kCntWPieces] : 0u);
   const uint32_t waves = gridDim.x * W;
   uint32_t streamed = 0, rounds = 0, probed = 0;
   // blocks of one XCD (every eighth) take neighbouring owners of the list,
   // whose edges share rows: its L2 then serves more of them
   const uint32_t per = gridDim.x / kXcds, vb = gridDim.x % kXcds ? blockIdx.x : blockIdx.x % kXcds * per + blockIdx.x / kXcds;
-  uint32_t idx = vb * W + wv, n_b = 0, n_e = 0, n_k = 0;  // the next owner, fetched one ahead
-  if (idx < count) n_b = wl_b[idx], n_e = wl_e[idx], n_k = wl_k[idx];
+  uint32_t n_b = 0, n_e = 0, n_f = 0, n_k = 0;  // the next owner or piece, fetched one ahead
+  auto fetch = [&](uint32_t i) {
+    if (i < owners) {
+      n_b = wl_b[i], n_e = wl_e[i], n_k = wl_k[i], n_f = 0;
+    } else if (PIECES && i < count) {
+      const uint4 q = pieces[i - owners];
+      n_b = q.x, n_e = q.y, n_f = q.z, n_k = q.w;
+    }
+  };
+  uint32_t idx = vb * W + wv;
+  fetch(idx);
   for (; idx < count; idx += waves) {
     const uint32_t bb = __builtin_amdgcn_readfirstlane(n_b), be = __builtin_amdgcn_readfirstlane(n_e);
     const uint32_t owned = __builtin_amdgcn_readfirstlane(n_k), l = be - bb;
-    if (idx + waves < count) n_b = wl_b[idx + waves], n_e = wl_e[idx + waves], n_k = wl_k[idx + waves];
+    const uint32_t first = PIECES ? bb + __builtin_amdgcn_readfirstlane(n_f) : bb;
+    fetch(idx + waves);
     uint4 ed = make_uint4(kNone, kNone, 0, 0);  // (entry, reverse entry, row start of a, d(a))
-    if (lane < owned) ed = A.uedge[bb + lane];
+    if (lane < owned) ed = A.uedge[first + lane];
     const uint32_t top = 4 * coarse_words(l), mask = top * 128 - 1;
     if (lane < top) own4[top + lane] = l >= kMinRow ? A.bits[A.fine0 + 4 * coarse_at(bb) + lane] : make_uint4(0, 0, 0, 0);
     wave_lds_sync();
@@ -915,7 +946,7 @@ __global__ void __launch_bounds__(kBlock, 6)
       const uint32_t ne = min(owned - base, (uint32_t)kWave);
       if (base) {
         ed = make_uint4(kNone, kNone, 0, 0);
-        if (lane < ne) ed = A.uedge[bb + base + lane];
+        if (lane < ne) ed = A.uedge[first + base + lane];
       }
       uint32_t cstar = 0;
       bool survive = false;
@@ -1145,7 +1176,7 @@ void launch_plan_filter(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s
   // the lists share arrays that the core pass initialises later
   k_plan_filter<<<grid_for(g->n, kBlock), kBlock, 0, s>>>(g->n, g->row_begin, g->row_end, b.cnt_u, b.work_u, b.units,
                                                           b.ucap / 2, b.ucap, (uint32_t*)b.label, (uint32_t*)b.parent,
-                                                          (uint32_t*)b.lo, b.cnt);
+                                                          (uint32_t*)b.lo, g->m < kPieceEntries, b.cnt);
 }
 
 bool filter_leaves_units(const sgc_dgraph* g) { return g->max_degree > std::min(kWaveRow, kWaveEdges); }
@@ -1182,10 +1213,15 @@ void launch_filter(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int 
   if (has_large) k_hash_units<<<cus * 2, 1024, 0, s>>>(A, io);
   io.in = b.units, io.in_step = 1, io.in_count = kCntFUnits1, io.queue = kCntFQueue1;
   if (has_small) k_bitmap_units<false><<<cus * 8, 256, 0, s>>>(A, io);
-  const uint64_t want = ((uint64_t)g->n + kBlock / kWave - 1) / (kBlock / kWave), cap = (uint64_t)cus * 6;
-  k_bitmap_wave<<<(uint32_t)(want < cap ? want : cap), kBlock, 0, s>>>(A, (const uint32_t*)b.label,
-                                                                       (const uint32_t*)b.parent,
-                                                                       (const uint32_t*)b.lo);
+  const bool cut = g->m < kPieceEntries;
+  const uint64_t want = ((uint64_t)g->n * (cut ? 2 : 1) + kBlock / kWave - 1) / (kBlock / kWave), cap = (uint64_t)cus * 6;
+  const uint32_t grid = (uint32_t)(want < cap ? want : cap);
+  const uint32_t *const wl_b = (const uint32_t*)b.label, *const wl_e = (const uint32_t*)b.parent,
+                 *const wl_k = (const uint32_t*)b.lo;
+  if (cut)
+    k_bitmap_wave<true><<<grid, kBlock, 0, s>>>(A, wl_b, wl_e, wl_k, wave_pieces(b.units, fcap));
+  else
+    k_bitmap_wave<false><<<grid, kBlock, 0, s>>>(A, wl_b, wl_e, wl_k, nullptr);
 }
 
 }  // namespace sgc
