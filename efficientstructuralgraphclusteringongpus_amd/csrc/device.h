@@ -65,6 +65,7 @@ enum Counter {
   kCntFQueue2 = 192,
   kCntHUnits = 208,   // units of the hash filter
   kCntHQueue = 224,
+  kCntRecords = 224,  // chips, which have no hash filter: packed edge records placed
   kCntPieces = 240,   // pieces of labelled rows for the classify pass
   kCntWPieces = 248,  // pieces of wave-filter owners beyond their first (the line is the other's only later)
   kStripe0 = 256,
@@ -227,12 +228,9 @@ struct PassBuffers {
   uint32_t* ny;
   uint32_t* nn;
   // Packed edge records of out-of-core chips (launch_prep_packed): each
-  // owner's first record (n, the exclusive prefix of its owned count) and
-  // its cursor (n), and the scan's scratch.
+  // owner's first record (n) and its cursor (n).
   uint32_t* rec_start = nullptr;
   uint32_t* rec_cur = nullptr;
-  void* scan_tmp = nullptr;
-  size_t scan_tmp_bytes = 0;
   uint32_t ucap;
   uint64_t* cnt;     // kCntWords
 };
@@ -330,11 +328,9 @@ void launch_init(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s);
 // With p.prune, also counts each row's degree-decided similar and dissimilar
 // entries (ny, nn).
 void launch_prep(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStream_t s, bool count_all = false);
-// Scratch bytes of the exclusive scan over n per-owner counts (packed records).
-size_t scan_scratch_bytes(uint32_t n);
 // Packed edge records, for chips whose record array holds fewer records than
 // the chip has entries: the prep kernel writes flags and per-owner counts,
-// the counts are scanned into b.rec_start (and copied to b.rec_cur); then
+// every owner gets its place in b.rec_start (and b.rec_cur); then
 // launch_similarity_packed decides the owned edges in `rounds` rounds, round
 // r taking the owners whose records start in [r w, (r + 1) w), packed into
 // b.uedge (which must hold w plus the largest owned count); rounds past the

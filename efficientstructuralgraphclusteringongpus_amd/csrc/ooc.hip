@@ -104,7 +104,7 @@ constexpr uint64_t kRowChipBytesPerEntry = 4 + 4 + 1;
 constexpr uint64_t kMaxChipEntries = 0xFFFFFFF0ull;
 
 struct ResidentLayout {
-  size_t rb, re, sd, par, lab, lo, hi, core, cntu, work, scan, scan_bytes, bytes;
+  size_t rb, re, sd, par, lab, lo, hi, core, cntu, work, bytes;
 };
 
 ResidentLayout resident_layout(uint32_t n) {
@@ -114,8 +114,6 @@ ResidentLayout resident_layout(uint32_t n) {
   r.sd = L.take((size_t)n * 4), r.par = L.take((size_t)n * 4), r.lab = L.take((size_t)n * 4);
   r.lo = L.take((size_t)n * 4), r.hi = L.take((size_t)n * 4), r.core = L.take(n);
   r.cntu = L.take((size_t)n * 4), r.work = L.take((size_t)n * 8);
-  r.scan_bytes = std::max<size_t>(scan_scratch_bytes(n), 1);
-  r.scan = L.take(r.scan_bytes);
   r.bytes = L.bytes;
   return r;
 }
@@ -329,8 +327,6 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
   // owner in lo's and sd's memory (free until the core phase)
   pb.rec_start = (uint32_t*)pb.lo;
   pb.rec_cur = pb.sd;
-  pb.scan_tmp = base + RLay.scan;
-  pb.scan_tmp_bytes = RLay.scan_bytes;
   R.chip = base + resident;
 
   // a page-locked graph is sent as it lies: only row offsets are staged.

@@ -27,8 +27,6 @@
 
 #include <algorithm>
 
-#include <hipcub/device/device_scan.hpp>
-
 #include "device.h"
 #include "device_util.h"
 
@@ -87,7 +85,7 @@ __device__ __forceinline__ uint32_t log2_pow2(uint32_t t) { return 31 - __clz(t)
 //   kRecRow     at the owner's own row range, uedge[rb[b] + slot];
 //   kRecCount   nowhere: flags and per-owner counts only (first of two passes);
 //   kRecCompact packed by owner: owner b's records start at rec_start[b],
-//               its exclusive prefix of the counts (second pass: the flags of
+//               its first place among the packed ones (second pass: the flags of
 //               the first are read back, owned = kFlagUDown).  One round
 //               writes the owners whose rec_start lies in [r0, r0 + w), at
 //               rec_cur[b] - r0 + slot (rec_cur: b's cursor, starting at
@@ -1189,12 +1187,6 @@ void launch_window_offsets(const sgc_dgraph* g, hipStream_t s) {
   k_window_offsets<<<grid_for(total, kBlock), kBlock, 0, s>>>(g->n, g->row_ptr, g->adj, g->wcount, g->woff);
 }
 
-size_t scan_scratch_bytes(uint32_t n) {
-  size_t bytes = 0;
-  (void)hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, (const uint32_t*)nullptr, (uint32_t*)nullptr, n);
-  return bytes;
-}
-
 void launch_prep(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, hipStream_t s, bool count_all) {
   if (g->m == 0) return;
   const uint32_t grid = grid_for(g->m, kBlock);
@@ -1307,14 +1299,34 @@ RowRanges chip_rows(const sgc_dgraph* g) {
   return RowRanges{{g->pair.lo0, g->pair.lo1}, {g->pair.hi0, g->pair.hi1}, 2};
 }
 
-// A second scanned range continues the first: out[i] += the first range's
-// last start + its last count.
-__global__ void __launch_bounds__(kBlock) k_scan_carry(uint32_t* __restrict__ out, uint32_t count,
-                                                       const uint32_t* __restrict__ last_start,
-                                                       const uint32_t* __restrict__ last_count) {
-  const uint32_t add = *last_start + *last_count;
-  const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < count; i += stride) out[i] += add;
+// Each owner's first record, and its cursor there: the blocks' owners one
+// after another in the order the blocks get their place, which the rounds do
+// not care about.  (A scan by a library, its carry to the second range and a
+// copy took up to seven launches a chip and 39 us; this takes 5.)
+__global__ void __launch_bounds__(kBlock) k_rec_starts(RowRanges rr, const uint32_t* __restrict__ cnt_u,
+                                                       uint32_t* __restrict__ rec_start,
+                                                       uint32_t* __restrict__ rec_cur, uint64_t* __restrict__ cnt) {
+  constexpr uint32_t V = 8;
+  unsigned long long* const ctr[1] = {(unsigned long long*)&cnt[kCntRecords]};
+  const uint64_t n0 = rr.hi[0] - rr.lo[0], n = n0 + (rr.count > 1 ? rr.hi[1] - rr.lo[1] : 0u);
+  const uint64_t tile = (uint64_t)kBlock * V;
+  for (uint64_t base = (uint64_t)blockIdx.x * tile; base < n; base += (uint64_t)gridDim.x * tile) {  // block-uniform
+    uint32_t x[V], c[V], at[1] = {0};
+#pragma unroll
+    for (uint32_t j = 0; j < V; ++j) {
+      const uint64_t i = base + j * kBlock + threadIdx.x;
+      x[j] = i < n0 ? rr.lo[0] + (uint32_t)i : rr.lo[1] + (uint32_t)(i - n0);
+      c[j] = i < n ? cnt_u[x[j]] : 0u;
+      at[0] += c[j];
+    }
+    block_reserve<1>(at, ctr);
+#pragma unroll
+    for (uint32_t j = 0; j < V; ++j)
+      if (base + j * kBlock + threadIdx.x < n) {
+        rec_start[x[j]] = rec_cur[x[j]] = at[0];
+        at[0] += c[j];
+      }
+  }
 }
 }  // namespace
 
@@ -1323,19 +1335,10 @@ void launch_prep_packed(const sgc_dgraph* g, const PassBuffers& b, ScanParams p,
   k_prep<false, false, kRecCount><<<grid_for(g->m, kBlock), kBlock, 0, s>>>(
       g->m, g->row_begin, g->row_end, g->adj, g->src, g->ndeg, g->mirror, p.eps, false, g->pair, b.flag, b.cnt_u,
       b.work_u, b.uedge, b.cnt, nullptr, nullptr);
-  // each owner's first record: an exclusive scan of the owned counts over
-  // the chip's rows, the second range continuing where the first ends
   const RowRanges rr = chip_rows(g);
-  for (int q = 0; q < rr.count; ++q) {
-    const uint32_t x0 = rr.lo[q], count = rr.hi[q] - rr.lo[q];
-    if (!count) continue;
-    size_t tmp_bytes = b.scan_tmp_bytes;
-    (void)hipcub::DeviceScan::ExclusiveSum(b.scan_tmp, tmp_bytes, b.cnt_u + x0, b.rec_start + x0, count, s);
-    if (q == 1 && rr.hi[0] > rr.lo[0])
-      k_scan_carry<<<grid_for(count, kBlock), kBlock, 0, s>>>(b.rec_start + x0, count, b.rec_start + rr.hi[0] - 1,
-                                                              b.cnt_u + rr.hi[0] - 1);
-    (void)hipMemcpyAsync(b.rec_cur + x0, b.rec_start + x0, (size_t)count * 4, hipMemcpyDeviceToDevice, s);
-  }
+  uint64_t rows = 0;
+  for (int q = 0; q < rr.count; ++q) rows += rr.hi[q] - rr.lo[q];
+  if (rows) k_rec_starts<<<grid_for(rows, kBlock * 8), kBlock, 0, s>>>(rr, b.cnt_u, b.rec_start, b.rec_cur, b.cnt);
 }
 
 void launch_similarity_packed(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int cu_count, int impl,
