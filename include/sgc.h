@@ -320,8 +320,9 @@ typedef struct {
  * resident throughout.  Outputs as sgc_scan (host arrays,
  * each optional) and bit-identical to it.  stats->ms_similarity fields are
  * device time summed over chips; the per-phase fields are filled when all
- * rows fit one chip; ms_total is wall time.  SGC_ENOMEM if the budget is
- * below sgc_ooc_min_budget. */
+ * rows fit one chip; ms_total is wall time.  The context keeps up to 256 MB
+ * of the pass's page-locked staging for the next one.  SGC_ENOMEM if the
+ * budget is below sgc_ooc_min_budget. */
 int sgc_scan_ooc(sgc_ctx* ctx, const sgc_host_graph* g, double eps, int32_t mu, uint64_t device_budget,
                  int32_t* labels, uint8_t* core, uint8_t* sim, sgc_stats* stats, sgc_ooc_stats* ooc);
 
