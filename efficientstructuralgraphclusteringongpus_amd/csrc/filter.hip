@@ -224,7 +224,9 @@ __global__ void __launch_bounds__(kBlock) k_pack_narrow(PackArgs A) {
 
 // Wide rows, one block each: the groups by class (each class from a group of
 // its own, the groups left over all padding), the bitmaps as above.  Rows
-// beyond kMaxThresholdRow are never streamed: no bitmap.
+// beyond kMaxThresholdRow are never streamed: no bitmap.  Every entry goes in,
+// whatever its degree: input that is not symmetric has neighbours without a
+// row, and one that is left out would count as a certain miss.
 __global__ void __launch_bounds__(kBlock) k_pack_wide(PackArgs A) {
   constexpr uint32_t C = 4;
   __shared__ __align__(16) uint32_t bits[8192];  // M(46338) = 2^18 bits; 4 M(1024) = 2^14
@@ -250,7 +252,7 @@ __global__ void __launch_bounds__(kBlock) k_pack_wide(PackArgs A) {
       }
 #pragma unroll
       for (uint32_t j = 0; j < C; ++j) {
-        if (!dv[j]) continue;
+        if (t0 + j * kBlock + threadIdx.x >= d) continue;
         atomicAdd(&h[vertex_class(v[j], dv[j], tab)], 1u);
         if (coarse) {
           const uint32_t hv = vertex_hash(v[j]);
@@ -290,7 +292,7 @@ __global__ void __launch_bounds__(kBlock) k_pack_wide(PackArgs A) {
       }
 #pragma unroll
       for (uint32_t j = 0; j < C; ++j) {
-        if (!dv[j]) continue;
+        if (t0 + j * kBlock + threadIdx.x >= d) continue;
         const uint32_t c = vertex_class(v[j], dv[j], tab), pos = atomicAdd(&cur[c], 1u);
         const uint32_t q = pos / kGroup, r = pos % kGroup, e = group_element(vertex_hash(v[j]));
         uint16_t* const g = A.groups + ((uint64_t)first[c] + q) * 8;

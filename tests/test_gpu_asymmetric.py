@@ -70,3 +70,30 @@ def test_server_rejects_asymmetric_graph(ctx):
         with pytest.raises(sgc.SGCError) as ei:
             srv.add_graph(g)
         assert ei.value.code == EFORMAT
+
+
+@pytest.mark.parametrize("shared,more,eps", [(400, 200, 0.5),    # bitmaps of a narrow and a wide row
+                                             (300, 1700, 0.3),   # large owner, both filters
+                                             (450, 3000, 0.2)])  # large owner, hash groups alone
+def test_neighbours_whose_own_row_is_empty(ctx, shared, more, eps):
+    """Two linked vertices list `shared` vertices with no row of their own,
+    one of them `more` such vertices besides: the filters must know every
+    neighbour they share, whatever its degree."""
+    n = 3 + shared + more
+    rows = [[] for _ in range(n)]
+    rows[0] = [1, *range(3, 3 + shared)]
+    rows[1] = [0, *range(3, n)]
+    rp = np.cumsum([0] + [len(r) for r in rows])
+    g = sgc.HostGraph.from_csr(rp, np.array(sum(rows, []), dtype=np.int32), check_symmetry=False)
+    want = (shared + 2) ** 2 >= eps * eps * (len(rows[0]) + 1) * (len(rows[1]) + 1)
+    say("empty rows", shared, more, eps, "similar", want)
+    dg = sgc.DeviceGraph(ctx, g)
+    try:
+        r = sgc.scan(ctx, dg, eps, 2, want_sim=True)
+        dg.tuning = sgc.Tuning(hash_tables=0)  # every edge counted
+        x = sgc.scan(ctx, dg, eps, 2, want_sim=True)
+        assert r.stats.u_edges == x.stats.u_edges == 1
+        assert bool(x.sim[0]) == want and bool(r.sim[0]) == want
+        assert np.array_equal(r.sim, x.sim) and np.array_equal(r.labels, x.labels)
+    finally:
+        dg.close()
