@@ -108,6 +108,11 @@ constexpr size_t kStageBytes = 512u << 10;
 constexpr int kBounces = 4;
 constexpr size_t kBounceBytes = 8u << 20;
 
+// Most memory of a freed graph's row copies that a context keeps: releasing it
+// takes 0.25 ms, and a caller that uploads, runs and releases graphs of 3e7
+// entries one after another (6.0 ms each) had 6.4 ms with it released each time.
+constexpr size_t kSpareBytes = 512u << 20;
+
 // Grow-only device (or page-locked host) allocation owned by a context.
 struct DevBuf {
   void* ptr = nullptr;
@@ -136,6 +141,9 @@ struct sgc_ctx {
   hipEvent_t bounce_done[sgc::kBounces] = {};
   sgc::DevBuf host_work;    // page-locked work memory of out-of-core passes
   bool prune = false;       // core-check pruning in passes that return no similarity flags (sgc_ctx_set_pruning)
+  size_t work_pass = 0;  // bytes of `work` that the passes so far needed (uploads reserve them, and may sort in more)
+  sgc_dgraph* packed = nullptr;  // the graphs that have compact row copies, linked by next_packed
+  sgc::DevBuf spare;     // the row copies' memory of a graph freed earlier, for the next one (sgc::kSpareBytes)
 };
 
 namespace sgc {
@@ -193,11 +201,15 @@ struct sgc_dgraph {
   uint32_t wcount = 0;
   // Compact copies of the rows for the filter stages (filter.hip: bitmaps
   // and hash groups, 9 bytes per entry); graphs of a serving engine, and
-  // uploads without room, have none (null).
+  // uploads without room, have none (null).  An allocation of their own: the
+  // context takes them back when it finds no room for something else.
   char* packed = nullptr;
-  // the allocations that hold the arrays above: one for all of them, or,
+  size_t packed_cap = 0;  // bytes of that allocation
+  sgc_dgraph* next_packed = nullptr;
+  sgc_dgraph** link_packed = nullptr;  // the pointer that holds this graph in the context's list, or null
+  // the allocations that hold the other arrays: one for all of them, or,
   // where that much was not free in one piece, one for each that was
-  void* blocks[5] = {};
+  void* blocks[4] = {};
 };
 
 namespace sgc {
@@ -259,8 +271,15 @@ inline size_t unit_capacity(uint64_t m) { return (size_t)(m / 2) + 2; }
 // some entry has no reverse entry.  SGC_OK otherwise.
 int check_unit_overflow(const uint64_t* cnt_host, uint64_t m);
 
+// Device memory of the context's device, or null.  Where there is not enough,
+// the context gives back what it can do without, if that makes room: spare
+// memory, work memory beyond a pass's, then its graphs' compact row copies.
+// Called with nothing of the work buffer in use.
+void* device_alloc(sgc_ctx* ctx, size_t bytes);
+// Frees g's compact row copies, or (keep) leaves their memory to its context.
+void drop_packed(sgc_dgraph* g, bool keep = false);
 // The context's work buffer grown to at least `bytes`, or null when the
-// device has not that much.
+// device has not that much (the buffer then has the size it had).
 void* work_memory(sgc_ctx* ctx, size_t bytes);
 // At least `bytes` of page-locked host memory, the context's until
 // release_host_work; null when the system will not lock that much.
@@ -292,8 +311,10 @@ void launch_fill_rows(const uint32_t* rp, uint32_t n, uint32_t m, uint32_t base,
 // Fills g->ndeg and g->mirror (after g->src), whichever are there.  Entries
 // without a reverse entry get mirror word 0xFFFFFFFF.  Works in the context's
 // work buffer; without its memory the reverse entries are searched one by
-// one.  May synchronise the stream.
+// one.  May synchronise the stream.  index_work_bytes: what it takes of the
+// buffer at most.
 hipError_t build_indexes(sgc_ctx* ctx, const sgc_dgraph* g);
+size_t index_work_bytes(const sgc_dgraph* g);
 // 2^20-id windows of the large-tier bitmap covering n ids, and the kernel
 // filling g->woff (see sgc_dgraph).
 uint32_t window_count(uint32_t n);

@@ -46,19 +46,19 @@ int scratch_ptr_for(int device, void** out) {
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
-int ensure(DevBuf& b, size_t bytes) {
+int ensure(sgc_ctx* ctx, DevBuf& b, size_t bytes) {
   if (b.bytes >= bytes) return SGC_OK;
+  const size_t had = b.bytes;
   if (b.ptr) (void)hipFree(b.ptr);
-  b.ptr = nullptr;
-  b.bytes = 0;
-  hipError_t e = hipMalloc(&b.ptr, bytes);
-  if (e != hipSuccess) {
-    b.ptr = nullptr;
-    (void)hipGetLastError();
-    return fail(SGC_ENOMEM, "device allocation of %zu bytes failed: %s", bytes, hipGetErrorString(e));
+  b = DevBuf();
+  for (const size_t want : {bytes, had}) {  // what it had is enough for others
+    if (want) b.ptr = device_alloc(ctx, want);
+    if (!b.ptr) continue;
+    b.bytes = want;
+    break;
   }
-  b.bytes = bytes;
-  return SGC_OK;
+  if (b.bytes >= bytes) return SGC_OK;
+  return fail(SGC_ENOMEM, "device allocation of %zu bytes failed: out of memory", bytes);
 }
 
 // Byte offsets of one pass's arrays for graph g inside a work buffer; `bytes`
@@ -114,8 +114,9 @@ void bind_pass(char* base, const PassLayout& L, const sgc_dgraph* g, uint64_t* c
 // hipMalloc when too small).
 int carve(sgc_ctx* ctx, const sgc_dgraph* g, PassBuffers* pb) {
   const PassLayout L = pass_layout(g);
-  int rc = ensure(ctx->work, L.bytes);
+  int rc = ensure(ctx, ctx->work, L.bytes);
   if (rc) return rc;
+  ctx->work_pass = std::max(ctx->work_pass, L.bytes);
   bind_pass((char*)ctx->work.ptr, L, g, (uint64_t*)ctx->counters.ptr, pb);
   return SGC_OK;
 }
@@ -148,7 +149,7 @@ extern "C" int sgc_ctx_create(int device, sgc_ctx** out) {
   strncpy(ctx->name, prop.name[0] ? prop.name : prop.gcnArchName, sizeof(ctx->name) - 1);
   ctx->cu_count = prop.multiProcessorCount;
   SGC_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
-  int rc = ensure(ctx->counters, kCntWords * sizeof(uint64_t));
+  int rc = ensure(ctx, ctx->counters, kCntWords * sizeof(uint64_t));
   if (rc) {
     delete ctx;
     return rc;
@@ -170,7 +171,13 @@ extern "C" void sgc_ctx_destroy(sgc_ctx* ctx) {
   (void)hipStreamSynchronize(ctx->stream);
   for (auto& e : ctx->ev)
     if (e) (void)hipEventDestroy(e);
-  if (ctx->work.ptr) (void)hipFree(ctx->work.ptr);
+  while (sgc_dgraph* g = ctx->packed) {  // graphs not freed yet
+    ctx->packed = g->next_packed;
+    g->next_packed = nullptr;
+    g->link_packed = nullptr;
+  }
+  for (DevBuf* b : {&ctx->work, &ctx->spare})
+    if (b->ptr) (void)hipFree(b->ptr);
   if (ctx->counters.ptr) (void)hipFree(ctx->counters.ptr);
   if (ctx->host_counters) (void)hipHostFree(ctx->host_counters);
   if (ctx->bounce) (void)hipHostFree(ctx->bounce);
@@ -321,8 +328,63 @@ hipError_t sgc::download(sgc_ctx* ctx, const HostCopy* copies, int count) {
   return e != hipSuccess ? e : w;
 }
 
+void* sgc::device_alloc(sgc_ctx* ctx, size_t bytes) {
+  void* p = nullptr;
+  auto get = [&]() {
+    if (hipMalloc(&p, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+    p = nullptr;
+    return false;
+  };
+  if (get()) return p;
+  size_t room = 0, total = 0;
+  if (hipMemGetInfo(&room, &total) != hipSuccess) return nullptr;
+  const size_t excess = ctx->work.bytes > ctx->work_pass ? ctx->work.bytes - ctx->work_pass : 0;
+  room += ctx->spare.bytes + excess;
+  for (const sgc_dgraph* g = ctx->packed; g; g = g->next_packed) room += g->packed_cap;
+  if (room < bytes) return nullptr;
+  if (ctx->spare.ptr) {
+    (void)hipFree(ctx->spare.ptr);
+    ctx->spare = DevBuf();
+    if (get()) return p;
+  }
+  if (excess) {
+    (void)hipFree(ctx->work.ptr);
+    ctx->work = DevBuf();
+    if (ctx->work_pass && hipMalloc(&ctx->work.ptr, ctx->work_pass) == hipSuccess)
+      ctx->work.bytes = ctx->work_pass;
+    else
+      ctx->work.ptr = nullptr;
+    if (get()) return p;
+  }
+  while (ctx->packed) {
+    drop_packed(ctx->packed);
+    if (get()) return p;
+  }
+  return nullptr;
+}
+
+void sgc::drop_packed(sgc_dgraph* g, bool keep) {
+  if (g->link_packed) {  // its context is there
+    *g->link_packed = g->next_packed;
+    if (g->next_packed) g->next_packed->link_packed = g->link_packed;
+    DevBuf& spare = g->ctx->spare;
+    if (keep && g->packed_cap <= kSpareBytes && g->packed_cap > spare.bytes) {
+      std::swap(spare.bytes, g->packed_cap);
+      void* const p = spare.ptr;
+      spare.ptr = g->packed;
+      g->packed = (char*)p;
+    }
+  }
+  g->link_packed = nullptr;
+  g->next_packed = nullptr;
+  if (g->packed) (void)hipFree(g->packed);
+  g->packed = nullptr;
+  g->packed_cap = 0;
+}
+
 void* sgc::work_memory(sgc_ctx* ctx, size_t bytes) {
-  if (ensure(ctx->work, bytes) == SGC_OK) return ctx->work.ptr;
+  if (ensure(ctx, ctx->work, bytes) == SGC_OK) return ctx->work.ptr;
   clear_error();
   return nullptr;
 }
@@ -372,6 +434,7 @@ int sgc::upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgr
   narrow_row_ptr(g, rp32.data(), &maxd);
   d->max_degree = (uint32_t)maxd;
   auto cleanup = [d]() {
+    drop_packed(d);
     for (void* p : d->blocks)
       if (p) (void)hipFree(p);
     delete d;
@@ -382,29 +445,25 @@ int sgc::upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgr
   // gathers them), the window-offset index (the kernels find window
   // boundaries while streaming; it grows with n^2: R-MAT-26 at edge factor 16
   // needs 17 GB, twice its adjacency, and a pass there runs 2.5 times faster
-  // with it) and the filter stages' compact rows (every edge goes to the
-  // exact kernels).  One allocation for all: seven of them cost an upload of
+  // with it).  One allocation for all: seven of them cost an upload of
   // R-MAT-20 and its release 1.9 ms, one 0.6.
   const size_t rp_bytes = align_up((g->n + 1) * 4, 256), m_bytes = align_up(std::max<size_t>(g->m, 1) * 4, 256);
-  const size_t need[5] = {rp_bytes + 2 * m_bytes, g->m ? m_bytes : 0, g->m ? m_bytes : 0,
-                          align_up(window_index_bytes(d->n, g->m), 256), scans && g->m ? packed_bytes(g->m) : 0};
-  char* at[5] = {};
-  if (hipMalloc(&d->blocks[0], need[0] + need[1] + need[2] + need[3] + need[4]) == hipSuccess) {
+  const size_t need[4] = {rp_bytes + 2 * m_bytes, g->m ? m_bytes : 0, g->m ? m_bytes : 0,
+                          align_up(window_index_bytes(d->n, g->m), 256)};
+  char* at[4] = {};
+  d->blocks[0] = device_alloc(ctx, need[0] + need[1] + need[2] + need[3]);
+  if (d->blocks[0]) {
     char* p = (char*)d->blocks[0];
-    for (int i = 0; i < 5; p += need[i++]) at[i] = need[i] ? p : nullptr;
+    for (int i = 0; i < 4; p += need[i++]) at[i] = need[i] ? p : nullptr;
   } else {
-    (void)hipGetLastError();
-    for (int i = 0; i < 5; ++i) {
-      d->blocks[i] = nullptr;
-      if (need[i] && hipMalloc(&d->blocks[i], need[i]) != hipSuccess) {
-        (void)hipGetLastError();
-        d->blocks[i] = nullptr;
-        if (i) continue;
-        cleanup();
-        return fail(SGC_ENOMEM, "device allocation for graph (n=%llu, m=%llu) failed", (unsigned long long)g->n,
-                    (unsigned long long)g->m);
-      }
+    for (int i = 0; i < 4; ++i) {
+      if (need[i]) d->blocks[i] = device_alloc(ctx, need[i]);
       at[i] = (char*)d->blocks[i];
+    }
+    if (!at[0]) {
+      cleanup();
+      return fail(SGC_ENOMEM, "device allocation for graph (n=%llu, m=%llu) failed", (unsigned long long)g->n,
+                  (unsigned long long)g->m);
     }
   }
   d->row_ptr = (uint32_t*)at[0];
@@ -416,9 +475,9 @@ int sgc::upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgr
   d->ndeg = (uint32_t*)at[2];
   d->woff = (uint32_t*)at[3];
   if (d->woff) d->wcount = window_count(d->n);
-  d->packed = at[4];
-  // the indexes are built in the buffer a pass works in, sized for that at once
-  (void)work_memory(ctx, pass_layout(d).bytes);
+  // the indexes are built in the buffer a pass works in, sized for both at once
+  const size_t pass = pass_layout(d).bytes;
+  if (!work_memory(ctx, std::max(pass, index_work_bytes(d)))) (void)work_memory(ctx, pass);
   hipError_t e = upload_bytes(ctx, d->row_ptr, rp32.data(), (g->n + 1) * 4, false);
   if (e == hipSuccess && g->m) e = upload_bytes(ctx, d->adj, g->adj, g->m * 4, g->pinned);
   if (e == hipSuccess) {
@@ -428,7 +487,28 @@ int sgc::upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgr
   if (e == hipSuccess) {
     launch_window_offsets(d, ctx->stream);
     e = hipGetLastError();
-    if (e == hipSuccess) e = build_packed_rows(ctx, d);
+  }
+  // The filter stages' compact rows (without them every edge goes to the exact
+  // kernels), from what is left when a pass has its memory.
+  if (e == hipSuccess && scans && d->mirror && d->ndeg && ctx->work.bytes >= pass) {
+    const size_t bytes = packed_bytes(g->m);
+    if (ctx->spare.bytes >= bytes && ctx->spare.bytes / 2 <= bytes) {
+      d->packed = (char*)ctx->spare.ptr;
+      d->packed_cap = ctx->spare.bytes;
+      ctx->spare = DevBuf();
+    } else if (hipMalloc((void**)&d->packed, bytes) == hipSuccess) {
+      d->packed_cap = bytes;
+    } else {
+      (void)hipGetLastError();
+      d->packed = nullptr;
+    }
+    if (d->packed) e = build_packed_rows(ctx, d);
+  }
+  if (d->packed) {
+    d->next_packed = ctx->packed;
+    if (d->next_packed) d->next_packed->link_packed = &d->next_packed;
+    d->link_packed = &ctx->packed;
+    ctx->packed = d;
   }
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) {
@@ -443,6 +523,7 @@ extern "C" void sgc_dgraph_free(sgc_dgraph* d) {
   if (!d) return;
   (void)hipSetDevice(d->ctx->device);
   (void)hipStreamSynchronize(d->ctx->stream);
+  drop_packed(d, true);
   for (void* p : d->blocks)
     if (p) (void)hipFree(p);
   delete d;
@@ -785,9 +866,8 @@ extern "C" int sgc_copy_bench(sgc_ctx* ctx, uint64_t bytes, double* ms) {
   clear_error();
   if (!ctx || bytes < 16) return fail(SGC_EINVAL, "bad argument");
   SGC_HIP(hipSetDevice(ctx->device));
-  void *a = nullptr, *b = nullptr;
-  if (hipMalloc(&a, bytes) != hipSuccess || hipMalloc(&b, bytes) != hipSuccess) {
-    (void)hipGetLastError();
+  void *const a = device_alloc(ctx, bytes), *const b = a ? device_alloc(ctx, bytes) : nullptr;
+  if (!b) {
     if (a) (void)hipFree(a);
     return fail(SGC_ENOMEM, "device allocation of 2 x %llu bytes failed", (unsigned long long)bytes);
   }

@@ -1145,13 +1145,12 @@ PackLayout pack_layout(uint64_t m) {
 size_t packed_bytes(uint64_t m) { return pack_layout(m).bytes; }
 
 hipError_t build_packed_rows(sgc_ctx* ctx, sgc_dgraph* g) {
-  if (!g->packed) return hipSuccess;
   hipStream_t s = ctx->stream;
   const uint32_t n = g->n, m = g->m;
   const PackLayout L = pack_layout(m);
-  char* const mem = g->mirror && g->ndeg ? (char*)work_memory(ctx, L.tmp_bytes) : nullptr;
+  char* const mem = (char*)work_memory(ctx, L.tmp_bytes);
   if (!mem) {  // every edge goes to the exact kernels
-    g->packed = nullptr;
+    drop_packed(g);
     return hipSuccess;
   }
   char* const out = g->packed;

@@ -1004,6 +1004,37 @@ static void launch_mirror(const sgc_dgraph* g, hipStream_t s) {
 // bucket's rows no longer fit LDS, or its items come one by one.
 constexpr uint32_t kSearchEntries = 1u << 21;
 
+// Work memory of the sort: keys out, values in and out, its scratch and the
+// mismatch count.
+struct SortLayout {
+  size_t vin, vout, tmp, bad, bytes, tmp_bytes;
+  int key_bits;
+};
+
+static SortLayout sort_layout(const sgc_dgraph* g, hipStream_t s) {
+  SortLayout L{};
+  const size_t m = g->m;
+  L.key_bits = 1;
+  while (L.key_bits < 32 && (1ull << L.key_bits) < (uint64_t)g->n) ++L.key_bits;
+  (void)hipcub::DeviceRadixSort::SortPairs(nullptr, L.tmp_bytes, (const uint32_t*)nullptr, (uint32_t*)nullptr,
+                                           (const uint64_t*)nullptr, (uint64_t*)nullptr, g->m, 0, L.key_bits, s);
+  L.vin = (m * 4 + 255) / 256 * 256;
+  L.vout = L.vin + m * 8;
+  L.tmp = L.vout + m * 8;
+  L.bad = L.tmp + (L.tmp_bytes + 255) / 256 * 256;
+  L.bytes = L.bad + 256;
+  return L;
+}
+
+static size_t split_bytes(uint32_t m) {
+  return (size_t)((m + (1u << kBucketBits) - 1) >> kBucketBits) * (kBucketCap * sizeof(SplitItem) + 4);
+}
+
+size_t index_work_bytes(const sgc_dgraph* g) {
+  if (!g->mirror || g->m <= kSearchEntries) return 0;
+  return g->m <= kSplitEntries && g->ndeg ? split_bytes(g->m) : sort_layout(g, g->ctx->stream).bytes;
+}
+
 static hipError_t build_mirror(sgc_ctx* ctx, const sgc_dgraph* g);
 
 hipError_t build_indexes(sgc_ctx* ctx, const sgc_dgraph* g) {
@@ -1011,7 +1042,7 @@ hipError_t build_indexes(sgc_ctx* ctx, const sgc_dgraph* g) {
   const uint32_t m = g->m;
   if (m > kSearchEntries && m <= kSplitEntries && g->mirror && g->ndeg) {
     const uint32_t buckets = (m + (1u << kBucketBits) - 1) >> kBucketBits;
-    char* const mem = (char*)work_memory(ctx, (size_t)buckets * (kBucketCap * sizeof(SplitItem) + 4));
+    char* const mem = (char*)work_memory(ctx, split_bytes(m));
     if (mem) {
       uint32_t* const cursor = (uint32_t*)(mem + (size_t)buckets * kBucketCap * sizeof(SplitItem));
       hipError_t e = hipMemsetAsync(cursor, 0, (size_t)buckets * 4, s);
@@ -1035,26 +1066,19 @@ static hipError_t build_mirror(sgc_ctx* ctx, const sgc_dgraph* g) {
     launch_mirror(g, s);
     return hipGetLastError();
   }
-  int bits = 1;
-  while (bits < 32 && (1ull << bits) < (uint64_t)g->n) ++bits;
-  size_t tmp_bytes = 0;
-  (void)hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, (const uint32_t*)nullptr, (uint32_t*)nullptr,
-                                           (const uint64_t*)nullptr, (uint64_t*)nullptr, m, 0, bits, s);
-  // keys out, values in and out, the sort's scratch and the mismatch count
-  const size_t o_keys = 0, o_vin = ((size_t)m * 4 + 255) / 256 * 256, o_vout = o_vin + (size_t)m * 8,
-               o_tmp = o_vout + (size_t)m * 8, o_bad = o_tmp + (tmp_bytes + 255) / 256 * 256;
-  char* const mem = (char*)work_memory(ctx, o_bad + 256);
+  SortLayout L = sort_layout(g, s);
+  char* const mem = (char*)work_memory(ctx, L.bytes);
   if (!mem) {
     launch_mirror(g, s);  // not enough room to sort: search each reverse entry
     return hipGetLastError();
   }
-  uint32_t* keys = (uint32_t*)(mem + o_keys);
-  uint64_t* vin = (uint64_t*)(mem + o_vin);
-  uint64_t* vout = (uint64_t*)(mem + o_vout);
-  unsigned long long* bad = (unsigned long long*)(mem + o_bad);
+  uint32_t* keys = (uint32_t*)mem;
+  uint64_t* vin = (uint64_t*)(mem + L.vin);
+  uint64_t* vout = (uint64_t*)(mem + L.vout);
+  unsigned long long* bad = (unsigned long long*)(mem + L.bad);
   k_rows_and_positions<<<grid_for(m, kBlock), kBlock, 0, s>>>(m, g->src, vin);
-  hipError_t e = hipcub::DeviceRadixSort::SortPairs(mem + o_tmp, tmp_bytes, (const uint32_t*)g->adj, keys, vin, vout,
-                                                     m, 0, bits, s);
+  hipError_t e = hipcub::DeviceRadixSort::SortPairs(mem + L.tmp, L.tmp_bytes, (const uint32_t*)g->adj, keys, vin,
+                                                     vout, m, 0, L.key_bits, s);
   if (e == hipSuccess) e = hipMemsetAsync(bad, 0, 8, s);
   if (e == hipSuccess) {
     k_mirror_from_sorted<<<grid_for(m, kBlock), kBlock, 0, s>>>(m, g->src, g->adj, keys, vout, g->mirror, bad);

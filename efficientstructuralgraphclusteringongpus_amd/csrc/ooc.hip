@@ -301,10 +301,9 @@ int run_ooc(OocRun& R, double eps, int32_t mu, uint64_t budget, int32_t* labels,
                 (unsigned long long)budget, (unsigned long long)(resident + chip_need + 8192));
 
   // ---- device and pinned host memory
-  if (hipMalloc(&R.dev, resident + chip_need) != hipSuccess) {
-    (void)hipGetLastError();
+  R.dev = device_alloc(ctx, resident + chip_need);
+  if (!R.dev)
     return fail(SGC_ENOMEM, "device allocation of %llu bytes failed", (unsigned long long)(resident + chip_need));
-  }
   char* base = (char*)R.dev;
   R.rb = (uint32_t*)(base + RLay.rb);
   R.re = (uint32_t*)(base + RLay.re);

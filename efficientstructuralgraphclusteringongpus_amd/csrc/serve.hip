@@ -485,12 +485,8 @@ int ensure_lanes(sgc_server* S) {
   for (BatchLane& L : S->lanes) {
     if (!L.stream) SGC_HIP(hipStreamCreateWithFlags(&L.stream, hipStreamNonBlocking));
     if (!L.h_table) SGC_HIP(hipHostMalloc((void**)&L.h_table, sizeof(BatchTable), hipHostMallocDefault));
-    if (!L.d_table) {
-      if (hipMalloc((void**)&L.d_table, sizeof(BatchTable)) != hipSuccess) {
-        (void)hipGetLastError();
-        return fail(SGC_ENOMEM, "batch table allocation failed");
-      }
-    }
+    if (!L.d_table) L.d_table = (BatchTable*)device_alloc(S->ctx, sizeof(BatchTable));
+    if (!L.d_table) return fail(SGC_ENOMEM, "batch table allocation failed");
     if (!L.start) SGC_HIP(hipEventCreate(&L.start));
     if (!L.done) SGC_HIP(hipEventCreate(&L.done));
     memset(L.h_table, 0, sizeof(BatchTable));
@@ -802,8 +798,8 @@ extern "C" int sgc_server_add_graph(sgc_server* S, const sgc_host_graph* hg, uin
   // one device and one page-locked allocation for all slots
   const size_t cn_bytes = align256(std::max<size_t>(m, 1) * 4), label_bytes = align256(std::max<size_t>(n, 1) * 4),
                host_bytes = label_bytes + align256(kCntWords * 8) + align256(sizeof(QueryParams));
-  if (hipMalloc((void**)&G->cn, cn_bytes + S->slots_per_graph * (slot_bytes(n, m) + kCntWords * 8)) != hipSuccess) {
-    (void)hipGetLastError();
+  G->cn = (uint32_t*)device_alloc(ctx, cn_bytes + S->slots_per_graph * (slot_bytes(n, m) + kCntWords * 8));
+  if (!G->cn) {
     free_graph(G);
     return fail(SGC_ENOMEM, "device allocation for graph of %u vertices failed", n);
   }

@@ -173,14 +173,19 @@ typedef struct sgc_dgraph sgc_dgraph;
 
 /* Copies a host CSR into HBM (uint32 offsets; requires m < 2^32, else
  * SGC_ERANGE - use sgc_scan_ooc for larger graphs) and builds the device
- * indexes (entry rows, reverse entries, neighbour degrees, window offsets, and
- * the compact row copies of the similarity filters), about 25 bytes of device
- * memory per entry in one allocation; what finds no room is left out.  A graph
- * not in page-locked memory (sgc_graph_pin) is staged through the context's
- * 32 MB of page-locked buffers, allocated at the first such copy and kept
- * until sgc_ctx_destroy.  The indexes are built in the context's work memory,
- * which is grown to what a pass over the graph needs; without that room the
- * reverse entries are searched one by one.  Synchronises the context stream. */
+ * indexes (entry rows, reverse entries, neighbour degrees, window offsets),
+ * about 16 bytes of device memory per entry in one allocation; what finds no
+ * room is left out.  A graph not in page-locked memory (sgc_graph_pin) is staged
+ * through the context's 32 MB of page-locked buffers, allocated at the first
+ * such copy and kept until sgc_ctx_destroy.  The indexes are built in the
+ * context's work memory, which is grown to what a pass over the graph needs;
+ * without that room the reverse entries are searched one by one.  From what is
+ * left then, 9 bytes per entry go to the compact row copies of the similarity
+ * filters.  Where a later allocation of the context finds no room, it gives back
+ * work memory that no pass has used and the row copies of its graphs; passes
+ * over these then count every edge.  Row copies of up to 512 MB stay with the
+ * context when their graph is freed, for the next upload, or until
+ * sgc_ctx_destroy.  Synchronises the context stream. */
 int sgc_dgraph_upload(sgc_ctx* ctx, const sgc_host_graph* g, sgc_dgraph** out);
 void sgc_dgraph_free(sgc_dgraph* dg);
 
