@@ -333,6 +333,14 @@ constexpr uint32_t kLargeEdges = 768;
 // the large owners' edges go to the hash filter at once.  R-MAT-24, with the
 // bitmaps first / without: eps 0.25 63.1 / 58.0 ms, eps 0.3 46.4 / 50.6.
 constexpr double kCoarseEps = 0.27;
+// Below this one most edges are similar and the exact kernels see that after
+// a few elements, where the hash filter reads the whole row to no end: there
+// the large owners' edges pass the bitmap kernel (which rejects next to
+// nothing) and are counted.  Similarity phase, with the hash filter / without:
+// R-MAT-22 eps 0.01 31.4 / 19.8 ms, 0.02 39.7 / 29.2, 0.03 48.4 / 40.6,
+// 0.05 49.0 / 54.5; R-MAT-24 eps 0.01 223 / 145, 0.02 323 / 271, 0.03 336 / 359,
+// 0.05 246 / 351.
+constexpr double kHashEps = 0.025;
 
 // Pieces an owner's edges are cut into for the wave filter, beyond its first
 // (row begin and end, first edge, edges): at most one for every 32 owned
@@ -1202,16 +1210,17 @@ void launch_filter(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int 
   uint4* const hash_units = b.units + fcap / 4;
   const bool coarse = p.eps >= kCoarseEps;
   io.in = b.units + fcap - 1, io.in_step = -1, io.in_count = kCntFUnits2, io.queue = kCntFQueue2;
-  io.next = coarse ? hash_units : nullptr;
+  const bool hashes = p.eps >= kHashEps;
+  io.next = hashes ? hash_units : nullptr;
   // kernels whose owners the graph cannot have are not launched (an owner
   // with more than kWaveEdges edges has a longer row than that)
   const bool has_large = g->max_degree > kSmallRow, has_small = g->max_degree > std::min(kWaveRow, kWaveEdges);
-  if (coarse && has_large) {
+  if ((coarse || !hashes) && has_large) {
     k_bitmap_units<true><<<cus * 2, 1024, 0, s>>>(A, io);
     io.in = hash_units, io.in_step = 1, io.in_count = kCntHUnits, io.queue = kCntHQueue;
   }
   io.next = nullptr;
-  if (has_large) k_hash_units<<<cus * 2, 1024, 0, s>>>(A, io);
+  if (hashes && has_large) k_hash_units<<<cus * 2, 1024, 0, s>>>(A, io);
   io.in = b.units, io.in_step = 1, io.in_count = kCntFUnits1, io.queue = kCntFQueue1;
   if (has_small) k_bitmap_units<false><<<cus * 8, 256, 0, s>>>(A, io);
   const bool cut = g->m < kPieceEntries;

@@ -66,6 +66,28 @@ def test_filter_matches_exact_kernels_and_oracle(ctx, sizes, fans):
         dg.close()
 
 
+@pytest.mark.parametrize("eps", [0.01, 0.02])
+def test_similar_edges_of_long_rows_are_not_read_in_full(ctx, eps):
+    """At low eps an edge between two rows of 4000 entries is similar after
+    about 90 common neighbours: no filter reads the row first.  Short rows are
+    read once at most."""
+    g = edge_graph((4000, 4990), (), seed=8)
+    deg = np.diff(g.row_ptr).astype(np.int64)
+    src = np.repeat(np.arange(g.n), deg)
+    lo, hi = np.minimum(deg[src], deg[g.adj]), np.maximum(deg[src], deg[g.adj])
+    left = (src < g.adj) & (lo + 1 >= (hi + 1) * eps * eps) & (eps * eps * (lo + 1) * (hi + 1) > 4)
+    long, short = int(lo[left & (lo > 1024)].sum()), int(lo[left & (lo <= 1024)].sum())
+    dg = sgc.DeviceGraph(ctx, g)
+    try:
+        r = sgc.scan(ctx, dg, eps, 3, want_sim=True)
+        labels, _, sim, _ = ob.orc_scan(g.row_ptr, g.adj, eps, 3)
+        say("eps", eps, "long rows", long, "short rows", short, "loaded", r.stats.loaded_elements)
+        assert np.array_equal(r.sim, sim) and np.array_equal(r.labels, labels)
+        assert r.stats.loaded_elements < short + long / 2
+    finally:
+        dg.close()
+
+
 @pytest.mark.parametrize("n,deg", [(40, 39), (3000, 900)])
 def test_filter_on_one_degree_class(ctx, n, deg):
     """Regular rows: every vertex has (nearly) the same degree, so the classes
