@@ -317,7 +317,7 @@ size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Device bytes of one query slot for a graph of n vertices, m entries.
 size_t slot_bytes(uint64_t n, uint64_t m) {
-  return align256(std::max<uint64_t>(m, 1)) + 5 * align256(n * 4 + 4) + align256(n + 1) + align256(kCntSlots * 8) +
+  return align256(std::max<uint64_t>(m, 1)) + 5 * align256(n * 4 + 4) + align256(n + 1) + align256(kCntWords * 8) +
          align256(sizeof(QueryParams));
 }
 
@@ -343,7 +343,7 @@ struct Slot {
 struct Graph {
   uint32_t id = 0;
   sgc_dgraph* dg = nullptr;
-  uint32_t* cn = nullptr;  // start of the graph's device memory: then the slots, then kCntWords per slot
+  uint32_t* cn = nullptr;  // start of the graph's device memory: then the slots
   float* ratio = nullptr;  // in the reverse-entry index's memory, which only the counting pass reads
   char* host_mem = nullptr;  // page-locked: the slots' labels, counters and parameters
   size_t bytes = 0;
@@ -798,7 +798,7 @@ extern "C" int sgc_server_add_graph(sgc_server* S, const sgc_host_graph* hg, uin
   // one device and one page-locked allocation for all slots
   const size_t cn_bytes = align256(std::max<size_t>(m, 1) * 4), label_bytes = align256(std::max<size_t>(n, 1) * 4),
                host_bytes = label_bytes + align256(kCntWords * 8) + align256(sizeof(QueryParams));
-  G->cn = (uint32_t*)device_alloc(ctx, cn_bytes + S->slots_per_graph * (slot_bytes(n, m) + kCntWords * 8));
+  G->cn = (uint32_t*)device_alloc(ctx, cn_bytes + S->slots_per_graph * slot_bytes(n, m));
   if (!G->cn) {
     free_graph(G);
     return fail(SGC_ENOMEM, "device allocation for graph of %u vertices failed", n);
@@ -849,7 +849,6 @@ extern "C" int sgc_server_add_graph(sgc_server* S, const sgc_host_graph* hg, uin
   }
   G->slots.resize(S->slots_per_graph);
   char* const base = (char*)G->cn + cn_bytes;
-  uint64_t* const cnt_mem = (uint64_t*)(base + S->slots_per_graph * slot_bytes(n, m));
   for (uint32_t i = 0; i < S->slots_per_graph; ++i) {
     Slot& sl = G->slots[i];
     char* p = base + i * slot_bytes(n, m);
@@ -867,8 +866,8 @@ extern "C" int sgc_server_add_graph(sgc_server* S, const sgc_host_graph* hg, uin
     p += align256((size_t)n * 4 + 4);
     sl.pb.core = (uint8_t*)p;
     p += align256((size_t)n + 1);
-    sl.pb.cnt = cnt_mem + (size_t)i * kCntWords;
-    p += align256(kCntSlots * 8);
+    sl.pb.cnt = (uint64_t*)p;
+    p += align256(kCntWords * 8);
     sl.d_params = (QueryParams*)p;
     sl.stream = S->next_stream;
     S->next_stream = (S->next_stream + 1) % kStreams;
