@@ -253,6 +253,7 @@ struct ScanParams {
   // core-check pruning (GPUSCAN++/GPUScan.cu:303): the workgroup tier defers
   // an edge whose endpoints are both decided (core or not) when it starts
   bool prune = false;
+  bool count_all = false;  // no filter stage (sgc_dgraph_autotune)
 };
 
 // Per-vertex state of the pruned core check, kept in PassBuffers::core until

@@ -11,6 +11,7 @@
 #include "GPUScan.h"
 #include "device.h"
 #include "graph_host.h"
+#include "tuning_sweep.h"
 
 using namespace sgc;
 
@@ -709,11 +710,11 @@ int run_pass(sgc_ctx* ctx, sgc_dgraph* g, double eps, int32_t mu, PassBuffers* p
 namespace {
 
 // Similarity-phase time of one pass (prep, plan and both tiers are run; the
-// similarity kernels alone are timed).
-int time_similarity(sgc_ctx* ctx, sgc_dgraph* g, double eps, PassBuffers* pb, double* ms) {
+// similarity kernels alone are timed), with its filter stages or without.
+int time_similarity(sgc_ctx* ctx, sgc_dgraph* g, double eps, bool filters, PassBuffers* pb, double* ms) {
   int rc = carve(ctx, g, pb);
   if (rc) return rc;
-  const ScanParams p{eps, 2};
+  const ScanParams p{eps, 2, false, !filters};
   hipStream_t s = ctx->stream;
   launch_init(g, *pb, s);
   launch_prep(g, *pb, p, s);
@@ -738,64 +739,19 @@ extern "C" int sgc_dgraph_autotune(sgc_ctx* ctx, sgc_dgraph* g, double eps, sgc_
   SGC_HIP(hipSetDevice(ctx->device));
   PassBuffers pb;
   uint32_t trials = 0;
-  auto measure = [&](const SimTuning& t, double* ms) -> int {
+  auto measure = [&](const SimTuning& t, bool filters, double* ms) -> int {
     g->tuning = t;
     double a = 0, b = 0;
-    int rc = time_similarity(ctx, g, eps, &pb, &a);
-    if (!rc) rc = time_similarity(ctx, g, eps, &pb, &b);
+    int rc = time_similarity(ctx, g, eps, filters, &pb, &a);
+    if (!rc) rc = time_similarity(ctx, g, eps, filters, &pb, &b);
     trials += 2;
     *ms = std::min(a, b);
     return rc;
   };
-  const SimTuning defaults;
-  double ms_default = 0;
-  int rc = measure(defaults, &ms_default);
-  if (rc) return rc;
-  SimTuning cur = defaults;
-  double cur_ms = ms_default;
-  const double large_work[] = {2097152.0, 8388608.0, 33554432.0};
-  const uint32_t small_deg[] = {128, 256, 512, 1024};
-  const double small_work[] = {65536.0, 262144.0, 1048576.0};
-  for (double v : large_work) {
-    SimTuning t = cur;
-    t.large_unit_work = v;
-    double ms;
-    if (v == cur.large_unit_work) continue;
-    if ((rc = measure(t, &ms))) return rc;
-    if (ms < cur_ms) cur = t, cur_ms = ms;
-  }
-  for (uint32_t v : small_deg) {
-    SimTuning t = cur;
-    t.small_max_degree = v;
-    double ms;
-    if (v == cur.small_max_degree) continue;
-    if ((rc = measure(t, &ms))) return rc;
-    if (ms < cur_ms) cur = t, cur_ms = ms;
-  }
-  for (double v : small_work) {
-    SimTuning t = cur;
-    t.small_unit_work = v;
-    double ms;
-    if (v == cur.small_unit_work) continue;
-    if ((rc = measure(t, &ms))) return rc;
-    if (ms < cur_ms) cur = t, cur_ms = ms;
-  }
-  {
-    SimTuning t = cur;
-    t.hash_tables = 1 - cur.hash_tables;
-    double ms;
-    if ((rc = measure(t, &ms))) return rc;
-    if (ms < cur_ms) cur = t, cur_ms = ms;
-  }
-  const uint32_t tiny_work[] = {0, 1024, 2048, 4096};
-  for (uint32_t v : tiny_work) {
-    SimTuning t = cur;
-    t.tiny_work = v;
-    double ms;
-    if (v == cur.tiny_work) continue;
-    if ((rc = measure(t, &ms))) return rc;
-    if (ms < cur_ms) cur = t, cur_ms = ms;
-  }
+  SimTuning cur;
+  g->tuning = cur;
+  double cur_ms = 0, ms_default = 0;
+  if (int rc = sweep_tuning(filter_stage(g, ScanParams{eps, 2}), measure, &cur, &cur_ms, &ms_default)) return rc;
   g->tuning = cur;
   if (best) {
     memset(best, 0, sizeof(*best));

@@ -1178,7 +1178,7 @@ hipError_t build_packed_rows(sgc_ctx* ctx, sgc_dgraph* g) {
 }
 
 bool filter_stage(const sgc_dgraph* g, ScanParams p) {
-  return g->packed && g->mirror && !p.prune && g->tuning.hash_tables != 0;
+  return g->packed && g->mirror && !p.prune && !p.count_all && g->tuning.hash_tables != 0;
 }
 
 void launch_plan_filter(const sgc_dgraph* g, const PassBuffers& b, hipStream_t s) {

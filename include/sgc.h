@@ -214,7 +214,9 @@ int sgc_dgraph_set_tuning(sgc_dgraph* dg, const sgc_tuning* t);
 /* Times the similarity phase of dg at eps under candidate knobs (coordinate
  * descent over large_unit_work, small_max_degree, small_unit_work,
  * hash_tables, tiny_work; best of two passes each), keeps the fastest on dg
- * and reports it. */
+ * and reports it.  Where the filter stages run, the knobs they do not read are
+ * timed in passes that count every edge; ms_similarity and ms_default are
+ * times of passes as sgc_scan runs them. */
 int sgc_dgraph_autotune(sgc_ctx* ctx, sgc_dgraph* dg, double eps, sgc_tuning* best);
 uint64_t sgc_dgraph_n(const sgc_dgraph* dg);
 uint64_t sgc_dgraph_m(const sgc_dgraph* dg);
