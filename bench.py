@@ -13,12 +13,13 @@ value = E * passes / (wall time of the K steps) in GTEPS (1e9
 similarity-edges/s), passes = 12 K.
 roofline: the similarity of the large owners (degree > 1024), most of a pass:
 the bitmap filter, the hash filter and the exact kernel for what they leave.
-Their DRAM bytes per pass come from the committed rocprofv3 counter summary of
+Their bytes past L2 per pass come from the committed rocprofv3 counter summary of
 this workload (profiles/large_owner_similarity_rmat24_counters.md: FETCH_SIZE
 and WRITE_SIZE of each of the 12 configurations, scaled by the same counters
 of a plain copy), summed over the passes actually timed and divided by their
 durations on the device clock: achieved GB/s, and frac against the 8 TB/s
-peak.  The algorithmic-byte model (sum over the owners' undecided edges of
+HBM peak (an upper bound on the share of DRAM bandwidth: the last-level cache
+serves some of that traffic).  The algorithmic-byte model (sum over the owners' undecided edges of
 4 * (s + min(l, s * ceil(log2(l + 1))))) is reported beside it under
 alg_model; the filters' compact rows, early exits and LDS-resident owner rows
 move far fewer bytes than that model, so its ratio to the peak passes 1.
@@ -410,7 +411,7 @@ def ooc_bench(sgc, ctx, args):
 
 
 def measured_traffic(args):
-    """DRAM bytes per pass of the large owners' similarity kernels for each
+    """Bytes past L2 per pass of the large owners' similarity kernels for each
     (eps, mu) of the default workload, from the committed rocprofv3 counter
     summary (FETCH_SIZE and WRITE_SIZE, each scaled by the plain-copy
     calibration); None for other workloads or without the summary."""
@@ -589,8 +590,9 @@ def main() -> int:
             "traffic_source": traffic["source"] if traffic else None,
             "avg_launch_ms": round(launch_ms, 4),
             "launches": passes,
-            "note": ("achieved = DRAM bytes of the timed passes' kernels (rocprofv3 FETCH_SIZE and WRITE_SIZE per "
-                     "configuration, scaled by a plain copy's counters) / their summed durations"),
+            "note": ("achieved = bytes past L2 of the timed passes' kernels (rocprofv3 FETCH_SIZE and WRITE_SIZE per "
+                     "configuration, scaled by a plain copy's counters) / their summed durations; the last-level "
+                     "cache serves part of them, so frac is an upper bound on the share of DRAM bandwidth"),
             "alg_model": {
                 "bytes_per_launch": large_bytes / passes,
                 "achieved": round(alg_achieved, 2),

@@ -298,7 +298,7 @@ __device__ __forceinline__ uint32_t team_sum(uint32_t v) {
 // (about two buckets per power of two, largest first): the teams of a wave
 // then take edges of about the same length, end their rounds and fetch their
 // next edges together, and the longest do not start last.  hist: 32 zeroed
-// words; called by every thread, with two barriers.  *todo: edges with size
+// words; called by every thread, with one barrier.  *todo: edges with size
 // > 0 (size < 2^16).
 __device__ __forceinline__ uint32_t order_by_size(uint32_t size, uint32_t* hist, uint32_t* todo) {
   const uint32_t lg = size ? 31 - __clz(size) : 0u;

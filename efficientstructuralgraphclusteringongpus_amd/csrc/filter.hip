@@ -33,7 +33,7 @@
 // Similarity phase on R-MAT-24 (2.6e8 edges), exact kernels alone -> with the
 // filters: eps 0.2 150 -> 67 ms, 0.3 119 -> 46, 0.4 80 -> 24, 0.6 32 -> 11,
 // 0.8 22 -> 8.  (Hash groups alone: 67, 51, 35, 17, 11.)  The build takes
-// about 8 ms of the upload.
+// 3.8 ms of the upload.  Lower eps: kHashEps.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1199,9 +1199,10 @@ void launch_filter(const sgc_dgraph* g, const PassBuffers& b, ScanParams p, int 
                      (const uint4*)(mem + L.coarse), (uint32_t)((L.fine - L.coarse) / 16),
                      b.uedge,  b.flag,
                      b.cnt};
-  // Units of owners above kWaveRow entries: fewer than m / 50 of each kind
-  // (an owner has its row's entries, a unit 64 edges unless it is an owner's
-  // last), so each of the four lists has room in an eighth of the array.
+  // Units of owners above kWaveRow entries: a unit has at least 32 edges unless
+  // it is its owner's last, m / 2 edges are owned and an owner has more than 256
+  // entries, so there are at most m / 64 + m / 257 of each kind and each of the
+  // four lists has room in an eighth of the array (m / 16).
   const uint32_t fcap = b.ucap / 2;
   UnitIO io;
   io.small_exact = b.units + fcap;
