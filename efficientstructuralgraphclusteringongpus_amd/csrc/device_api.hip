@@ -47,6 +47,27 @@ int scratch_ptr_for(int device, void** out) {
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
+// Guards what contexts know of their graphs' row copies (sgc_ctx::packed and
+// spare, sgc_dgraph::packed and its links): a graph may be freed on any thread,
+// while its context works on another, or after its context.
+std::mutex g_packed_mu;
+
+// Takes g out of its context's list, if it is in one.
+void unlink_packed(sgc_dgraph* g) {
+  if (!g->link_packed) return;
+  *g->link_packed = g->next_packed;
+  if (g->next_packed) g->next_packed->link_packed = g->link_packed;
+  g->link_packed = nullptr;
+  g->next_packed = nullptr;
+}
+
+void free_packed(sgc_dgraph* g) {
+  unlink_packed(g);
+  if (g->packed) (void)hipFree(g->packed);
+  g->packed = nullptr;
+  g->packed_cap = 0;
+}
+
 int ensure(sgc_ctx* ctx, DevBuf& b, size_t bytes) {
   if (b.bytes >= bytes) return SGC_OK;
   const size_t had = b.bytes;
@@ -172,10 +193,9 @@ extern "C" void sgc_ctx_destroy(sgc_ctx* ctx) {
   (void)hipStreamSynchronize(ctx->stream);
   for (auto& e : ctx->ev)
     if (e) (void)hipEventDestroy(e);
-  while (sgc_dgraph* g = ctx->packed) {  // graphs not freed yet
-    ctx->packed = g->next_packed;
-    g->next_packed = nullptr;
-    g->link_packed = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(g_packed_mu);
+    while (ctx->packed) unlink_packed(ctx->packed);  // graphs not freed yet
   }
   for (DevBuf* b : {&ctx->work, &ctx->spare})
     if (b->ptr) (void)hipFree(b->ptr);
@@ -338,6 +358,7 @@ void* sgc::device_alloc(sgc_ctx* ctx, size_t bytes) {
     return false;
   };
   if (get()) return p;
+  std::lock_guard<std::mutex> lock(g_packed_mu);
   size_t room = 0, total = 0;
   if (hipMemGetInfo(&room, &total) != hipSuccess) return nullptr;
   const size_t excess = ctx->work.bytes > ctx->work_pass ? ctx->work.bytes - ctx->work_pass : 0;
@@ -359,29 +380,22 @@ void* sgc::device_alloc(sgc_ctx* ctx, size_t bytes) {
     if (get()) return p;
   }
   while (ctx->packed) {
-    drop_packed(ctx->packed);
+    free_packed(ctx->packed);
     if (get()) return p;
   }
   return nullptr;
 }
 
 void sgc::drop_packed(sgc_dgraph* g, bool keep) {
-  if (g->link_packed) {  // its context is there
-    *g->link_packed = g->next_packed;
-    if (g->next_packed) g->next_packed->link_packed = g->link_packed;
-    DevBuf& spare = g->ctx->spare;
-    if (keep && g->packed_cap <= kSpareBytes && g->packed_cap > spare.bytes) {
-      std::swap(spare.bytes, g->packed_cap);
-      void* const p = spare.ptr;
-      spare.ptr = g->packed;
-      g->packed = (char*)p;
-    }
+  std::lock_guard<std::mutex> lock(g_packed_mu);
+  // in a list: its context is there
+  if (keep && g->link_packed && g->packed_cap <= kSpareBytes && g->packed_cap > g->ctx->spare.bytes) {
+    void* const p = g->ctx->spare.ptr;
+    g->ctx->spare.ptr = g->packed;
+    g->packed = (char*)p;
+    std::swap(g->ctx->spare.bytes, g->packed_cap);
   }
-  g->link_packed = nullptr;
-  g->next_packed = nullptr;
-  if (g->packed) (void)hipFree(g->packed);
-  g->packed = nullptr;
-  g->packed_cap = 0;
+  free_packed(g);
 }
 
 void* sgc::work_memory(sgc_ctx* ctx, size_t bytes) {
@@ -493,19 +507,23 @@ int sgc::upload_graph(sgc_ctx* ctx, const sgc_host_graph* g, bool scans, sgc_dgr
   // kernels), from what is left when a pass has its memory.
   if (e == hipSuccess && scans && d->mirror && d->ndeg && ctx->work.bytes >= pass) {
     const size_t bytes = packed_bytes(g->m);
-    if (ctx->spare.bytes >= bytes && ctx->spare.bytes / 2 <= bytes) {
-      d->packed = (char*)ctx->spare.ptr;
-      d->packed_cap = ctx->spare.bytes;
-      ctx->spare = DevBuf();
-    } else if (hipMalloc((void**)&d->packed, bytes) == hipSuccess) {
-      d->packed_cap = bytes;
-    } else {
+    {
+      std::lock_guard<std::mutex> lock(g_packed_mu);
+      if (ctx->spare.bytes >= bytes && ctx->spare.bytes / 2 <= bytes) {
+        d->packed = (char*)ctx->spare.ptr;
+        d->packed_cap = ctx->spare.bytes;
+        ctx->spare = DevBuf();
+      }
+    }
+    if (!d->packed && hipMalloc((void**)&d->packed, bytes) == hipSuccess) d->packed_cap = bytes;
+    if (!d->packed_cap) {
       (void)hipGetLastError();
       d->packed = nullptr;
     }
     if (d->packed) e = build_packed_rows(ctx, d);
   }
   if (d->packed) {
+    std::lock_guard<std::mutex> lock(g_packed_mu);
     d->next_packed = ctx->packed;
     if (d->next_packed) d->next_packed->link_packed = &d->next_packed;
     d->link_packed = &ctx->packed;

@@ -3,6 +3,8 @@ need: with the device filled up to a chosen rest, what runs without the
 copies still runs, with the same results (needs an MI355X)."""
 from __future__ import annotations
 
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -96,3 +98,22 @@ def test_graphs_closed_in_any_order():
             graphs[i].close()
             for k in left:
                 assert np.array_equal(sgc.scan(c, graphs[k], 0.5, 2).labels, labels)
+
+
+def test_graphs_freed_on_another_thread():
+    """While the context's own thread uploads, scans and frees."""
+    g = sgc.HostGraph.rmat(12, 8, seed=3)
+    with sgc.Context(0) as c:
+        own = sgc.DeviceGraph(c, g)
+        labels = sgc.scan(c, own, 0.5, 2).labels
+        for _ in range(4):
+            others = [sgc.DeviceGraph(c, g) for _ in range(8)]
+            freeing = threading.Thread(target=lambda: [dg.close() for dg in others])
+            freeing.start()
+            for _ in range(4):
+                dg = sgc.DeviceGraph(c, g)
+                assert np.array_equal(sgc.scan(c, dg, 0.5, 2).labels, labels)
+                dg.close()
+            freeing.join()
+            assert np.array_equal(sgc.scan(c, own, 0.5, 2).labels, labels)
+        own.close()
